@@ -169,3 +169,28 @@ def test_forward_large_tiles(pkg, dn_ref, dev):
     print("256x256 head vs emulated", err, flush=True)
     assert err < 3e-2
     d.destroy()
+
+
+@pytest.mark.parametrize("H,W", [(8, 8), (24, 40), (40, 104), (64, 32)])
+def test_weight_gradients_do_not_depend_on_the_split(pkg, dn_ref, dev, H, W):
+    """The mean loss over eight copies of one image has the gradients of the
+    image alone (every activation and stored gradient is the same but for an
+    exact factor 1/8), summed over eight times the tiles in another split. Only
+    FP32 summation order differs: below 1e-4 per layer (a tile lost or counted
+    twice is of order 1/tiles: 1e-2 or more at these sizes)."""
+    import torch
+    offs, _ = dn_ref.offsets()
+    grads = []
+    bits, xv, _ = _inputs(11, 1, H, W)
+    for B in (1, 8):
+        d = pkg.Denoiser(8 * 40 * 104, seed=1)
+        d.set_params(dn_ref.init_like_gpu_shapes(seed=2))
+        X = torch.from_numpy(np.repeat(bits, B, 0).view(np.int16)).to(dev)
+        T = torch.full((B, H, W, 3), -5.0, device=dev)
+        d.train_step(B, H, W, X, T, 0.0, want_loss=False)
+        grads.append(d.params(1).astype(np.float64))
+        d.destroy()
+    for i, (wo, bo) in enumerate(offs):
+        cout = dn_ref.LAYERS[i][1]
+        assert _rel(grads[1][wo:bo], grads[0][wo:bo]) < 1e-4, i
+        assert _rel(grads[1][bo:bo + cout], grads[0][bo:bo + cout]) < 1e-4, i

@@ -20,9 +20,10 @@
 //     one's output kept in LDS (recomputed on the halo).
 //   * k_conv: the generic implicit GEMM, kept for the 1x1 head in training
 //     and its input gradient.
-//   * k_wgrad: weight gradients, M = output channels, N = input channels,
-//     K = pixels; 32-pixel tiles staged through LDS transposed, split over
-//     pixel ranges into partials reduced in a fixed order (deterministic).
+//   * k_wgrad: weight and bias gradients, M = output channels, N = input
+//     channels, K = pixels; tiles with their halo staged once for all taps and
+//     read with transposing LDS reads, split over pixel ranges into partials
+//     reduced in a fixed order (deterministic).
 //   * upsampling (training), pooling / upsampling backward, ReLU-mask, loss,
 //     Adam and weight layout kernels.
 #include <hip/hip_runtime.h>
@@ -682,97 +683,219 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
 }
 
 // --------------------------------------------------------------- wgrad ----
+// Weight and bias gradients of one layer: dW[co][t][ci] = sum over pixels p
+// of G[p][co] X[p + t][ci], db[co] = sum of G[p][co]; a GEMM with M = output
+// channels, N = input channels (per tap) and K = pixels on MFMA 16x16x32.
+//
+// Both operands need 8 consecutive K (pixels) of one channel per lane while
+// the tensors are NHWC. The tiles stay in LDS as they lie in memory
+// ([pixel][channel]) and are read with the transposing LDS read
+// (ds_read_b64_tr_b16: 16 lanes read a 4 pixel x 16 channel block and each
+// gets one channel's 4 pixels), so a horizontal tap is only an address offset
+// of one pixel and one input halo serves all nine taps. A workgroup walks
+// 8-row x 32-pixel tiles of its pixel range; a wave reads every input row
+// fragment once per horizontal tap and uses it for the (up to three) output
+// rows of the vertical taps. Channel tiles: 64 x 64 per workgroup (each wave
+// 32 x 32, 36 accumulators) or, for narrow layers, 32 channels on one or both
+// sides with the four waves splitting the tile's rows and summing through LDS
+// at the end. The bias rides along as one MFMA per row against ones.
+// Partials per pixel range are reduced in a fixed order (deterministic).
+// What bounds it: LDS reads (about 0.5-0.8 of the MFMA cycles) and the
+// staging latency of each tile. Before: nine passes over both tensors (one
+// per tap) with 2-byte transposing LDS stores, and a bias pass of its own
+// with too few workgroups.
 struct WgradArgs {
     const uint16_t* g; int ldg; int cout;    // output gradient (ReLU mask applied)
     const uint16_t* x; int ldx; int cin;     // layer input
-    float* part;                             // [splits][cout][taps*cin]
-    int B, H, W, splits, chunk;              // pixels per split (multiple of 32)
+    float* part;                             // [splits][cout * taps * cin weights, cout biases]
+    int B, H, W;
+    int tilesX, tilesY, tiles, splits;       // 8 x 32 pixel tiles; split s takes tiles [s, s + 1) * tiles / splits
 };
 
-constexpr int kLdsRow = 40;   // 32 pixels + 8 padding (bf16 elements)
+constexpr int kWgRows = 8, kWgPx = 32;
 
-// grid: (ceil(cout/64), ceil(cin/64), taps*splits). Tile 64 (co) x 64 (ci);
-// wave w: co [32*(w>>1), +32) x ci [32*(w&1), +32).
-template <int TAPS>
-__global__ __launch_bounds__(kBlock) void k_wgrad(WgradArgs a) {
-    __shared__ __attribute__((aligned(16))) uint16_t Gt[64 * kLdsRow];
-    __shared__ __attribute__((aligned(16))) uint16_t Xt[64 * kLdsRow];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int co0 = blockIdx.x * 64, ci0 = blockIdx.y * 64;
-    const int t = blockIdx.z % TAPS, split = blockIdx.z / TAPS;
-    const int dy = TAPS == 9 ? t / 3 - 1 : 0, dx = TAPS == 9 ? t % 3 - 1 : 0;
-    const int P = a.B * a.H * a.W;
-    const int pBeg = split * a.chunk, pEnd = min(P, pBeg + a.chunk);
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+
+template <int TAPS, int MT, int NT, int WC, int WI>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_wgrad(WgradArgs a) {
+    constexpr int WK = 4 / (WC * WI);              // waves splitting the rows
+    constexpr int RW = kWgRows / WK;               // output rows per wave and tile
+    constexpr int HALO = TAPS == 9 ? 1 : 0, NR = TAPS == 9 ? 3 : 1;
+    constexpr int GC = 16 * MT * WC, XC = 16 * NT * WI;          // channels staged per pixel
+    constexpr int XW = kWgPx + 2 * HALO, XH = kWgRows + 2 * HALO;
+    constexpr int GP = kWgRows * kWgPx * GC / 8, XP = XH * XW * XC / 8;   // 16-byte pieces
+    constexpr int ACC = TAPS * MT * NT * 256;      // accumulators of one wave (floats)
+    constexpr int RED = WK > 1 ? (ACC + MT * 256) * 4 : 0;
+    constexpr int STAGE = (GP + XP) * 16;
+    __shared__ __attribute__((aligned(16))) unsigned char smem[STAGE > RED ? STAGE : RED];
+    uint4* const sg = (uint4*)smem;
+    uint4* const sx = sg + GP;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int row = lane & 15, kg = lane >> 4;
-    const int wco = 32 * (wave >> 1), wci = 32 * (wave & 1);
-    // loader: thread -> (pixel lp = tid/8, channel chunk 8*(tid%8))
-    const int lp = threadIdx.x >> 3, lc = 8 * (threadIdx.x & 7);
-    f32x4 acc[2][2];
-    for (int r = 0; r < 2; r++)
-        for (int j = 0; j < 2; j++) acc[r][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int p0 = pBeg; p0 < pEnd; p0 += 32) {
-        const int p = p0 + lp;
-        uint4 gv = make_uint4(0, 0, 0, 0), xv = make_uint4(0, 0, 0, 0);
-        if (p < pEnd) {
-            if (co0 + lc < a.cout) gv = *(const uint4*)(a.g + (size_t)p * a.ldg + co0 + lc);
-            const int xx = p % a.W, q = p / a.W, yy = q % a.H, bb = q / a.H;
-            const int sy = yy + dy, sx = xx + dx;
-            if (sy >= 0 && sy < a.H && sx >= 0 && sx < a.W && ci0 + lc < a.cin)
-                xv = *(const uint4*)(a.x + ((size_t)(bb * a.H + sy) * a.W + sx) * a.ldx + ci0 + lc);
+    const int wc = wave % WC, wi = (wave / WC) % WI, wk = wave / (WC * WI);
+    const int co0 = blockIdx.x * GC, ci0 = blockIdx.y * XC;
+    const bool bias = blockIdx.y == 0 && wi == 0;  // wave-uniform
+    // 16-byte piece c of pixel px of a row lies at piece swz(px, c) of the row:
+    // with 128-byte pixels the 32-byte channel pairs are rotated by px / 2, so
+    // that the four pixels of a transposing read touch different banks. The
+    // row enters only as a constant offset, so that a lane keeps a handful of
+    // addresses for all rows.
+    auto swz = [](int px, int c, int pieces) { return px * pieces + (pieces == 8 ? c ^ (px & 6) : c); };
+    // fragment of 8 pixels (from pixel px0 + 8 kg of a row) x 16 channels (tile c) as K x M / K x N operand
+    auto frag = [&](const uint4* rowBase, int px0, int c, int pieces) {
+        s16x4 h[2];
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const int q = px0 + 8 * kg + (row >> 2) + 4 * k;
+            const uint2* src = (const uint2*)(rowBase + swz(q, 2 * c + ((row >> 1) & 1), pieces)) + (row & 1);
+            h[k] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)src);
         }
-        const uint16_t* ge = (const uint16_t*)&gv;
-        const uint16_t* xe = (const uint16_t*)&xv;
-        for (int e = 0; e < 8; e++) {
-            Gt[(lc + e) * kLdsRow + lp] = ge[e];
-            Xt[(lc + e) * kLdsRow + lp] = xe[e];
+        struct { s16x4 a, b; } f{h[0], h[1]};
+        return __builtin_bit_cast(bf16x8, f);
+    };
+    f32x4 acc[TAPS][MT][NT], accb[MT];
+#pragma unroll
+    for (int t = 0; t < TAPS; t++)
+#pragma unroll
+        for (int r = 0; r < MT; r++)
+#pragma unroll
+            for (int j = 0; j < NT; j++) acc[t][r][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < MT; r++) accb[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const uint32_t one2 = 0x3f803f80u;             // two BF16 ones
+    const bf16x8 ones = __builtin_bit_cast(bf16x8, make_uint4(one2, one2, one2, one2));
+
+    const int t0 = (int)((long long)a.tiles * blockIdx.z / a.splits);
+    const int t1 = (int)((long long)a.tiles * (blockIdx.z + 1) / a.splits);
+    for (int tile = t0; tile < t1; tile++) {
+        const int tx = tile % a.tilesX, q = tile / a.tilesX, ty = q % a.tilesY, bb = q / a.tilesY;
+        const int x0 = tx * kWgPx, y0 = ty * kWgRows;
+        __syncthreads();                           // the previous tile's reads are done
+#pragma unroll 4
+        for (int e = tid; e < GP; e += kBlock) {
+            const int c = e % (GC / 8), p = e / (GC / 8);
+            const int y = y0 + p / kWgPx, x = x0 + p % kWgPx;
+            uint4 v = make_uint4(0, 0, 0, 0);
+            if (y < a.H && x < a.W) v = *(const uint4*)(a.g + ((size_t)(bb * a.H + y) * a.W + x) * a.ldg + co0 + 8 * c);
+            sg[p / kWgPx * (kWgPx * GC / 8) + swz(p % kWgPx, c, GC / 8)] = v;
+        }
+#pragma unroll 4
+        for (int e = tid; e < XP; e += kBlock) {
+            const int c = e % (XC / 8), p = e / (XC / 8);
+            const int y = y0 - HALO + p / XW, x = x0 - HALO + p % XW;
+            uint4 v = make_uint4(0, 0, 0, 0);
+            if (y >= 0 && y < a.H && x >= 0 && x < a.W)
+                v = *(const uint4*)(a.x + ((size_t)(bb * a.H + y) * a.W + x) * a.ldx + ci0 + 8 * c);
+            sx[p / XW * (XW * XC / 8) + swz(p % XW, c, XC / 8)] = v;
         }
         __syncthreads();
-        bf16x8 av[2], bv[2];
-        for (int r = 0; r < 2; r++)
-            av[r] = __builtin_bit_cast(bf16x8, *(const uint4*)&Gt[(wco + r * 16 + row) * kLdsRow + 8 * kg]);
-        for (int j = 0; j < 2; j++)
-            bv[j] = __builtin_bit_cast(bf16x8, *(const uint4*)&Xt[(wci + j * 16 + row) * kLdsRow + 8 * kg]);
-        for (int r = 0; r < 2; r++)
-            for (int j = 0; j < 2; j++)
-                acc[r][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[r], bv[j], acc[r][j], 0, 0, 0);
-        __syncthreads();
+        bf16x8 ga[RW][MT];
+#pragma unroll
+        for (int xr = 0; xr < RW + 2 * HALO; xr++) {
+            if (xr < RW) {
+#pragma unroll
+                for (int r = 0; r < MT; r++) {
+                    ga[xr][r] = frag(sg + (wk * RW + xr) * (kWgPx * GC / 8), 0, wc * MT + r, GC / 8);
+                    if (bias) accb[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga[xr][r], ones, accb[r], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int dx = 0; dx < NR; dx++) {
+                bf16x8 xb[NT];
+#pragma unroll
+                for (int j = 0; j < NT; j++) xb[j] = frag(sx + (wk * RW + xr) * (XW * XC / 8), dx, wi * NT + j, XC / 8);
+#pragma unroll
+                for (int dy = 0; dy < NR; dy++) {
+                    const int ro = xr - dy;        // output row whose tap dy reads this input row
+                    if (ro < 0 || ro >= RW) continue;
+#pragma unroll
+                    for (int r = 0; r < MT; r++)
+#pragma unroll
+                        for (int j = 0; j < NT; j++)
+                            acc[dy * NR + dx][r][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                ga[ro][r], xb[j], acc[dy * NR + dx][r][j], 0, 0, 0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);     // rows in order: fragments of later rows would spill
+        }
     }
-    const int K = TAPS * a.cin;
-    float* out = a.part + (size_t)split * a.cout * K;
-    for (int r = 0; r < 2; r++)
-        for (int j = 0; j < 2; j++) {
-            const int ci = ci0 + wci + j * 16 + row;
-            if (ci >= a.cin) continue;
-            for (int i = 0; i < 4; i++) {
-                const int co = co0 + wco + r * 16 + 4 * kg + i;
-                if (co < a.cout) out[(size_t)co * K + t * a.cin + ci] = acc[r][j][i];
+    // the row-splitting waves' sums, in wave order
+    if constexpr (WK > 1) {
+        float* red = (float*)smem;
+        constexpr int SUB = WC * WI;               // waves of one row group
+        static_assert(SUB * RED <= 160 * 1024, "LDS");
+        for (int k = 1; k < WK; k++) {
+            __syncthreads();
+            for (int sub = 0; sub < SUB; sub++) {
+                // one (wc, wi) pair at a time through the buffer
+                __syncthreads();
+                if (wk == k && wave % SUB == sub) {
+#pragma unroll
+                    for (int t = 0; t < TAPS; t++)
+#pragma unroll
+                        for (int r = 0; r < MT; r++)
+#pragma unroll
+                            for (int j = 0; j < NT; j++)
+                                *(f32x4*)(red + (((t * MT + r) * NT + j) * 64 + lane) * 4) = acc[t][r][j];
+#pragma unroll
+                    for (int r = 0; r < MT; r++) *(f32x4*)(red + ACC + (r * 64 + lane) * 4) = accb[r];
+                }
+                __syncthreads();
+                if (wk == 0 && wave % SUB == sub) {
+#pragma unroll
+                    for (int t = 0; t < TAPS; t++)
+#pragma unroll
+                        for (int r = 0; r < MT; r++)
+#pragma unroll
+                            for (int j = 0; j < NT; j++)
+                                acc[t][r][j] += *(const f32x4*)(red + (((t * MT + r) * NT + j) * 64 + lane) * 4);
+#pragma unroll
+                    for (int r = 0; r < MT; r++) accb[r] += *(const f32x4*)(red + ACC + (r * 64 + lane) * 4);
+                }
             }
         }
-}
-
-// grad[k] = sum over splits of part[s][k], in split order
-__global__ __launch_bounds__(kBlock) void k_reduce_splits(const float* part, int splits, size_t n, float* grad) {
-    for (size_t k = blockIdx.x * (size_t)kBlock + threadIdx.x; k < n; k += (size_t)gridDim.x * kBlock) {
-        float s = 0.0f;
-        for (int i = 0; i < splits; i++) s += part[(size_t)i * n + k];
-        grad[k] = s;
+        if (wk != 0) return;
     }
+    const int K = TAPS * a.cin;
+    float* out = a.part + (size_t)blockIdx.z * ((size_t)a.cout * K + a.cout);
+#pragma unroll
+    for (int r = 0; r < MT; r++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int co = co0 + (wc * MT + r) * 16 + 4 * kg + i;
+            if (co >= a.cout) continue;
+#pragma unroll
+            for (int t = 0; t < TAPS; t++)
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+                    out[(size_t)co * K + t * a.cin + ci0 + (wi * NT + j) * 16 + row] = acc[t][r][j][i];
+            if (bias && row == 0) out[(size_t)a.cout * K + co] = accb[r][i];
+        }
 }
 
-// bias gradient partials: block b sums pixels [b*chunk, ...) of 64 channels
-__global__ __launch_bounds__(kBlock) void k_bias_part(const uint16_t* g, int ldg, int cout, int P, int chunk,
-                                                      float* part) {
-    __shared__ float red[kBlock];
-    const int c = blockIdx.y * 64 + (threadIdx.x & 63), sub = threadIdx.x >> 6;
-    const int pBeg = blockIdx.x * chunk, pEnd = min(P, pBeg + chunk);
-    float s = 0.0f;
-    if (c < cout)
-        for (int p = pBeg + sub; p < pEnd; p += 4) s += bf2f(g[(size_t)p * ldg + c]);
-    red[threadIdx.x] = s;
+// grad[k] = sum over splits of part[s][k], four interleaved runs of splits
+// per column added in a fixed order (deterministic). 64 columns per
+// workgroup, one wave per run: the few columns of the narrow layers then have
+// enough loads in flight.
+__global__ __launch_bounds__(kBlock) void k_reduce_splits(const float* part, int splits, size_t n, float* grad) {
+    __shared__ float red[4][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const size_t k = blockIdx.x * (size_t)64 + lane;
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
+    if (k < n) {
+        int i = w;
+        for (; i + 12 < splits; i += 16) {
+            float v[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = part[(size_t)(i + 4 * j) * n + k];
+#pragma unroll
+            for (int j = 0; j < 4; j++) s[j] += v[j];
+        }
+        for (; i < splits; i += 4) s[0] += part[(size_t)i * n + k];
+    }
+    red[w][lane] = (s[0] + s[1]) + (s[2] + s[3]);
     __syncthreads();
-    if (sub == 0 && c < cout)
-        part[(size_t)blockIdx.x * cout + c] = ((red[threadIdx.x] + red[threadIdx.x + 64]) + red[threadIdx.x + 128]) +
-                                              red[threadIdx.x + 192];
+    if (w == 0 && k < n) grad[k] = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
 }
 
 // ---------------------------------------------------------- elementwise ----
@@ -1105,25 +1228,37 @@ static void conv_dx(Net& N, int li, const uint16_t* g, int ldg, uint16_t* dx, in
     else launch_conv3(a, L.d.cin, s);
 }
 
+// Weight and bias gradient of layer li into N.g (weights, then biases, as the
+// layer's parameters lie). Splits: two workgroups per CU (512), one per CU for
+// the 64 x 64 channel tiles, whose partials are large (both measured at
+// 8 x 256 x 256: 512 against 256 workgroups is 53 against 80 us for the
+// 32-channel layers; the 64 x 64 ones take 39 against 41 us but their
+// reduction half as long with 256); fewer where a split would get no tile of
+// its own or the partials would not fit. One step's weight and bias gradients
+// at that size: 8.2 ms before this kernel, 0.7 ms now.
+template <int TAPS, int MT, int NT, int WC, int WI>
+static void launch_wgrad(Net& N, WgradArgs a, size_t n, float* grad) {
+    const int gx = (a.cout + 16 * MT * WC - 1) / (16 * MT * WC), gy = a.cin / (16 * NT * WI);
+    constexpr int groups = WC * WI == 4 ? 256 : 512;
+    a.splits = std::max(1, std::min(a.tiles, groups / (gx * gy)));
+    while (a.splits > 1 && (size_t)a.splits * n > N.partFloats) a.splits--;
+    hipLaunchKernelGGL((k_wgrad<TAPS, MT, NT, WC, WI>), dim3(gx, gy, a.splits), dim3(kBlock), 0, N.stream, a);
+    hipLaunchKernelGGL(k_reduce_splits, dim3((unsigned)((n + 63) / 64)), dim3(kBlock), 0, N.stream, N.part, a.splits, n,
+                       grad);
+}
+
 static void conv_dw(Net& N, int li, const uint16_t* g, int ldg, const uint16_t* x, int ldx, int B, int H, int W) {
     const Layer& L = N.L[li];
-    const int P = B * H * W;
-    const size_t K = (size_t)L.d.taps * L.d.cin, n = (size_t)L.d.cout * K;
-    int splits = std::max(1, std::min(64, P / 2048));
-    while (splits > 1 && (size_t)splits * n > N.partFloats) splits--;
-    const int chunk = rup((P + splits - 1) / splits, 32);
-    splits = (P + chunk - 1) / chunk;
-    WgradArgs a{g, ldg, L.d.cout, x, ldx, L.d.cin, N.part, B, H, W, splits, chunk};
-    dim3 grid((L.d.cout + 63) / 64, (L.d.cin + 63) / 64, L.d.taps * splits);
-    if (L.d.taps == 9) hipLaunchKernelGGL(k_wgrad<9>, grid, dim3(kBlock), 0, N.stream, a);
-    else hipLaunchKernelGGL(k_wgrad<1>, grid, dim3(kBlock), 0, N.stream, a);
-    hipLaunchKernelGGL(k_reduce_splits, dim3(grid_for(n)), dim3(kBlock), 0, N.stream, N.part, splits, n, N.g + L.wOff);
-    // bias: partials over pixel chunks, then the same fixed-order reduction
-    const int bchunk = 4096, nb = (P + bchunk - 1) / bchunk;
-    hipLaunchKernelGGL(k_bias_part, dim3(nb, (L.d.cout + 63) / 64), dim3(kBlock), 0, N.stream, g, ldg, L.d.cout, P,
-                       bchunk, N.part);
-    hipLaunchKernelGGL(k_reduce_splits, dim3(grid_for(L.d.cout)), dim3(kBlock), 0, N.stream, N.part, nb,
-                       (size_t)L.d.cout, N.g + L.bOff);
+    const size_t n = (size_t)L.d.cout * L.d.taps * L.d.cin + L.d.cout;
+    WgradArgs a{g, ldg, L.d.cout, x, ldx, L.d.cin, N.part, B, H, W, (W + kWgPx - 1) / kWgPx,
+                (H + kWgRows - 1) / kWgRows, 0, 1};
+    a.tiles = a.tilesX * a.tilesY * B;
+    float* grad = N.g + L.wOff;
+    if (L.d.taps == 1) launch_wgrad<1, 1, 2, 1, 1>(N, a, n, grad);               // the head: 16-channel gradient rows
+    else if (L.d.cin == 16) launch_wgrad<9, 2, 1, 1, 1>(N, a, n, grad);
+    else if (L.d.cout % 64) launch_wgrad<9, 2, 2, 1, 1>(N, a, n, grad);
+    else if (L.d.cin % 64) launch_wgrad<9, 2, 2, 2, 1>(N, a, n, grad);
+    else launch_wgrad<9, 2, 2, 2, 2>(N, a, n, grad);
 }
 
 static void relu_bwd(Net& N, uint16_t* g, int ldg, const uint16_t* y, int ldy, int c, int P) {
@@ -1347,7 +1482,7 @@ CudaDenoiser_t cudaBVH_denoiserCreate(int maxPixels, uint64_t seed) {
         {&N.gA2, lv1 * 64}, {&N.gP1, lv1 * 32}, {&N.gA0, lv0 * 32}};
     size_t actBytes = 0;
     for (auto& b : bufs) actBytes += (b.elems * 2 + 255) & ~(size_t)255;
-    N.partFloats = std::max<size_t>(16u << 20, (size_t)(P / 4096 + 1) * 256);
+    N.partFloats = 16u << 20;
     const size_t fBytes = (lv0 * 3 * 2 + N.partFloats + 8192) * 4;
     if (hipMalloc(&N.act, actBytes + fBytes) != hipSuccess ||
         hipMalloc((void**)&N.w, N.nParams * 4 * 4) != hipSuccess || hipMalloc((void**)&N.wbuf, wbytes) != hipSuccess) {

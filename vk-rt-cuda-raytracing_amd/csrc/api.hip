@@ -61,35 +61,8 @@ static void host_parallel(size_t n, F&& f) {
     for (auto& x : th) x.join();
 }
 
-// Bounds of n x 9 host floats as a sequential std::min / std::max pass
-// computes them (per-chunk passes combined in order give the same values,
-// signed zeros included), centre and diagonal extent.
-static void set_bounds(CudaBVHHandle* h, const float* tri9, int n) {
-    const unsigned nt = 8;
-    std::vector<float> cmn(3 * nt, 1e30f), cmx(3 * nt, -1e30f);
-    const size_t chunk = (size_t(n) + nt - 1) / nt;
-    std::vector<std::thread> th;
-    auto work = [&](unsigned t) {
-        const size_t b = std::min<size_t>(n, t * chunk), e = std::min<size_t>(n, (t + 1) * chunk);
-        float mn[3] = {1e30f, 1e30f, 1e30f}, mx[3] = {-1e30f, -1e30f, -1e30f};   // in registers
-        for (size_t i = b; i < e; i++)
-            for (int k = 0; k < 9; k++) {
-                const float x = tri9[9 * i + k];
-                mn[k % 3] = std::min(mn[k % 3], x);
-                mx[k % 3] = std::max(mx[k % 3], x);
-            }
-        for (int a = 0; a < 3; a++) { cmn[3 * t + a] = mn[a]; cmx[3 * t + a] = mx[a]; }
-    };
-    if (n < (1 << 16)) {
-        for (unsigned t = 0; t < nt; t++) work(t);
-    } else {
-        for (unsigned t = 1; t < nt; t++) th.emplace_back(work, t);
-        work(0);
-        for (auto& x : th) x.join();
-    }
-    float bmin[3] = {1e30f, 1e30f, 1e30f}, bmax[3] = {-1e30f, -1e30f, -1e30f};
-    for (unsigned t = 0; t < nt; t++)
-        for (int a = 0; a < 3; a++) { bmin[a] = std::min(bmin[a], cmn[3 * t + a]); bmax[a] = std::max(bmax[a], cmx[3 * t + a]); }
+// Scene box, its centre and diagonal from the device build's bounds.
+static void set_bounds(CudaBVHHandle* h, const float* bmin, const float* bmax) {
     for (int a = 0; a < 3; a++) { h->bboxMin[a] = bmin[a]; h->bboxMax[a] = bmax[a]; h->bboxCenter[a] = (bmin[a] + bmax[a]) * 0.5f; }
     const float ex = bmax[0] - bmin[0], ey = bmax[1] - bmin[1], ez = bmax[2] - bmin[2];
     h->bboxExtent = sqrtf(ex * ex + ey * ey + ez * ez);
@@ -142,13 +115,13 @@ static bool ensure_exports(CudaBVHHandle* h) {
 
 // Completes a handle whose device structure (d_nodes4, d_tris, d_leafOfPrim,
 // d_ordered, d_nodes2 for a single tree, numNodes4, depth4) is set: the
-// bounds from the n x 9 host triangles (original order), the traversal
-// scratch and the default launch configurations; the host exports follow on
-// first use. Frees the handle and returns nullptr on failure.
-static CudaBVHHandle* make_handle(CudaBVHHandle* h, const float* tri9, int n) {
+// bounds, the traversal scratch and the default launch configurations; the
+// host exports follow on first use. Frees the handle and returns nullptr on
+// failure.
+static CudaBVHHandle* make_handle(CudaBVHHandle* h, const float* bmin, const float* bmax, int n) {
     h->numTris = n;
     h->numOrdered = n;
-    set_bounds(h, tri9, n);
+    set_bounds(h, bmin, bmax);
     if (rtk::alloc_scratch(h->scratch) != 0) {
         free_handle_device(h);
         delete h;
@@ -167,15 +140,15 @@ static CudaBVHHandle* make_handle(CudaBVHHandle* h, const float* tri9, int n) {
     return h;
 }
 
-// Builds a handle from n x 9 floats (original order). d_tri9 (nullable): the
-// same triangles already on the device (not freed here). With sceneOff the
+// Builds a handle from n x 9 floats (original order) on the host (tri9) or
+// already on the device (d_tri9, not freed here). With sceneOff the
 // handle is a forest of numScenes trees (roots4: each tree's BVH4 root).
 static CudaBVHHandle* build_impl(const float* tri9, int n, int maxLeaf, const int* sceneOff = nullptr,
                                  int numScenes = 1, std::vector<int>* roots4 = nullptr,
                                  const float* d_tri9 = nullptr, std::vector<rt::Node2>* forestNodes2 = nullptr,
                                  std::vector<int>* forestOrdered = nullptr) {
     rt::clear_error();
-    if (!tri9 || n <= 0) { set_error("cudaBVH_build: need tris != NULL and numTris > 0 (got %d)", n); return nullptr; }
+    if ((!tri9 && !d_tri9) || n <= 0) { set_error("cudaBVH_build: need tris != NULL and numTris > 0 (got %d)", n); return nullptr; }
     if (n > (1 << 27)) { set_error("cudaBVH_build: %d triangles exceed the leaf encoding (2^27)", n); return nullptr; }
     auto* h = new CudaBVHHandle();
     hipStream_t s = hstream(h);
@@ -223,7 +196,7 @@ static CudaBVHHandle* build_impl(const float* tri9, int n, int maxLeaf, const in
     }
     {
         const double t2 = clk();
-        CudaBVHHandle* r = make_handle(h, tri9, n);
+        CudaBVHHandle* r = make_handle(h, g.bmin, g.bmax, n);
         const double t3 = clk();
         if (r) {
             r->buildStats[0] = float(t1 - t0); r->buildStats[1] = float(t2 - t1);
@@ -385,15 +358,12 @@ CudaBVH_t cudaBVH_buildDevice(const void* d_vertices, int numVertices, int verte
         set_error("cudaBVH_buildDevice: cannot allocate %zu bytes", size_t(numTris) * 36);
         return nullptr;
     }
-    std::vector<float> host(size_t(numTris) * 9);
     int bad = 0;
     hipError_t e = hipMemset(d_bad, 0, sizeof(int));
     if (e == hipSuccess)
         e = rtk::launch_gather_tris(d_vertices, numVertices, vertexStride, d_indices, indexBytes, numTris, d_tri, d_bad,
                                     nullptr);
-    // the host copy feeds the reference's host-side exports (SoA, packed, DFS)
     if (e == hipSuccess) e = hipMemcpy(&bad, d_bad, sizeof(int), hipMemcpyDeviceToHost);
-    if (e == hipSuccess && !bad) e = hipMemcpy(host.data(), d_tri, host.size() * 4, hipMemcpyDeviceToHost);
     hipFree(d_bad);
     if (e != hipSuccess || bad) {
         hipFree(d_tri);
@@ -401,7 +371,7 @@ CudaBVH_t cudaBVH_buildDevice(const void* d_vertices, int numVertices, int verte
         else set_error("cudaBVH_buildDevice: gather failed: %s", hipGetErrorString(e));
         return nullptr;
     }
-    CudaBVHHandle* h = build_impl(host.data(), numTris, 4, nullptr, 1, nullptr, d_tri);
+    CudaBVHHandle* h = build_impl(nullptr, numTris, 4, nullptr, 1, nullptr, d_tri);
     hipFree(d_tri);
     return h;
 }
@@ -461,7 +431,6 @@ int cudaBVH_buildManyDevice(const CudaGeometry* geoms, const int* geomOffsets, i
         set_error("%s: cannot allocate %lld triangles", fn, total);
         return -1;
     }
-    std::vector<float> host(size_t(total) * 9);
     int bad = 0;
     hipError_t e = hipMemset(dBad, 0, sizeof(int));
     for (int k = 0; k < numBlas && e == hipSuccess; k++) {
@@ -474,7 +443,6 @@ int cudaBVH_buildManyDevice(const CudaGeometry* geoms, const int* geomOffsets, i
         }
     }
     if (e == hipSuccess) e = hipMemcpy(&bad, dBad, sizeof(int), hipMemcpyDeviceToHost);
-    if (e == hipSuccess && !bad) e = hipMemcpy(host.data(), dTri, host.size() * 4, hipMemcpyDeviceToHost);
     hipFree(dBad);
     if (e != hipSuccess || bad) {
         hipFree(dTri);
@@ -488,7 +456,7 @@ int cudaBVH_buildManyDevice(const CudaGeometry* geoms, const int* geomOffsets, i
         return -1;
     };
     for (int k : small) {
-        out[k] = build_impl(host.data() + 9 * size_t(start[k]), (int)count[k], 4, nullptr, 1, nullptr,
+        out[k] = build_impl(nullptr, (int)count[k], 4, nullptr, 1, nullptr,
                             dTri + 9 * size_t(start[k]));
         if (!out[k]) return fail_all();
     }
@@ -498,7 +466,7 @@ int cudaBVH_buildManyDevice(const CudaGeometry* geoms, const int* geomOffsets, i
         for (int i = 0; i < R; i++) off[i + 1] = off[i] + (int)count[big[i]];
         std::vector<int> roots4, ford;
         std::vector<rt::Node2> fn2;
-        CudaBVHHandle* forest = build_impl(host.data(), off[R], 4, off.data(), R, &roots4, dTri, &fn2, &ford);
+        CudaBVHHandle* forest = build_impl(nullptr, off[R], 4, off.data(), R, &roots4, dTri, &fn2, &ford);
         if (!forest) return fail_all();
         // BVH2 subtree sizes: the trees lie one after another in pre-order
         std::vector<int> sz(fn2.size(), 1);
@@ -541,7 +509,13 @@ int cudaBVH_buildManyDevice(const CudaGeometry* geoms, const int* geomOffsets, i
             }
             h->depth4 = bvh4_depth(hn4);
             root2 += sz[root2];
-            out[k] = make_handle(h, host.data() + 9 * size_t(t0), nt);
+            float bmin[3], bmax[3];
+            if (rt::mesh_bounds(dTri + 9 * size_t(t0), nt, nullptr, bmin, bmax) == 0) {
+                out[k] = make_handle(h, bmin, bmax, nt);
+            } else {
+                free_handle_device(h);
+                delete h;
+            }
             if (!out[k]) { cudaBVH_destroy(forest); return fail_all(); }
         }
         cudaBVH_destroy(forest);

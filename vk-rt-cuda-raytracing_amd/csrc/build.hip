@@ -6,27 +6,33 @@
 // triangles) with two rules made exact: the partition is taken on the
 // evaluated bin boundary and is stable, and a node whose centroids coincide on
 // every axis splits at the middle of its range. Under those rules the tree is
-// a pure function of the input, and this level-synchronous GPU build yields
-// bit for bit the tree of a recursive host build:
+// a pure function of the input, and this build yields bit for bit the tree of
+// a recursive host build:
 //
-//  * per level, every primitive of an unfinished node is binned on the three
-//    axes with atomics (box min/max as order-preserving integers, which makes
-//    the result independent of atomic order; LDS-privatised when a workgroup's
-//    chunk lies in one node);
-//  * one thread per node evaluates the 45 SAH candidates in the host order;
-//  * a device-wide exclusive scan of the go-left flags gives every primitive
-//    its stable position in the child range;
-//  * child boxes and centroid bounds are min/max reductions over the moved
-//    primitives;
-//  * finally nodes are renumbered in depth-first pre-order (subtree sizes
-//    bottom-up, offsets top-down), and the BVH2 is collapsed into the
-//    reference's 64-byte BVH4 nodes (backend :31-34, :391-418), FP16 bounds
-//    rounded outward. Which BVH2 nodes become BVH4 nodes is a surface-area
-//    choice (dynamic programming over the BVH2, bottom-up costs then top-down
-//    slot counts, one launch per BVH2 level each way): the least total area
-//    of BVH4 nodes, i.e. the fewest expected node visits, with up to four
-//    slots per node. The reference opens both children of every other level,
-//    which leaves 45 % of the nodes 2-wide on the 3.4 M-triangle terrain.
+//  * top phase, one level at a time, for nodes of more than kSmall
+//    primitives: bins in LDS per 4096-primitive chunk of a node, merged with
+//    atomics (box min/max as order-preserving integers, so the order does not
+//    matter); one workgroup per node evaluates the 45 SAH candidates in the
+//    host order and, from the chunks' bin counts, where each chunk's left
+//    primitives go; a stable scatter moves the chunk and reduces the
+//    children's box and centroid bounds;
+//  * bottom phase, one launch: a workgroup takes a node of at most kSmall
+//    primitives with its boxes in LDS and builds the whole subtree, one wave
+//    per node and level, then the subtree's collapse costs;
+//  * a node's depth-first pre-order number needs no renumbering passes: it is
+//    twice the number of leaves before its first primitive (one scan of the
+//    leaf-start flags) plus the left turns on its path (less one per earlier
+//    tree of a forest);
+//  * the BVH2 is collapsed into the reference's 64-byte BVH4 nodes (backend
+//    :31-34, :391-418), FP16 bounds rounded outward. Which BVH2 nodes become
+//    BVH4 nodes is a surface-area choice (dynamic programming over the BVH2,
+//    bottom-up costs then top-down slot counts): the least total area of BVH4
+//    nodes, i.e. the fewest expected node visits, with up to four slots per
+//    node. The reference opens both children of every other level, which
+//    leaves 45 % of the nodes 2-wide on the 3.4 M-triangle terrain.
+//
+// What bounds it: LDS atomics and dependent LDS steps of the bottom phase, the
+// memory passes (two per level) and launches (four per level) of the top one.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -43,7 +49,14 @@ constexpr int kBinInts = 7;                 // box min xyz, max xyz (ordered int
 constexpr int kAxisInts = kBins * kBinInts;
 constexpr int kSlotInts = 3 * kAxisInts;
 constexpr int kThreads = 256;
-constexpr int kChunk = 2048;                // primitives per workgroup in the binning passes
+
+// Nodes of at most kSmall primitives are built to their leaves by one
+// workgroup (k_subtree); larger ones are split level by level in chunks of
+// kChunk primitives.
+constexpr int kSmall = 2048;
+constexpr int kTopThreads = 512;
+constexpr int kPerThread = 8;
+constexpr int kChunk = kTopThreads * kPerThread;
 
 __device__ __forceinline__ int f2o(float f) {
     const int i = __float_as_int(f);
@@ -63,40 +76,100 @@ __device__ __forceinline__ int bin_of(float c, float cmin, float cmax) {
     return b < 0 ? 0 : (b >= kBins ? kBins - 1 : b);
 }
 
+// --- cross-lane primitives (DPP) ---
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp(int old, int v) {
+    return __builtin_amdgcn_update_dpp(old, v, CTRL, ROWS, 0xf, false);
+}
+// min / max over the 64 lanes (every lane active), wave-uniform result
+__device__ __forceinline__ int wave_min(int v) {
+    v = min(v, dpp<0x111, 0xf>(v, v)); v = min(v, dpp<0x112, 0xf>(v, v));
+    v = min(v, dpp<0x114, 0xf>(v, v)); v = min(v, dpp<0x118, 0xf>(v, v));
+    v = min(v, dpp<0x142, 0xa>(v, v)); v = min(v, dpp<0x143, 0xc>(v, v));
+    return __builtin_amdgcn_readlane(v, 63);
+}
+__device__ __forceinline__ int wave_max(int v) {
+    v = max(v, dpp<0x111, 0xf>(v, v)); v = max(v, dpp<0x112, 0xf>(v, v));
+    v = max(v, dpp<0x114, 0xf>(v, v)); v = max(v, dpp<0x118, 0xf>(v, v));
+    v = max(v, dpp<0x142, 0xa>(v, v)); v = max(v, dpp<0x143, 0xc>(v, v));
+    return __builtin_amdgcn_readlane(v, 63);
+}
+__device__ __forceinline__ float wave_minf(float x) { return o2f(wave_min(f2o(x))); }
+// lane l's value as seen from D lanes to the left (row_shr) / right (row_shl)
+// within its 16-lane row; `none` beyond the row
+template <int D> __device__ __forceinline__ int from_left(int none, int v) { return dpp<0x110 + D, 0xf>(none, v); }
+template <int D> __device__ __forceinline__ int from_right(int none, int v) { return dpp<0x100 + D, 0xf>(none, v); }
+template <int D> __device__ __forceinline__ float from_left(float none, float v) {
+    return __int_as_float(from_left<D>(__float_as_int(none), __float_as_int(v)));
+}
+template <int D> __device__ __forceinline__ float from_right(float none, float v) {
+    return __int_as_float(from_right<D>(__float_as_int(none), __float_as_int(v)));
+}
+__device__ __forceinline__ float lane_of(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// ------------------------------- data ----------------------------------------
+// A tree node while it is being built covers the primitives at positions
+// [s, s + c). lt: left turns on its path from the root; tree: its scene.
+struct Seg { int s, c, lt, tree; };
+
+// An internal node of the top phase. left / right: >= 0 a top node, < 0 the
+// subtree -1 - ref.
+struct Top { int s, m, lt, tree, left, right; float box[6]; };   // m: first primitive of the right child
+
+// A subtree of at most kSmall primitives. buf: which of the two index buffers
+// holds its primitives; bounds: box and centroid bounds (ordered ints).
+// level: BVH2 level of its root; levels: its own (set by k_subtree).
+struct Small { Seg g; int buf, level, levels, pad; int bounds[12]; };
+
+// A node of a subtree: box, first primitive, left turns, and either the left
+// child's record (the right one follows) with the split position m, or -1 and
+// the primitive count in m.
+struct Rec { float4 a; float2 b; int s, lt; int child, m, pad[2]; };
+
 struct Build {
-    int n, maxLeaf;
-    const float* pbox;      // [n][6] primitive boxes, original index
-    const float4* cen;      // [n] centroids
-    int* idx;               // [n] primitive at position
-    int* pnode;             // [n] node of position
-    int* idx2;
-    int* pnode2;
-    int* flag;              // [n] go-left flag
-    int* rank;              // [n] exclusive scan of flag
-    int* nbox;              // [cap][6] ordered ints
-    int* ncen;              // [cap][6] ordered ints (centroid bounds)
-    int* ns;                // [cap] range start
-    int* ncnt;              // [cap] primitive count
-    int* nleft;             // [cap] -1 for a leaf
-    int* nright;
-    int* ndepth;
-    int* nodeSlot;          // [cap] slot of an active node
-    int* act;               // [n] active nodes of the level
-    int* bins;              // [m][3][16][7]
-    int* sAxis;             // [m] split axis (-1: middle split)
-    int* sBin;
-    int* sNl;               // left count
-    int* small;             // [cap] node whose level was done by k_small_level (bounds written there)
-    int* bigSlot;           // [cap] bins slot of a node of more than kSmall primitives
-    int* bigCount;          // bins slots handed out this level
+    int n, maxLeaf, numScenes, maxBig;
+    float4* pbox;            // [n][2] primitive boxes, original index
+    int* idx[2];             // [n] primitive at position (ping-pong of the top phase)
+    int* ordered;            // [n] final order
+    int* leafFlag;           // [n] 1 where a leaf starts
+    const int* off;          // [numScenes + 1] scene offsets
+    const int* primBase;     // [numScenes + 1] chunks of kChunk primitives before each scene
+    int* rootAcc;            // [numScenes][12] root bounds (ordered ints)
+    int* rootRef;            // [numScenes] top node or -1 - subtree
+    unsigned long long* bnd; // [6] mesh bounds as (ordered value, first position) keys
+    // active nodes of a level (ping-pong)
+    Seg* act[2];             // [maxBig]
+    int* actAcc[2];          // [maxBig][12]
+    int* chunkBase[2];       // [maxBig + 1] chunks before each active node
+    int* bins[2];            // [2 maxBig][3][16][7]
+    int* childAcc;           // [2 maxBig][12]
+    int* sAxis;              // [maxBig] split axis (-1: middle split)
+    int* sBin;               // last left bin
+    int* sNl;                // left count
+    int* chunkHist;          // [chunks][48] primitives per axis and bin
+    int* chunkLeft;          // [chunks] left primitives of the node before the chunk
+    int* count;              // [8]: 0 active nodes, 1 their chunks, 2 subtrees, 4 / 5 leaf and head totals, 6 / 7 BVH4 / BVH2 levels
+    int* topLevel;           // [kMaxTopLevels + 1] first top node of each level
+    Top* top;                // top nodes, level by level
+    float4* topCost;
+    int2* topAsg;            // (slots presented as, BVH4 level)
+    Small* small;
+    float4* smallCost;
+    int2* smallAsg;
+    Rec* rec;                // subtree records: from 2 * first position
+    float4* cost;            // collapse costs, as rec
+    unsigned short* lvl;     // first record of each level of a subtree, from 2 * first position
+    int* leafRank;           // [n] leaves before a position
 };
 
-// Nodes of at most kSmall primitives take one level per launch inside one
-// wave (k_small_level): LDS bins, SAH, stable partition and child bounds
-// without global atomics. Larger nodes use the device-wide passes.
-constexpr int kSmall = 2048;
+__device__ __forceinline__ int pre_of(const Build& b, int s, int lt, int tree) { return 2 * b.leafRank[s] + lt - tree; }
 
-// ---------------------------------------------------------------------------
 // Scene of primitive i: the last s with off[s] <= i (off: numScenes+1 ascending offsets).
 __device__ __forceinline__ int scene_of(const int* off, int numScenes, int i) {
     int lo = 0, hi = numScenes - 1;
@@ -107,445 +180,491 @@ __device__ __forceinline__ int scene_of(const int* off, int numScenes, int i) {
     return lo;
 }
 
-__global__ void k_prims(const float* __restrict__ tris, int n, float* pbox, float4* cen, int* idx, int* pnode,
-                        const int* off, int numScenes) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float* t = tris + 9 * (size_t)i;
-    float mn[3], mx[3];
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-        mn[a] = fminf(fminf(t[a], t[3 + a]), t[6 + a]) + 0.0f;   // + 0: -0 -> +0
-        mx[a] = fmaxf(fmaxf(t[a], t[3 + a]), t[6 + a]) + 0.0f;
-        pbox[6 * (size_t)i + a] = mn[a];
-        pbox[6 * (size_t)i + 3 + a] = mx[a];
+// Segment of chunk c: the last j < m with base[j] <= c (a 64-ary search, the
+// same in every wave).
+__device__ __forceinline__ int find_seg(const int* base, int m, int c) {
+    const int lane = threadIdx.x & 63;
+    int lo = 0, len = m;
+    while (len > 1) {
+        const int step = (len + 63) >> 6;
+        const int k = lo + lane * step;
+        const bool le = lane * step < len && base[k] <= c;
+        const int hits = __popcll(__ballot(le));
+        lo += (hits - 1) * step;
+        len = min(step, m - lo);
     }
-    cen[i] = make_float4((mn[0] + mx[0]) * .5f, (mn[1] + mx[1]) * .5f, (mn[2] + mx[2]) * .5f, 0.f);
-    idx[i] = i;
-    pnode[i] = numScenes == 1 ? 0 : scene_of(off, numScenes, i);
+    return lo;
 }
 
-// Roots: node s spans scene s's primitives; slots[s] is its active slot (or -1).
-__global__ void k_init_roots(Build b, const int* off, const int* slots, int numScenes) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= numScenes) return;
-    b.ns[s] = off[s]; b.ncnt[s] = off[s + 1] - off[s];
-    b.nleft[s] = -1; b.nright[s] = -1; b.ndepth[s] = 0;
-    b.nodeSlot[s] = slots[s];
-    if (slots[s] >= 0) b.act[slots[s]] = s;
+__device__ __forceinline__ void load_box(const float4* pbox, int p, float (&v)[6]) {
+    const float4 a = pbox[2 * (size_t)p];
+    const float2 b = *(const float2*)&pbox[2 * (size_t)p + 1];
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y;
 }
+// Centroid of a primitive box (one float expression everywhere).
+__device__ __forceinline__ float centroid(const float (&v)[6], int a) { return (v[a] + v[3 + a]) * .5f; }
 
-__global__ void k_init_nodes(int* nbox, int* ncen, int* small, int first, int count) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    small[first + i] = 0;
-    const size_t o = 6 * (size_t)(first + i);
+// Bounds of up to kPerThread primitives per thread (box and centroid, ordered
+// ints), reduced over the workgroup into dst with 12 atomics.
+template <int NT>
+struct BoundsAcc {
+    int v[12];
+    __device__ __forceinline__ void init() {
 #pragma unroll
-    for (int a = 0; a < 3; a++) {
-        nbox[o + a] = kOrdPosInf; nbox[o + 3 + a] = kOrdNegInf;
-        ncen[o + a] = kOrdPosInf; ncen[o + 3 + a] = kOrdNegInf;
+        for (int k = 0; k < 12; k++) v[k] = (k % 6) < 3 ? kOrdPosInf : kOrdNegInf;
     }
-}
-
-// Box and centroid bounds of every node at or above levelBase, reduced over
-// its primitives (LDS first when the chunk lies in one node).
-__global__ __launch_bounds__(kThreads) void k_node_bounds(Build b, int levelBase) {
-    // The nodes bounded here (children of nodes of more than kSmall
-    // primitives) are at most four per chunk: at most two such parents
-    // overlap kChunk consecutive positions. Each gets an LDS accumulator,
-    // claimed by node id; global atomics only if a fifth ever showed up.
-    __shared__ int key[4];
-    __shared__ int lb[4][12];
-    const int c0 = blockIdx.x * kChunk, c1 = min(c0 + kChunk, b.n);
-    if (threadIdx.x < 4) key[threadIdx.x] = -1;
-    if (threadIdx.x < 48) lb[threadIdx.x / 12][threadIdx.x % 12] = (threadIdx.x % 6) < 3 ? kOrdPosInf : kOrdNegInf;
-    __syncthreads();
-    for (int i = c0 + threadIdx.x; i < c1; i += kThreads) {
-        const int node = b.pnode[i];
-        if (node < levelBase || b.small[node]) continue;
-        int j = 0;
-        for (; j < 4; j++) {
-            const int k = key[j];
-            if (k == node) break;
-            if (k == -1) {
-                const int prev = atomicCAS(&key[j], -1, node);
-                if (prev == -1 || prev == node) break;
-            }
-        }
-        const int p = b.idx[i];
-        const float* pb = b.pbox + 6 * (size_t)p;
-        const float4 c = b.cen[p];
-        const float cv[3] = {c.x, c.y, c.z};
-        int* nb = j < 4 ? &lb[j][0] : b.nbox + 6 * (size_t)node;
-        int* nc = j < 4 ? &lb[j][6] : b.ncen + 6 * (size_t)node;
+    __device__ __forceinline__ void add(const float (&bx)[6]) {
 #pragma unroll
         for (int a = 0; a < 3; a++) {
-            atomicMin(&nb[a], f2o(pb[a])); atomicMax(&nb[3 + a], f2o(pb[3 + a]));
-            atomicMin(&nc[a], f2o(cv[a])); atomicMax(&nc[3 + a], f2o(cv[a]));
+            v[a] = min(v[a], f2o(bx[a])); v[3 + a] = max(v[3 + a], f2o(bx[3 + a]));
+            const int c = f2o(centroid(bx, a));
+            v[6 + a] = min(v[6 + a], c); v[9 + a] = max(v[9 + a], c);
         }
     }
-    __syncthreads();
-    if (threadIdx.x < 48) {
-        const int j = threadIdx.x / 12, k = threadIdx.x % 12, u = key[j];
-        if (u >= 0) {
-            int* dst = (k < 6 ? b.nbox : b.ncen) + 6 * (size_t)u + (k % 6);
-            if ((k % 6) < 3) atomicMin(dst, lb[j][k]); else atomicMax(dst, lb[j][k]);
+    // lds: NT / 64 * 12 ints; every thread of the workgroup calls it
+    __device__ __forceinline__ void flush(int* lds, int* dst) {
+        const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma unroll
+        for (int k = 0; k < 12; k++) {
+            const int r = (k % 6) < 3 ? wave_min(v[k]) : wave_max(v[k]);
+            if (lane == 0) lds[w * 12 + k] = r;
         }
+        __syncthreads();
+        if (threadIdx.x < 12) {
+            const int k = threadIdx.x;
+            int r = lds[k];
+            for (int j = 1; j < NT / 64; j++) r = (k % 6) < 3 ? min(r, lds[j * 12 + k]) : max(r, lds[j * 12 + k]);
+            if ((k % 6) < 3) atomicMin(&dst[k], r); else atomicMax(&dst[k], r);
+        }
+        __syncthreads();
     }
-}
+};
 
-// Bins slots of the level's nodes of more than kSmall primitives (the others
-// bin in LDS): at most n / (kSmall + 1) + numScenes of them; which node gets
-// which slot does not matter.
-__global__ void k_big_slots(Build b, int m) {
-    const int slot = blockIdx.x * blockDim.x + threadIdx.x;
-    if (slot >= m) return;
-    const int node = b.act[slot];
-    if (b.ncnt[node] > kSmall) b.bigSlot[node] = atomicAdd(b.bigCount, 1);
-}
-
-__global__ void k_zero_int(int* w) { *w = 0; }
-
-__global__ void k_clear_bins(int* bins, int slots) {
+__global__ void k_build_init(Build b, int slots) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= slots * kSlotInts) return;
-    const int f = i % kBinInts;
-    bins[i] = f < 3 ? kOrdPosInf : (f < 6 ? kOrdNegInf : 0);
-}
-
-__device__ __forceinline__ void bin_prim(const Build& b, int node, int p, int* dst /*[3][16][7]*/) {
-    const float* pb = b.pbox + 6 * (size_t)p;
-    const float4 c = b.cen[p];
-    const float cv[3] = {c.x, c.y, c.z};
-    const int* nc = b.ncen + 6 * (size_t)node;
-    int bx[6];
-#pragma unroll
-    for (int k = 0; k < 6; k++) bx[k] = f2o(pb[k]);
-#pragma unroll
-    for (int ax = 0; ax < 3; ax++) {
-        const float cmin = o2f(nc[ax]), cmax = o2f(nc[3 + ax]);
-        if (cmax - cmin < 1e-8f) continue;
-        int* d = dst + ax * kAxisInts + bin_of(cv[ax], cmin, cmax) * kBinInts;
-#pragma unroll
-        for (int k = 0; k < 3; k++) { atomicMin(&d[k], bx[k]); atomicMax(&d[3 + k], bx[3 + k]); }
-        atomicAdd(&d[6], 1);
-    }
-}
-
-__global__ __launch_bounds__(kThreads) void k_bin(Build b) {
-    // A node of more than kSmall (>= kChunk) primitives that overlaps this
-    // chunk holds its first or its last position, so the chunk bins into at
-    // most two LDS copies (those two nodes) and flushes them once.
-    __shared__ int lb[2][kSlotInts];
-    __shared__ int nodes2[2];
-    const int c0 = blockIdx.x * kChunk, c1 = min(c0 + kChunk, b.n);
-    if (threadIdx.x == 0) {
-        const int a = b.pnode[c0], z = b.pnode[c1 - 1];
-        nodes2[0] = b.ncnt[a] > kSmall ? a : -1;
-        nodes2[1] = (z != a && b.ncnt[z] > kSmall) ? z : -1;
-    }
-    for (int i = threadIdx.x; i < 2 * kSlotInts; i += kThreads) {
-        const int f = (i % kSlotInts) % kBinInts;
-        lb[i / kSlotInts][i % kSlotInts] = f < 3 ? kOrdPosInf : (f < 6 ? kOrdNegInf : 0);
-    }
-    __syncthreads();
-    const int na = nodes2[0], nz = nodes2[1];
-    if (na < 0 && nz < 0) return;
-    for (int i = c0 + threadIdx.x; i < c1; i += kThreads) {
-        const int node = b.pnode[i];
-        if (node == na) bin_prim(b, node, b.idx[i], lb[0]);
-        else if (node == nz) bin_prim(b, node, b.idx[i], lb[1]);
-    }
-    __syncthreads();
-    for (int q = 0; q < 2; q++) {
-        const int u = nodes2[q];
-        if (u < 0) continue;
-        int* g = b.bins + (size_t)b.bigSlot[u] * kSlotInts;
-        for (int i = threadIdx.x; i < kSlotInts; i += kThreads) {
-            const int f = i % kBinInts;
-            const int v = lb[q][i];
-            if (f == 6) { if (v) atomicAdd(&g[i], v); }
-            else if (f < 3) { if (v != kOrdPosInf) atomicMin(&g[i], v); }
-            else if (v != kOrdNegInf) atomicMax(&g[i], v);
-        }
-    }
-}
-
-// SAH over 3 axes x 15 boundaries in the host order (axis-major, strict <)
-// from the node's bins ([3][16][7], global or LDS): split axis (-1: middle
-// split), last left bin and left count.
-__device__ __forceinline__ void sah_choose(const int* bins, const int* nb, const int* nc, int cnt, int& bestAxis,
-                                           int& bestBin, int& bestNl) {
-    const float pA = area(o2f(nb[0]), o2f(nb[1]), o2f(nb[2]), o2f(nb[3]), o2f(nb[4]), o2f(nb[5]));
-    float bestCost = 1e30f;
-    bestAxis = -1; bestBin = -1; bestNl = 0;
-    for (int ax = 0; ax < 3; ax++) {
-        const float cmin = o2f(nc[ax]), cmax = o2f(nc[3 + ax]);
-        if (cmax - cmin < 1e-8f) continue;
-        const int* B = bins + ax * kAxisInts;
-        float R[kBins][6];
-        int rc[kBins];
-        for (int k = 0; k < 6; k++) R[kBins - 1][k] = o2f(B[(kBins - 1) * kBinInts + k]);
-        rc[kBins - 1] = B[(kBins - 1) * kBinInts + 6];
-        for (int q = kBins - 2; q >= 0; q--) {
-            for (int k = 0; k < 3; k++) {
-                R[q][k] = fminf(R[q + 1][k], o2f(B[q * kBinInts + k]));
-                R[q][3 + k] = fmaxf(R[q + 1][3 + k], o2f(B[q * kBinInts + 3 + k]));
-            }
-            rc[q] = rc[q + 1] + B[q * kBinInts + 6];
-        }
-        float L[6];
-        for (int k = 0; k < 6; k++) L[k] = o2f(B[k]);
-        int lc = B[6];
-        for (int q = 0; q < kBins - 1; q++) {
-            if (q > 0) {
-                for (int k = 0; k < 3; k++) {
-                    L[k] = fminf(L[k], o2f(B[q * kBinInts + k]));
-                    L[3 + k] = fmaxf(L[3 + k], o2f(B[q * kBinInts + 3 + k]));
-                }
-                lc += B[q * kBinInts + 6];
-            }
-            if (lc == 0 || rc[q + 1] == 0) continue;
-            const float cost = (float)lc * area(L[0], L[1], L[2], L[3], L[4], L[5]) / pA +
-                               (float)rc[q + 1] * area(R[q + 1][0], R[q + 1][1], R[q + 1][2], R[q + 1][3],
-                                                        R[q + 1][4], R[q + 1][5]) / pA + 1.f;
-            if (cost < bestCost) { bestCost = cost; bestAxis = ax; bestBin = q; bestNl = lc; }
-        }
-    }
-    if (bestAxis < 0) bestNl = cnt / 2;                      // coincident centroids: middle split
-}
-
-// Children of a split node: ids childBase + 2 slot (+1), ranges, depth.
-__device__ __forceinline__ void make_children(const Build& b, int node, int slot, int childBase, int nl) {
-    const int L = childBase + 2 * slot, R = L + 1;
-    const int s = b.ns[node], d = b.ndepth[node] + 1, cnt = b.ncnt[node];
-    b.nleft[node] = L; b.nright[node] = R;
-    b.ns[L] = s; b.ncnt[L] = nl; b.ns[R] = s + nl; b.ncnt[R] = cnt - nl;
-    b.ndepth[L] = d; b.ndepth[R] = d;
-    b.nleft[L] = b.nright[L] = b.nleft[R] = b.nright[R] = -1;
-}
-
-// One thread per active node of more than kSmall primitives: SAH from the
-// device-wide bins, then the two children.
-__global__ void k_sah(Build b, int m, int childBase) {
-    const int slot = blockIdx.x * blockDim.x + threadIdx.x;
-    if (slot >= m) return;
-    const int node = b.act[slot];
-    const int cnt = b.ncnt[node];
-    if (cnt <= kSmall) return;
-    int ax, bin, nl;
-    sah_choose(b.bins + (size_t)b.bigSlot[node] * kSlotInts, b.nbox + 6 * (size_t)node, b.ncen + 6 * (size_t)node, cnt, ax,
-               bin, nl);
-    b.sAxis[slot] = ax;
-    b.sBin[slot] = bin;
-    b.sNl[slot] = nl;
-    make_children(b, node, slot, childBase, nl);
-}
-
-// One level of every active node of at most kSmall primitives, one wave per
-// node: bins in LDS, the SAH choice, the two children, the stable partition
-// of its primitives into idx2 / pnode2 (ballot ranks, left ones first) and
-// the children's box and centroid bounds, written directly (small[child] = 1
-// tells k_node_bounds to leave them alone). Same results as the device-wide
-// passes, which skip these nodes.
-__global__ __launch_bounds__(64) void k_small_level(Build b, int m, int childBase) {
-    __shared__ int lb[kSlotInts];
-    __shared__ int cb[24];                   // left box, left centroids, right box, right centroids
-    __shared__ int choice[3];
-    const int slot = blockIdx.x;
-    if (slot >= m) return;
-    const int node = b.act[slot];
-    const int cnt = b.ncnt[node];
-    if (cnt > kSmall) return;                // uniform per workgroup
-    const int lane = threadIdx.x;
-    for (int i = lane; i < kSlotInts; i += 64) {
+    if (i < b.numScenes * 12) b.rootAcc[i] = (i % 6) < 3 ? kOrdPosInf : kOrdNegInf;
+    if (i < 6) b.bnd[i] = ~0ull;
+    if (i < 8) b.count[i] = 0;
+    if (i == 0) b.topLevel[0] = 0;
+    if (i < slots * kSlotInts) {
         const int f = i % kBinInts;
+        b.bins[0][i] = f < 3 ? kOrdPosInf : (f < 6 ? kOrdNegInf : 0);
+    }
+}
+
+// ------------------------------- top phase -----------------------------------
+// Primitive boxes and identity order, the scenes' root bounds and the bounds
+// of the whole mesh. The mesh bounds keep, as a sequential std::min / std::max
+// pass over the triangles would, the first of equal values (the sign of a
+// zero) and skip NaN: each axis reduces a 64-bit key of the ordered value and
+// the position of the coordinate.
+__global__ __launch_bounds__(kTopThreads) void k_prims(Build b, const float* __restrict__ tris, int chunks) {
+    __shared__ int lds[kTopThreads / 64 * 12];
+    __shared__ unsigned long long lk[kTopThreads / 64][6];
+    const int j = find_seg(b.primBase, b.numScenes, blockIdx.x);
+    const int s = b.off[j], c = b.off[j + 1] - s;
+    const int p0 = (blockIdx.x - b.primBase[j]) * kChunk;
+    BoundsAcc<kTopThreads> acc;
+    acc.init();
+    unsigned long long key[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) key[k] = ~0ull;
+    for (int k = 0; k < kPerThread; k++) {
+        const int q = p0 + k * kTopThreads + threadIdx.x;
+        if (q >= c) break;
+        const int i = s + q;
+        const float* t = tris + 9 * (size_t)i;
+        float x[9], v[6];
+#pragma unroll
+        for (int e = 0; e < 9; e++) x[e] = t[e];
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+            v[a] = fminf(fminf(x[a], x[3 + a]), x[6 + a]) + 0.0f;   // + 0: -0 -> +0
+            v[3 + a] = fmaxf(fmaxf(x[a], x[3 + a]), x[6 + a]) + 0.0f;
+        }
+        b.pbox[2 * (size_t)i] = make_float4(v[0], v[1], v[2], v[3]);
+        b.pbox[2 * (size_t)i + 1] = make_float4(v[4], v[5], 0.f, 0.f);
+        b.idx[0][i] = i;
+        acc.add(v);
+#pragma unroll
+        for (int e = 0; e < 9; e++) {
+            if (x[e] == x[e]) {
+                const int a = e % 3;
+                const unsigned int o = (unsigned int)f2o(x[e] + 0.0f) ^ 0x80000000u;
+                const unsigned int pos = 3u * (unsigned int)i + (unsigned int)(e / 3);
+                const unsigned long long lo = (unsigned long long)o << 32 | pos;
+                const unsigned long long hi = (unsigned long long)~o << 32 | pos;
+                if (lo < key[a]) key[a] = lo;
+                if (hi < key[3 + a]) key[3 + a] = hi;
+            }
+        }
+    }
+    acc.flush(lds, b.rootAcc + 12 * (size_t)j);
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+        unsigned long long v = key[k];
+        for (int d = 32; d > 0; d >>= 1) {
+            const unsigned long long o = __shfl_xor(v, d, 64);
+            if (o < v) v = o;
+        }
+        if ((threadIdx.x & 63) == 0) lk[threadIdx.x >> 6][k] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x < 6) {
+        unsigned long long v = lk[0][threadIdx.x];
+        for (int w = 1; w < kTopThreads / 64; w++) v = min(v, lk[w][threadIdx.x]);
+        atomicMin(&b.bnd[threadIdx.x], v);
+    }
+}
+
+// Bounds of n triangles alone (one tree of a forest): the keys of k_prims.
+__global__ __launch_bounds__(kTopThreads) void k_mesh_keys(const float* __restrict__ tris, int n,
+                                                           unsigned long long* bnd) {
+    unsigned long long key[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) key[k] = ~0ull;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+#pragma unroll
+        for (int e = 0; e < 9; e++) {
+            const float x = tris[9 * (size_t)i + e];
+            if (x == x) {
+                const int a = e % 3;
+                const unsigned int o = (unsigned int)f2o(x + 0.0f) ^ 0x80000000u;
+                const unsigned int pos = 3u * (unsigned int)i + (unsigned int)(e / 3);
+                const unsigned long long lo = (unsigned long long)o << 32 | pos;
+                const unsigned long long hi = (unsigned long long)~o << 32 | pos;
+                if (lo < key[a]) key[a] = lo;
+                if (hi < key[3 + a]) key[3 + a] = hi;
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+        unsigned long long v = key[k];
+        for (int d = 32; d > 0; d >>= 1) {
+            const unsigned long long o = __shfl_xor(v, d, 64);
+            if (o < v) v = o;
+        }
+        if ((threadIdx.x & 63) == 0) atomicMin(&bnd[k], v);
+    }
+}
+__global__ void k_keys_init(unsigned long long* bnd) {
+    if (threadIdx.x < 6) bnd[threadIdx.x] = ~0ull;
+}
+// Keys -> the coordinates they name; an axis without a value below 1e30
+// (above -1e30) keeps that bound, as the sequential pass does.
+__global__ void k_mesh_bounds(const float* tris, const unsigned long long* bnd, float* out) {
+    const int k = threadIdx.x;
+    if (k >= 6) return;
+    float r = k < 3 ? 1e30f : -1e30f;
+    if (bnd[k] != ~0ull) {
+        const unsigned int pos = (unsigned int)bnd[k];
+        const float x = tris[9 * (size_t)(pos / 3) + 3 * (pos % 3) + k % 3];
+        if (k < 3 ? x < r : r < x) r = x;
+    }
+    out[k] = r;
+}
+
+// Next level's active nodes: the children (2 m of them, or with `init` the
+// numScenes roots) of more than kSmall primitives in order, with their chunk
+// numbering; the others become subtrees. One workgroup. `out` is the parity
+// of the arrays written (and of the index buffer that holds the children's
+// primitives).
+__global__ __launch_bounds__(1024) void k_top_next(Build b, int out, int init, int level) {
+    __shared__ int lds[1024 / 64 + 1];
+    const int in = out ^ 1;
+    const int m = init ? 0 : b.count[0], kids = init ? b.numScenes : 2 * m;
+    const int topBase = init ? 0 : b.topLevel[level];
+    const int smallBase = b.count[2];
+    __syncthreads();                       // every thread has read count before it changes
+    int nbig = 0, nsmall = 0, nchunks = 0;
+    for (int k0 = 0; k0 < kids; k0 += 1024) {
+        const int k = k0 + threadIdx.x;
+        const bool valid = k < kids;
+        Seg g{0, 0, 0, 0};
+        const int* acc = nullptr;
+        if (valid && init) {
+            g = Seg{b.off[k], b.off[k + 1] - b.off[k], 0, k};
+            acc = b.rootAcc + 12 * (size_t)k;
+        } else if (valid) {
+            const Seg p = b.act[in][k >> 1];
+            const int nl = b.sNl[k >> 1];
+            g = (k & 1) ? Seg{p.s + nl, p.c - nl, p.lt, p.tree} : Seg{p.s, nl, p.lt + 1, p.tree};
+            acc = b.childAcc + 12 * (size_t)k;
+        }
+        const bool big = valid && g.c > kSmall;
+        const int chunks = big ? (g.c + kChunk - 1) / kChunk : 0;
+        int tb, ts, tc;
+        const int rb = nbig + rts::block_exclusive_scan<1024>(big ? 1 : 0, lds, &tb);
+        const int rs = nsmall + rts::block_exclusive_scan<1024>(valid && !big ? 1 : 0, lds, &ts);
+        const int rc = nchunks + rts::block_exclusive_scan<1024>(chunks, lds, &tc);
+        if (valid) {
+            int ref;
+            if (big) {
+                b.act[out][rb] = g;
+                b.chunkBase[out][rb] = rc;
+                for (int q = 0; q < 12; q++) b.actAcc[out][12 * (size_t)rb + q] = acc[q];
+                ref = topBase + m + rb;            // top nodes are numbered level by level
+            } else {
+                Small& sm = b.small[smallBase + rs];
+                sm.g = g;
+                sm.buf = out;
+                sm.level = init ? 0 : level + 1;
+                for (int q = 0; q < 12; q++) sm.bounds[q] = acc[q];
+                ref = -1 - (smallBase + rs);
+            }
+            if (init) b.rootRef[k] = ref;
+            else if (k & 1) b.top[topBase + (k >> 1)].right = ref;
+            else b.top[topBase + (k >> 1)].left = ref;
+        }
+        nbig += tb; nsmall += ts; nchunks += tc;
+    }
+    if (threadIdx.x == 0) {
+        b.chunkBase[out][nbig] = nchunks;
+        b.count[0] = nbig;
+        b.count[1] = nchunks;
+        b.count[2] = smallBase + nsmall;
+        b.topLevel[init ? 0 : level + 1] = topBase + m;
+    }
+}
+
+// Bins of one chunk of an active node: LDS copies (a coherent mesh puts a
+// wave's primitives in one bin, and one copy would serialise its atomics),
+// merged into the node's bins; the chunk's counts per bin stay for the
+// partition.
+constexpr int kBinCopies = 8;
+constexpr int kCopyStride = kSlotInts + 9;        // copies start on different banks
+__global__ __launch_bounds__(kTopThreads) void k_top_bin(Build b, int cur) {
+    __shared__ int lb[kBinCopies * kCopyStride];
+    if ((int)blockIdx.x >= b.count[1]) return;
+    const int j = find_seg(b.chunkBase[cur], b.count[0], blockIdx.x);
+    const Seg g = b.act[cur][j];
+    const int p0 = ((int)blockIdx.x - b.chunkBase[cur][j]) * kChunk;
+    const int* nc = b.actAcc[cur] + 12 * (size_t)j + 6;
+    float cmin[3], cmax[3];
+    bool use[3];
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        cmin[a] = o2f(nc[a]); cmax[a] = o2f(nc[3 + a]);
+        use[a] = !(cmax[a] - cmin[a] < 1e-8f);
+    }
+    for (int i = threadIdx.x; i < kBinCopies * kCopyStride; i += kTopThreads) {
+        const int f = (i % kCopyStride) % kBinInts;
         lb[i] = f < 3 ? kOrdPosInf : (f < 6 ? kOrdNegInf : 0);
     }
-    if (lane < 24) cb[lane] = (lane % 6) < 3 ? kOrdPosInf : kOrdNegInf;
     __syncthreads();
-    const int s = b.ns[node];
-    for (int i = lane; i < cnt; i += 64) bin_prim(b, node, b.idx[s + i], lb);
+    int* mine = lb + (threadIdx.x % kBinCopies) * kCopyStride;
+    const int* idx = b.idx[cur] + g.s;
+#pragma unroll 2
+    for (int k = 0; k < kPerThread; k++) {
+        const int i = p0 + k * kTopThreads + threadIdx.x;
+        if (i >= g.c) break;
+        float v[6];
+        load_box(b.pbox, idx[i], v);
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+            if (!use[a]) continue;
+            int* d = mine + a * kAxisInts + bin_of(centroid(v, a), cmin[a], cmax[a]) * kBinInts;
+#pragma unroll
+            for (int e = 0; e < 3; e++) { atomicMin(&d[e], f2o(v[e])); atomicMax(&d[3 + e], f2o(v[3 + e])); }
+            atomicAdd(&d[6], 1);
+        }
+    }
     __syncthreads();
-    if (lane == 0) {
-        int ax, bin, nl;
-        sah_choose(lb, b.nbox + 6 * (size_t)node, b.ncen + 6 * (size_t)node, cnt, ax, bin, nl);
-        choice[0] = ax; choice[1] = bin; choice[2] = nl;
-        b.sAxis[slot] = ax; b.sBin[slot] = bin; b.sNl[slot] = nl;
-        make_children(b, node, slot, childBase, nl);
+    int* out = b.bins[cur] + (size_t)j * kSlotInts;
+    for (int i = threadIdx.x; i < kSlotInts; i += kTopThreads) {
+        const int f = i % kBinInts;
+        int v = lb[i];
+        for (int k = 1; k < kBinCopies; k++) {
+            const int o = lb[k * kCopyStride + i];
+            v = f < 3 ? min(v, o) : (f < 6 ? max(v, o) : v + o);
+        }
+        if (f == 6) {
+            b.chunkHist[(size_t)blockIdx.x * (3 * kBins) + i / kBinInts] = v;
+            if (v) atomicAdd(&out[i], v);
+        } else if (f < 3) {
+            if (v != kOrdPosInf) atomicMin(&out[i], v);
+        } else if (v != kOrdNegInf) {
+            atomicMax(&out[i], v);
+        }
+    }
+}
+
+// SAH over 3 axes x 15 boundaries in one wave: lane 16 a + q holds bin q of
+// axis a; box prefixes and suffixes are scans within the 16-lane rows, and the
+// first candidate of least cost in the host order (axis-major, strict <) wins.
+struct Sah {
+    int axis, bin, nl;         // split (axis -1: middle split), last left bin, left count; wave-uniform
+    int src;                   // the winning lane
+    float L[6], R[6];          // this lane's candidate: left and right box
+    bool nan;                  // some bin's box holds a NaN (wave-uniform)
+};
+__device__ __forceinline__ void sah_wave(const int* bins, float pA, bool use0, bool use1, bool use2, int cnt, Sah& r) {
+    const int lane = threadIdx.x & 63;
+    const int ax = lane >> 4, q = lane & 15;
+    float bx[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    int n = 0;
+    if (lane < 3 * kBins) {
+        const int* B = bins + lane * kBinInts;
+#pragma unroll
+        for (int k = 0; k < 6; k++) bx[k] = o2f(B[k]);
+        n = B[6];
+    }
+    r.nan = __any(bx[0] != bx[0] || bx[1] != bx[1] || bx[2] != bx[2] || bx[3] != bx[3] || bx[4] != bx[4] || bx[5] != bx[5]);
+    int ln = n, rn = n;
+    float S[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) r.L[k] = S[k] = bx[k];
+#define RTB_SCAN(D)                                                                                     \
+    {                                                                                                   \
+        _Pragma("unroll") for (int k = 0; k < 3; k++) {                                                 \
+            r.L[k] = fminf(r.L[k], from_left<D>(INFINITY, r.L[k]));                                     \
+            r.L[3 + k] = fmaxf(r.L[3 + k], from_left<D>(-INFINITY, r.L[3 + k]));                        \
+            S[k] = fminf(S[k], from_right<D>(INFINITY, S[k]));                                          \
+            S[3 + k] = fmaxf(S[3 + k], from_right<D>(-INFINITY, S[3 + k]));                             \
+        }                                                                                               \
+        ln += from_left<D>(0, ln);                                                                      \
+        rn += from_right<D>(0, rn);                                                                     \
+    }
+    RTB_SCAN(1) RTB_SCAN(2) RTB_SCAN(4) RTB_SCAN(8)
+#undef RTB_SCAN
+#pragma unroll
+    for (int k = 0; k < 6; k++) r.R[k] = from_right<1>(k < 3 ? INFINITY : -INFINITY, S[k]);
+    rn = from_right<1>(0, rn);
+    const bool use = ax == 0 ? use0 : (ax == 1 ? use1 : (ax == 2 && use2));
+    const float cost = (float)ln * area(r.L[0], r.L[1], r.L[2], r.L[3], r.L[4], r.L[5]) / pA +
+                       (float)rn * area(r.R[0], r.R[1], r.R[2], r.R[3], r.R[4], r.R[5]) / pA + 1.f;
+    const bool ok = use && q < kBins - 1 && ln != 0 && rn != 0 && cost < 1e30f;
+    const float least = wave_minf(ok ? cost : INFINITY);
+    const uint64_t best = __ballot(ok && cost == least);
+    if (best == 0) {                               // coincident centroids: middle split
+        r.axis = -1; r.bin = -1; r.nl = cnt / 2; r.src = 0;
+    } else {
+        r.src = __ffsll((unsigned long long)best) - 1;
+        r.axis = r.src >> 4;
+        r.bin = r.src & 15;
+        r.nl = __builtin_amdgcn_readlane(ln, r.src);
+    }
+}
+
+// One workgroup per active node: the SAH choice (first wave), the top node,
+// the children's empty bounds, cleared bins for two nodes of the next level,
+// and the left primitives before each of the node's chunks.
+__global__ __launch_bounds__(kThreads) void k_top_split(Build b, int cur, int level) {
+    __shared__ int choice[3];
+    __shared__ int lds[kThreads / 64 + 1];
+    const int j = blockIdx.x;
+    if (j >= b.count[0]) return;
+    const Seg g = b.act[cur][j];
+    const int* nb = b.actAcc[cur] + 12 * (size_t)j;
+    if (threadIdx.x < 64) {
+        float bx[6], cb[6];
+#pragma unroll
+        for (int k = 0; k < 6; k++) { bx[k] = o2f(nb[k]); cb[k] = o2f(nb[6 + k]); }
+        Sah r;
+        sah_wave(b.bins[cur] + (size_t)j * kSlotInts, area(bx[0], bx[1], bx[2], bx[3], bx[4], bx[5]),
+                 !(cb[3] - cb[0] < 1e-8f), !(cb[4] - cb[1] < 1e-8f), !(cb[5] - cb[2] < 1e-8f), g.c, r);
+        if (threadIdx.x == 0) {
+            choice[0] = r.axis; choice[1] = r.bin; choice[2] = r.nl;
+            b.sAxis[j] = r.axis; b.sBin[j] = r.bin; b.sNl[j] = r.nl;
+            Top& t = b.top[b.topLevel[level] + j];
+            t.s = g.s; t.m = g.s + r.nl; t.lt = g.lt; t.tree = g.tree;
+#pragma unroll
+            for (int k = 0; k < 6; k++) t.box[k] = bx[k];
+        }
+    }
+    if (threadIdx.x < 24) b.childAcc[24 * (size_t)j + threadIdx.x] = (threadIdx.x % 6) < 3 ? kOrdPosInf : kOrdNegInf;
+    int* clr = b.bins[cur ^ 1] + 2 * (size_t)j * kSlotInts;
+    for (int i = threadIdx.x; i < 2 * kSlotInts; i += kThreads) {
+        const int f = i % kBinInts;
+        clr[i] = f < 3 ? kOrdPosInf : (f < 6 ? kOrdNegInf : 0);
     }
     __syncthreads();
     const int ax = choice[0], bin = choice[1], nl = choice[2];
-    const int L = childBase + 2 * slot, R = L + 1;
-    const int* nc = b.ncen + 6 * (size_t)node;
-    const float cmin = ax >= 0 ? o2f(nc[ax]) : 0.f, cmax = ax >= 0 ? o2f(nc[3 + ax]) : 0.f;
-    int leftBefore = 0;
-    for (int base = 0; base < cnt; base += 64) {
-        const int i = base + lane;
-        const bool valid = i < cnt;
-        int p = 0;
-        bool left = false;
-        if (valid) {
-            p = b.idx[s + i];
+    const int c0 = b.chunkBase[cur][j], nch = b.chunkBase[cur][j + 1] - c0;
+    int carry = 0;
+    for (int q0 = 0; q0 < nch; q0 += kThreads) {
+        const int q = q0 + threadIdx.x;
+        int left = 0;
+        if (q < nch) {
             if (ax < 0) {
-                left = i < nl;
+                left = max(0, min(nl - q * kChunk, kChunk));
             } else {
-                const float4 c = b.cen[p];
-                const float cv = ax == 0 ? c.x : (ax == 1 ? c.y : c.z);
-                left = bin_of(cv, cmin, cmax) <= bin;
+                const int* h = b.chunkHist + (size_t)(c0 + q) * (3 * kBins) + ax * kBins;
+                for (int k = 0; k <= bin; k++) left += h[k];
             }
         }
-        const uint64_t lm = __ballot(valid && left);
-        const int lr = __popcll(lm & ((1ull << lane) - 1ull));
-        if (valid) {
-            const int pos = left ? s + leftBefore + lr : s + nl + (i - leftBefore - lr);
-            b.idx2[pos] = p;
-            b.pnode2[pos] = left ? L : R;
-            const float* pb = b.pbox + 6 * (size_t)p;
-            const float4 c = b.cen[p];
-            const float cv[3] = {c.x, c.y, c.z};
-            int* d = cb + (left ? 0 : 12);
+        int tot;
+        const int ex = rts::block_exclusive_scan<kThreads>(left, lds, &tot);
+        if (q < nch) b.chunkLeft[c0 + q] = carry + ex;
+        carry += tot;
+    }
+}
+
+// Stable partition of one chunk into the other index buffer, and the
+// children's box and centroid bounds. A thread takes kPerThread consecutive
+// primitives, so one scan of the per-thread left counts ranks the chunk.
+__global__ __launch_bounds__(kTopThreads) void k_top_scatter(Build b, int cur) {
+    __shared__ int lds[kTopThreads / 64 * 12 + 1];
+    if ((int)blockIdx.x >= b.count[1]) return;
+    const int j = find_seg(b.chunkBase[cur], b.count[0], blockIdx.x);
+    const Seg g = b.act[cur][j];
+    const int p0 = ((int)blockIdx.x - b.chunkBase[cur][j]) * kChunk;
+    const int ax = b.sAxis[j], bin = b.sBin[j], nl = b.sNl[j];
+    const int* nc = b.actAcc[cur] + 12 * (size_t)j + 6;
+    const float cmin = ax >= 0 ? o2f(nc[ax]) : 0.f, cmax = ax >= 0 ? o2f(nc[3 + ax]) : 0.f;
+    const int* idx = b.idx[cur] + g.s;
+    const int i0 = p0 + (int)threadIdx.x * kPerThread;
+    int p[kPerThread];
+    unsigned int lm = 0;
+    BoundsAcc<kTopThreads> accL, accR;
+    accL.init();
+    accR.init();
 #pragma unroll
-            for (int a = 0; a < 3; a++) {
-                atomicMin(&d[a], f2o(pb[a])); atomicMax(&d[3 + a], f2o(pb[3 + a]));
-                atomicMin(&d[6 + a], f2o(cv[a])); atomicMax(&d[9 + a], f2o(cv[a]));
-            }
-        }
-        leftBefore += __popcll(lm);
-    }
-    __syncthreads();
-    if (lane < 24) {
-        const int child = lane < 12 ? L : R, k = lane % 12;
-        int* dst = (k < 6 ? b.nbox : b.ncen) + 6 * (size_t)child + (k % 6);
-        *dst = cb[lane];
-    }
-    if (lane == 0) { b.small[L] = 1; b.small[R] = 1; }
-}
-
-__global__ void k_flags(Build b) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= b.n) return;
-    const int node = b.pnode[i];
-    int f = 0;
-    if (b.ncnt[node] > b.maxLeaf && b.ncnt[node] > kSmall) {
-        const int slot = b.nodeSlot[node];
-        const int ax = b.sAxis[slot];
+    for (int k = 0; k < kPerThread; k++) p[k] = i0 + k < g.c ? idx[i0 + k] : -1;
+#pragma unroll
+    for (int k = 0; k < kPerThread; k++) {
+        if (p[k] < 0) continue;
+        float v[6];
+        load_box(b.pbox, p[k], v);
+        bool left;
         if (ax < 0) {
-            f = (i - b.ns[node]) < b.sNl[slot];
+            left = i0 + k < nl;
         } else {
-            const float4 c = b.cen[b.idx[i]];
-            const float cv = ax == 0 ? c.x : (ax == 1 ? c.y : c.z);
-            const int* nc = b.ncen + 6 * (size_t)node;
-            f = bin_of(cv, o2f(nc[ax]), o2f(nc[3 + ax])) <= b.sBin[slot];
+            const float c = ax == 0 ? centroid(v, 0) : (ax == 1 ? centroid(v, 1) : centroid(v, 2));
+            left = bin_of(c, cmin, cmax) <= bin;
         }
+        if (left) { lm |= 1u << k; accL.add(v); }
+        else accR.add(v);
     }
-    b.flag[i] = f;
-}
-
-__global__ void k_scatter(Build b) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= b.n) return;
-    const int node = b.pnode[i];
-    if (b.ncnt[node] <= b.maxLeaf) {
-        b.idx2[i] = b.idx[i];
-        b.pnode2[i] = node;
-        return;
+    int tot;
+    int before = b.chunkLeft[blockIdx.x] + rts::block_exclusive_scan<kTopThreads>(__popc(lm), lds, &tot);
+    int* o = b.idx[cur ^ 1] + g.s;
+#pragma unroll
+    for (int k = 0; k < kPerThread; k++) {
+        if (p[k] < 0) continue;
+        if (lm >> k & 1) { o[before] = p[k]; before++; }
+        else o[nl + (i0 + k - before)] = p[k];
     }
-    if (b.ncnt[node] <= kSmall) return;          // partitioned by k_small_level
-    const int slot = b.nodeSlot[node];
-    const int s = b.ns[node], nl = b.sNl[slot];
-    const int lr = b.rank[i] - b.rank[s];
-    int pos, child;
-    if (b.flag[i]) { pos = s + lr; child = b.nleft[node]; }
-    else { pos = s + nl + ((i - s) - lr); child = b.nright[node]; }
-    b.idx2[pos] = b.idx[i];
-    b.pnode2[pos] = child;
+    accL.flush(lds, b.childAcc + 24 * (size_t)j);
+    accR.flush(lds, b.childAcc + 24 * (size_t)j + 12);
 }
 
-__global__ void k_next_active(Build b, int first, int count, const int* rank, int* act2) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    const int node = first + i;
-    if (b.ncnt[node] > b.maxLeaf) {
-        act2[rank[i]] = node;
-        b.nodeSlot[node] = rank[i];
-    }
-}
-
-__global__ void k_active_flags(const int* ncnt, int first, int count, int maxLeaf, int* f) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < count) f[i] = ncnt[first + i] > maxLeaf;
-}
-
-// ------------------------------- pre-order renumbering -----------------------
-__global__ void k_sizes(const int* nleft, const int* nright, int* size, int first, int count) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    const int v = first + i;
-    size[v] = nleft[v] < 0 ? 1 : 1 + size[nleft[v]] + size[nright[v]];
-}
-
-// Pre-order positions of the roots: trees one after the other.
-__global__ void k_root_pre(const int* size, int* pre, int numScenes) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    int acc = 0;
-    for (int s = 0; s < numScenes; s++) { pre[s] = acc; acc += size[s]; }
-}
-
-__global__ void k_root4(const int* pre, const int* b4id, int numScenes, int* root4) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < numScenes) root4[s] = b4id[pre[s]];
-}
-
-__global__ void k_preorder(const int* nleft, const int* nright, const int* size, int* pre, int first, int count) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    const int v = first + i;
-    if (nleft[v] < 0) return;
-    pre[nleft[v]] = pre[v] + 1;
-    pre[nright[v]] = pre[v] + 1 + size[nleft[v]];
-}
-
-// Pre-order BVH2 (rt::Node2 layout: box[6], left, right, triStart, triCount)
-// and the collapse's starting state: every tree root presents itself as one
-// slot (assign 1) and is the head of its BVH4 root at BVH4 level 0.
-__global__ void k_emit_bvh2(Build b, const int* pre, int count, rt::Node2* out, int* head, int* assign, int* lev4) {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= count) return;
-    const int p = pre[v];
-    rt::Node2 nd;
-    for (int k = 0; k < 3; k++) {
-        nd.box.mn[k] = o2f(b.nbox[6 * (size_t)v + k]);
-        nd.box.mx[k] = o2f(b.nbox[6 * (size_t)v + 3 + k]);
-    }
-    const bool leaf = b.nleft[v] < 0;
-    nd.left = leaf ? 0 : pre[b.nleft[v]];
-    nd.right = leaf ? 0 : pre[b.nright[v]];
-    nd.triStart = leaf ? b.ns[v] : 0;
-    nd.triCount = leaf ? b.ncnt[v] : 0;
-    out[p] = nd;
-    head[p] = 0;
-    assign[p] = b.ndepth[v] == 0 ? 1 : 0;
-    lev4[p] = 0;
-}
-
+// ------------------------------- collapse ------------------------------------
 // --- BVH2 -> BVH4 collapse (same rule and float operation order as the
 // oracle's collapse_costs / collapse_split / collapse_gather) ---
-// cost[p] = (c1, c2, c3, c4): least total area of the BVH4 nodes needed to
-// present subtree p as k slots; a leaf is one free slot; for an internal p,
-// g_k = min over a of c_a(left) + c_{k-a}(right), c1 = area(p) + min g_k.
+// cost = (c1, c2, c3, c4): least total area of the BVH4 nodes needed to
+// present a subtree as k slots; a leaf is one free slot; for an internal node,
+// g_k = min over a of c_a(left) + c_{k-a}(right), c1 = area + min g_k.
 constexpr float kCostInf = 3.0e38f;
 
-__global__ void k_collapse_cost(const rt::Node2* n2, const int* pre, int first, int count, float4* cost) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    const int p = pre[first + i];
-    const rt::Node2& nd = n2[p];
-    if (nd.triCount > 0) { cost[p] = make_float4(0.0f, kCostInf, kCostInf, kCostInf); return; }
-    const float4 L = cost[nd.left], R = cost[nd.right];
+__device__ __forceinline__ float4 leaf_cost() { return make_float4(0.0f, kCostInf, kCostInf, kCostInf); }
+__device__ __forceinline__ float4 node_cost(float ar, const float4& L, const float4& R) {
     const float l[4] = {L.x, L.y, L.z, L.w}, r[4] = {R.x, R.y, R.z, R.w};
     float g[5] = {kCostInf, kCostInf, kCostInf, kCostInf, kCostInf};
+#pragma unroll
     for (int k = 2; k <= 4; k++)
+#pragma unroll
         for (int a = 1; a < k; a++) {
             const float x = l[a - 1] + r[k - a - 1];
             if (x < g[k]) g[k] = x;
@@ -553,50 +672,376 @@ __global__ void k_collapse_cost(const rt::Node2* n2, const int* pre, int first, 
     float best = g[2];
     if (g[3] < best) best = g[3];
     if (g[4] < best) best = g[4];
-    const float ar = area(nd.box.mn[0], nd.box.mn[1], nd.box.mn[2], nd.box.mx[0], nd.box.mx[1], nd.box.mx[2]);
-    cost[p] = make_float4(ar + best, g[2], g[3], g[4]);
+    return make_float4(ar + best, g[2], g[3], g[4]);
 }
 
-// Left slot count of subtree p presented as m slots (ties: the smaller).
-__device__ __forceinline__ int collapse_left(const rt::Node2& nd, const float4* cost, int m) {
-    const float4 L = cost[nd.left], R = cost[nd.right];
-    const float l[4] = {L.x, L.y, L.z, L.w}, r[4] = {R.x, R.y, R.z, R.w};
-    int ba = 1;
-    float bx = kCostInf;
-    for (int a = 1; a < m; a++) {
-        const float x = l[a - 1] + r[m - a - 1];
-        if (x < bx) { bx = x; ba = a; }
-    }
-    return ba;
-}
-
-// Top-down, one BVH2 level per launch: an internal node presented as one
-// slot heads a BVH4 node of its cheapest width k (ties: the narrower) and
-// hands its children their slot counts; a node presented as m >= 2 slots is
-// dissolved into its parent's node and splits m between its children. lev4:
-// BVH4 level of a head / of the node whose slots a dissolved node fills.
-__global__ void k_collapse_assign(const rt::Node2* n2, const int* pre, int first, int count, const float4* cost,
-                                  int* assign, int* head, int* lev4) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    const int p = pre[first + i];
-    const rt::Node2& nd = n2[p];
-    const int m = assign[p];
-    if (nd.triCount > 0 || m == 0) return;
-    int k = m, cl = lev4[p];
+// Top-down step at an internal node presented as m slots at BVH4 level lev
+// (m 0: not reached): a node presented as one slot heads a BVH4 node of its
+// cheapest width (ties: the narrower); one presented as m >= 2 slots is
+// dissolved into its parent's node. Returns the children's (slots, level) and
+// whether the node is a head. lev: BVH4 level of a head / of the node whose
+// slots a dissolved node fills.
+__device__ __forceinline__ bool assign_slots(const float4& c, const float4& L, const float4& R, int m, int lev, int2& al,
+                                             int2& ar) {
+    al = ar = make_int2(0, 0);
+    if (m == 0) return false;
+    int k = m, cl = lev;
     if (m == 1) {
-        const float4 c = cost[p];
         k = 2;
         if (c.z < c.y) k = 3;
         if (c.w < (k == 3 ? c.z : c.y)) k = 4;
-        head[p] = 1;
-        cl = lev4[p] + 1;
+        cl = lev + 1;
     }
-    const int a = collapse_left(nd, cost, k);
-    assign[nd.left] = a;
-    assign[nd.right] = k - a;
-    lev4[nd.left] = cl;
-    lev4[nd.right] = cl;
+    // left slots of k (ties: the smaller)
+    const float l[4] = {L.x, L.y, L.z, L.w}, r[4] = {R.x, R.y, R.z, R.w};
+    int ba = 1;
+    float bx = kCostInf;
+#pragma unroll
+    for (int a = 1; a < 4; a++) {
+        if (a >= k) break;
+        const int o = k - a - 1;
+        const float x = l[a - 1] + (o == 0 ? r[0] : (o == 1 ? r[1] : r[2]));
+        if (x < bx) { bx = x; ba = a; }
+    }
+    al = make_int2(ba, cl);
+    ar = make_int2(k - ba, cl);
+    return m == 1;
+}
+
+// ------------------------------- subtrees ------------------------------------
+// A whole subtree per workgroup: primitive boxes in LDS, level by level, one
+// wave per node (nodes of at most 64 primitives stay in registers: one
+// primitive per lane). Leaves write their part of the final order at once.
+// MAXQ: most active nodes of a level (kSmall / (maxLeaf + 1)).
+constexpr int kSubThreads = 512, kSubWaves = kSubThreads / 64;
+
+template <int MAXQ>
+struct SubLds {
+    float box[6][kSmall];
+    unsigned short perm[2][kSmall];
+    unsigned int seg[2][MAXQ];                 // start | count << 12
+    unsigned short rec[2][MAXQ];
+    float pA[2][MAXQ];                         // area of the node's box
+    int bins[kSubWaves][kSlotInts];
+    int qn[2], recs;
+};
+
+template <int MAXQ>
+__global__ __launch_bounds__(kSubThreads) void k_subtree(Build b) {
+    __shared__ __attribute__((aligned(16))) SubLds<MAXQ> S;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const Small& sm = b.small[blockIdx.x];
+    const Seg g = sm.g;
+    const int* idxIn = b.idx[sm.buf] + g.s;
+    int* ordered = b.ordered + g.s;
+    int* leafFlag = b.leafFlag + g.s;
+    Rec* rec = b.rec + 2 * (size_t)g.s;
+    unsigned short* lvl = b.lvl + 2 * (size_t)g.s;
+    float rb[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) rb[k] = o2f(sm.bounds[k]);
+    const bool rootLeaf = g.c <= b.maxLeaf;
+    for (int i = tid; i < g.c; i += kSubThreads) {
+        const int p = idxIn[i];
+        float v[6];
+        load_box(b.pbox, p, v);
+#pragma unroll
+        for (int k = 0; k < 6; k++) S.box[k][i] = v[k];
+        S.perm[0][i] = (unsigned short)i;
+        if (rootLeaf) { ordered[i] = p; leafFlag[i] = i == 0; }
+    }
+    if (tid == 0) {
+        rec[0].a = make_float4(rb[0], rb[1], rb[2], rb[3]);
+        rec[0].b = make_float2(rb[4], rb[5]);
+        rec[0].s = g.s; rec[0].lt = g.lt;
+        if (rootLeaf) { rec[0].child = -1; rec[0].m = g.c; }
+        S.recs = 1;
+        S.qn[0] = rootLeaf ? 0 : 1;
+        S.qn[1] = 0;
+        S.seg[0][0] = (unsigned int)g.c << 12;
+        S.rec[0][0] = 0;
+        S.pA[0][0] = area(rb[0], rb[1], rb[2], rb[3], rb[4], rb[5]);
+        lvl[0] = 0;
+        lvl[1] = 1;
+    }
+    __syncthreads();
+    int level = 0;
+    int* const lb = S.bins[w];
+    for (int cur = 0;; cur ^= 1, level++) {
+        const int qn = S.qn[cur];
+        if (qn == 0) break;
+        const unsigned short* perm = S.perm[cur];
+        unsigned short* perm2 = S.perm[cur ^ 1];
+        for (int j = w; j < qn; j += kSubWaves) {
+            const unsigned int sg = S.seg[cur][j];
+            const int start = __builtin_amdgcn_readfirstlane((int)(sg & 0xfffu));
+            const int cnt = __builtin_amdgcn_readfirstlane((int)(sg >> 12));
+            const int rid = __builtin_amdgcn_readfirstlane((int)S.rec[cur][j]);
+            const float pA = S.pA[cur][j];
+            const bool one = cnt <= 64;            // the node's primitives fit the wave's lanes
+            int myp = 0;
+            float v[6] = {0, 0, 0, 0, 0, 0};
+            // centroid bounds
+            int cb[6] = {kOrdPosInf, kOrdPosInf, kOrdPosInf, kOrdNegInf, kOrdNegInf, kOrdNegInf};
+            for (int i = lane; i < cnt; i += 64) {
+                myp = perm[start + i];
+#pragma unroll
+                for (int k = 0; k < 6; k++) v[k] = S.box[k][myp];
+#pragma unroll
+                for (int a = 0; a < 3; a++) {
+                    const int c = f2o(centroid(v, a));
+                    cb[a] = min(cb[a], c); cb[3 + a] = max(cb[3 + a], c);
+                }
+            }
+            float cmin[3], cmax[3];
+            bool use[3];
+#pragma unroll
+            for (int a = 0; a < 3; a++) {
+                cmin[a] = o2f(wave_min(cb[a])); cmax[a] = o2f(wave_max(cb[3 + a]));
+                use[a] = !(cmax[a] - cmin[a] < 1e-8f);
+            }
+            // bins
+            for (int i = lane; i < kSlotInts; i += 64) {
+                const int f = i % kBinInts;
+                lb[i] = f < 3 ? kOrdPosInf : (f < 6 ? kOrdNegInf : 0);
+            }
+            wave_lds_fence();
+            int mb[3] = {0, 0, 0};
+            for (int i = lane; i < cnt; i += 64) {
+                if (!one) {
+                    myp = perm[start + i];
+#pragma unroll
+                    for (int k = 0; k < 6; k++) v[k] = S.box[k][myp];
+                }
+#pragma unroll
+                for (int a = 0; a < 3; a++) {
+                    if (!use[a]) continue;
+                    mb[a] = bin_of(centroid(v, a), cmin[a], cmax[a]);
+                    int* d = lb + a * kAxisInts + mb[a] * kBinInts;
+#pragma unroll
+                    for (int e = 0; e < 3; e++) { atomicMin(&d[e], f2o(v[e])); atomicMax(&d[3 + e], f2o(v[3 + e])); }
+                    atomicAdd(&d[6], 1);
+                }
+            }
+            wave_lds_fence();
+            Sah r;
+            sah_wave(lb, pA, use[0], use[1], use[2], cnt, r);
+            const int ax = r.axis, bin = r.bin, nl = r.nl, nr = cnt - nl;
+            const bool leafL = nl <= b.maxLeaf, leafR = nr <= b.maxLeaf;
+            // stable partition
+            const bool exact = ax < 0 || r.nan;    // child boxes by reduction (see below)
+            int xb[12];
+#pragma unroll
+            for (int k = 0; k < 12; k++) xb[k] = (k % 6) < 3 ? kOrdPosInf : kOrdNegInf;
+            const float smin = ax == 1 ? cmin[1] : (ax == 2 ? cmin[2] : cmin[0]);
+            const float smax = ax == 1 ? cmax[1] : (ax == 2 ? cmax[2] : cmax[0]);
+            int leftBefore = 0;
+            for (int base = 0; base < cnt; base += 64) {
+                const int i = base + lane;
+                const bool valid = i < cnt;
+                bool left = false;
+                if (valid) {
+                    if (!one) {
+                        myp = perm[start + i];
+                        if (ax >= 0) mb[0] = bin_of((S.box[ax][myp] + S.box[3 + ax][myp]) * .5f, smin, smax);
+                    } else {
+                        mb[0] = ax == 1 ? mb[1] : (ax == 2 ? mb[2] : mb[0]);
+                    }
+                    left = ax < 0 ? i < nl : mb[0] <= bin;
+                    if (exact) {
+#pragma unroll
+                        for (int e = 0; e < 3; e++) {
+                            const int lo = f2o(S.box[e][myp]), hi = f2o(S.box[3 + e][myp]);
+                            if (left) { xb[e] = min(xb[e], lo); xb[3 + e] = max(xb[3 + e], hi); }
+                            else { xb[6 + e] = min(xb[6 + e], lo); xb[9 + e] = max(xb[9 + e], hi); }
+                        }
+                    }
+                }
+                const uint64_t lm = __ballot(valid && left);
+                const int lr = leftBefore + __popcll(lm & ((1ull << lane) - 1ull));
+                if (valid) {
+                    const int pos = start + (left ? lr : nl + (i - lr));
+                    if (left ? leafL : leafR) {
+                        ordered[pos] = idxIn[myp];
+                        leafFlag[pos] = pos == start + (left ? 0 : nl);
+                    } else {
+                        perm2[pos] = (unsigned short)myp;
+                    }
+                }
+                leftBefore += __popcll(lm);
+            }
+            // children: their boxes are the winning candidate's; a middle
+            // split has none, and with a NaN box the scans (which skip NaN)
+            // could differ from a reduction over ordered integers
+            float cx[12];
+            if (exact) {
+#pragma unroll
+                for (int k = 0; k < 12; k++) cx[k] = o2f((k % 6) < 3 ? wave_min(xb[k]) : wave_max(xb[k]));
+            } else {
+#pragma unroll
+                for (int k = 0; k < 6; k++) { cx[k] = lane_of(r.L[k], r.src); cx[6 + k] = lane_of(r.R[k], r.src); }
+            }
+            int base = 0, qpos = 0;
+            if (lane == 0) {
+                base = atomicAdd(&S.recs, 2);
+                qpos = atomicAdd(&S.qn[cur ^ 1], (leafL ? 0 : 1) + (leafR ? 0 : 1));
+            }
+            base = __builtin_amdgcn_readfirstlane(base);
+            qpos = __builtin_amdgcn_readfirstlane(qpos);
+            if (lane < 2) {                        // lane 0: left child, lane 1: right child
+                const bool R = lane == 1, leaf = R ? leafR : leafL;
+                const int cs = R ? start + nl : start, cc = R ? nr : nl;
+                const float x0 = R ? cx[6] : cx[0], x1 = R ? cx[7] : cx[1], x2 = R ? cx[8] : cx[2];
+                const float x3 = R ? cx[9] : cx[3], x4 = R ? cx[10] : cx[4], x5 = R ? cx[11] : cx[5];
+                Rec& c = rec[base + lane];
+                const int lt = rec[rid].lt;
+                c.a = make_float4(x0, x1, x2, x3);
+                c.b = make_float2(x4, x5);
+                c.s = g.s + cs;
+                c.lt = R ? lt : lt + 1;
+                if (leaf) {
+                    c.child = -1; c.m = cc;
+                } else {
+                    const int q = qpos + (R && !leafL ? 1 : 0);
+                    S.seg[cur ^ 1][q] = (unsigned int)cs | (unsigned int)cc << 12;
+                    S.rec[cur ^ 1][q] = (unsigned short)(base + lane);
+                    S.pA[cur ^ 1][q] = area(x0, x1, x2, x3, x4, x5);
+                }
+                if (lane == 0) { rec[rid].child = base; rec[rid].m = g.s + start + nl; }
+            }
+        }
+        __syncthreads();
+        if (tid == 0) { S.qn[cur] = 0; lvl[level + 2] = (unsigned short)S.recs; }
+        __syncthreads();
+    }
+    // collapse costs, bottom-up; levels [0, level] hold records
+    const int total = S.recs;
+    __syncthreads();
+    float4* cst = (float4*)&S;
+    static_assert(sizeof(SubLds<MAXQ>) >= (2 * kSmall - 1) * sizeof(float4), "collapse costs fit the LDS");
+    float4* gc = b.cost + 2 * (size_t)g.s;
+    for (int L = level; L >= 0; L--) {
+        const int r0 = lvl[L], r1 = L == level ? total : lvl[L + 1];
+        for (int k = r0 + tid; k < r1; k += kSubThreads) {
+            const Rec& rc = rec[k];
+            float4 c = leaf_cost();
+            if (rc.child >= 0)
+                c = node_cost(area(rc.a.x, rc.a.y, rc.a.z, rc.a.w, rc.b.x, rc.b.y), cst[rc.child], cst[rc.child + 1]);
+            cst[k] = c;
+            gc[k] = c;
+        }
+        __syncthreads();
+    }
+    if (tid == 0) {
+        lvl[level + 1] = (unsigned short)total;
+        b.smallCost[blockIdx.x] = cst[0];
+        b.small[blockIdx.x].levels = level + 1;
+    }
+}
+
+// ------------------------------- numbering and emission -----------------------
+// depth: BVH4 levels, BVH2 levels
+struct Emit { rt::Node2* n2; int* head; int* assign; int* depth; };
+
+__device__ __forceinline__ void emit_node(const Emit& e, int p, const float (&bx)[6], int left, int right, int triStart,
+                                          int triCount, bool head, int m) {
+    rt::Node2 nd;
+#pragma unroll
+    for (int k = 0; k < 3; k++) { nd.box.mn[k] = bx[k]; nd.box.mx[k] = bx[3 + k]; }
+    nd.left = left; nd.right = right; nd.triStart = triStart; nd.triCount = triCount;
+    e.n2[p] = nd;
+    e.head[p] = head ? 1 : 0;
+    e.assign[p] = m;
+}
+
+// The top nodes: costs bottom-up, then slots top-down and their BVH2 nodes
+// (one workgroup; a few thousand nodes at most in a balanced tree).
+__global__ __launch_bounds__(1024) void k_top_collapse(Build b, Emit e, int levels) {
+    __shared__ int dmax;
+    auto cost_of = [&](int ref) { return ref >= 0 ? b.topCost[ref] : b.smallCost[-1 - ref]; };
+    if (threadIdx.x == 0) dmax = 0;
+    for (int L = levels - 1; L >= 0; L--) {
+        const int t0 = b.topLevel[L], t1 = b.topLevel[L + 1];
+        for (int k = t0 + (int)threadIdx.x; k < t1; k += 1024) {
+            const Top& t = b.top[k];
+            b.topCost[k] = node_cost(area(t.box[0], t.box[1], t.box[2], t.box[3], t.box[4], t.box[5]), cost_of(t.left),
+                                     cost_of(t.right));
+        }
+        __syncthreads();
+    }
+    auto set = [&](int ref, int2 a) { if (ref >= 0) b.topAsg[ref] = a; else b.smallAsg[-1 - ref] = a; };
+    for (int k = threadIdx.x; k < b.numScenes; k += 1024) set(b.rootRef[k], make_int2(1, 0));
+    __syncthreads();
+    int depth = 0;
+    for (int L = 0; L < levels; L++) {
+        const int t0 = b.topLevel[L], t1 = b.topLevel[L + 1];
+        for (int k = t0 + (int)threadIdx.x; k < t1; k += 1024) {
+            const Top& t = b.top[k];
+            const int2 a = b.topAsg[k];
+            int2 al, ar;
+            const bool head = assign_slots(b.topCost[k], cost_of(t.left), cost_of(t.right), a.x, a.y, al, ar);
+            set(t.left, al);
+            set(t.right, ar);
+            const int p = pre_of(b, t.s, t.lt, t.tree);
+            emit_node(e, p, t.box, p + 1, pre_of(b, t.m, t.lt, t.tree), 0, 0, head, a.x);
+            if (head) depth = max(depth, a.y + 1);
+        }
+        __syncthreads();
+    }
+    atomicMax(&dmax, depth);
+    __syncthreads();
+    if (threadIdx.x == 0 && dmax) atomicMax(e.depth, dmax);
+}
+
+// A subtree's slots top-down and its BVH2 nodes.
+__global__ __launch_bounds__(kThreads) void k_sub_emit(Build b, Emit e) {
+    __shared__ unsigned int asg[2 * kSmall];      // slots | BVH4 level << 4
+    __shared__ int dmax;
+    const Small& sm = b.small[blockIdx.x];
+    const Seg g = sm.g;
+    const Rec* rec = b.rec + 2 * (size_t)g.s;
+    const float4* cost = b.cost + 2 * (size_t)g.s;
+    const unsigned short* lvl = b.lvl + 2 * (size_t)g.s;
+    const int levels = sm.levels;
+    if (threadIdx.x == 0) {
+        const int2 a = b.smallAsg[blockIdx.x];
+        asg[0] = (unsigned int)a.x | (unsigned int)a.y << 4;
+        dmax = 0;
+    }
+    __syncthreads();
+    int depth = 0;
+    for (int L = 0; L < levels; L++) {
+        const int r0 = lvl[L], r1 = lvl[L + 1];
+        for (int k = r0 + (int)threadIdx.x; k < r1; k += kThreads) {
+            const Rec rc = rec[k];
+            const float bx[6] = {rc.a.x, rc.a.y, rc.a.z, rc.a.w, rc.b.x, rc.b.y};
+            const int p = pre_of(b, rc.s, rc.lt, g.tree);
+            const int m = (int)(asg[k] & 15u), lev = (int)(asg[k] >> 4);
+            if (rc.child < 0) {
+                emit_node(e, p, bx, 0, 0, rc.s, rc.m, false, m);
+            } else {
+                int2 al, ar;
+                const bool head = assign_slots(cost[k], cost[rc.child], cost[rc.child + 1], m, lev, al, ar);
+                asg[rc.child] = (unsigned int)al.x | (unsigned int)al.y << 4;
+                asg[rc.child + 1] = (unsigned int)ar.x | (unsigned int)ar.y << 4;
+                emit_node(e, p, bx, p + 1, pre_of(b, rc.m, rc.lt, g.tree), 0, 0, head, m);
+                if (head) depth = max(depth, lev + 1);
+            }
+        }
+        __syncthreads();
+    }
+    if (depth) atomicMax(&dmax, depth);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        atomicMax(&e.depth[0], dmax);
+        atomicMax(&e.depth[1], sm.level + levels);
+    }
+}
+
+// BVH4 root of each tree (a root is the head at its pre-order position).
+__global__ void k_root4(Build b, const int* b4id, int* root4) {
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s < b.numScenes) root4[s] = b4id[pre_of(b, b.off[s], 0, s)];
 }
 
 __device__ __forceinline__ uint16_t h_bits(_Float16 h) { return __builtin_bit_cast(uint16_t, h); }
@@ -629,8 +1074,8 @@ __device__ __forceinline__ int32_t leaf_code(int first, int count) { return -((f
 // exclusive count of heads before p, i.e. the node's pre-order BVH4 index.
 // Its slots are the nodes of assign 1 below it, reached through dissolved
 // nodes (assign >= 2), left to right, so they stay in BVH2 pre-order.
-__global__ void k_emit_bvh4(const rt::Node2* n2, const int* head, const int* b4id, const int* assign,
-                            const int* lev4, int count, uint4* out, int* depth4) {
+__global__ void k_emit_bvh4(const rt::Node2* n2, const int* head, const int* b4id, const int* assign, int count,
+                            uint4* out) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= count || !head[p]) return;
     const rt::Node2& nd = n2[p];
@@ -669,11 +1114,10 @@ __global__ void k_emit_bvh4(const rt::Node2* n2, const int* head, const int* b4i
     o[2] = make_uint4(hz[0] | (uint32_t)hz[1] << 16, hz[2] | (uint32_t)hz[3] << 16, hz[4] | (uint32_t)hz[5] << 16,
                       hz[6] | (uint32_t)hz[7] << 16);
     o[3] = make_uint4((uint32_t)child[0], (uint32_t)child[1], (uint32_t)child[2], (uint32_t)child[3]);
-    atomicMax(depth4, lev4[p] + 1);
 }
 
 // A tree whose root is a leaf (n <= maxLeaf): one BVH4 node with one slot.
-__global__ void k_emit_leaf_root(const rt::Node2* n2, uint4* out, int* depth4) {
+__global__ void k_emit_leaf_root(const rt::Node2* n2, uint4* out) {
     const rt::Node2& r = n2[0];
     uint16_t h[3][8];
     for (int a = 0; a < 3; a++) {
@@ -685,7 +1129,6 @@ __global__ void k_emit_leaf_root(const rt::Node2* n2, uint4* out, int* depth4) {
         out[a] = make_uint4(h[a][0] | (uint32_t)h[a][1] << 16, h[a][2] | (uint32_t)h[a][3] << 16,
                             h[a][4] | (uint32_t)h[a][5] << 16, h[a][6] | (uint32_t)h[a][7] << 16);
     out[3] = make_uint4((uint32_t)leaf_code(r.triStart, r.triCount), 0xffffffffu, 0xffffffffu, 0xffffffffu);
-    *depth4 = 1;
 }
 
 // Leaf-order triangles {v0.xyz, bits(id)}, {v1.xyz, 0}, {v2.xyz, 0} and the
@@ -841,21 +1284,46 @@ static double now_ms() {
     return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now().time_since_epoch()).count();
 }
 
-struct DevBuf {
-    std::vector<void*> ptrs;
-    template <class T> T* get(size_t count) {
-        void* p = nullptr;
-        if (hipMalloc(&p, std::max<size_t>(count, 1) * sizeof(T)) != hipSuccess) return nullptr;
-        ptrs.push_back(p);
-        return (T*)p;
+// One device allocation cut into pieces. The build needs some thirty arrays;
+// each hipFree of a large one costs 0.3 ms, one for all of them the same.
+struct Slab {
+    struct Piece { void** p; size_t bytes; };
+    std::vector<Piece> want;
+    void* base = nullptr;
+    template <class T> void add(T** p, size_t count) {
+        want.push_back({(void**)p, (std::max<size_t>(count, 1) * sizeof(T) + 255) & ~size_t(255)});
     }
-    ~DevBuf() { for (void* p : ptrs) hipFree(p); }
+    bool alloc() {
+        size_t total = 0;
+        for (const Piece& w : want) total += w.bytes;
+        if (hipMalloc(&base, total) != hipSuccess) { base = nullptr; return false; }
+        char* c = (char*)base;
+        for (const Piece& w : want) { *w.p = c; c += w.bytes; }
+        return true;
+    }
+    ~Slab() { if (base) hipFree(base); }
 };
 
 #define BUILD_CHECK(cond, msg)              \
     do {                                    \
         if (!(cond)) { set_error("%s", msg); return -1; } \
     } while (0)
+
+int mesh_bounds(const float* d_tris, int n, hipStream_t s, float* mn, float* mx) {
+    unsigned long long* key = nullptr;
+    if (hipMalloc((void**)&key, 128) != hipSuccess) { set_error("mesh bounds: out of device memory"); return -1; }
+    float* out = (float*)(key + 8);
+    float h[6];
+    hipLaunchKernelGGL(rtb::k_keys_init, dim3(1), dim3(64), 0, s, key);
+    hipLaunchKernelGGL(rtb::k_mesh_keys, dim3(std::min((n + 511) / 512, 1024)), dim3(rtb::kTopThreads), 0, s, d_tris, n, key);
+    hipLaunchKernelGGL(rtb::k_mesh_bounds, dim3(1), dim3(64), 0, s, d_tris, key, out);
+    hipError_t e = hipMemcpyAsync(h, out, sizeof h, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    hipFree(key);
+    if (e != hipSuccess) { set_error("mesh bounds: %s", hipGetErrorString(e)); return -1; }
+    for (int a = 0; a < 3; a++) { mn[a] = h[a]; mx[a] = h[3 + a]; }
+    return 0;
+}
 
 // Builds the BVH on the device from d_tris (n x 9 floats, original order).
 // Outputs (device, allocated here): nodes4 (numNodes4 x 64 B), leaf-order
@@ -869,165 +1337,162 @@ int gpu_build(const float* d_tris, int n, int maxLeaf, hipStream_t s, GpuBVH& ou
         double t0;
         ~Report() { if (verbose()) fprintf(stderr, "[CudaBVH] gpu_build: %.2f ms incl. workspace free\n", now_ms() - t0); }
     } report{tBegin};
-    DevBuf tmp;
     const int R = numScenes;
-    std::vector<int> hOff = sceneOff ? std::vector<int>(sceneOff, sceneOff + R + 1) : std::vector<int>{0, n};
-    std::vector<int> hSlots(R, -1);
-    int m = 0;
+    // host tables: scene offsets, then chunks of kChunk primitives before each scene
+    std::vector<int> tab(2 * (size_t)(R + 1));
+    int* hOff = tab.data();
+    int* hBase = tab.data() + R + 1;
+    int largest = 0, big0 = 0;
+    for (int k = 0; k <= R; k++) hOff[k] = sceneOff ? sceneOff[k] : k * n;
+    hBase[0] = 0;
     for (int k = 0; k < R; k++) {
         const int c = hOff[k + 1] - hOff[k];
         if (c <= 0 || (R > 1 && c <= maxLeaf)) {
             set_error("gpu build: scene %d has %d primitives (a batch needs more than %d per scene)", k, c, maxLeaf);
             return -1;
         }
-        if (c > maxLeaf) hSlots[k] = m++;
+        largest = std::max(largest, c);
+        big0 += c > kSmall;
+        hBase[k + 1] = hBase[k] + (c + kChunk - 1) / kChunk;
     }
-    int* dOff = tmp.get<int>(R + 1);
-    int* dSlots = tmp.get<int>(R);
-    BUILD_CHECK(dOff && dSlots, "gpu build: out of device memory");
-    if (hipMemcpyAsync(dOff, hOff.data(), (R + 1) * sizeof(int), hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipMemcpyAsync(dSlots, hSlots.data(), R * sizeof(int), hipMemcpyHostToDevice, s) != hipSuccess) {
-        set_error("gpu build: upload failed");
-        return -1;
-    }
+    const size_t N = (size_t)n;
     Build b{};
-    b.n = n; b.maxLeaf = maxLeaf;
-    const size_t cap = 2 * (size_t)n;
-    float* pbox = tmp.get<float>(6 * (size_t)n);
-    float4* cen = tmp.get<float4>(n);
-    b.pbox = pbox; b.cen = cen;
-    b.idx = tmp.get<int>(n); b.pnode = tmp.get<int>(n);
-    b.idx2 = tmp.get<int>(n); b.pnode2 = tmp.get<int>(n);
-    b.flag = tmp.get<int>(n + 1); b.rank = tmp.get<int>(n + 1);
-    b.nbox = tmp.get<int>(6 * cap); b.ncen = tmp.get<int>(6 * cap);
-    b.ns = tmp.get<int>(cap); b.ncnt = tmp.get<int>(cap);
-    b.nleft = tmp.get<int>(cap); b.nright = tmp.get<int>(cap); b.ndepth = tmp.get<int>(cap);
-    b.nodeSlot = tmp.get<int>(cap);
-    b.small = tmp.get<int>(cap);
-    b.bigSlot = tmp.get<int>(cap);
-    b.bigCount = tmp.get<int>(1);
-    const int maxBig = n / (kSmall + 1) + R + 1;
-    b.bins = tmp.get<int>((size_t)maxBig * kSlotInts);
-    b.act = tmp.get<int>(n); int* act2 = tmp.get<int>(n);
-    b.sAxis = tmp.get<int>(n); b.sBin = tmp.get<int>(n); b.sNl = tmp.get<int>(n);
-    int* tiles = tmp.get<int>(scan_tiles_needed((int)cap) + 8);
-    int* dcount = tmp.get<int>(4);
-    BUILD_CHECK(pbox && cen && b.idx && b.pnode && b.idx2 && b.pnode2 && b.flag && b.rank && b.nbox && b.ncen &&
-                b.ns && b.ncnt && b.nleft && b.nright && b.ndepth && b.nodeSlot && b.small && b.bigSlot && b.bigCount &&
-                b.bins && b.act && act2 && b.sAxis &&
-                b.sBin && b.sNl && tiles && dcount, "gpu build: out of device memory");
-
-    const int T = kThreads;
-    auto grid = [](long long items) { return dim3((unsigned)((items + kThreads - 1) / kThreads)); };
-    const int chunks = (n + kChunk - 1) / kChunk;
-    hipLaunchKernelGGL(k_prims, grid(n), dim3(T), 0, s, d_tris, n, pbox, cen, b.idx, b.pnode, dOff, R);
-    hipLaunchKernelGGL(k_init_roots, grid(R), dim3(T), 0, s, b, dOff, dSlots, R);
-    hipLaunchKernelGGL(k_init_nodes, grid(R), dim3(T), 0, s, b.nbox, b.ncen, b.small, 0, R);
-    hipLaunchKernelGGL(k_node_bounds, dim3(chunks), dim3(T), 0, s, b, 0);
-
-    std::vector<int> levelStart = {0, R};     // node ids of level L: [levelStart[L], levelStart[L+1])
-    int nodeCount = R;
-    while (m > 0) {
-        const int childBase = nodeCount;
-        hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, s, b.bigCount);
-        hipLaunchKernelGGL(k_big_slots, grid(m), dim3(T), 0, s, b, m);
-        hipLaunchKernelGGL(k_clear_bins, grid((long long)maxBig * kSlotInts), dim3(T), 0, s, b.bins, maxBig);
-        hipLaunchKernelGGL(k_init_nodes, grid(2 * m), dim3(T), 0, s, b.nbox, b.ncen, b.small, childBase, 2 * m);
-        hipLaunchKernelGGL(k_bin, dim3(chunks), dim3(T), 0, s, b);
-        hipLaunchKernelGGL(k_sah, grid(m), dim3(T), 0, s, b, m, childBase);
-        hipLaunchKernelGGL(k_small_level, dim3(m), dim3(64), 0, s, b, m, childBase);
-        hipLaunchKernelGGL(k_flags, grid(n), dim3(T), 0, s, b);
-        scan_exclusive(b.flag, b.rank, n, dcount, tiles, s);
-        hipLaunchKernelGGL(k_scatter, grid(n), dim3(T), 0, s, b);
-        std::swap(b.idx, b.idx2);
-        std::swap(b.pnode, b.pnode2);
-        hipLaunchKernelGGL(k_node_bounds, dim3(chunks), dim3(T), 0, s, b, childBase);
-        // next level's active nodes: children with more than maxLeaf primitives, in id order
-        hipLaunchKernelGGL(k_active_flags, grid(2 * m), dim3(T), 0, s, b.ncnt, childBase, 2 * m, maxLeaf, b.flag);
-        scan_exclusive(b.flag, b.rank, 2 * m, dcount, tiles, s);
-        hipLaunchKernelGGL(k_next_active, grid(2 * m), dim3(T), 0, s, b, childBase, 2 * m, b.rank, act2);
-        std::swap(b.act, act2);
-        nodeCount += 2 * m;
-        levelStart.push_back(nodeCount);
-        int next = 0;
-        if (hipMemcpyAsync(&next, dcount, 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
-            hipStreamSynchronize(s) != hipSuccess) {
-            set_error("gpu build: level %zu failed", levelStart.size() - 2);
-            return -1;
-        }
-        m = next;
+    b.n = n; b.maxLeaf = maxLeaf; b.numScenes = R;
+    b.maxBig = n / (kSmall + 1) + 1;              // active nodes of one level
+    const size_t maxChunks = N / kChunk + b.maxBig + 1;
+    Slab slab;
+    int *dTab = nullptr, *tiles = nullptr, *head = nullptr, *assign = nullptr, *b4id = nullptr, *dRoot4 = nullptr;
+    float* dBounds = nullptr;
+    slab.add(&dTab, 2 * (size_t)(R + 1));
+    slab.add(&b.pbox, 2 * N);
+    slab.add(&b.idx[0], N); slab.add(&b.idx[1], N);
+    slab.add(&b.leafFlag, N); slab.add(&b.leafRank, N);
+    slab.add(&b.rootAcc, 12 * (size_t)R); slab.add(&b.rootRef, R); slab.add(&b.bnd, 6);
+    for (int k = 0; k < 2; k++) {
+        slab.add(&b.act[k], b.maxBig); slab.add(&b.actAcc[k], 12 * (size_t)b.maxBig);
+        slab.add(&b.chunkBase[k], b.maxBig + 1); slab.add(&b.bins[k], 2 * (size_t)b.maxBig * kSlotInts);
     }
-    // pre-order renumbering
-    int* size = tmp.get<int>(nodeCount);
-    int* pre = tmp.get<int>(nodeCount);
-    int* head = tmp.get<int>(nodeCount + 1);
-    int* b4id = tmp.get<int>(nodeCount + 1);
-    int* assign = tmp.get<int>(nodeCount);
-    int* lev4 = tmp.get<int>(nodeCount);
-    float4* ccost = tmp.get<float4>(nodeCount);
-    BUILD_CHECK(size && pre && head && b4id && assign && lev4 && ccost, "gpu build: out of device memory");
-    const int levels = (int)levelStart.size() - 1;
-    for (int L = levels - 1; L >= 0; L--) {
-        const int f = levelStart[L], c = levelStart[L + 1] - f;
-        hipLaunchKernelGGL(k_sizes, grid(c), dim3(T), 0, s, b.nleft, b.nright, size, f, c);
-    }
-    hipLaunchKernelGGL(k_root_pre, dim3(1), dim3(1), 0, s, size, pre, R);
-    for (int L = 0; L < levels; L++) {
-        const int f = levelStart[L], c = levelStart[L + 1] - f;
-        hipLaunchKernelGGL(k_preorder, grid(c), dim3(T), 0, s, b.nleft, b.nright, size, pre, f, c);
-    }
-    out.numNodes2 = nodeCount;
-    if (hipMalloc((void**)&out.nodes2, (size_t)nodeCount * sizeof(Node2)) != hipSuccess) {
+    slab.add(&b.childAcc, 24 * (size_t)b.maxBig);
+    slab.add(&b.sAxis, b.maxBig); slab.add(&b.sBin, b.maxBig); slab.add(&b.sNl, b.maxBig);
+    slab.add(&b.chunkHist, maxChunks * 3 * kBins); slab.add(&b.chunkLeft, maxChunks);
+    slab.add(&b.count, 8);
+    slab.add(&b.topLevel, N + 2);                 // a level splits at least one node
+    slab.add(&b.top, N); slab.add(&b.topCost, N); slab.add(&b.topAsg, N);
+    slab.add(&b.small, N); slab.add(&b.smallCost, N); slab.add(&b.smallAsg, N);
+    slab.add(&b.rec, 2 * N); slab.add(&b.cost, 2 * N); slab.add(&b.lvl, 2 * N + 2);
+    slab.add(&head, 2 * N); slab.add(&assign, 2 * N); slab.add(&b4id, 2 * N);
+    slab.add(&tiles, scan_tiles_needed((int)std::min<size_t>(2 * N, 0x7fffffff)) + 8);
+    slab.add(&dRoot4, R);
+    slab.add(&dBounds, 8);
+    BUILD_CHECK(slab.alloc(), "gpu build: out of device memory");
+    if (hipMalloc((void**)&out.ordered, N * 4) != hipSuccess || hipMalloc(&out.tris, N * 48) != hipSuccess ||
+        hipMalloc((void**)&out.leafOf, N * 4) != hipSuccess) {
         set_error("gpu build: out of device memory");
         return -1;
     }
-    hipLaunchKernelGGL(k_emit_bvh2, grid(nodeCount), dim3(T), 0, s, b, pre, nodeCount, out.nodes2, head, assign, lev4);
-    for (int L = levels - 1; L >= 0; L--) {
-        const int f = levelStart[L], c = levelStart[L + 1] - f;
-        hipLaunchKernelGGL(k_collapse_cost, grid(c), dim3(T), 0, s, out.nodes2, pre, f, c, ccost);
-    }
-    for (int L = 0; L < levels; L++) {
-        const int f = levelStart[L], c = levelStart[L + 1] - f;
-        hipLaunchKernelGGL(k_collapse_assign, grid(c), dim3(T), 0, s, out.nodes2, pre, f, c, ccost, assign, head, lev4);
-    }
-    scan_exclusive(head, b4id, nodeCount, dcount, tiles, s);
-    int heads = 0;
-    if (hipMemcpyAsync(&heads, dcount, 4, hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess) {
-        set_error("gpu build: renumbering failed");
+    b.ordered = out.ordered;
+    b.off = dTab; b.primBase = dTab + R + 1;
+    if (hipMemcpyAsync(dTab, tab.data(), tab.size() * sizeof(int), hipMemcpyHostToDevice, s) != hipSuccess) {
+        set_error("gpu build: upload failed");
         return -1;
     }
+    const int T = kThreads;
+    auto grid = [](long long items) { return dim3((unsigned)((items + kThreads - 1) / kThreads)); };
+    const int slots0 = std::max(big0, 1);
+    hipLaunchKernelGGL(k_build_init, grid(std::max(R * 12, slots0 * kSlotInts)), dim3(T), 0, s, b, slots0);
+    hipLaunchKernelGGL(k_prims, dim3(hBase[R]), dim3(kTopThreads), 0, s, b, d_tris, hBase[R]);
+    hipLaunchKernelGGL(k_mesh_bounds, dim3(1), dim3(64), 0, s, d_tris, b.bnd, dBounds);
+    hipLaunchKernelGGL(k_top_next, dim3(1), dim3(1024), 0, s, b, 0, 1, 0);
+    // Levels until no node of more than kSmall primitives is left. The
+    // largest scene needs at least log2(c / kSmall) levels, so the first
+    // read-back of the node count (a wait for the device) comes after those.
+    int levels = 0, cur = 0;
+    if (big0 > 0) {
+        int need = 0;
+        while (((long long)kSmall << need) < largest) need++;
+        long long nodes = big0;
+        for (;;) {
+            const int gn = (int)std::min<long long>(nodes, b.maxBig);
+            const int gc = (int)std::min<long long>((long long)(N / kChunk) + gn + 1, (long long)maxChunks);
+            hipLaunchKernelGGL(k_top_bin, dim3(gc), dim3(kTopThreads), 0, s, b, cur);
+            hipLaunchKernelGGL(k_top_split, dim3(gn), dim3(T), 0, s, b, cur, levels);
+            hipLaunchKernelGGL(k_top_scatter, dim3(gc), dim3(kTopThreads), 0, s, b, cur);
+            hipLaunchKernelGGL(k_top_next, dim3(1), dim3(1024), 0, s, b, cur ^ 1, 0, levels);
+            cur ^= 1;
+            levels++;
+            nodes = std::min<long long>(2 * nodes, b.maxBig);
+            if (levels < need) continue;
+            int m = 0;
+            if (hipMemcpyAsync(&m, b.count, 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
+                hipStreamSynchronize(s) != hipSuccess) {
+                set_error("gpu build: level %d failed", levels - 1);
+                return -1;
+            }
+            if (m == 0) break;
+            nodes = m;
+        }
+    }
+    int hc[8] = {0};
+    if (hipMemcpyAsync(hc, b.count, sizeof hc, hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess) {
+        set_error("gpu build: top levels failed");
+        return -1;
+    }
+    const int numSmall = hc[2];
+    // subtrees: narrow queues (more workgroups per CU) where the leaves hold four
+    if (maxLeaf >= 4)
+        hipLaunchKernelGGL((k_subtree<kSmall / 5 + 1>), dim3(numSmall), dim3(kSubThreads), 0, s, b);
+    else
+        hipLaunchKernelGGL((k_subtree<kSmall / 2 + 1>), dim3(numSmall), dim3(kSubThreads), 0, s, b);
+    scan_exclusive(b.leafFlag, b.leafRank, n, b.count + 4, tiles, s);
+    int leaves = 0;
+    if (hipMemcpyAsync(&leaves, b.count + 4, 4, hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess) {
+        set_error("gpu build: subtrees failed");
+        return -1;
+    }
+    const int nodeCount = 2 * leaves - R;
+    out.numNodes2 = nodeCount;
+    if (leaves <= 0 || hipMalloc((void**)&out.nodes2, (size_t)nodeCount * sizeof(Node2)) != hipSuccess) {
+        set_error("gpu build: out of device memory");
+        return -1;
+    }
+    const Emit em{out.nodes2, head, assign, b.count + 6};
+    hipLaunchKernelGGL(k_top_collapse, dim3(1), dim3(1024), 0, s, b, em, levels);
+    hipLaunchKernelGGL(k_sub_emit, dim3(numSmall), dim3(T), 0, s, b, em);
+    scan_exclusive(head, b4id, nodeCount, b.count + 5, tiles, s);
+    hipLaunchKernelGGL(k_leaf_tris, grid(n), dim3(T), 0, s, d_tris, b.ordered, n, (float4*)out.tris, out.leafOf, b.off, R);
+    float hb[6];
+    int fin[3] = {0, 0, 0};                       // heads, BVH4 and BVH2 levels
+    if (hipMemcpyAsync(fin, b.count + 5, sizeof fin, hipMemcpyDeviceToHost, s) != hipSuccess ||
+        hipMemcpyAsync(hb, dBounds, sizeof hb, hipMemcpyDeviceToHost, s) != hipSuccess ||
+        hipStreamSynchronize(s) != hipSuccess) {
+        set_error("gpu build: numbering failed");
+        return -1;
+    }
+    for (int a = 0; a < 3; a++) { out.bmin[a] = hb[a]; out.bmax[a] = hb[3 + a]; }
+    const int heads = fin[0];
     out.numNodes4 = std::max(heads, 1);
-    int* dDepth = dcount + 1;
-    hipMemsetAsync(dDepth, 0, sizeof(int), s);
-    if (hipMalloc(&out.nodes4, (size_t)out.numNodes4 * 64) != hipSuccess ||
-        hipMalloc(&out.tris, (size_t)n * 48) != hipSuccess || hipMalloc((void**)&out.leafOf, (size_t)n * 4) != hipSuccess ||
-        hipMalloc((void**)&out.ordered, (size_t)n * 4) != hipSuccess) {
+    out.depth4 = std::max(fin[1], 1);             // a leaf root is one node
+    if (hipMalloc(&out.nodes4, (size_t)out.numNodes4 * 64) != hipSuccess) {
         set_error("gpu build: out of device memory");
         return -1;
     }
     if (heads > 0)
-        hipLaunchKernelGGL(k_emit_bvh4, grid(nodeCount), dim3(T), 0, s, out.nodes2, head, b4id, assign, lev4,
-                           nodeCount, (uint4*)out.nodes4, dDepth);
+        hipLaunchKernelGGL(k_emit_bvh4, grid(nodeCount), dim3(T), 0, s, out.nodes2, head, b4id, assign, nodeCount,
+                           (uint4*)out.nodes4);
     else
-        hipLaunchKernelGGL(k_emit_leaf_root, dim3(1), dim3(1), 0, s, out.nodes2, (uint4*)out.nodes4, dDepth);
-    hipLaunchKernelGGL(k_leaf_tris, grid(n), dim3(T), 0, s, d_tris, b.idx, n, (float4*)out.tris, out.leafOf, dOff, R);
+        hipLaunchKernelGGL(k_emit_leaf_root, dim3(1), dim3(1), 0, s, out.nodes2, (uint4*)out.nodes4);
     if (roots4) {
-        int* dRoot4 = tmp.get<int>(R);
-        BUILD_CHECK(dRoot4, "gpu build: out of device memory");
-        hipLaunchKernelGGL(k_root4, grid(R), dim3(T), 0, s, pre, b4id, R, dRoot4);
+        hipLaunchKernelGGL(k_root4, grid(R), dim3(T), 0, s, b, b4id, dRoot4);
         roots4->assign(R, 0);
         if (hipMemcpyAsync(roots4->data(), dRoot4, R * sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess) {
             set_error("gpu build: root download failed");
             return -1;
         }
     }
-    hipMemcpyAsync(out.ordered, b.idx, (size_t)n * 4, hipMemcpyDeviceToDevice, s);
-    hipMemcpyAsync(&out.depth4, dDepth, 4, hipMemcpyDeviceToHost, s);
     hipError_t e = hipStreamSynchronize(s);
     if (e == hipSuccess) e = hipGetLastError();
     if (e != hipSuccess) { set_error("gpu build failed: %s", hipGetErrorString(e)); return -1; }
-    if (verbose()) fprintf(stderr, "[CudaBVH] gpu_build: %d levels, %.2f ms to the last kernel\n", levels, now_ms() - tBegin);
-    out.levels = levels;
+    out.levels = fin[2];
     return 0;
 }
 

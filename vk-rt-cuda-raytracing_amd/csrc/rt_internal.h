@@ -48,7 +48,8 @@ struct GpuBVH {
     void* tris = nullptr;                          // leaf order, 48 B per triangle
     int* leafOf = nullptr;                         // original index -> leaf position
     int* ordered = nullptr;                        // leaf position -> original index
-    int levels = 0;
+    int levels = 0;                                // BVH2 levels
+    float bmin[3], bmax[3];                        // mesh bounds (mesh_bounds' values)
 };
 // Builds one BVH, or with sceneOff (numScenes+1 host offsets into d_tris) a
 // forest of numScenes independent BVHs in one level-synchronous pass: node
@@ -56,6 +57,10 @@ struct GpuBVH {
 // their index within their scene; roots4 receives each tree's BVH4 root.
 int gpu_build(const float* d_tris, int n, int maxLeaf, hipStream_t s, GpuBVH& out, const int* sceneOff = nullptr,
               int numScenes = 1, std::vector<int>* roots4 = nullptr);
+// Bounds of n x 9 device floats as a sequential std::min / std::max pass over
+// the triangles computes them (from 1e30 / -1e30; the first of equal values,
+// NaN skipped). Waits for stream s. 0 on success.
+int mesh_bounds(const float* d_tris, int n, hipStream_t s, float* mn, float* mx);
 void scan_exclusive(const int* in, int* out, int n, int* total, int* tiles, hipStream_t s);
 int scan_tiles_needed(int n);
 

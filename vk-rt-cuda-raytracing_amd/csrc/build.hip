@@ -46,8 +46,8 @@ namespace rtb {
 
 constexpr int kBins = 16;
 constexpr int kBinInts = 7;                 // box min xyz, max xyz (ordered ints), count
-constexpr int kAxisInts = kBins * kBinInts;
-constexpr int kSlotInts = 3 * kAxisInts;
+constexpr int kCells = 3 * kBins;           // bins of the three axes
+constexpr int kSlotInts = kBinInts * kCells;   // a node's bins: [7][3][16]
 constexpr int kThreads = 256;
 
 // Nodes of at most kSmall primitives are built to their leaves by one
@@ -240,6 +240,12 @@ struct BoundsAcc {
     }
 };
 
+// Empty value of word i of (consecutive) bins.
+__device__ __forceinline__ int empty_bin(int i) {
+    const int f = i % kSlotInts / kCells;
+    return f < 3 ? kOrdPosInf : (f < 6 ? kOrdNegInf : 0);
+}
+
 __global__ void k_build_init(Build b, int slots) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < b.numScenes * 12) b.rootAcc[i] = (i % 6) < 3 ? kOrdPosInf : kOrdNegInf;
@@ -247,8 +253,7 @@ __global__ void k_build_init(Build b, int slots) {
     if (i < 8) b.count[i] = 0;
     if (i == 0) b.topLevel[0] = 0;
     if (i < slots * kSlotInts) {
-        const int f = i % kBinInts;
-        b.bins[0][i] = f < 3 ? kOrdPosInf : (f < 6 ? kOrdNegInf : 0);
+        b.bins[0][i] = empty_bin(i);
     }
 }
 
@@ -448,10 +453,7 @@ __global__ __launch_bounds__(kTopThreads) void k_top_bin(Build b, int cur) {
         cmin[a] = o2f(nc[a]); cmax[a] = o2f(nc[3 + a]);
         use[a] = !(cmax[a] - cmin[a] < 1e-8f);
     }
-    for (int i = threadIdx.x; i < kBinCopies * kCopyStride; i += kTopThreads) {
-        const int f = (i % kCopyStride) % kBinInts;
-        lb[i] = f < 3 ? kOrdPosInf : (f < 6 ? kOrdNegInf : 0);
-    }
+    for (int i = threadIdx.x; i < kBinCopies * kCopyStride; i += kTopThreads) lb[i] = empty_bin(i % kCopyStride);
     __syncthreads();
     int* mine = lb + (threadIdx.x % kBinCopies) * kCopyStride;
     const int* idx = b.idx[cur] + g.s;
@@ -464,23 +466,26 @@ __global__ __launch_bounds__(kTopThreads) void k_top_bin(Build b, int cur) {
 #pragma unroll
         for (int a = 0; a < 3; a++) {
             if (!use[a]) continue;
-            int* d = mine + a * kAxisInts + bin_of(centroid(v, a), cmin[a], cmax[a]) * kBinInts;
+            int* d = mine + a * kBins + bin_of(centroid(v, a), cmin[a], cmax[a]);
 #pragma unroll
-            for (int e = 0; e < 3; e++) { atomicMin(&d[e], f2o(v[e])); atomicMax(&d[3 + e], f2o(v[3 + e])); }
-            atomicAdd(&d[6], 1);
+            for (int e = 0; e < 3; e++) {
+                atomicMin(&d[e * kCells], f2o(v[e]));
+                atomicMax(&d[(3 + e) * kCells], f2o(v[3 + e]));
+            }
+            atomicAdd(&d[6 * kCells], 1);
         }
     }
     __syncthreads();
     int* out = b.bins[cur] + (size_t)j * kSlotInts;
     for (int i = threadIdx.x; i < kSlotInts; i += kTopThreads) {
-        const int f = i % kBinInts;
+        const int f = i / kCells;
         int v = lb[i];
         for (int k = 1; k < kBinCopies; k++) {
             const int o = lb[k * kCopyStride + i];
             v = f < 3 ? min(v, o) : (f < 6 ? max(v, o) : v + o);
         }
         if (f == 6) {
-            b.chunkHist[(size_t)blockIdx.x * (3 * kBins) + i / kBinInts] = v;
+            b.chunkHist[(size_t)blockIdx.x * kCells + i - 6 * kCells] = v;
             if (v) atomicAdd(&out[i], v);
         } else if (f < 3) {
             if (v != kOrdPosInf) atomicMin(&out[i], v);
@@ -490,51 +495,93 @@ __global__ __launch_bounds__(kTopThreads) void k_top_bin(Build b, int cur) {
     }
 }
 
-// SAH over 3 axes x 15 boundaries in one wave: lane 16 a + q holds bin q of
-// axis a; box prefixes and suffixes are scans within the 16-lane rows, and the
-// first candidate of least cost in the host order (axis-major, strict <) wins.
-struct Sah {
-    int axis, bin, nl;         // split (axis -1: middle split), last left bin, left count; wave-uniform
-    int src;                   // the winning lane
-    float L[6], R[6];          // this lane's candidate: left and right box
-    bool nan;                  // some bin's box holds a NaN (wave-uniform)
-};
-__device__ __forceinline__ void sah_wave(const int* bins, float pA, bool use0, bool use1, bool use2, int cnt, Sah& r) {
-    const int lane = threadIdx.x & 63;
-    const int ax = lane >> 4, q = lane & 15;
-    float bx[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    int n = 0;
-    if (lane < 3 * kBins) {
-        const int* B = bins + lane * kBinInts;
-#pragma unroll
-        for (int k = 0; k < 6; k++) bx[k] = o2f(B[k]);
-        n = B[6];
-    }
-    r.nan = __any(bx[0] != bx[0] || bx[1] != bx[1] || bx[2] != bx[2] || bx[3] != bx[3] || bx[4] != bx[4] || bx[5] != bx[5]);
+// SAH candidates of one axis, a 16-lane row per node: the lane of bin q holds
+// the candidate that splits after it. In: its bin (ordered ints, count); out:
+// left and right box and counts (row scans). Integers order and combine as
+// the floats do; with a NaN in some box (`nan`, wave-uniform) the scans run on
+// floats, whose min / max skip it.
+struct Cand { float L[6], R[6]; int nl, nr; };
+__device__ __forceinline__ void sah_scan(const int (&B)[6], int n, bool nan, Cand& c) {
     int ln = n, rn = n;
-    float S[6];
+    if (!nan) {
+        int L[6], S[6];
 #pragma unroll
-    for (int k = 0; k < 6; k++) r.L[k] = S[k] = bx[k];
+        for (int k = 0; k < 6; k++) L[k] = S[k] = B[k];
 #define RTB_SCAN(D)                                                                                     \
     {                                                                                                   \
         _Pragma("unroll") for (int k = 0; k < 3; k++) {                                                 \
-            r.L[k] = fminf(r.L[k], from_left<D>(INFINITY, r.L[k]));                                     \
-            r.L[3 + k] = fmaxf(r.L[3 + k], from_left<D>(-INFINITY, r.L[3 + k]));                        \
+            L[k] = min(L[k], from_left<D>(kOrdPosInf, L[k]));                                           \
+            L[3 + k] = max(L[3 + k], from_left<D>(kOrdNegInf, L[3 + k]));                               \
+            S[k] = min(S[k], from_right<D>(kOrdPosInf, S[k]));                                          \
+            S[3 + k] = max(S[3 + k], from_right<D>(kOrdNegInf, S[3 + k]));                              \
+        }                                                                                               \
+        ln += from_left<D>(0, ln);                                                                      \
+        rn += from_right<D>(0, rn);                                                                     \
+    }
+        RTB_SCAN(1) RTB_SCAN(2) RTB_SCAN(4) RTB_SCAN(8)
+#undef RTB_SCAN
+#pragma unroll
+        for (int k = 0; k < 6; k++) {
+            c.L[k] = o2f(L[k]);
+            c.R[k] = o2f(from_right<1>(k < 3 ? kOrdPosInf : kOrdNegInf, S[k]));
+        }
+    } else {
+        float L[6], S[6];
+#pragma unroll
+        for (int k = 0; k < 6; k++) L[k] = S[k] = o2f(B[k]);
+#define RTB_SCAN(D)                                                                                     \
+    {                                                                                                   \
+        _Pragma("unroll") for (int k = 0; k < 3; k++) {                                                 \
+            L[k] = fminf(L[k], from_left<D>(INFINITY, L[k]));                                           \
+            L[3 + k] = fmaxf(L[3 + k], from_left<D>(-INFINITY, L[3 + k]));                              \
             S[k] = fminf(S[k], from_right<D>(INFINITY, S[k]));                                          \
             S[3 + k] = fmaxf(S[3 + k], from_right<D>(-INFINITY, S[3 + k]));                             \
         }                                                                                               \
         ln += from_left<D>(0, ln);                                                                      \
         rn += from_right<D>(0, rn);                                                                     \
     }
-    RTB_SCAN(1) RTB_SCAN(2) RTB_SCAN(4) RTB_SCAN(8)
+        RTB_SCAN(1) RTB_SCAN(2) RTB_SCAN(4) RTB_SCAN(8)
 #undef RTB_SCAN
 #pragma unroll
-    for (int k = 0; k < 6; k++) r.R[k] = from_right<1>(k < 3 ? INFINITY : -INFINITY, S[k]);
-    rn = from_right<1>(0, rn);
+        for (int k = 0; k < 6; k++) {
+            c.L[k] = L[k];
+            c.R[k] = from_right<1>(k < 3 ? INFINITY : -INFINITY, S[k]);
+        }
+    }
+    c.nl = ln;
+    c.nr = from_right<1>(0, rn);
+}
+// An ordered integer outside [-inf, +inf] is a NaN.
+__device__ __forceinline__ bool ord_nan(int o) { return o > kOrdPosInf || o < kOrdNegInf; }
+__device__ __forceinline__ float sah_cost(const Cand& c, float pA) {
+    return (float)c.nl * area(c.L[0], c.L[1], c.L[2], c.L[3], c.L[4], c.L[5]) / pA +
+           (float)c.nr * area(c.R[0], c.R[1], c.R[2], c.R[3], c.R[4], c.R[5]) / pA + 1.f;
+}
+
+// SAH over 3 axes x 15 boundaries in one wave: lane 16 a + q holds bin q of
+// axis a; the first candidate of least cost in the host order (axis-major,
+// strict <) wins.
+struct Sah {
+    int axis, bin, nl;         // split (axis -1: middle split), last left bin, left count; wave-uniform
+    int src;                   // the winning lane
+    Cand c;                    // this lane's candidate
+    bool nan;                  // some bin's box holds a NaN (wave-uniform)
+};
+__device__ __forceinline__ void sah_wave(const int* bins, float pA, bool use0, bool use1, bool use2, int cnt, Sah& r) {
+    const int lane = threadIdx.x & 63;
+    const int ax = lane >> 4, q = lane & 15;
+    int B[6] = {kOrdPosInf, kOrdPosInf, kOrdPosInf, kOrdNegInf, kOrdNegInf, kOrdNegInf};
+    int n = 0;
+    if (lane < kCells) {
+#pragma unroll
+        for (int k = 0; k < 6; k++) B[k] = bins[k * kCells + lane];
+        n = bins[6 * kCells + lane];
+    }
+    r.nan = __any(ord_nan(B[0]) || ord_nan(B[1]) || ord_nan(B[2]) || ord_nan(B[3]) || ord_nan(B[4]) || ord_nan(B[5]));
+    sah_scan(B, n, r.nan, r.c);
     const bool use = ax == 0 ? use0 : (ax == 1 ? use1 : (ax == 2 && use2));
-    const float cost = (float)ln * area(r.L[0], r.L[1], r.L[2], r.L[3], r.L[4], r.L[5]) / pA +
-                       (float)rn * area(r.R[0], r.R[1], r.R[2], r.R[3], r.R[4], r.R[5]) / pA + 1.f;
-    const bool ok = use && q < kBins - 1 && ln != 0 && rn != 0 && cost < 1e30f;
+    const float cost = sah_cost(r.c, pA);
+    const bool ok = use && q < kBins - 1 && r.c.nl != 0 && r.c.nr != 0 && cost < 1e30f;
     const float least = wave_minf(ok ? cost : INFINITY);
     const uint64_t best = __ballot(ok && cost == least);
     if (best == 0) {                               // coincident centroids: middle split
@@ -543,7 +590,7 @@ __device__ __forceinline__ void sah_wave(const int* bins, float pA, bool use0, b
         r.src = __ffsll((unsigned long long)best) - 1;
         r.axis = r.src >> 4;
         r.bin = r.src & 15;
-        r.nl = __builtin_amdgcn_readlane(ln, r.src);
+        r.nl = __builtin_amdgcn_readlane(r.c.nl, r.src);
     }
 }
 
@@ -575,10 +622,7 @@ __global__ __launch_bounds__(kThreads) void k_top_split(Build b, int cur, int le
     }
     if (threadIdx.x < 24) b.childAcc[24 * (size_t)j + threadIdx.x] = (threadIdx.x % 6) < 3 ? kOrdPosInf : kOrdNegInf;
     int* clr = b.bins[cur ^ 1] + 2 * (size_t)j * kSlotInts;
-    for (int i = threadIdx.x; i < 2 * kSlotInts; i += kThreads) {
-        const int f = i % kBinInts;
-        clr[i] = f < 3 ? kOrdPosInf : (f < 6 ? kOrdNegInf : 0);
-    }
+    for (int i = threadIdx.x; i < 2 * kSlotInts; i += kThreads) clr[i] = empty_bin(i);
     __syncthreads();
     const int ax = choice[0], bin = choice[1], nl = choice[2];
     const int c0 = b.chunkBase[cur][j], nch = b.chunkBase[cur][j + 1] - c0;
@@ -590,7 +634,7 @@ __global__ __launch_bounds__(kThreads) void k_top_split(Build b, int cur, int le
             if (ax < 0) {
                 left = max(0, min(nl - q * kChunk, kChunk));
             } else {
-                const int* h = b.chunkHist + (size_t)(c0 + q) * (3 * kBins) + ax * kBins;
+                const int* h = b.chunkHist + (size_t)(c0 + q) * kCells + ax * kBins;
                 for (int k = 0; k <= bin; k++) left += h[k];
             }
         }
@@ -709,22 +753,298 @@ __device__ __forceinline__ bool assign_slots(const float4& c, const float4& L, c
 }
 
 // ------------------------------- subtrees ------------------------------------
-// A whole subtree per workgroup: primitive boxes in LDS, level by level, one
-// wave per node (nodes of at most 64 primitives stay in registers: one
-// primitive per lane). Leaves write their part of the final order at once.
+// A whole subtree per workgroup: primitive boxes in LDS, level by level. A
+// wave takes one node (up to 64 primitives stay in registers, one per lane),
+// or four nodes of at most kTiny primitives, a 16-lane row each: most inner
+// nodes are that small, and the SAH of one costs nearly as many instructions
+// as of four. Leaves write their part of the final order at once.
 // MAXQ: most active nodes of a level (kSmall / (maxLeaf + 1)).
 constexpr int kSubThreads = 512, kSubWaves = kSubThreads / 64;
+constexpr int kTiny = 16;
 
 template <int MAXQ>
 struct SubLds {
     float box[6][kSmall];
     unsigned short perm[2][kSmall];
+    // active nodes: larger ones from the front, tiny ones from the back
     unsigned int seg[2][MAXQ];                 // start | count << 12
     unsigned short rec[2][MAXQ];
+    unsigned short lt[2][MAXQ];                // left turns below the subtree's root
     float pA[2][MAXQ];                         // area of the node's box
-    int bins[kSubWaves][kSlotInts];
-    int qn[2], recs;
+    int bins[kSubWaves][kBinInts * 64];
+    int nbig[2], ntiny[2], next, recs;
 };
+
+// Where a subtree's nodes go.
+struct SubOut { Rec* rec; int s, lt, maxLeaf; };
+
+// The two children of node `rid`: records, and queue entries of those that
+// are not leaves. Called by lane 0 of a wave or by one lane per node.
+template <int MAXQ>
+__device__ __forceinline__ void sub_children(SubLds<MAXQ>& S, const SubOut& o, int nxt, int rid, int lt, int start, int cnt,
+                                             int nl, const float (&L)[6], const float (&R)[6]) {
+    const int base = atomicAdd(&S.recs, 2);
+    o.rec[rid].child = base;
+    o.rec[rid].m = o.s + start + nl;
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const int cs = k ? start + nl : start, cc = k ? cnt - nl : nl, cl = k ? lt : lt + 1;
+        const float x[6] = {k ? R[0] : L[0], k ? R[1] : L[1], k ? R[2] : L[2], k ? R[3] : L[3], k ? R[4] : L[4],
+                            k ? R[5] : L[5]};
+        Rec& c = o.rec[base + k];
+        c.a = make_float4(x[0], x[1], x[2], x[3]);
+        c.b = make_float2(x[4], x[5]);
+        c.s = o.s + cs;
+        c.lt = o.lt + cl;
+        if (cc <= o.maxLeaf) {
+            c.child = -1;
+            c.m = cc;
+        } else {
+            const int q = cc > kTiny ? atomicAdd(&S.nbig[nxt], 1) : MAXQ - 1 - atomicAdd(&S.ntiny[nxt], 1);
+            S.seg[nxt][q] = (unsigned int)cs | (unsigned int)cc << 12;
+            S.rec[nxt][q] = (unsigned short)(base + k);
+            S.lt[nxt][q] = (unsigned short)cl;
+            S.pA[nxt][q] = area(x[0], x[1], x[2], x[3], x[4], x[5]);
+        }
+    }
+}
+
+// One node by one wave.
+template <int MAXQ>
+__device__ __forceinline__ void sub_node(SubLds<MAXQ>& S, const SubOut& o, int cur, int j, int* lb, const int* idxIn,
+                                         int* ordered, int* leafFlag) {
+    const int lane = threadIdx.x & 63;
+    const unsigned int sg = S.seg[cur][j];
+    const int start = __builtin_amdgcn_readfirstlane((int)(sg & 0xfffu));
+    const int cnt = __builtin_amdgcn_readfirstlane((int)(sg >> 12));
+    const float pA = S.pA[cur][j];
+    const unsigned short* perm = S.perm[cur];
+    unsigned short* perm2 = S.perm[cur ^ 1];
+    const bool one = cnt <= 64;                // the node's primitives fit the wave's lanes
+    int myp = 0;
+    float v[6] = {0, 0, 0, 0, 0, 0};
+    // centroid bounds
+    int cb[6] = {kOrdPosInf, kOrdPosInf, kOrdPosInf, kOrdNegInf, kOrdNegInf, kOrdNegInf};
+    for (int i = lane; i < cnt; i += 64) {
+        myp = perm[start + i];
+#pragma unroll
+        for (int k = 0; k < 6; k++) v[k] = S.box[k][myp];
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+            const int c = f2o(centroid(v, a));
+            cb[a] = min(cb[a], c); cb[3 + a] = max(cb[3 + a], c);
+        }
+    }
+    float cmin[3], cmax[3];
+    bool use[3];
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        cmin[a] = o2f(wave_min(cb[a])); cmax[a] = o2f(wave_max(cb[3 + a]));
+        use[a] = !(cmax[a] - cmin[a] < 1e-8f);
+    }
+    // bins
+    if (lane < kCells) {
+#pragma unroll
+        for (int f = 0; f < kBinInts; f++) lb[f * kCells + lane] = f < 3 ? kOrdPosInf : (f < 6 ? kOrdNegInf : 0);
+    }
+    wave_lds_fence();
+    int mb[3] = {0, 0, 0};
+    for (int i = lane; i < cnt; i += 64) {
+        if (!one) {
+            myp = perm[start + i];
+#pragma unroll
+            for (int k = 0; k < 6; k++) v[k] = S.box[k][myp];
+        }
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+            if (!use[a]) continue;
+            mb[a] = bin_of(centroid(v, a), cmin[a], cmax[a]);
+            int* d = lb + a * kBins + mb[a];
+#pragma unroll
+            for (int e = 0; e < 3; e++) {
+                atomicMin(&d[e * kCells], f2o(v[e]));
+                atomicMax(&d[(3 + e) * kCells], f2o(v[3 + e]));
+            }
+            atomicAdd(&d[6 * kCells], 1);
+        }
+    }
+    wave_lds_fence();
+    Sah r;
+    sah_wave(lb, pA, use[0], use[1], use[2], cnt, r);
+    const int ax = r.axis, bin = r.bin, nl = r.nl;
+    const bool leafL = nl <= o.maxLeaf, leafR = cnt - nl <= o.maxLeaf;
+    // Stable partition. The children's boxes are the winning candidate's; a
+    // middle split has none, and with a NaN box the scans (which skip NaN)
+    // could differ from a reduction over ordered integers, so those reduce.
+    const bool exact = ax < 0 || r.nan;
+    const float smin = ax == 1 ? cmin[1] : (ax == 2 ? cmin[2] : cmin[0]);
+    const float smax = ax == 1 ? cmax[1] : (ax == 2 ? cmax[2] : cmax[0]);
+    int xb[12];
+#pragma unroll
+    for (int k = 0; k < 12; k++) xb[k] = (k % 6) < 3 ? kOrdPosInf : kOrdNegInf;
+    int leftBefore = 0;
+    for (int base = 0; base < cnt; base += 64) {
+        const int i = base + lane;
+        const bool valid = i < cnt;
+        bool left = false;
+        if (valid) {
+            if (!one) {
+                myp = perm[start + i];
+                if (ax >= 0) mb[0] = bin_of((S.box[ax][myp] + S.box[3 + ax][myp]) * .5f, smin, smax);
+            } else {
+                mb[0] = ax == 1 ? mb[1] : (ax == 2 ? mb[2] : mb[0]);
+            }
+            left = ax < 0 ? i < nl : mb[0] <= bin;
+            if (exact) {
+#pragma unroll
+                for (int e = 0; e < 3; e++) {
+                    const int lo = f2o(S.box[e][myp]), hi = f2o(S.box[3 + e][myp]);
+                    if (left) { xb[e] = min(xb[e], lo); xb[3 + e] = max(xb[3 + e], hi); }
+                    else { xb[6 + e] = min(xb[6 + e], lo); xb[9 + e] = max(xb[9 + e], hi); }
+                }
+            }
+        }
+        const uint64_t lm = __ballot(valid && left);
+        const int lr = leftBefore + __popcll(lm & ((1ull << lane) - 1ull));
+        if (valid) {
+            const int pos = start + (left ? lr : nl + (i - lr));
+            if (left ? leafL : leafR) {
+                ordered[pos] = idxIn[myp];
+                leafFlag[pos] = pos == start + (left ? 0 : nl);
+            } else {
+                perm2[pos] = (unsigned short)myp;
+            }
+        }
+        leftBefore += __popcll(lm);
+    }
+    float L[6], R[6];
+    if (exact) {
+#pragma unroll
+        for (int k = 0; k < 6; k++) {
+            L[k] = o2f(k < 3 ? wave_min(xb[k]) : wave_max(xb[k]));
+            R[k] = o2f(k < 3 ? wave_min(xb[6 + k]) : wave_max(xb[6 + k]));
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < 6; k++) { L[k] = lane_of(r.c.L[k], r.src); R[k] = lane_of(r.c.R[k], r.src); }
+    }
+    if (lane == 0) sub_children(S, o, cur ^ 1, S.rec[cur][j], S.lt[cur][j], start, cnt, nl, L, R);
+}
+
+// min / max over a 16-lane row, in every lane of it
+__device__ __forceinline__ int row_min(int v) {
+    v = min(v, dpp<0x128, 0xf>(v, v)); v = min(v, dpp<0x124, 0xf>(v, v));   // rotations by 8, 4, 2, 1
+    v = min(v, dpp<0x122, 0xf>(v, v)); return min(v, dpp<0x121, 0xf>(v, v));
+}
+__device__ __forceinline__ int row_max(int v) {
+    v = max(v, dpp<0x128, 0xf>(v, v)); v = max(v, dpp<0x124, 0xf>(v, v));
+    v = max(v, dpp<0x122, 0xf>(v, v)); return max(v, dpp<0x121, 0xf>(v, v));
+}
+
+// Four tiny nodes by one wave: queue entries [t0, min(t0 + 4, count)) counted
+// from the back, one per 16-lane row, one axis at a time. Each lane keeps its
+// cheapest candidate of the three axes (the first of equals); the row's least
+// (cost, axis, bin) wins and that lane writes the children. Rows that need
+// the general path (no candidate, a NaN box) are left to sub_node.
+template <int MAXQ>
+__device__ __forceinline__ void sub_tiny(SubLds<MAXQ>& S, const SubOut& o, int cur, int t0, int count, int* lb,
+                                         const int* idxIn, int* ordered, int* leafFlag) {
+    const int lane = threadIdx.x & 63, row = lane >> 4, q = lane & 15;
+    const bool node = t0 + row < count;
+    const int j = node ? MAXQ - 1 - (t0 + row) : MAXQ - 1;
+    const unsigned int sg = S.seg[cur][j];
+    const int start = (int)(sg & 0xfffu), cnt = node ? (int)(sg >> 12) : 0;
+    const float pA = S.pA[cur][j];
+    const bool valid = q < cnt;
+    int myp = 0;
+    float v[6] = {0, 0, 0, 0, 0, 0};
+    int ob[6] = {kOrdPosInf, kOrdPosInf, kOrdPosInf, kOrdNegInf, kOrdNegInf, kOrdNegInf};
+    float cen[3], cmin[3], cmax[3];
+    bool use[3];
+    if (valid) {
+        myp = S.perm[cur][start + q];
+#pragma unroll
+        for (int k = 0; k < 6; k++) { v[k] = S.box[k][myp]; ob[k] = f2o(v[k]); }
+    }
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        cen[a] = centroid(v, a);
+        const int c = f2o(cen[a]);
+        cmin[a] = o2f(row_min(valid ? c : kOrdPosInf));
+        cmax[a] = o2f(row_max(valid ? c : kOrdNegInf));
+        use[a] = !(cmax[a] - cmin[a] < 1e-8f);
+    }
+    const bool nan = __any(ord_nan(ob[0]) || ord_nan(ob[1]) || ord_nan(ob[2]) || ord_nan(ob[3]) || ord_nan(ob[4]) ||
+                           ord_nan(ob[5]));
+    int best = -1;                                 // axis * 16 + bin of this lane's cheapest candidate
+    float bestCost = INFINITY;
+    int nl = 0, mybin[3] = {0, 0, 0};
+    float L[6], R[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) L[k] = R[k] = 0.f;
+    if (!nan) {
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+            // one axis' bins of the four nodes: [7][64], a lane's bin in its column
+#pragma unroll
+            for (int f = 0; f < kBinInts; f++) lb[f * 64 + lane] = f < 3 ? kOrdPosInf : (f < 6 ? kOrdNegInf : 0);
+            wave_lds_fence();
+            if (valid && use[a]) {
+                mybin[a] = bin_of(cen[a], cmin[a], cmax[a]);
+                int* d = lb + row * 16 + mybin[a];
+#pragma unroll
+                for (int e = 0; e < 3; e++) {
+                    atomicMin(&d[e * 64], ob[e]);
+                    atomicMax(&d[(3 + e) * 64], ob[3 + e]);
+                }
+                atomicAdd(&d[6 * 64], 1);
+            }
+            wave_lds_fence();
+            int B[6];
+#pragma unroll
+            for (int k = 0; k < 6; k++) B[k] = lb[k * 64 + lane];
+            const int n = lb[6 * 64 + lane];
+            wave_lds_fence();
+            Cand c;
+            sah_scan(B, n, false, c);
+            const float cost = sah_cost(c, pA);
+            if (use[a] && q < kBins - 1 && c.nl != 0 && c.nr != 0 && cost < 1e30f && cost < bestCost) {
+                bestCost = cost;
+                best = a * 16 + q;
+                nl = c.nl;
+#pragma unroll
+                for (int k = 0; k < 6; k++) { L[k] = c.L[k]; R[k] = c.R[k]; }
+            }
+        }
+    }
+    constexpr int kNone = 1 << 20;
+    const int least = row_min(f2o(bestCost));
+    const int key = best >= 0 && f2o(bestCost) == least ? best : kNone;
+    const int wk = row_min(key);
+    const bool won = node && wk != kNone;          // the row has a split
+    const int rnl = row_max(key == wk ? nl : -1);
+    const int ax = wk >> 4;
+    const bool left = valid && (ax == 0 ? mybin[0] : (ax == 1 ? mybin[1] : mybin[2])) <= (wk & 15);
+    const unsigned int lm = (unsigned int)(__ballot(left) >> (row * 16)) & 0xffffu;
+    if (won && valid) {
+        const int lr = __popc(lm & ((1u << q) - 1u));
+        const int pos = start + (left ? lr : rnl + (q - lr));
+        if ((left ? rnl : cnt - rnl) <= o.maxLeaf) {
+            ordered[pos] = idxIn[myp];
+            leafFlag[pos] = pos == start + (left ? 0 : rnl);
+        } else {
+            S.perm[cur ^ 1][pos] = (unsigned short)myp;
+        }
+    }
+    if (won && key == wk) sub_children(S, o, cur ^ 1, S.rec[cur][j], S.lt[cur][j], start, cnt, nl, L, R);
+    uint64_t rest = __ballot(node && !won && q == 0);
+    while (rest) {
+        const int r = (__ffsll((unsigned long long)rest) - 1) >> 4;
+        rest &= rest - 1;
+        wave_lds_fence();
+        sub_node(S, o, cur, MAXQ - 1 - (t0 + r), lb, idxIn, ordered, leafFlag);
+    }
+}
 
 template <int MAXQ>
 __global__ __launch_bounds__(kSubThreads) void k_subtree(Build b) {
@@ -737,6 +1057,7 @@ __global__ __launch_bounds__(kSubThreads) void k_subtree(Build b) {
     int* leafFlag = b.leafFlag + g.s;
     Rec* rec = b.rec + 2 * (size_t)g.s;
     unsigned short* lvl = b.lvl + 2 * (size_t)g.s;
+    const SubOut o{rec, g.s, g.lt, b.maxLeaf};
     float rb[6];
 #pragma unroll
     for (int k = 0; k < 6; k++) rb[k] = o2f(sm.bounds[k]);
@@ -756,11 +1077,15 @@ __global__ __launch_bounds__(kSubThreads) void k_subtree(Build b) {
         rec[0].s = g.s; rec[0].lt = g.lt;
         if (rootLeaf) { rec[0].child = -1; rec[0].m = g.c; }
         S.recs = 1;
-        S.qn[0] = rootLeaf ? 0 : 1;
-        S.qn[1] = 0;
-        S.seg[0][0] = (unsigned int)g.c << 12;
-        S.rec[0][0] = 0;
-        S.pA[0][0] = area(rb[0], rb[1], rb[2], rb[3], rb[4], rb[5]);
+        S.next = 0;
+        const bool tiny = g.c <= kTiny;
+        S.nbig[0] = !rootLeaf && !tiny; S.ntiny[0] = !rootLeaf && tiny;
+        S.nbig[1] = S.ntiny[1] = 0;
+        const int q = tiny ? MAXQ - 1 : 0;
+        S.seg[0][q] = (unsigned int)g.c << 12;
+        S.rec[0][q] = 0;
+        S.lt[0][q] = 0;
+        S.pA[0][q] = area(rb[0], rb[1], rb[2], rb[3], rb[4], rb[5]);
         lvl[0] = 0;
         lvl[1] = 1;
     }
@@ -768,150 +1093,19 @@ __global__ __launch_bounds__(kSubThreads) void k_subtree(Build b) {
     int level = 0;
     int* const lb = S.bins[w];
     for (int cur = 0;; cur ^= 1, level++) {
-        const int qn = S.qn[cur];
-        if (qn == 0) break;
-        const unsigned short* perm = S.perm[cur];
-        unsigned short* perm2 = S.perm[cur ^ 1];
-        for (int j = w; j < qn; j += kSubWaves) {
-            const unsigned int sg = S.seg[cur][j];
-            const int start = __builtin_amdgcn_readfirstlane((int)(sg & 0xfffu));
-            const int cnt = __builtin_amdgcn_readfirstlane((int)(sg >> 12));
-            const int rid = __builtin_amdgcn_readfirstlane((int)S.rec[cur][j]);
-            const float pA = S.pA[cur][j];
-            const bool one = cnt <= 64;            // the node's primitives fit the wave's lanes
-            int myp = 0;
-            float v[6] = {0, 0, 0, 0, 0, 0};
-            // centroid bounds
-            int cb[6] = {kOrdPosInf, kOrdPosInf, kOrdPosInf, kOrdNegInf, kOrdNegInf, kOrdNegInf};
-            for (int i = lane; i < cnt; i += 64) {
-                myp = perm[start + i];
-#pragma unroll
-                for (int k = 0; k < 6; k++) v[k] = S.box[k][myp];
-#pragma unroll
-                for (int a = 0; a < 3; a++) {
-                    const int c = f2o(centroid(v, a));
-                    cb[a] = min(cb[a], c); cb[3 + a] = max(cb[3 + a], c);
-                }
-            }
-            float cmin[3], cmax[3];
-            bool use[3];
-#pragma unroll
-            for (int a = 0; a < 3; a++) {
-                cmin[a] = o2f(wave_min(cb[a])); cmax[a] = o2f(wave_max(cb[3 + a]));
-                use[a] = !(cmax[a] - cmin[a] < 1e-8f);
-            }
-            // bins
-            for (int i = lane; i < kSlotInts; i += 64) {
-                const int f = i % kBinInts;
-                lb[i] = f < 3 ? kOrdPosInf : (f < 6 ? kOrdNegInf : 0);
-            }
+        const int nbig = S.nbig[cur], ntiny = S.ntiny[cur], items = nbig + (ntiny + 3) / 4;
+        if (items == 0) break;
+        for (;;) {
+            int it = 0;
+            if (lane == 0) it = atomicAdd(&S.next, 1);
+            it = __builtin_amdgcn_readfirstlane(it);
+            if (it >= items) break;
+            if (it < nbig) sub_node(S, o, cur, it, lb, idxIn, ordered, leafFlag);
+            else sub_tiny(S, o, cur, 4 * (it - nbig), ntiny, lb, idxIn, ordered, leafFlag);
             wave_lds_fence();
-            int mb[3] = {0, 0, 0};
-            for (int i = lane; i < cnt; i += 64) {
-                if (!one) {
-                    myp = perm[start + i];
-#pragma unroll
-                    for (int k = 0; k < 6; k++) v[k] = S.box[k][myp];
-                }
-#pragma unroll
-                for (int a = 0; a < 3; a++) {
-                    if (!use[a]) continue;
-                    mb[a] = bin_of(centroid(v, a), cmin[a], cmax[a]);
-                    int* d = lb + a * kAxisInts + mb[a] * kBinInts;
-#pragma unroll
-                    for (int e = 0; e < 3; e++) { atomicMin(&d[e], f2o(v[e])); atomicMax(&d[3 + e], f2o(v[3 + e])); }
-                    atomicAdd(&d[6], 1);
-                }
-            }
-            wave_lds_fence();
-            Sah r;
-            sah_wave(lb, pA, use[0], use[1], use[2], cnt, r);
-            const int ax = r.axis, bin = r.bin, nl = r.nl, nr = cnt - nl;
-            const bool leafL = nl <= b.maxLeaf, leafR = nr <= b.maxLeaf;
-            // stable partition
-            const bool exact = ax < 0 || r.nan;    // child boxes by reduction (see below)
-            int xb[12];
-#pragma unroll
-            for (int k = 0; k < 12; k++) xb[k] = (k % 6) < 3 ? kOrdPosInf : kOrdNegInf;
-            const float smin = ax == 1 ? cmin[1] : (ax == 2 ? cmin[2] : cmin[0]);
-            const float smax = ax == 1 ? cmax[1] : (ax == 2 ? cmax[2] : cmax[0]);
-            int leftBefore = 0;
-            for (int base = 0; base < cnt; base += 64) {
-                const int i = base + lane;
-                const bool valid = i < cnt;
-                bool left = false;
-                if (valid) {
-                    if (!one) {
-                        myp = perm[start + i];
-                        if (ax >= 0) mb[0] = bin_of((S.box[ax][myp] + S.box[3 + ax][myp]) * .5f, smin, smax);
-                    } else {
-                        mb[0] = ax == 1 ? mb[1] : (ax == 2 ? mb[2] : mb[0]);
-                    }
-                    left = ax < 0 ? i < nl : mb[0] <= bin;
-                    if (exact) {
-#pragma unroll
-                        for (int e = 0; e < 3; e++) {
-                            const int lo = f2o(S.box[e][myp]), hi = f2o(S.box[3 + e][myp]);
-                            if (left) { xb[e] = min(xb[e], lo); xb[3 + e] = max(xb[3 + e], hi); }
-                            else { xb[6 + e] = min(xb[6 + e], lo); xb[9 + e] = max(xb[9 + e], hi); }
-                        }
-                    }
-                }
-                const uint64_t lm = __ballot(valid && left);
-                const int lr = leftBefore + __popcll(lm & ((1ull << lane) - 1ull));
-                if (valid) {
-                    const int pos = start + (left ? lr : nl + (i - lr));
-                    if (left ? leafL : leafR) {
-                        ordered[pos] = idxIn[myp];
-                        leafFlag[pos] = pos == start + (left ? 0 : nl);
-                    } else {
-                        perm2[pos] = (unsigned short)myp;
-                    }
-                }
-                leftBefore += __popcll(lm);
-            }
-            // children: their boxes are the winning candidate's; a middle
-            // split has none, and with a NaN box the scans (which skip NaN)
-            // could differ from a reduction over ordered integers
-            float cx[12];
-            if (exact) {
-#pragma unroll
-                for (int k = 0; k < 12; k++) cx[k] = o2f((k % 6) < 3 ? wave_min(xb[k]) : wave_max(xb[k]));
-            } else {
-#pragma unroll
-                for (int k = 0; k < 6; k++) { cx[k] = lane_of(r.L[k], r.src); cx[6 + k] = lane_of(r.R[k], r.src); }
-            }
-            int base = 0, qpos = 0;
-            if (lane == 0) {
-                base = atomicAdd(&S.recs, 2);
-                qpos = atomicAdd(&S.qn[cur ^ 1], (leafL ? 0 : 1) + (leafR ? 0 : 1));
-            }
-            base = __builtin_amdgcn_readfirstlane(base);
-            qpos = __builtin_amdgcn_readfirstlane(qpos);
-            if (lane < 2) {                        // lane 0: left child, lane 1: right child
-                const bool R = lane == 1, leaf = R ? leafR : leafL;
-                const int cs = R ? start + nl : start, cc = R ? nr : nl;
-                const float x0 = R ? cx[6] : cx[0], x1 = R ? cx[7] : cx[1], x2 = R ? cx[8] : cx[2];
-                const float x3 = R ? cx[9] : cx[3], x4 = R ? cx[10] : cx[4], x5 = R ? cx[11] : cx[5];
-                Rec& c = rec[base + lane];
-                const int lt = rec[rid].lt;
-                c.a = make_float4(x0, x1, x2, x3);
-                c.b = make_float2(x4, x5);
-                c.s = g.s + cs;
-                c.lt = R ? lt : lt + 1;
-                if (leaf) {
-                    c.child = -1; c.m = cc;
-                } else {
-                    const int q = qpos + (R && !leafL ? 1 : 0);
-                    S.seg[cur ^ 1][q] = (unsigned int)cs | (unsigned int)cc << 12;
-                    S.rec[cur ^ 1][q] = (unsigned short)(base + lane);
-                    S.pA[cur ^ 1][q] = area(x0, x1, x2, x3, x4, x5);
-                }
-                if (lane == 0) { rec[rid].child = base; rec[rid].m = g.s + start + nl; }
-            }
         }
         __syncthreads();
-        if (tid == 0) { S.qn[cur] = 0; lvl[level + 2] = (unsigned short)S.recs; }
+        if (tid == 0) { S.nbig[cur] = S.ntiny[cur] = 0; S.next = 0; lvl[level + 2] = (unsigned short)S.recs; }
         __syncthreads();
     }
     // collapse costs, bottom-up; levels [0, level] hold records
@@ -1374,7 +1568,7 @@ int gpu_build(const float* d_tris, int n, int maxLeaf, hipStream_t s, GpuBVH& ou
     }
     slab.add(&b.childAcc, 24 * (size_t)b.maxBig);
     slab.add(&b.sAxis, b.maxBig); slab.add(&b.sBin, b.maxBig); slab.add(&b.sNl, b.maxBig);
-    slab.add(&b.chunkHist, maxChunks * 3 * kBins); slab.add(&b.chunkLeft, maxChunks);
+    slab.add(&b.chunkHist, maxChunks * kCells); slab.add(&b.chunkLeft, maxChunks);
     slab.add(&b.count, 8);
     slab.add(&b.topLevel, N + 2);                 // a level splits at least one node
     slab.add(&b.top, N); slab.add(&b.topCost, N); slab.add(&b.topAsg, N);

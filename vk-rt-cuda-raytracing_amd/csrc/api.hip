@@ -35,11 +35,13 @@ static int ensure_cwbvh(CudaBVH_t bvh);
 static void async_release(CudaBVH_t bvh);
 
 static void free_handle_device(CudaBVHHandle* h) {
-    hipFree(h->d_nodes4); hipFree(h->d_tris); hipFree(h->d_leafOfPrim); hipFree(h->d_work); hipFree(h->d_sortWs);
+    hipDeviceSynchronize();          // traces on any stream may still read the arrays
+    rt::dev_free(h->d_nodes4); rt::dev_free(h->d_tris); rt::dev_free(h->d_leafOfPrim);
+    hipFree(h->d_work); hipFree(h->d_sortWs);
     h->d_sortWs = nullptr; h->sortWsBytes = 0;
     hipFree(h->d_cwNodes); hipFree(h->d_cwTris);
     h->d_cwNodes = h->d_cwTris = nullptr;
-    hipFree(h->d_nodes2); hipFree(h->d_ordered);
+    rt::dev_free(h->d_nodes2); rt::dev_free(h->d_ordered);
     h->d_nodes2 = nullptr; h->d_ordered = nullptr;
     rtk::free_scratch(h->scratch);
     hipHostFree(h->h_pinned);
@@ -160,17 +162,19 @@ static CudaBVHHandle* build_impl(const float* tri9, int n, int maxLeaf, const in
     const double t0 = clk();
     double t1 = t0;
     if (!d_in) {
-        HIP_TRY(hipMalloc((void**)&d_own, size_t(n) * 36), goto fail);
-        HIP_TRY(hipMemcpyAsync(d_own, tri9, size_t(n) * 36, hipMemcpyHostToDevice, s), hipFree(d_own); goto fail);
+        d_own = (float*)rt::dev_alloc(size_t(n) * 36);
+        if (!d_own) { set_error("cudaBVH_build: cannot allocate %d triangles", n); goto fail; }
+        HIP_TRY(hipMemcpyAsync(d_own, tri9, size_t(n) * 36, hipMemcpyHostToDevice, s), rt::dev_release(d_own); goto fail);
         d_in = d_own;
     }
     hipStreamSynchronize(s);          // the build syncs anyway; this separates the upload time
     t1 = clk();
     if (rt::gpu_build(d_in, n, maxLeaf, s, g, sceneOff, numScenes, roots4) != 0) {
-        hipFree(d_own); hipFree(g.nodes2); hipFree(g.nodes4); hipFree(g.tris); hipFree(g.leafOf); hipFree(g.ordered);
+        hipDeviceSynchronize();
+        for (void* p : {(void*)d_own, (void*)g.nodes2, g.nodes4, g.tris, (void*)g.leafOf, (void*)g.ordered}) rt::dev_free(p);
         goto fail;
     }
-    hipFree(d_own);
+    rt::dev_free(d_own);                // the build has waited for its stream
     h->d_nodes4 = g.nodes4;
     h->d_tris = g.tris;
     h->d_leafOfPrim = g.leafOf;
@@ -191,7 +195,7 @@ static CudaBVHHandle* build_impl(const float* tri9, int n, int maxLeaf, const in
             forestOrdered->resize(n);
             e = hipMemcpy(forestOrdered->data(), g.ordered, size_t(n) * 4, hipMemcpyDeviceToHost);
         }
-        hipFree(g.nodes2);
+        rt::dev_free(g.nodes2);
         if (e != hipSuccess) { set_error("copying the forest back failed: %s", hipGetErrorString(e)); goto fail; }
     }
     {
@@ -353,8 +357,8 @@ CudaBVH_t cudaBVH_buildDevice(const void* d_vertices, int numVertices, int verte
     }
     float* d_tri = nullptr;
     int* d_bad = nullptr;
-    if (hipMalloc((void**)&d_tri, size_t(numTris) * 36) != hipSuccess || hipMalloc((void**)&d_bad, sizeof(int)) != hipSuccess) {
-        hipFree(d_tri);
+    if (!(d_tri = (float*)rt::dev_alloc(size_t(numTris) * 36)) || hipMalloc((void**)&d_bad, sizeof(int)) != hipSuccess) {
+        rt::dev_free(d_tri);
         set_error("cudaBVH_buildDevice: cannot allocate %zu bytes", size_t(numTris) * 36);
         return nullptr;
     }
@@ -366,13 +370,13 @@ CudaBVH_t cudaBVH_buildDevice(const void* d_vertices, int numVertices, int verte
     if (e == hipSuccess) e = hipMemcpy(&bad, d_bad, sizeof(int), hipMemcpyDeviceToHost);
     hipFree(d_bad);
     if (e != hipSuccess || bad) {
-        hipFree(d_tri);
+        rt::dev_release(d_tri);
         if (bad) set_error("cudaBVH_buildDevice: an index is >= numVertices (%d)", numVertices);
         else set_error("cudaBVH_buildDevice: gather failed: %s", hipGetErrorString(e));
         return nullptr;
     }
     CudaBVHHandle* h = build_impl(nullptr, numTris, 4, nullptr, 1, nullptr, d_tri);
-    hipFree(d_tri);
+    rt::dev_free(d_tri);                // the build has waited for its stream
     return h;
 }
 
@@ -426,8 +430,8 @@ int cudaBVH_buildManyDevice(const CudaGeometry* geoms, const int* geomOffsets, i
     if (total > (1ll << 28)) { set_error("%s: %lld triangles in all", fn, total); return -1; }
     float* dTri = nullptr;
     int* dBad = nullptr;
-    if (hipMalloc((void**)&dTri, size_t(total) * 36) != hipSuccess || hipMalloc((void**)&dBad, sizeof(int)) != hipSuccess) {
-        hipFree(dTri);
+    if (!(dTri = (float*)rt::dev_alloc(size_t(total) * 36)) || hipMalloc((void**)&dBad, sizeof(int)) != hipSuccess) {
+        rt::dev_free(dTri);
         set_error("%s: cannot allocate %lld triangles", fn, total);
         return -1;
     }
@@ -445,14 +449,14 @@ int cudaBVH_buildManyDevice(const CudaGeometry* geoms, const int* geomOffsets, i
     if (e == hipSuccess) e = hipMemcpy(&bad, dBad, sizeof(int), hipMemcpyDeviceToHost);
     hipFree(dBad);
     if (e != hipSuccess || bad) {
-        hipFree(dTri);
+        rt::dev_release(dTri);
         if (bad) set_error("%s: an index is >= its geometry's numVertices", fn);
         else set_error("%s: gather failed: %s", fn, hipGetErrorString(e));
         return -1;
     }
     auto fail_all = [&]() {
         for (int k = 0; k < numBlas; k++) { cudaBVH_destroy(out[k]); out[k] = nullptr; }
-        hipFree(dTri);
+        rt::dev_release(dTri);
         return -1;
     };
     for (int k : small) {
@@ -489,13 +493,14 @@ int cudaBVH_buildManyDevice(const CudaGeometry* geoms, const int* geomOffsets, i
             std::vector<int> ord(ford.begin() + t0, ford.begin() + t0 + nt);
             for (int& x : ord) x -= t0;
             h->numNodes2 = int(sub.size());
-            const bool ok = hipMalloc(&h->d_nodes4, hn4.size()) == hipSuccess &&
-                            hipMalloc(&h->d_nodes2, sub.size() * sizeof(rt::Node2)) == hipSuccess &&
-                            hipMalloc((void**)&h->d_ordered, size_t(nt) * 4) == hipSuccess &&
+            h->d_nodes4 = rt::dev_alloc(hn4.size());
+            h->d_nodes2 = rt::dev_alloc(sub.size() * sizeof(rt::Node2));
+            h->d_ordered = (int*)rt::dev_alloc(size_t(nt) * 4);
+            h->d_tris = rt::dev_alloc(size_t(nt) * 48);
+            h->d_leafOfPrim = (int*)rt::dev_alloc(size_t(nt) * 4);
+            const bool ok = h->d_nodes4 && h->d_nodes2 && h->d_ordered && h->d_tris && h->d_leafOfPrim &&
                             hipMemcpy(h->d_nodes2, sub.data(), sub.size() * sizeof(rt::Node2), hipMemcpyHostToDevice) == hipSuccess &&
                             hipMemcpy(h->d_ordered, ord.data(), size_t(nt) * 4, hipMemcpyHostToDevice) == hipSuccess &&
-                            hipMalloc(&h->d_tris, size_t(nt) * 48) == hipSuccess &&
-                            hipMalloc((void**)&h->d_leafOfPrim, size_t(nt) * 4) == hipSuccess &&
                             rtk::launch_slice_forest(forest->d_nodes4, first4, h->numNodes4, forest->d_tris,
                                                      forest->d_leafOfPrim, t0, nt, h->d_nodes4, h->d_tris,
                                                      h->d_leafOfPrim, nullptr) == 0 &&
@@ -520,14 +525,13 @@ int cudaBVH_buildManyDevice(const CudaGeometry* geoms, const int* geomOffsets, i
         }
         cudaBVH_destroy(forest);
     }
-    hipFree(dTri);
+    rt::dev_release(dTri);
     return 0;
 }
 
 void cudaBVH_destroy(CudaBVH_t bvh) {
     if (!bvh) return;
     async_release(bvh);          // the background tracer no longer renders from it
-    if (bvh->stream) hipStreamSynchronize(hstream(bvh)); else hipDeviceSynchronize();
     free_handle_device(bvh);
     delete bvh;
 }
@@ -893,6 +897,7 @@ int cudaBVH_getPackedTris(CudaBVH_t bvh, float** outData) {
 void cudaBVH_resetDevice(void) {
     g_async.stop();
     hipDeviceSynchronize();
+    rt::dev_trim();
 }
 
 CudaBVH_t cudaBVH_buildFromAABBs(const float* aabbs, int numAABBs) {

@@ -127,13 +127,15 @@ struct Top { int s, m, lt, tree, left, right; float box[6]; };   // m: first pri
 // level: BVH2 level of its root; levels: its own (set by k_subtree).
 struct Small { Seg g; int buf, level, levels, pad; int bounds[12]; };
 
-// A node of a subtree: box, first primitive, left turns, and either the left
-// child's record (the right one follows) with the split position m, or -1 and
-// the primitive count in m.
-struct Rec { float4 a; float2 b; int s, lt; int child, m, pad[2]; };
+// A node of a subtree: box, first primitive and left turns (both counted from
+// the subtree's), and either the left child's record (the right one follows)
+// with the split position m, or kLeaf and the primitive count in m.
+struct Rec { float4 a; float2 b; unsigned short s, lt, child, m; };
+constexpr unsigned short kLeaf = 0xffff;
 
 struct Build {
     int n, maxLeaf, numScenes, maxBig;
+    int maxNodes;            // top nodes, and subtrees, that there is room for
     float4* pbox;            // [n][2] primitive boxes, original index
     int* idx[2];             // [n] primitive at position (ping-pong of the top phase)
     int* ordered;            // [n] final order
@@ -154,8 +156,8 @@ struct Build {
     int* sNl;                // left count
     int* chunkHist;          // [chunks][48] primitives per axis and bin
     int* chunkLeft;          // [chunks] left primitives of the node before the chunk
-    int* count;              // [8]: 0 active nodes, 1 their chunks, 2 subtrees, 4 / 5 leaf and head totals, 6 / 7 BVH4 / BVH2 levels
-    int* topLevel;           // [kMaxTopLevels + 1] first top node of each level
+    int* count;              // [8]: 0 active nodes, 1 their chunks, 2 subtrees, 3 set when maxNodes is exceeded, 4 / 5 leaf and head totals, 6 / 7 BVH4 / BVH2 levels
+    int* topLevel;           // [maxNodes + 2] first top node of each level
     Top* top;                // top nodes, level by level
     float4* topCost;
     int2* topAsg;            // (slots presented as, BVH4 level)
@@ -263,7 +265,7 @@ __global__ void k_build_init(Build b, int slots) {
 // pass over the triangles would, the first of equal values (the sign of a
 // zero) and skip NaN: each axis reduces a 64-bit key of the ordered value and
 // the position of the coordinate.
-__global__ __launch_bounds__(kTopThreads) void k_prims(Build b, const float* __restrict__ tris, int chunks) {
+__global__ __launch_bounds__(kTopThreads) void k_prims(Build b, const float* __restrict__ tris) {
     __shared__ int lds[kTopThreads / 64 * 12];
     __shared__ unsigned long long lk[kTopThreads / 64][6];
     const int j = find_seg(b.primBase, b.numScenes, blockIdx.x);
@@ -410,6 +412,8 @@ __global__ __launch_bounds__(1024) void k_top_next(Build b, int out, int init, i
                 b.chunkBase[out][rb] = rc;
                 for (int q = 0; q < 12; q++) b.actAcc[out][12 * (size_t)rb + q] = acc[q];
                 ref = topBase + m + rb;            // top nodes are numbered level by level
+            } else if (smallBase + rs >= b.maxNodes) {
+                ref = -1;                          // no room (flagged below): the build starts over
             } else {
                 Small& sm = b.small[smallBase + rs];
                 sm.g = g;
@@ -425,9 +429,11 @@ __global__ __launch_bounds__(1024) void k_top_next(Build b, int out, int init, i
         nbig += tb; nsmall += ts; nchunks += tc;
     }
     if (threadIdx.x == 0) {
+        const bool full = smallBase + nsmall > b.maxNodes || topBase + m + nbig > b.maxNodes;
         b.chunkBase[out][nbig] = nchunks;
-        b.count[0] = nbig;
-        b.count[1] = nchunks;
+        b.count[0] = full ? 0 : nbig;
+        b.count[1] = full ? 0 : nchunks;
+        if (full) b.count[3] = 1;
         b.count[2] = smallBase + nsmall;
         b.topLevel[init ? 0 : level + 1] = topBase + m;
     }
@@ -776,7 +782,7 @@ struct SubLds {
 };
 
 // Where a subtree's nodes go.
-struct SubOut { Rec* rec; int s, lt, maxLeaf; };
+struct SubOut { Rec* rec; int maxLeaf; };
 
 // The two children of node `rid`: records, and queue entries of those that
 // are not leaves. Called by lane 0 of a wave or by one lane per node.
@@ -784,8 +790,8 @@ template <int MAXQ>
 __device__ __forceinline__ void sub_children(SubLds<MAXQ>& S, const SubOut& o, int nxt, int rid, int lt, int start, int cnt,
                                              int nl, const float (&L)[6], const float (&R)[6]) {
     const int base = atomicAdd(&S.recs, 2);
-    o.rec[rid].child = base;
-    o.rec[rid].m = o.s + start + nl;
+    o.rec[rid].child = (unsigned short)base;
+    o.rec[rid].m = (unsigned short)(start + nl);
 #pragma unroll
     for (int k = 0; k < 2; k++) {
         const int cs = k ? start + nl : start, cc = k ? cnt - nl : nl, cl = k ? lt : lt + 1;
@@ -794,11 +800,11 @@ __device__ __forceinline__ void sub_children(SubLds<MAXQ>& S, const SubOut& o, i
         Rec& c = o.rec[base + k];
         c.a = make_float4(x[0], x[1], x[2], x[3]);
         c.b = make_float2(x[4], x[5]);
-        c.s = o.s + cs;
-        c.lt = o.lt + cl;
+        c.s = (unsigned short)cs;
+        c.lt = (unsigned short)cl;
         if (cc <= o.maxLeaf) {
-            c.child = -1;
-            c.m = cc;
+            c.child = kLeaf;
+            c.m = (unsigned short)cc;
         } else {
             const int q = cc > kTiny ? atomicAdd(&S.nbig[nxt], 1) : MAXQ - 1 - atomicAdd(&S.ntiny[nxt], 1);
             S.seg[nxt][q] = (unsigned int)cs | (unsigned int)cc << 12;
@@ -1057,7 +1063,7 @@ __global__ __launch_bounds__(kSubThreads) void k_subtree(Build b) {
     int* leafFlag = b.leafFlag + g.s;
     Rec* rec = b.rec + 2 * (size_t)g.s;
     unsigned short* lvl = b.lvl + 2 * (size_t)g.s;
-    const SubOut o{rec, g.s, g.lt, b.maxLeaf};
+    const SubOut o{rec, b.maxLeaf};
     float rb[6];
 #pragma unroll
     for (int k = 0; k < 6; k++) rb[k] = o2f(sm.bounds[k]);
@@ -1074,8 +1080,8 @@ __global__ __launch_bounds__(kSubThreads) void k_subtree(Build b) {
     if (tid == 0) {
         rec[0].a = make_float4(rb[0], rb[1], rb[2], rb[3]);
         rec[0].b = make_float2(rb[4], rb[5]);
-        rec[0].s = g.s; rec[0].lt = g.lt;
-        if (rootLeaf) { rec[0].child = -1; rec[0].m = g.c; }
+        rec[0].s = rec[0].lt = 0;
+        if (rootLeaf) { rec[0].child = kLeaf; rec[0].m = (unsigned short)g.c; }
         S.recs = 1;
         S.next = 0;
         const bool tiny = g.c <= kTiny;
@@ -1119,7 +1125,7 @@ __global__ __launch_bounds__(kSubThreads) void k_subtree(Build b) {
         for (int k = r0 + tid; k < r1; k += kSubThreads) {
             const Rec& rc = rec[k];
             float4 c = leaf_cost();
-            if (rc.child >= 0)
+            if (rc.child != kLeaf)
                 c = node_cost(area(rc.a.x, rc.a.y, rc.a.z, rc.a.w, rc.b.x, rc.b.y), cst[rc.child], cst[rc.child + 1]);
             cst[k] = c;
             gc[k] = c;
@@ -1135,7 +1141,7 @@ __global__ __launch_bounds__(kSubThreads) void k_subtree(Build b) {
 
 // ------------------------------- numbering and emission -----------------------
 // depth: BVH4 levels, BVH2 levels
-struct Emit { rt::Node2* n2; int* head; int* assign; int* depth; };
+struct Emit { rt::Node2* n2; int* head; unsigned char* assign; int* depth; };
 
 __device__ __forceinline__ void emit_node(const Emit& e, int p, const float (&bx)[6], int left, int right, int triStart,
                                           int triCount, bool head, int m) {
@@ -1145,7 +1151,7 @@ __device__ __forceinline__ void emit_node(const Emit& e, int p, const float (&bx
     nd.left = left; nd.right = right; nd.triStart = triStart; nd.triCount = triCount;
     e.n2[p] = nd;
     e.head[p] = head ? 1 : 0;
-    e.assign[p] = m;
+    e.assign[p] = (unsigned char)m;
 }
 
 // The top nodes: costs bottom-up, then slots top-down and their BVH2 nodes
@@ -1209,16 +1215,16 @@ __global__ __launch_bounds__(kThreads) void k_sub_emit(Build b, Emit e) {
         for (int k = r0 + (int)threadIdx.x; k < r1; k += kThreads) {
             const Rec rc = rec[k];
             const float bx[6] = {rc.a.x, rc.a.y, rc.a.z, rc.a.w, rc.b.x, rc.b.y};
-            const int p = pre_of(b, rc.s, rc.lt, g.tree);
+            const int lt = g.lt + rc.lt, p = pre_of(b, g.s + rc.s, lt, g.tree);
             const int m = (int)(asg[k] & 15u), lev = (int)(asg[k] >> 4);
-            if (rc.child < 0) {
-                emit_node(e, p, bx, 0, 0, rc.s, rc.m, false, m);
+            if (rc.child == kLeaf) {
+                emit_node(e, p, bx, 0, 0, g.s + rc.s, rc.m, false, m);
             } else {
                 int2 al, ar;
                 const bool head = assign_slots(cost[k], cost[rc.child], cost[rc.child + 1], m, lev, al, ar);
                 asg[rc.child] = (unsigned int)al.x | (unsigned int)al.y << 4;
                 asg[rc.child + 1] = (unsigned int)ar.x | (unsigned int)ar.y << 4;
-                emit_node(e, p, bx, p + 1, pre_of(b, rc.m, rc.lt, g.tree), 0, 0, head, m);
+                emit_node(e, p, bx, p + 1, pre_of(b, g.s + rc.m, lt, g.tree), 0, 0, head, m);
                 if (head) depth = max(depth, lev + 1);
             }
         }
@@ -1268,7 +1274,7 @@ __device__ __forceinline__ int32_t leaf_code(int first, int count) { return -((f
 // exclusive count of heads before p, i.e. the node's pre-order BVH4 index.
 // Its slots are the nodes of assign 1 below it, reached through dissolved
 // nodes (assign >= 2), left to right, so they stay in BVH2 pre-order.
-__global__ void k_emit_bvh4(const rt::Node2* n2, const int* head, const int* b4id, const int* assign, int count,
+__global__ void k_emit_bvh4(const rt::Node2* n2, const int* head, const int* b4id, const unsigned char* assign, int count,
                             uint4* out) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= count || !head[p]) return;
@@ -1478,8 +1484,7 @@ static double now_ms() {
     return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now().time_since_epoch()).count();
 }
 
-// One device allocation cut into pieces. The build needs some thirty arrays;
-// each hipFree of a large one costs 0.3 ms, one for all of them the same.
+// One device allocation cut into pieces (the build needs some thirty arrays).
 struct Slab {
     struct Piece { void** p; size_t bytes; };
     std::vector<Piece> want;
@@ -1490,12 +1495,14 @@ struct Slab {
     bool alloc() {
         size_t total = 0;
         for (const Piece& w : want) total += w.bytes;
-        if (hipMalloc(&base, total) != hipSuccess) { base = nullptr; return false; }
+        base = dev_alloc(total);
+        if (!base) return false;
         char* c = (char*)base;
         for (const Piece& w : want) { *w.p = c; c += w.bytes; }
         return true;
     }
-    ~Slab() { if (base) hipFree(base); }
+    bool idle = false;               // the build has waited for its last kernel
+    ~Slab() { if (idle) dev_free(base); else dev_release(base); }
 };
 
 #define BUILD_CHECK(cond, msg)              \
@@ -1523,8 +1530,10 @@ int mesh_bounds(const float* d_tris, int n, hipStream_t s, float* mn, float* mx)
 // Outputs (device, allocated here): nodes4 (numNodes4 x 64 B), leaf-order
 // triangles (n x 48 B), leafOf (n ints), ordered (n ints, leaf order ->
 // original index), nodes2 (pre-order rt::Node2). Returns 0 on success.
-int gpu_build(const float* d_tris, int n, int maxLeaf, hipStream_t s, GpuBVH& out, const int* sceneOff,
-              int numScenes, std::vector<int>* roots4) {
+// With room for maxNodes top nodes and subtrees; full is set (and -1 returned)
+// when they do not suffice.
+static int build_with_room(const float* d_tris, int n, int maxLeaf, hipStream_t s, GpuBVH& out, const int* sceneOff,
+                           int numScenes, std::vector<int>* roots4, size_t maxNodes, bool& full) {
     using namespace rtb;
     const double tBegin = verbose() ? now_ms() : 0.0;
     struct Report {
@@ -1554,8 +1563,11 @@ int gpu_build(const float* d_tris, int n, int maxLeaf, hipStream_t s, GpuBVH& ou
     b.n = n; b.maxLeaf = maxLeaf; b.numScenes = R;
     b.maxBig = n / (kSmall + 1) + 1;              // active nodes of one level
     const size_t maxChunks = N / kChunk + b.maxBig + 1;
+    const size_t M = maxNodes;
+    b.maxNodes = (int)M;
     Slab slab;
-    int *dTab = nullptr, *tiles = nullptr, *head = nullptr, *assign = nullptr, *b4id = nullptr, *dRoot4 = nullptr;
+    int *dTab = nullptr, *tiles = nullptr, *head = nullptr, *b4id = nullptr, *dRoot4 = nullptr;
+    unsigned char* assign = nullptr;
     float* dBounds = nullptr;
     slab.add(&dTab, 2 * (size_t)(R + 1));
     slab.add(&b.pbox, 2 * N);
@@ -1570,17 +1582,19 @@ int gpu_build(const float* d_tris, int n, int maxLeaf, hipStream_t s, GpuBVH& ou
     slab.add(&b.sAxis, b.maxBig); slab.add(&b.sBin, b.maxBig); slab.add(&b.sNl, b.maxBig);
     slab.add(&b.chunkHist, maxChunks * kCells); slab.add(&b.chunkLeft, maxChunks);
     slab.add(&b.count, 8);
-    slab.add(&b.topLevel, N + 2);                 // a level splits at least one node
-    slab.add(&b.top, N); slab.add(&b.topCost, N); slab.add(&b.topAsg, N);
-    slab.add(&b.small, N); slab.add(&b.smallCost, N); slab.add(&b.smallAsg, N);
+    slab.add(&b.topLevel, M + 2);                 // a level splits at least one node
+    slab.add(&b.top, M); slab.add(&b.topCost, M); slab.add(&b.topAsg, M);
+    slab.add(&b.small, M); slab.add(&b.smallCost, M); slab.add(&b.smallAsg, M);
     slab.add(&b.rec, 2 * N); slab.add(&b.cost, 2 * N); slab.add(&b.lvl, 2 * N + 2);
     slab.add(&head, 2 * N); slab.add(&assign, 2 * N); slab.add(&b4id, 2 * N);
     slab.add(&tiles, scan_tiles_needed((int)std::min<size_t>(2 * N, 0x7fffffff)) + 8);
     slab.add(&dRoot4, R);
     slab.add(&dBounds, 8);
     BUILD_CHECK(slab.alloc(), "gpu build: out of device memory");
-    if (hipMalloc((void**)&out.ordered, N * 4) != hipSuccess || hipMalloc(&out.tris, N * 48) != hipSuccess ||
-        hipMalloc((void**)&out.leafOf, N * 4) != hipSuccess) {
+    out.ordered = (int*)dev_alloc(N * 4);
+    out.tris = dev_alloc(N * 48);
+    out.leafOf = (int*)dev_alloc(N * 4);
+    if (!out.ordered || !out.tris || !out.leafOf) {
         set_error("gpu build: out of device memory");
         return -1;
     }
@@ -1594,7 +1608,7 @@ int gpu_build(const float* d_tris, int n, int maxLeaf, hipStream_t s, GpuBVH& ou
     auto grid = [](long long items) { return dim3((unsigned)((items + kThreads - 1) / kThreads)); };
     const int slots0 = std::max(big0, 1);
     hipLaunchKernelGGL(k_build_init, grid(std::max(R * 12, slots0 * kSlotInts)), dim3(T), 0, s, b, slots0);
-    hipLaunchKernelGGL(k_prims, dim3(hBase[R]), dim3(kTopThreads), 0, s, b, d_tris, hBase[R]);
+    hipLaunchKernelGGL(k_prims, dim3(hBase[R]), dim3(kTopThreads), 0, s, b, d_tris);
     hipLaunchKernelGGL(k_mesh_bounds, dim3(1), dim3(64), 0, s, d_tris, b.bnd, dBounds);
     hipLaunchKernelGGL(k_top_next, dim3(1), dim3(1024), 0, s, b, 0, 1, 0);
     // Levels until no node of more than kSmall primitives is left. The
@@ -1631,6 +1645,10 @@ int gpu_build(const float* d_tris, int n, int maxLeaf, hipStream_t s, GpuBVH& ou
         set_error("gpu build: top levels failed");
         return -1;
     }
+    if (hc[3]) {
+        full = true;
+        return -1;
+    }
     const int numSmall = hc[2];
     // subtrees: narrow queues (more workgroups per CU) where the leaves hold four
     if (maxLeaf >= 4)
@@ -1645,7 +1663,7 @@ int gpu_build(const float* d_tris, int n, int maxLeaf, hipStream_t s, GpuBVH& ou
     }
     const int nodeCount = 2 * leaves - R;
     out.numNodes2 = nodeCount;
-    if (leaves <= 0 || hipMalloc((void**)&out.nodes2, (size_t)nodeCount * sizeof(Node2)) != hipSuccess) {
+    if (leaves <= 0 || !(out.nodes2 = (Node2*)dev_alloc((size_t)nodeCount * sizeof(Node2)))) {
         set_error("gpu build: out of device memory");
         return -1;
     }
@@ -1666,7 +1684,7 @@ int gpu_build(const float* d_tris, int n, int maxLeaf, hipStream_t s, GpuBVH& ou
     const int heads = fin[0];
     out.numNodes4 = std::max(heads, 1);
     out.depth4 = std::max(fin[1], 1);             // a leaf root is one node
-    if (hipMalloc(&out.nodes4, (size_t)out.numNodes4 * 64) != hipSuccess) {
+    if (!(out.nodes4 = dev_alloc((size_t)out.numNodes4 * 64))) {
         set_error("gpu build: out of device memory");
         return -1;
     }
@@ -1687,7 +1705,25 @@ int gpu_build(const float* d_tris, int n, int maxLeaf, hipStream_t s, GpuBVH& ou
     if (e == hipSuccess) e = hipGetLastError();
     if (e != hipSuccess) { set_error("gpu build failed: %s", hipGetErrorString(e)); return -1; }
     out.levels = fin[2];
+    slab.idle = true;
     return 0;
+}
+
+// The subtrees of a tree hold hundreds to 2048 primitives each; room for one
+// per 128 is enough for all but trees that split off a few primitives at a
+// time, level after level, and those start over with room for the worst case.
+int gpu_build(const float* d_tris, int n, int maxLeaf, hipStream_t s, GpuBVH& out, const int* sceneOff,
+              int numScenes, std::vector<int>* roots4) {
+    const size_t N = (size_t)std::max(n, 1), room = std::min(N, N / 128 + 1024 + (size_t)numScenes);
+    bool full = false;
+    int rc = build_with_room(d_tris, n, maxLeaf, s, out, sceneOff, numScenes, roots4, room, full);
+    if (rc != 0 && full) {
+        for (void* p : {(void*)out.ordered, out.tris, (void*)out.leafOf}) dev_release(p);
+        out = GpuBVH();
+        full = false;
+        rc = build_with_room(d_tris, n, maxLeaf, s, out, sceneOff, numScenes, roots4, N, full);
+    }
+    return rc;
 }
 
 }  // namespace rt

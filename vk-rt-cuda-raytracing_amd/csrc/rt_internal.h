@@ -61,6 +61,13 @@ int gpu_build(const float* d_tris, int n, int maxLeaf, hipStream_t s, GpuBVH& ou
 // the triangles computes them (from 1e30 / -1e30; the first of equal values,
 // NaN skipped). Waits for stream s. 0 on success.
 int mesh_bounds(const float* d_tris, int n, hipStream_t s, float* mn, float* mx);
+// Device memory with a bounded cache of freed blocks (devmem.hip). nullptr when
+// out of memory. dev_free: no device work uses the block any longer;
+// dev_release waits for the device first (as hipFree does). Both accept nullptr.
+void* dev_alloc(size_t bytes);
+void dev_free(void* p);
+void dev_release(void* p);
+void dev_trim();                                   // gives the cached blocks back
 void scan_exclusive(const int* in, int* out, int n, int* total, int* tiles, hipStream_t s);
 int scan_tiles_needed(int n);
 

@@ -1248,7 +1248,8 @@ int alloc_scratch(rt::TraceScratch& sc) {
 }
 
 void free_scratch(rt::TraceScratch& sc) {
-    hipFree(sc.spill); hipFree(sc.counter); hipFree(sc.status); hipFree(sc.tiles); hipFree(sc.hits);
+    rt::dev_release(sc.spill);
+    hipFree(sc.counter); hipFree(sc.status); hipFree(sc.tiles); hipFree(sc.hits);
     hipFree(sc.tileCost); hipFree(sc.tileOrder); hipFree(sc.tilePred);
     sc.spill = nullptr; sc.spillBytes = 0; sc.counter = nullptr; sc.status = nullptr;
     sc.tiles = nullptr; sc.tileCap = 0; sc.hits = nullptr; sc.hitsBytes = 0;
@@ -1295,10 +1296,11 @@ int grow_spill(rt::TraceScratch& sc, size_t need) {
         rt::set_error("fixed traversal scratch too small: %zu bytes of spill needed, %zu held", need, sc.spillBytes);
         return -1;
     }
-    hipFree(sc.spill);
-    sc.spill = nullptr; sc.spillBytes = 0;
+    rt::dev_release(sc.spill);
     sc.gen++;
-    if (hipMalloc(&sc.spill, need) != hipSuccess) {
+    sc.spillBytes = 0;
+    sc.spill = rt::dev_alloc(need);
+    if (!sc.spill) {
         rt::set_error("cannot allocate %zu bytes of traversal stack spill", need);
         return -1;
     }

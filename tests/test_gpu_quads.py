@@ -1,0 +1,175 @@
+"""Traversal with four lanes per ray: launches whose rays all run that way (the
+default below a ray count per class), and the hand-over of a wave's last rays
+to it in the larger and in the explicitly configured launches. The reference is
+the CPU oracle on the exported tree or the counted one-lane traversal; every
+value is computed by the same expressions in all of them, so IDs and bits are
+equal."""
+import numpy as np
+import pytest
+
+from conftest import hit_buffers, to_dev
+
+pytestmark = pytest.mark.gpu
+KEYS = ("t", "prim_id", "u", "v")
+
+
+def _bits(x):
+    x = np.asarray(x)
+    return x.view(np.uint32) if x.dtype == np.float32 else x
+
+
+def _rays(n, seed, flat=0.0):
+    """Rays into [-1, 1]^3, a share of them along an axis from a grid (their
+    origins lie on box planes), some with short intervals."""
+    rng = np.random.default_rng(seed)
+    r = np.zeros((8, n), np.float32)
+    d = rng.normal(size=(3, n))
+    r[0:3] = rng.uniform(-1.2, 1.2, (3, n))
+    r[3:6] = d / np.linalg.norm(d, axis=0)
+    f = rng.random(n) < flat
+    r[0:3, f] = 0.25 * rng.integers(-4, 5, (3, int(f.sum())))
+    r[3:6, f] = 0.0
+    r[3 + rng.integers(0, 3, int(f.sum())), np.flatnonzero(f)] = rng.choice([-1.0, 1.0], int(f.sum()))
+    r[7] = np.where(rng.random(n) < 0.2, rng.uniform(0.05, 1.0, n), 1e30)
+    return r
+
+
+def _soup(nt, seed, size=0.08, grid=False):
+    rng = np.random.default_rng(seed)
+    t = rng.uniform(-1, 1, (nt, 1, 3)) + rng.normal(scale=size, size=(nt, 3, 3))
+    if grid:
+        t = np.round(t * 4) / 4                       # coincident and degenerate triangles, ties in t
+    return t.astype(np.float32).reshape(nt, 9)
+
+
+def _closest(b, rays, dev, counted=False, **kw):
+    import torch
+    n = rays.shape[1]
+    R, H = to_dev(rays, dev), hit_buffers(n + 64, dev)
+    for h in H.values():
+        h.fill_(-3)
+    out = [H[k][:n] for k in KEYS]
+    if counted:
+        c = [torch.empty(n, dtype=torch.int32, device=dev) for _ in range(2)]
+        b.trace_closest_counted(R, *out, *c)
+    else:
+        b.trace_closest(R, *out, **kw)
+    torch.cuda.synchronize()
+    got = {k: H[k].cpu().numpy() for k in KEYS}
+    assert all((got[k][n:] == -3).all() for k in KEYS)
+    return {k: got[k][:n] for k in KEYS}
+
+
+def _any(b, rays, dev, counted=False):
+    import torch
+    n = rays.shape[1]
+    occ = torch.full((n + 64,), 7, dtype=torch.uint8, device=dev)
+    if counted:
+        c = [torch.empty(n, dtype=torch.int32, device=dev) for _ in range(2)]
+        b.trace_any_counted(to_dev(rays, dev), occ[:n], *c)
+    else:
+        b.trace_any(to_dev(rays, dev), occ[:n])
+    torch.cuda.synchronize()
+    occ = occ.cpu().numpy()
+    assert (occ[n:] == 7).all()
+    return occ[:n]
+
+
+def _same(a, b):
+    for k in KEYS:
+        assert np.array_equal(_bits(a[k]), _bits(b[k])), (k, int((_bits(a[k]) != _bits(b[k])).sum()))
+
+
+@pytest.mark.parametrize("nt,grid", [(1, False), (3, False), (40, True), (20000, False)])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 64, 65, 3001])
+def test_small_launches(pkg, oracle, dev, n, nt, grid):
+    """Ray counts at and beside a wave's 16 rays, trees from one leaf up,
+    flat rays mixed in; closest hits and occlusion as the oracle's, with the
+    borrowed scratch too, and through every configured schedule."""
+    rays = _rays(n, 5 * n + nt, flat=0.3)
+    with pkg.BVH.build(_soup(nt, nt, size=0.4 if nt < 100 else 0.08, grid=grid)) as b:
+        nodes, lt, pid = b.node_data(), np.ascontiguousarray(b.tri_data().T), b.leaf_prim_ids()
+        r = oracle.trace_closest(nodes, lt, pid, rays)
+        ref = {"t": r["t"], "prim_id": r["id"], "u": r["u"], "v": r["v"]}
+        occ = oracle.trace_any(nodes, lt, pid, rays)["occ"]
+        _same(_closest(b, rays, dev), ref)
+        assert np.array_equal(_any(b, rays, dev), occ)
+        H = hit_buffers(n, dev)
+        b.trace_closest_no_alloc(to_dev(rays, dev), *[H[k] for k in KEYS])
+        import torch
+        torch.cuda.synchronize()
+        _same({k: H[k].cpu().numpy() for k in KEYS}, ref)
+        for sched in (pkg.SCHEDULE_BATCH, pkg.SCHEDULE_REFILL):
+            b.set_trace_config(pkg.CLASS_INCOHERENT, sched, 4, 1)
+            b.set_trace_config(pkg.CLASS_ANY, sched, 4, 1)
+            _same(_closest(b, rays, dev), ref)
+            assert np.array_equal(_any(b, rays, dev), occ)
+
+
+@pytest.mark.parametrize("depth", [4, 8])
+def test_deep_tree(pkg, dev, depth):
+    """A tree whose stacks pass both LDS depths: triangles in nested shells of
+    geometrically shrinking size, so that boxes nest and few rays skip any."""
+    rng = np.random.default_rng(3)
+    k = np.arange(6000)
+    s = (0.5 ** (k / 150.0))[:, None, None]
+    tris = (s * rng.normal(size=(6000, 3, 3))).astype(np.float32).reshape(-1, 9)
+    rays = _rays(3000, 11)
+    rays[0:3] *= rng.uniform(0.0, 1.0, 3000).astype(np.float32) ** 8
+    with pkg.BVH.build(tris) as b:
+        assert 3 * b.depth + 4 > 24
+        ref, occ = _closest(b, rays, dev, counted=True), _any(b, rays, dev, counted=True)
+        _same(_closest(b, rays, dev), ref)
+        assert np.array_equal(_any(b, rays, dev), occ)
+        for sched in (pkg.SCHEDULE_BATCH, pkg.SCHEDULE_REFILL):
+            b.set_trace_config(pkg.CLASS_INCOHERENT, sched, depth, 1)
+            b.set_trace_config(pkg.CLASS_ANY, sched, depth, 1)
+            _same(_closest(b, rays, dev), ref)
+            assert np.array_equal(_any(b, rays, dev), occ)
+        assert b.trace_status() == 0
+
+
+@pytest.mark.parametrize("n", [1 << 18, (1 << 18) + 1, (1 << 19) + 17])
+def test_both_sides_of_the_ray_count_rule(pkg, dev, n):
+    """Launches at, and just past, the ray counts where the kernels change; a
+    queue of the same capacity holding fewer rays."""
+    import torch
+    rays = _rays(n, n, flat=0.02)
+    with pkg.BVH.build(_soup(30000, 8, size=0.03)) as b:
+        ref, occ = _closest(b, rays, dev, counted=True), _any(b, rays, dev, counted=True)
+        _same(_closest(b, rays, dev), ref)
+        assert np.array_equal(_any(b, rays, dev), occ)
+        m = n // 3 + 5
+        cnt = torch.tensor([m], dtype=torch.int32, device=dev)
+        R, H = to_dev(rays, dev), hit_buffers(n, dev)
+        for h in H.values():
+            h.fill_(-3)
+        o = torch.full((n,), 7, dtype=torch.uint8, device=dev)
+        b.trace_closest_queued(n, cnt, R, *[H[k] for k in KEYS])
+        b.trace_any_queued(n, cnt, R, o)
+        torch.cuda.synchronize()
+        _same({k: H[k][:m].cpu().numpy() for k in KEYS}, {k: ref[k][:m] for k in KEYS})
+        assert all((H[k][m:] == -3).all().item() for k in KEYS)
+        assert np.array_equal(o[:m].cpu().numpy(), occ[:m]) and (o[m:] == 7).all().item()
+
+
+@pytest.mark.parametrize("W,H", [(1, 1), (3, 5), (4, 4), (61, 33), (677, 679)])
+def test_pinhole_images(pkg, oracle, scenes, dev, W, H):
+    """4 x 4 pixel tiles cut off at the right and bottom edge, and an image
+    past the ray count where the batch kernel takes over (677 x 679, plain and
+    cost-ordered): every pixel as the explicit rays' counted trace."""
+    import torch
+    cam = scenes.parity_camera(W, H)
+    rays = oracle.gen_pinhole(scenes.cam_array(cam), W, H)
+    c = pkg.camera(cam["o"], cam["f"], cam["r"], cam["u"], cam["scale_x"], cam["scale_y"])
+    with pkg.BVH.build(scenes.random_triangles(20000, seed=2)) as b:
+        ref = _closest(b, rays, dev, counted=True)
+        for flags in (0, pkg.FLAG_COST_ORDER, pkg.FLAG_COST_ORDER):
+            hb = hit_buffers(W * H + 64, dev)
+            for h in hb.values():
+                h.fill_(-3)
+            b.trace_pinhole_closest(W, H, c, *[hb[k] for k in KEYS], flags=flags)
+            torch.cuda.synchronize()
+            got = {k: hb[k].cpu().numpy() for k in KEYS}
+            _same({k: got[k][:W * H] for k in KEYS}, ref)
+            assert all((got[k][W * H:] == -3).all() for k in KEYS)

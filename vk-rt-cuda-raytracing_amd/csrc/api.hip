@@ -1235,6 +1235,7 @@ int cudaBVH_setTraceConfig(CudaBVH_t bvh, int rayClass, int schedule, int ldsDep
     bvh->tune[rayClass].schedule = schedule;
     bvh->tune[rayClass].ldsDepth = ldsDepth;
     bvh->tune[rayClass].blocksPerCU = blocksPerCU;
+    bvh->tune[rayClass].chosen = true;
     return 0;
 }
 
@@ -1294,6 +1295,7 @@ int cudaBVH_autotune(CudaBVH_t bvh, int rayClass, int width, int height, const C
                 bvh->tune[rayClass].schedule = sch;
                 bvh->tune[rayClass].ldsDepth = d;
                 bvh->tune[rayClass].blocksPerCU = b;
+                bvh->tune[rayClass].chosen = true;       // times this schedule whatever the ray count
                 rtk::TraceArgs a = base;
                 rc = rtk::launch_trace(bvh, bvh->scratch, a, mode, false, coherent, false, s);   // warm-up
                 hipEventRecord(e0, s);
@@ -1321,6 +1323,7 @@ int cudaBVH_autotune(CudaBVH_t bvh, int rayClass, int width, int height, const C
     hipEventDestroy(e0); hipEventDestroy(e1);
     hipFree(out);
     bvh->tune[rayClass] = rc == 0 ? best : saved;
+    bvh->tune[rayClass].chosen = saved.chosen;
     if (numResults) *numResults = row;
     return rc;
 }

@@ -96,6 +96,7 @@ struct TraceConfig {
     int schedule = kScheduleBatch;
     int ldsDepth = 16;
     int blocksPerCU = 0;
+    bool chosen = false;                // set by the caller: small launches keep this schedule too
 };
 
 // Resources of one traversal kernel, read once per kernel (hipFuncGetAttributes

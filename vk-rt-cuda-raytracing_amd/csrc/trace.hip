@@ -17,6 +17,7 @@
 // t. Any-hit pushes children unsorted in slot order (v10_pipeline.cu:241-244).
 #include "rt_device.h"
 #include "rt_internal.h"
+#include "rt_quad.h"
 #include "trace_launch.h"
 
 #include <algorithm>
@@ -135,6 +136,10 @@ struct Result {
     bool occluded;
     int visits, tests;
     int steps;         // loop steps of the ray (batch schedule)
+    // a ray handed over to a quad (batch schedule): what it visits next and its stack
+    bool open;
+    int ref, sp;
+    float tn;
 };
 
 // Closest-hit result of ray ri. The while-while kernel, whose lanes finish
@@ -328,6 +333,13 @@ __global__ void k_fill_i32(int* p, int n, int v) {
 // the short ones sharing its SIMD (on that view: 0.55 to 0.46 ms per launch).
 constexpr int kPrioSteps = 32;   // loop steps per wave-priority level
 
+// Rays left in a wave when four lanes take each of them over (rt_quad.h): as
+// many as it has quads.
+constexpr int kQuadRays = 16;
+
+// A leaf cursor (triangles [first, first + count)) as a leaf code.
+__device__ __forceinline__ int cursor_code(int first, int count) { return -((first << 3) | (count - 1)) - 2; }
+
 template <int MODE, bool MT, bool FLAT, int LDSD, int BLOCK>
 __device__ __forceinline__ void trace_ray(const TraceArgs& a, const Ray& r, int* s_ref, float* s_tn, int tid,
                                              int gtid, Result& res, int root, int pc) {
@@ -432,6 +444,186 @@ __device__ __forceinline__ void trace_ray(const TraceArgs& a, const Ray& r, int*
     res.occluded = found; res.visits = visits; res.tests = tests; res.steps = steps;
 }
 
+// The same steps for a whole wave at once, ending when at most kQuadRays
+// lanes still hold a ray (res.open): those go on in quads (finish_quads).
+// Uncounted watertight launches. Every lane calls it; `live` lanes hold a ray.
+// The loop is wave-uniform: with lanes leaving it one by one, each value of
+// theirs that is needed afterwards took a second register (105 VGPRs instead
+// of 80).
+template <int MODE, int LDSD, int BLOCK>
+__device__ __forceinline__ void trace_wave(const TraceArgs& a, const Ray& r, bool live, bool flat, int* s_ref, float* s_tn, int tid,
+                                           int gtid, Result& res, int root, int pc) {
+    const uint4* __restrict__ nodes = a.nodes;
+    const float4* __restrict__ tris = a.tris;
+    int sp = 0, ref = root, bid = -1, lts = 0, ltc = 0;
+    float tn = -INFINITY, best = r.tmax, bu = 0.f, bv = 0.f;
+    bool has = live, found = false;
+    auto push = [&](int rf, float t) {
+        if (sp < LDSD) {
+            s_ref[sp * BLOCK + tid] = rf;
+            s_tn[sp * BLOCK + tid] = t;
+        } else if (sp < a.maxStack) {
+            a.spill[spill_index<LDSD>(a, sp, gtid)] = make_int2(rf, __float_as_int(t));
+        } else {
+            atomicOr(a.status, 1);
+            return;
+        }
+        sp++;
+    };
+    int steps = 0;
+    for (;;) {
+        if (__popcll(__ballot(has)) <= a.quadRays) break;
+        steps++;
+        if (steps == kPrioSteps) __builtin_amdgcn_s_setprio(1);
+        else if (steps == 2 * kPrioSteps) __builtin_amdgcn_s_setprio(2);
+        else if (steps == 3 * kPrioSteps) __builtin_amdgcn_s_setprio(3);
+        if (!has) continue;
+        bool cont = false;
+        if (ltc == 0 && ref < 0 && (MODE == kModeAny || tn <= best)) {
+            const int enc = -(ref + 2);
+            lts = enc >> 3; ltc = (enc & 7) + 1;
+        }
+        if (ltc > 0) {
+            // two triangles per step when the leaf has two left (as trace_ray)
+            const int ti = lts;
+            const bool two = ltc > 1;
+            const int tj = two ? ti + 1 : ti;
+            const float4 p0 = tris[3 * ti], p1 = tris[3 * ti + 1], p2 = tris[3 * ti + 2];
+            const float4 q0 = tris[3 * tj], q1 = tris[3 * tj + 1], q2 = tris[3 * tj + 2];
+            auto test = [&](const float4& a0, const float4& a1, const float4& a2) {
+                float t, u, v;
+                if (rtd::isect_watertight_wave(r, pc, a0, a1, a2, t, u, v) && t > r.tmin && t < r.tmax) {
+                    if constexpr (MODE == kModeAny) return true;
+                    const int id = __float_as_int(a0.w);
+                    if (t < best || (t == best && id < bid)) { best = t; bid = id; bu = u; bv = v; }
+                }
+                return false;
+            };
+            if (test(p0, p1, p2) || (two && test(q0, q1, q2))) { found = true; has = false; continue; }
+            lts += two ? 2 : 1;
+            ltc -= two ? 2 : 1;
+            cont = ltc > 0;
+        } else if (ref >= 0 && (MODE == kModeAny || tn <= best)) {
+            int nxt = ref;
+            float nt = 0.f;
+            if constexpr (MODE == kModeAny) {
+                if (flat) visit_any<true>(nodes, r, nxt, push);
+                else visit_any<false>(nodes, r, nxt, push);
+            } else {
+                if (flat) visit_closest<true>(nodes, r, best, nxt, nt, push);
+                else visit_closest<false>(nodes, r, best, nxt, nt, push);
+            }
+            if (nxt != -1) { ref = nxt; tn = nt; cont = true; }
+        }
+        if (!cont) {
+            if (sp == 0) {
+                has = false;
+            } else {
+                sp--;
+                if (sp < LDSD) {
+                    ref = s_ref[sp * BLOCK + tid];
+                    tn = s_tn[sp * BLOCK + tid];
+                } else {
+                    // non-temporal: kept apart from the LDS read, as in trace_ray
+                    typedef int v2i __attribute__((ext_vector_type(2)));
+                    const v2i e = __builtin_nontemporal_load((const v2i*)&a.spill[spill_index<LDSD>(a, sp, gtid)]);
+                    ref = e.x; tn = __int_as_float(e.y);
+                }
+            }
+        }
+    }
+    __builtin_amdgcn_s_setprio(0);
+    res.t = best; res.u = bu; res.v = bv; res.id = bid;
+    res.occluded = found; res.steps = steps;
+    res.open = has;
+    res.ref = ltc > 0 ? cursor_code(lts, ltc) : ref;
+    res.tn = tn;
+    res.sp = sp;
+}
+
+// Rays that a wave has left (lanes with `open`, at most kQuadRays of them) go
+// on with four lanes each: quad k takes over the k-th open lane's ray, its
+// closest hit so far and its stack (in place, in that lane's column). Every
+// lane of the wave calls it. The ray itself is read (or generated) again:
+// moving it across lanes held both copies in registers at once (97 VGPRs
+// instead of 80). Results go straight to the output arrays. Returns the
+// longest quad's steps.
+template <int MODE, bool PIN, int LDSD, int BLOCK>
+__device__ __forceinline__ int finish_quads(const TraceArgs& a, bool open, bool flat, int ref, float tn, int sp, float best,
+                                            float bu, float bv, int bid, int ri, int* s_ref, float* s_tn, int tid,
+                                            int gtid) {
+    constexpr bool ANY = MODE == kModeAny;
+    // opaque copies: otherwise every lane-dependent address of this phase is
+    // computed ahead of the caller's loops and held through them
+    asm volatile("" : "+v"(tid), "+v"(gtid));
+    const uint64_t mask = __ballot(open);
+    const int lane = tid & 63, src = rtq::source_lane(mask, lane), from = src < 0 ? lane : src;
+    rtq::Ray4 q;
+    ri = rtq::take(from, ri);
+    q.ref = rtq::take(from, ref);
+    q.tn = rtq::take(from, tn);
+    q.sp = rtq::take(from, sp);
+    if constexpr (!ANY) {
+        q.best = q.t = rtq::take(from, best);
+        q.id = rtq::take(from, bid);
+        q.u = rtq::take(from, bu); q.v = rtq::take(from, bv);
+        if ((lane & 3) != 0) { q.t = INFINITY; q.id = -1; }   // one lane holds the hit so far
+    }
+    q.col = from - lane;                           // the ray's stack column, as an offset to this lane's
+    q.found = false;
+    if (src >= 0) {
+        Ray r;
+        if constexpr (PIN) {
+            const int py = ri / a.W;
+            rtd::pinhole_ray(a.cam, ri - py * a.W, py, a.W, a.H, r);
+        } else {
+            r.ox = a.ox[ri]; r.oy = a.oy[ri]; r.oz = a.oz[ri];
+            r.dx = a.dx[ri]; r.dy = a.dy[ri]; r.dz = a.dz[ri];
+            r.tmin = a.tmin[ri]; r.tmax = a.tmax[ri];
+        }
+        rtd::ray_setup(r);
+        rtq::set_ray(q, r);
+    }
+    int steps = 0;
+    if (src >= 0) {
+        __builtin_amdgcn_s_setprio(3);
+        auto push = [&](rtq::Ray4& z, int at, int rf, float t) {
+            if (at < LDSD) {
+                s_ref[at * BLOCK + tid + z.col] = rf;
+                s_tn[at * BLOCK + tid + z.col] = t;
+            } else {
+                a.spill[spill_index<LDSD>(a, at, gtid + z.col)] = make_int2(rf, __float_as_int(t));
+            }
+        };
+        auto pop = [&](rtq::Ray4& z, int at, int& rf, float& t) {
+            if (at < LDSD) {
+                rf = s_ref[at * BLOCK + tid + z.col];
+                t = s_tn[at * BLOCK + tid + z.col];
+            } else {
+                typedef int v2i __attribute__((ext_vector_type(2)));
+                const v2i e = __builtin_nontemporal_load((const v2i*)&a.spill[spill_index<LDSD>(a, at, gtid + z.col)]);
+                rf = e.x; t = __int_as_float(e.y);
+            }
+        };
+        steps = flat ? rtq::traverse<ANY, true>(q, lane, a.nodes, a.tris, a.maxStack, a.status, push, pop)
+                     : rtq::traverse<ANY, false>(q, lane, a.nodes, a.tris, a.maxStack, a.status, push, pop);
+        __builtin_amdgcn_s_setprio(0);
+        if constexpr (!ANY) rtq::reduce(q);
+        if ((lane & 3) == 0) {
+            if constexpr (ANY) {
+                a.occ[ri] = q.found ? 1 : 0;
+            } else {
+                const bool hit = q.id >= 0;
+                a.t[ri] = hit ? q.t : RT_MISS_T;
+                if (a.id) a.id[ri] = q.id;
+                if (a.u) a.u[ri] = hit ? q.u : 0.f;
+                if (a.v) a.v[ri] = hit ? q.v : 0.f;
+            }
+        }
+    }
+    return rtd::wave_max(steps);
+}
+
 // Refill schedule: the batch schedule's one-short-step loop (a node visit or
 // one or two triangles per iteration, as trace_ray), but a lane whose ray finished
 // takes the next work item from the wave's pool of 64 (one 8x8 tile for
@@ -465,6 +657,7 @@ __global__ __launch_bounds__(BLOCK) void k_trace_refill(TraceArgs a) {
     // written one by one, a ray's four results each dirtied an L2 sector of
     // its own. Two pools per wave are held; a third evicts the older one
     // (its gathered results go out, its later rays are written directly).
+    constexpr bool QUAD = !MT && MODE != kModeShade;
     constexpr bool POOL = MODE == kModeClosest && !PIN;
     constexpr int kSlots = 2;
     __shared__ float4 s_rec[POOL ? (BLOCK / 64) * kSlots * 64 : 1];
@@ -576,6 +769,10 @@ __global__ __launch_bounds__(BLOCK) void k_trace_refill(TraceArgs a) {
             if (exhausted && poolNext >= poolEnd) break;
             continue;
         }
+        if constexpr (QUAD) {
+            // nothing left to take: the last rays go on with four lanes each
+            if (exhausted && poolNext >= poolEnd && __popcll(__ballot(has)) <= a.quadRays) break;
+        }
         const bool waveFlat = __any(has && flat);
         if (!has) continue;
         bool cont = false, fin = false, found = false;
@@ -658,15 +855,113 @@ __global__ __launch_bounds__(BLOCK) void k_trace_refill(TraceArgs a) {
         }
 
     }
+    if constexpr (QUAD) {
+        if constexpr (POOL) {
+            // gathered results go out; the remaining rays write theirs directly
+            for (int sl = 0; sl < kSlots; sl++)
+                if (sbase[sl] >= 0) flush(sl);
+        }
+        if (__any(has))
+            finish_quads<MODE, PIN, LDSD, BLOCK>(a, has, __any(has && flat), ltc > 0 ? cursor_code(lts, ltc) : ref, tn, sp,
+                                                 best, bu, bv, bid, ri, s_ref, s_tn, tid, gtid);
+    }
+}
+
+// Small launches: four lanes per ray from the start, 16 rays (a 4x4 pixel tile
+// for pinhole rays) per wave and workgroup, no work counter. A launch of a few
+// thousand rays leaves most of the chip idle at one lane per ray, and its time
+// is the chain of its longest ray.
+constexpr int kQuadLds = 24;                       // LDS stack entries per quad
+
+template <int MODE, bool PIN>
+__global__ __launch_bounds__(64) void k_trace_quad(TraceArgs a) {
+    constexpr bool ANY = MODE == kModeAny;
+    __shared__ int s_ref[kQuadLds * 16];
+    __shared__ float s_tn[kQuadLds * 16];
+    const int lane = threadIdx.x, qd = lane >> 2;
+    const int tilesX = (a.W + 3) >> 2;
+    const int n = PIN ? tilesX * ((a.H + 3) >> 2) * 16 : (a.nDev ? min(*a.nDev, a.n) : a.n);
+    for (int base = blockIdx.x * 16; base < n; base += gridDim.x * 16) {
+        int ri = base + qd, px = 0, py = 0;
+        bool live = ri < n;
+        if constexpr (PIN) {
+            const int tile = base >> 4, ty = tile / tilesX;
+            px = (tile - ty * tilesX) * 4 + (qd & 3);
+            py = ty * 4 + (qd >> 2);
+            live = px < a.W && py < a.H;
+            ri = py * a.W + px;
+        }
+        Ray r;
+        rtq::Ray4 q;
+        bool flat = false;
+        if (live) {
+            if constexpr (PIN) {
+                rtd::pinhole_ray(a.cam, px, py, a.W, a.H, r);
+            } else {
+                r.ox = a.ox[ri]; r.oy = a.oy[ri]; r.oz = a.oz[ri];
+                r.dx = a.dx[ri]; r.dy = a.dy[ri]; r.dz = a.dz[ri];
+                r.tmin = a.tmin[ri]; r.tmax = a.tmax[ri];
+            }
+            rtd::ray_setup(r);
+            flat = rtd::ray_flat(r);
+            rtq::set_ray(q, r);
+            q.best = r.tmax;
+            q.t = INFINITY; q.u = q.v = 0.f; q.id = -1;
+            if ((lane & 3) == 0) q.t = r.tmax;
+            q.ref = ray_root(a, ri); q.tn = -INFINITY;
+            q.sp = 0; q.col = qd;
+            q.found = false;
+        }
+        const bool anyFlat = __any(flat);
+        if (!live) continue;
+        const size_t column = (size_t)blockIdx.x * 16;
+        auto push = [&](rtq::Ray4& z, int at, int rf, float t) {
+            if (at < kQuadLds) {
+                s_ref[at * 16 + z.col] = rf;
+                s_tn[at * 16 + z.col] = t;
+            } else {
+                a.spill[(size_t)(at - kQuadLds) * a.spillStride + column + z.col] = make_int2(rf, __float_as_int(t));
+            }
+        };
+        auto pop = [&](rtq::Ray4& z, int at, int& rf, float& t) {
+            if (at < kQuadLds) {
+                rf = s_ref[at * 16 + z.col];
+                t = s_tn[at * 16 + z.col];
+            } else {
+                const int2 e = a.spill[(size_t)(at - kQuadLds) * a.spillStride + column + z.col];
+                rf = e.x; t = __int_as_float(e.y);
+            }
+        };
+        if (anyFlat) rtq::traverse<ANY, true>(q, lane, a.nodes, a.tris, a.maxStack, a.status, push, pop);
+        else rtq::traverse<ANY, false>(q, lane, a.nodes, a.tris, a.maxStack, a.status, push, pop);
+        if constexpr (!ANY) rtq::reduce(q);
+        if ((lane & 3) == 0) {
+            if constexpr (ANY) {
+                a.occ[ri] = q.found ? 1 : 0;
+            } else {
+                const bool hit = q.id >= 0;
+                a.t[ri] = hit ? q.t : RT_MISS_T;
+                if (a.id) a.id[ri] = q.id;
+                if (a.u) a.u[ri] = hit ? q.u : 0.f;
+                if (a.v) a.v[ri] = hit ? q.v : 0.f;
+            }
+        }
+    }
 }
 
 // Batch schedule: each wave takes 64 rays (one 8x8 pixel tile for pinhole
 // rays) with one atomicAdd and runs until all 64 are done. Best for coherent
-// rays, whose lanes stay in step. Compiled for seven waves per SIMD (72
-// VGPRs, no scratch): with an LDS stack of 8 entries seven fit, and the
-// 1080p primaries ran ~2 % faster than at six.
+// rays, whose lanes stay in step. Uncounted watertight launches hand a wave's
+// last kQuadRays rays to quads, four lanes each: a launch's end is the chain
+// of steps of its slowest tiles, mostly run by waves with few rays left. That
+// takes 91 VGPRs (85 for any hit), five waves per SIMD instead of seven: on a
+// 0.5 M triangle terrain the pinhole launch of 1280 x 720 went from 318 to
+// 299 us and of 768 x 768 from 270 to 233 us, the cost-ordered one of
+// 1024 x 1024 from 279 to 243 us; the cost-ordered 1080p one, which the order
+// keeps busy to its end, from 366 to 385 us (on a triangle soup of 1 M from
+// 468 to 415). Squeezed to six waves it spilled registers to scratch.
 template <int MODE, bool MT, bool PIN, bool COUNT, int LDSD, int BLOCK>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(7))) void k_trace_batch(TraceArgs a) {
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_trace_batch(TraceArgs a) {
     __shared__ int s_ref[LDSD * BLOCK];
     __shared__ float s_tn[LDSD * BLOCK];
     const int tid = threadIdx.x;
@@ -714,12 +1009,22 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(7))) void
         // the live lanes' shared watertight axis permutation (-1: mixed)
         const int pc = MT ? -1 : rtd::wave_perm(r, live);
         int bsteps = 0;
-        if (live) {
-            Result res;
-            const int root = ray_root(a, ri);
-            if (anyFlat) trace_ray<MODE, MT, true, LDSD, BLOCK>(a, r, s_ref, s_tn, tid, gtid, res, root, pc);
-            else trace_ray<MODE, MT, false, LDSD, BLOCK>(a, r, s_ref, s_tn, tid, gtid, res, root, pc);
-
+        constexpr bool QUAD = !MT && !COUNT && MODE != kModeShade;
+        Result res;
+        if constexpr (QUAD) {
+            const int root = live ? ray_root(a, ri) : 0;
+            trace_wave<MODE, LDSD, BLOCK>(a, r, live, anyFlat, s_ref, s_tn, tid, gtid, res, root, pc);
+            bsteps = res.steps;
+        } else {
+            res.open = false;
+            if (live) {
+                const int root = ray_root(a, ri);
+                if (anyFlat) trace_ray<MODE, MT, true, LDSD, BLOCK>(a, r, s_ref, s_tn, tid, gtid, res, root, pc);
+                else trace_ray<MODE, MT, false, LDSD, BLOCK>(a, r, s_ref, s_tn, tid, gtid, res, root, pc);
+                bsteps = res.steps;
+            }
+        }
+        if (live && !res.open) {
             if constexpr (MODE == kModeAny) {
                 a.occ[ri] = res.occluded ? 1 : 0;
             } else if constexpr (MODE == kModeClosest) {
@@ -735,13 +1040,18 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(7))) void
                 a.cntNodes[ri] = res.visits;
                 a.cntTris[ri] = res.tests;
             }
-            bsteps = res.steps;
+        }
+        int qsteps = 0;
+        if constexpr (QUAD) {
+            if (__any(res.open))
+                qsteps = finish_quads<MODE, PIN, LDSD, BLOCK>(a, res.open, anyFlat, res.ref, res.tn, res.sp, res.t, res.u,
+                                                              res.v, res.id, ri, s_ref, s_tn, tid, gtid);
         }
         // a cost-ordered launch records the batch's step count (its slowest
         // lane's) for the next launch's order, row-major by tile position
         if constexpr (PIN && !COUNT) {
             if (a.tileCost) {
-                const int m = rtd::wave_max(bsteps);
+                const int m = rtd::wave_max(bsteps) + qsteps / 2;   // a quad's step is about half as long
                 if (lane == 0 && (unsigned)tile < (unsigned)a.nTiles) a.tileCost[ty * a.tilesX + tx] = m;
             }
         }
@@ -1187,6 +1497,7 @@ static int launch_kernel(const CudaBVHHandle* h, rt::TraceScratch& sc, TraceArgs
     a.spillStride = perWave ? threads / 64 : threads;
     a.counter = sc.counter;
     a.status = sc.status;
+    a.quadRays = rtq::fits(h->numNodes4, h->numOrdered) ? kQuadRays : 0;
     a.nodes = (const uint4*)h->d_nodes4;
     a.tris = (const float4*)h->d_tris;
     // staged hit records (not with the borrowed fixed scratch, which has no room for them)
@@ -1204,6 +1515,39 @@ static int launch_kernel(const CudaBVHHandle* h, rt::TraceScratch& sc, TraceArgs
                            a.v);
     }
     hipError_t e = hipGetLastError();
+    if (e != hipSuccess) { rt::set_error("trace launch failed: %s", hipGetErrorString(e)); return -1; }
+    return 0;
+}
+
+// Launch of k_trace_quad: one wave per workgroup, 16 rays each, as many
+// workgroups as there are rays, or as the stack spill has columns for. The
+// spill is sized as for the 256-thread kernels at full occupancy, whatever the
+// ray count: a launch that takes one of them after this one finds its room
+// (growing it would allocate, which a stream capture does not allow).
+template <int MODE, bool PIN>
+static int launch_quads(const CudaBVHHandle* h, rt::TraceScratch& sc, TraceArgs& a, int ldsDepth, hipStream_t s) {
+    static rt::KernelInfo ki;
+    auto kern = k_trace_quad<MODE, PIN>;
+    a.maxStack = 3 * h->depth4 + 4;
+    if (!sc.fixed && a.maxStack > ldsDepth) {
+        const size_t lanes = (size_t)num_cus() * 2048;
+        if (grow_spill(sc, (size_t)(a.maxStack - ldsDepth) * lanes * sizeof(int2)) != 0) return -1;
+    }
+    int grid = PIN ? ((a.W + 3) / 4) * ((a.H + 3) / 4) : (a.n + 15) / 16;
+    if (a.maxStack > kQuadLds) {
+        const size_t perGroup = (size_t)(a.maxStack - kQuadLds) * 16 * sizeof(int2);
+        grid = (int)std::min<size_t>((size_t)grid, sc.spillBytes / perGroup);
+        if (grid < 1) { rt::set_error("fixed traversal scratch too small for a tree of depth %d", h->depth4); return -1; }
+    }
+    rt::note_launch(kern, 64, ki, 0, 0, nullptr);
+    rt::note_launch(kern, 64, ki, ki.maxBlocks, grid, sc.launchInfo);
+    a.spill = (int2*)sc.spill;
+    a.spillStride = grid * 16;
+    a.status = sc.status;
+    a.nodes = (const uint4*)h->d_nodes4;
+    a.tris = (const float4*)h->d_tris;
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(64), 0, s, a);
+    const hipError_t e = hipGetLastError();
     if (e != hipSuccess) { rt::set_error("trace launch failed: %s", hipGetErrorString(e)); return -1; }
     return 0;
 }
@@ -1340,11 +1684,32 @@ static int launch_tuned(const CudaBVHHandle* h, rt::TraceScratch& sc, TraceArgs&
     return launch_depth<MODE, PIN, rt::kScheduleBatch>(h, sc, a, cfg, s);
 }
 
+// Launches of up to this many rays (a queue's capacity where the rays are
+// queued) give each ray four lanes from its root on (k_trace_quad): such a
+// launch leaves the chip's waves short of work, and its time is the chain of
+// steps of its longest rays. Larger ones fill the chip, and there the batch
+// and refill kernels, which hand a wave's last rays to quads, take fewer
+// instructions per ray. Measured, quads from the root / hand-over / neither
+// (us; a 0.5 M triangle terrain and a 1 M triangle soup of camera, secondary
+// and shadow rays):
+//   pinhole    0.26 M rays 152 / 190 / 242, 210 / 252 / 304; 0.41 M 186 / 214 / 243,
+//              257 / 271 / 329; 0.59 M 237 / 233 / 270, 311 / 306 / 344
+//   closest    0.22 M rays 198 / 214 / 273, 273 / 270 / 357; 0.35 M 257 / 231 / 298
+//   any hit    0.35 M rays 108 / 140 / 161; 0.50 M 135 / 161 / 183; 0.57 M (soup) 345 / 343 / 383
+constexpr int kQuadPinhole = 7 << 16, kQuadClosest = 1 << 18, kQuadAny = 1 << 19;
+
 int launch_trace(const CudaBVHHandle* h, rt::TraceScratch& sc, TraceArgs& a, int mode, bool mt, bool pinhole,
                  bool counted, hipStream_t s) {
     if (alloc_scratch(sc) != 0) return -1;
     if (a.n <= 0) return 0;
     const rt::TraceConfig& cfg = h->tune[mode == kModeAny ? rt::kClassAny : (pinhole ? rt::kClassCoherent : rt::kClassIncoherent)];
+    if (!mt && !counted && mode != kModeShade && !cfg.chosen &&
+        a.n <= (mode == kModeAny ? kQuadAny : pinhole ? kQuadPinhole : kQuadClosest) && rtq::fits(h->numNodes4, h->numOrdered)) {
+        const int d = cfg.ldsDepth;
+        if (mode == kModeClosest) return pinhole ? launch_quads<kModeClosest, true>(h, sc, a, d, s)
+                                                 : launch_quads<kModeClosest, false>(h, sc, a, d, s);
+        return pinhole ? launch_quads<kModeAny, true>(h, sc, a, d, s) : launch_quads<kModeAny, false>(h, sc, a, d, s);
+    }
     if (!mt && !counted) {
         if (mode == kModeClosest) return pinhole ? launch_tuned<kModeClosest, true>(h, sc, a, cfg, s)
                                                  : launch_tuned<kModeClosest, false>(h, sc, a, cfg, s);

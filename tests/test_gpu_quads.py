@@ -129,7 +129,7 @@ def test_deep_tree(pkg, dev, depth):
         assert b.trace_status() == 0
 
 
-@pytest.mark.parametrize("n", [1 << 18, (1 << 18) + 1, (1 << 19) + 17])
+@pytest.mark.parametrize("n", [9 << 15, (9 << 15) + 1, 25 << 14, (25 << 14) + 1, 9 << 16, (9 << 16) + 17])
 def test_both_sides_of_the_ray_count_rule(pkg, dev, n):
     """Launches at, and just past, the ray counts where the kernels change; a
     queue of the same capacity holding fewer rays."""
@@ -153,11 +153,11 @@ def test_both_sides_of_the_ray_count_rule(pkg, dev, n):
         assert np.array_equal(o[:m].cpu().numpy(), occ[:m]) and (o[m:] == 7).all().item()
 
 
-@pytest.mark.parametrize("W,H", [(1, 1), (3, 5), (4, 4), (61, 33), (677, 679)])
+@pytest.mark.parametrize("W,H", [(1, 1), (3, 5), (4, 4), (61, 33), (848, 851), (1025, 1025)])
 def test_pinhole_images(pkg, oracle, scenes, dev, W, H):
     """4 x 4 pixel tiles cut off at the right and bottom edge, and an image
-    past the ray count where the batch kernel takes over (677 x 679, plain and
-    cost-ordered): every pixel as the explicit rays' counted trace."""
+    past the ray counts where the batch kernel takes over (848 x 851 in cost
+    order, 1025 x 1025 also in plain order): every pixel as the explicit rays' counted trace."""
     import torch
     cam = scenes.parity_camera(W, H)
     rays = oracle.gen_pinhole(scenes.cam_array(cam), W, H)

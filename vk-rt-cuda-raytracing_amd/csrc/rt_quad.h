@@ -36,12 +36,14 @@ __device__ __forceinline__ float quad_perm(float v) { return __int_as_float(quad
 constexpr int kXor1 = 0xb1, kXor2 = 0x4e;             // quad_perm [1,0,3,2], [2,3,0,1]
 constexpr int kRot1 = 0x39, kRot2 = 0x4e, kRot3 = 0x93;   // lane c reads lane (c + k) & 3
 
-// A ray held by the four lanes of a quad. t, u, v, id: this lane's own closest
-// candidate; best: the quad's closest distance.
+// A ray held by the four lanes of a quad, in the axis order (x, y, z here) of
+// its watertight test throughout: the slab test is the same in any order. t,
+// u, v, id: this lane's closest candidate, at first the hit so far or (tmax,
+// -1) in every lane; best: the quad's closest distance. tmax: any hit only.
 struct Ray4 {
-    float ox, oy, oz, ix, iy, iz;
-    float okx, oky, okz, Sx, Sy, Sz, tmin, tmax;      // permuted origin, shear
-    uint32_t kxo, kyo, kzo;                           // byte offsets of the permuted components
+    float ox, oy, oz, ix, iy, iz, Sx, Sy, Sz, tmin, tmax;
+    float far;                                        // infinite for a flat ray, else NaN (see visit)
+    uint32_t kx, ky, kz;                              // the axes
     float t, u, v, best;
     int id;
     int ref, sp, col;                                 // node to visit next, stack entries, stack column
@@ -51,30 +53,32 @@ struct Ray4 {
 
 // Fills the ray part from a set-up ray (rtd::ray_setup).
 __device__ __forceinline__ void set_ray(Ray4& q, const rtd::Ray& r) {
-    q.ox = r.ox; q.oy = r.oy; q.oz = r.oz;
-    q.ix = r.ix; q.iy = r.iy; q.iz = r.iz;
+    q.ox = rtd::sel3(r.kx, r.ox, r.oy, r.oz);
+    q.oy = rtd::sel3(r.ky, r.ox, r.oy, r.oz);
+    q.oz = rtd::sel3(r.kz, r.ox, r.oy, r.oz);
+    q.ix = rtd::sel3(r.kx, r.ix, r.iy, r.iz);
+    q.iy = rtd::sel3(r.ky, r.ix, r.iy, r.iz);
+    q.iz = rtd::sel3(r.kz, r.ix, r.iy, r.iz);
     q.Sx = r.Sx; q.Sy = r.Sy; q.Sz = r.Sz;
     q.tmin = r.tmin; q.tmax = r.tmax;
-    q.okx = rtd::sel3(r.kx, r.ox, r.oy, r.oz);
-    q.oky = rtd::sel3(r.ky, r.ox, r.oy, r.oz);
-    q.okz = rtd::sel3(r.kz, r.ox, r.oy, r.oz);
-    q.kxo = 4u * r.kx; q.kyo = 4u * r.ky; q.kzo = 4u * r.kz;
+    q.kx = r.kx; q.ky = r.ky; q.kz = r.kz;
+    q.far = rtd::ray_flat(r) ? INFINITY : NAN;
 }
 
 // Watertight test of triangle ti (3 x float4), components addressed in the
 // ray's axis order; the arithmetic of rtd::isect_watertight.
 __device__ __forceinline__ bool isect(const Ray4& q, const void* tris, int ti, float& t, float& u, float& v, int& id) {
     const char* tb = (const char*)tris;
-    const uint32_t o = (uint32_t)ti * 48u, ox = o + q.kxo, oy = o + q.kyo, oz = o + q.kzo;
+    const uint32_t o = (uint32_t)ti * 48u, ox = o + 4u * q.kx, oy = o + 4u * q.ky, oz = o + 4u * q.kz;
     auto ld = [&](uint32_t off, int vertex) { return *(const float*)(tb + off + 16 * vertex); };
     const float ax = ld(ox, 0), bx = ld(ox, 1), cx = ld(ox, 2);
     const float ay = ld(oy, 0), by = ld(oy, 1), cy = ld(oy, 2);
     const float az = ld(oz, 0), bz = ld(oz, 1), cz = ld(oz, 2);
     id = *(const int*)(tb + o + 12);
-    const float Akz = az - q.okz, Bkz = bz - q.okz, Ckz = cz - q.okz;
-    const float Ax = (ax - q.okx) - q.Sx * Akz, Ay = (ay - q.oky) - q.Sy * Akz;
-    const float Bx = (bx - q.okx) - q.Sx * Bkz, By = (by - q.oky) - q.Sy * Bkz;
-    const float Cx = (cx - q.okx) - q.Sx * Ckz, Cy = (cy - q.oky) - q.Sy * Ckz;
+    const float Akz = az - q.oz, Bkz = bz - q.oz, Ckz = cz - q.oz;
+    const float Ax = (ax - q.ox) - q.Sx * Akz, Ay = (ay - q.oy) - q.Sy * Akz;
+    const float Bx = (bx - q.ox) - q.Sx * Bkz, By = (by - q.oy) - q.Sy * Bkz;
+    const float Cx = (cx - q.ox) - q.Sx * Ckz, Cy = (cy - q.oy) - q.Sy * Ckz;
     float U = Cx * By - Cy * Bx;
     float V = Ax * Cy - Ay * Cx;
     float W = Bx * Ay - By * Ax;
@@ -94,90 +98,106 @@ __device__ __forceinline__ bool isect(const Ray4& q, const void* tris, int ti, f
     return true;
 }
 
+// Offsets in a node of a lane's child: its entry and exit bound per axis
+// (exit: entry with bit 3 turned) and its child word.
+struct Slot { uint32_t x, y, z, child; };
+
+__device__ __forceinline__ Slot slot(const Ray4& q, int c) {
+    auto entry = [&](float inv, uint32_t axis) { return 16u * axis + 2u * c + (__float_as_uint(inv) >> 31) * 8u; };
+    return {entry(q.ix, q.kx), entry(q.iy, q.ky), entry(q.iz, q.kz), 48u + 4u * c};
+}
+
+// Visits node `node` of the array at nb: this lane's child, then the quad's
+// order of the hit ones. The nearest becomes q.ref, the others are pushed.
+// False when no child is hit.
+//
+// Of a flat ray (an infinite reciprocal) the distance to a plane through its
+// origin is 0 * inf = NaN: such an axis bounds nothing, and the NaN-ignoring
+// max / min leave it out, which is what rt_device.h's FLAT variant computes
+// with its -inf / +inf; q.far and tmin stand in where all three are NaN. (An
+// origin and direction of NaN themselves still hit nothing: q.far is NaN.)
+template <bool ANY, class Push>
+__device__ __forceinline__ bool visit(Ray4& q, int c, int sh, const char* nb, uint32_t o, const Slot& e, int maxStack,
+                                      int* status, Push&& push) {
+    auto half = [&](uint32_t off) { return (uint32_t)*(const uint16_t*)(nb + off); };
+    const uint32_t oX = o + e.x, oY = o + e.y, oZ = o + e.z;
+    const uint32_t hx = half(oX), hy = half(oY), hz = half(oZ);
+    const uint32_t gx = half(oX ^ 8u), gy = half(oY ^ 8u), gz = half(oZ ^ 8u);
+    const int child = *(const int*)(nb + (o + e.child));
+    const float t1x = rtd::h_sub<false>(hx, q.ox) * q.ix, t2x = rtd::h_sub<false>(gx, q.ox) * q.ix;
+    const float t1y = rtd::h_sub<false>(hy, q.oy) * q.iy, t2y = rtd::h_sub<false>(gy, q.oy) * q.iy;
+    const float t1z = rtd::h_sub<false>(hz, q.oz) * q.iz, t2z = rtd::h_sub<false>(gz, q.oz) * q.iz;
+    const float tN = fmaxf(fmaxf(fmaxf(t1x, t1y), t1z), q.tmin);
+    const float tF = fminf(fminf(fminf(t2x, t2y), t2z), q.far) * RT_ROBUST_TFAR;
+    const float limit = ANY ? q.tmax : q.best;
+    const bool hit = (tN <= tF) && (tN <= limit) && child != -1;
+    const uint32_t hm = (uint32_t)(__ballot(hit) >> sh) & 15u;
+    if (!hm) return false;
+    // rank of this lane's child among the quad's hits, nearest first: keys of
+    // the entry distance (from 0 up) with the lane in the two low bits, so
+    // that no two are equal
+    const int key = hit ? (__float_as_int(fmaxf(tN, 0.0f)) & ~3) | c : 0x7ffffffc | c;
+    const int k1 = quad_perm<kRot1>(key), k2 = quad_perm<kRot2>(key), k3 = quad_perm<kRot3>(key);
+    const int rank = -(((k1 - key) >> 31) + ((k2 - key) >> 31) + ((k3 - key) >> 31));
+    const int n = __popc(hm);
+    const int at = q.sp + n - 1 - rank;
+    if (hit && rank > 0 && at < maxStack) push(q, at, child, tN);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the quad's lanes read each other's entries
+    q.sp += n - 1;
+    if (q.sp > maxStack) { q.sp = maxStack; atomicOr(status, 1); }
+    const bool first = hit && rank == 0;
+    int rf = first ? child : 0, tb = first ? __float_as_int(tN) : 0;
+    rf |= quad_perm<kXor1>(rf); tb |= quad_perm<kXor1>(tb);
+    q.ref = rf | quad_perm<kXor2>(rf);
+    q.tn = __int_as_float(tb | quad_perm<kXor2>(tb));
+    return true;
+}
+
+// Tests leaf `ref`, a triangle per lane. closer(t, id): whether a hit replaces
+// this lane's candidate. True when an any-hit ray is done.
+template <bool ANY, class Closer>
+__device__ __forceinline__ bool leaf(Ray4& q, int c, int sh, const void* tris, int ref, Closer&& closer) {
+    const int enc = -(ref + 2), ts = enc >> 3, cnt = (enc & 7) + 1;
+    bool hit = false;
+    for (int b = 0; b < cnt; b += 4) {
+        if (b + c < cnt) {
+            float t, u, v;
+            int id;
+            if (isect(q, tris, ts + b + c, t, u, v, id) && t > q.tmin) {
+                if (ANY) hit |= t < q.tmax;
+                else if (closer(t, id)) { q.t = t; q.id = id; q.u = u; q.v = v; }
+            }
+        }
+    }
+    if (ANY) return ((__ballot(hit) >> sh) & 15u) != 0;
+    const float m = fminf(q.t, quad_perm<kXor1>(q.t));
+    q.best = fminf(m, quad_perm<kXor2>(m));
+    return false;
+}
+
 // Traverses from q.ref (a node or a leaf code) until the ray is done. ANY:
-// stops at the first hit (q.found). FLAT: the slab variant for rays with an
-// infinite reciprocal (chosen per wave). push(q, pos, ref, tn) and pop(q, pos,
+// stops at the first hit (q.found). push(q, pos, ref, tn) and pop(q, pos,
 // ref, tn) access entry pos < maxStack of the quad's stack; more entries (none
 // in a tree of the depth that maxStack was made for) are dropped and flagged
 // in *status. Control flow is the same in the four lanes of a quad. Returns
 // the steps taken.
-template <bool ANY, bool FLAT, class Push, class Pop>
+template <bool ANY, class Push, class Pop>
 __device__ __forceinline__ int traverse(Ray4& q, int lane, const void* nodes, const void* tris, int maxStack, int* status,
                                         Push&& push, Pop&& pop) {
     const int c = lane & 3, sh = lane & 60;
-    const char* nb = (const char*)nodes;
-    // offsets in a node of this lane's entry and exit bound per axis
-    auto entry = [&](float inv, int axis) {
-        return 16u * axis + 2u * c + (FLAT ? 0u : (__float_as_uint(inv) >> 31) * 8u);
-    };
-    const uint32_t eX = entry(q.ix, 0), eY = entry(q.iy, 1), eZ = entry(q.iz, 2), eC = 48u + 4u * c;
-    auto half = [&](uint32_t off) { return (uint32_t)*(const uint16_t*)(nb + off); };
+    const Slot e = slot(q, c);
     int steps = 0;
     for (;;) {
         steps++;
         if (q.ref < 0) {
             if (ANY || q.tn <= q.best) {
-                const int enc = -(q.ref + 2), ts = enc >> 3, cnt = (enc & 7) + 1;
-                bool hit = false;
-                for (int b = 0; b < cnt; b += 4) {
-                    if (b + c < cnt) {
-                        float t, u, v;
-                        int id;
-                        if (isect(q, tris, ts + b + c, t, u, v, id) && t > q.tmin && t < q.tmax) {
-                            if (ANY) hit = true;
-                            else if (t < q.t || (t == q.t && id < q.id)) { q.t = t; q.id = id; q.u = u; q.v = v; }
-                        }
-                    }
-                }
-                if (ANY) {
-                    if ((__ballot(hit) >> sh) & 15u) { q.found = true; break; }
-                } else {
-                    float m = fminf(q.t, quad_perm<kXor1>(q.t));
-                    q.best = fminf(m, quad_perm<kXor2>(m));
+                if (leaf<ANY>(q, c, sh, tris, q.ref, [&](float t, int id) { return t < q.t || (t == q.t && id < q.id); })) {
+                    q.found = true;
+                    break;
                 }
             }
         } else if (ANY || q.tn <= q.best) {
-            const uint32_t o = (uint32_t)q.ref << 6, oX = o + eX, oY = o + eY, oZ = o + eZ;
-            const uint32_t hx = half(oX), hy = half(oY), hz = half(oZ);
-            const uint32_t gx = half(oX ^ 8u), gy = half(oY ^ 8u), gz = half(oZ ^ 8u);
-            const int child = *(const int*)(nb + (o + eC));
-            float t1x = rtd::h_sub<false>(hx, q.ox) * q.ix, t2x = rtd::h_sub<false>(gx, q.ox) * q.ix;
-            float t1y = rtd::h_sub<false>(hy, q.oy) * q.iy, t2y = rtd::h_sub<false>(gy, q.oy) * q.iy;
-            float t1z = rtd::h_sub<false>(hz, q.oz) * q.iz, t2z = rtd::h_sub<false>(gz, q.oz) * q.iz;
-            float tN, tF;
-            if (FLAT) {
-                t1x = t1x != t1x ? -q.ix : t1x; t2x = t2x != t2x ? q.ix : t2x;
-                t1y = t1y != t1y ? -q.iy : t1y; t2y = t2y != t2y ? q.iy : t2y;
-                t1z = t1z != t1z ? -q.iz : t1z; t2z = t2z != t2z ? q.iz : t2z;
-                tN = fmaxf(fmaxf(fminf(t1x, t2x), fminf(t1y, t2y)), fminf(t1z, t2z));
-                tF = fminf(fminf(fmaxf(t1x, t2x), fmaxf(t1y, t2y)), fmaxf(t1z, t2z)) * RT_ROBUST_TFAR;
-            } else {
-                tN = fmaxf(fmaxf(t1x, t1y), t1z);
-                tF = fminf(fminf(t2x, t2y), t2z) * RT_ROBUST_TFAR;
-            }
-            const float limit = ANY ? q.tmax : q.best;
-            const bool hit = (tN <= tF) && (tF >= q.tmin) && (tN <= limit) && child != -1;
-            const uint32_t hm = (uint32_t)(__ballot(hit) >> sh) & 15u;
-            if (hm) {
-                // rank of this lane's child among the quad's hits, nearest
-                // first: keys of the entry distance (from 0 up) with the lane
-                // in the two low bits, so that no two are equal
-                const int key = hit ? (__float_as_int(fmaxf(tN, 0.0f)) & ~3) | c : 0x7ffffffc | c;
-                const int k1 = quad_perm<kRot1>(key), k2 = quad_perm<kRot2>(key), k3 = quad_perm<kRot3>(key);
-                const int rank = -(((k1 - key) >> 31) + ((k2 - key) >> 31) + ((k3 - key) >> 31));
-                const int n = __popc(hm);
-                const int at = q.sp + n - 1 - rank;
-                if (hit && rank > 0 && at < maxStack) push(q, at, child, tN);
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the quad's lanes read each other's entries
-                q.sp += n - 1;
-                if (q.sp > maxStack) { q.sp = maxStack; atomicOr(status, 1); }
-                const bool first = hit && rank == 0;
-                int rf = first ? child : 0, tb = first ? __float_as_int(tN) : 0;
-                rf |= quad_perm<kXor1>(rf); tb |= quad_perm<kXor1>(tb);
-                q.ref = rf | quad_perm<kXor2>(rf);
-                q.tn = __int_as_float(tb | quad_perm<kXor2>(tb));
-                continue;
-            }
+            if (visit<ANY>(q, c, sh, (const char*)nodes, (uint32_t)q.ref << 6, e, maxStack, status, push)) continue;
         }
         if (q.sp == 0) break;
         q.sp--;

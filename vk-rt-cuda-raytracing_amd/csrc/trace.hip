@@ -448,8 +448,7 @@ __device__ __forceinline__ void trace_ray(const TraceArgs& a, const Ray& r, int*
 // lanes still hold a ray (res.open): those go on in quads (finish_quads).
 // Uncounted watertight launches. Every lane calls it; `live` lanes hold a ray.
 // The loop is wave-uniform: with lanes leaving it one by one, each value of
-// theirs that is needed afterwards took a second register (105 VGPRs instead
-// of 80).
+// theirs that is needed afterwards took a second register (25 VGPRs more).
 template <int MODE, int LDSD, int BLOCK>
 __device__ __forceinline__ void trace_wave(const TraceArgs& a, const Ray& r, bool live, bool flat, int* s_ref, float* s_tn, int tid,
                                            int gtid, Result& res, int root, int pc) {
@@ -545,11 +544,11 @@ __device__ __forceinline__ void trace_wave(const TraceArgs& a, const Ray& r, boo
 // on with four lanes each: quad k takes over the k-th open lane's ray, its
 // closest hit so far and its stack (in place, in that lane's column). Every
 // lane of the wave calls it. The ray itself is read (or generated) again:
-// moving it across lanes held both copies in registers at once (97 VGPRs
-// instead of 80). Results go straight to the output arrays. Returns the
+// moving it across lanes held both copies in registers at once (17 VGPRs
+// more). Results go straight to the output arrays. Returns the
 // longest quad's steps.
 template <int MODE, bool PIN, int LDSD, int BLOCK>
-__device__ __forceinline__ int finish_quads(const TraceArgs& a, bool open, bool flat, int ref, float tn, int sp, float best,
+__device__ __forceinline__ int finish_quads(const TraceArgs& a, bool open, int ref, float tn, int sp, float best,
                                             float bu, float bv, int bid, int ri, int* s_ref, float* s_tn, int tid,
                                             int gtid) {
     constexpr bool ANY = MODE == kModeAny;
@@ -567,7 +566,6 @@ __device__ __forceinline__ int finish_quads(const TraceArgs& a, bool open, bool 
         q.best = q.t = rtq::take(from, best);
         q.id = rtq::take(from, bid);
         q.u = rtq::take(from, bu); q.v = rtq::take(from, bv);
-        if ((lane & 3) != 0) { q.t = INFINITY; q.id = -1; }   // one lane holds the hit so far
     }
     q.col = from - lane;                           // the ray's stack column, as an offset to this lane's
     q.found = false;
@@ -605,8 +603,7 @@ __device__ __forceinline__ int finish_quads(const TraceArgs& a, bool open, bool 
                 rf = e.x; t = __int_as_float(e.y);
             }
         };
-        steps = flat ? rtq::traverse<ANY, true>(q, lane, a.nodes, a.tris, a.maxStack, a.status, push, pop)
-                     : rtq::traverse<ANY, false>(q, lane, a.nodes, a.tris, a.maxStack, a.status, push, pop);
+        steps = rtq::traverse<ANY>(q, lane, a.nodes, a.tris, a.maxStack, a.status, push, pop);
         __builtin_amdgcn_s_setprio(0);
         if constexpr (!ANY) rtq::reduce(q);
         if ((lane & 3) == 0) {
@@ -862,7 +859,7 @@ __global__ __launch_bounds__(BLOCK) void k_trace_refill(TraceArgs a) {
                 if (sbase[sl] >= 0) flush(sl);
         }
         if (__any(has))
-            finish_quads<MODE, PIN, LDSD, BLOCK>(a, has, __any(has && flat), ltc > 0 ? cursor_code(lts, ltc) : ref, tn, sp,
+            finish_quads<MODE, PIN, LDSD, BLOCK>(a, has, ltc > 0 ? cursor_code(lts, ltc) : ref, tn, sp,
                                                  best, bu, bv, bid, ri, s_ref, s_tn, tid, gtid);
     }
 }
@@ -893,7 +890,6 @@ __global__ __launch_bounds__(64) void k_trace_quad(TraceArgs a) {
         }
         Ray r;
         rtq::Ray4 q;
-        bool flat = false;
         if (live) {
             if constexpr (PIN) {
                 rtd::pinhole_ray(a.cam, px, py, a.W, a.H, r);
@@ -903,16 +899,13 @@ __global__ __launch_bounds__(64) void k_trace_quad(TraceArgs a) {
                 r.tmin = a.tmin[ri]; r.tmax = a.tmax[ri];
             }
             rtd::ray_setup(r);
-            flat = rtd::ray_flat(r);
             rtq::set_ray(q, r);
             q.best = r.tmax;
-            q.t = INFINITY; q.u = q.v = 0.f; q.id = -1;
-            if ((lane & 3) == 0) q.t = r.tmax;
+            q.t = r.tmax; q.u = q.v = 0.f; q.id = -1;
             q.ref = ray_root(a, ri); q.tn = -INFINITY;
             q.sp = 0; q.col = qd;
             q.found = false;
         }
-        const bool anyFlat = __any(flat);
         if (!live) continue;
         const size_t column = (size_t)blockIdx.x * 16;
         auto push = [&](rtq::Ray4& z, int at, int rf, float t) {
@@ -932,8 +925,7 @@ __global__ __launch_bounds__(64) void k_trace_quad(TraceArgs a) {
                 rf = e.x; t = __int_as_float(e.y);
             }
         };
-        if (anyFlat) rtq::traverse<ANY, true>(q, lane, a.nodes, a.tris, a.maxStack, a.status, push, pop);
-        else rtq::traverse<ANY, false>(q, lane, a.nodes, a.tris, a.maxStack, a.status, push, pop);
+        rtq::traverse<ANY>(q, lane, a.nodes, a.tris, a.maxStack, a.status, push, pop);
         if constexpr (!ANY) rtq::reduce(q);
         if ((lane & 3) == 0) {
             if constexpr (ANY) {
@@ -954,14 +946,13 @@ __global__ __launch_bounds__(64) void k_trace_quad(TraceArgs a) {
 // rays, whose lanes stay in step. Uncounted watertight launches hand a wave's
 // last kQuadRays rays to quads, four lanes each: a launch's end is the chain
 // of steps of its slowest tiles, mostly run by waves with few rays left. That
-// takes 91 VGPRs (85 for any hit), five waves per SIMD instead of seven: on a
-// 0.5 M triangle terrain the pinhole launch of 1280 x 720 went from 318 to
-// 299 us and of 768 x 768 from 270 to 233 us, the cost-ordered one of
-// 1024 x 1024 from 279 to 243 us; the cost-ordered 1080p one, which the order
-// keeps busy to its end, from 366 to 385 us (on a triangle soup of 1 M from
-// 468 to 415). Squeezed to six waves it spilled registers to scratch.
+// takes 79 VGPRs, six waves per SIMD instead of seven (at seven it spilled up
+// to 7 to scratch): on a 0.5 M triangle terrain the cost-ordered pinhole launch
+// of 1024 x 1024 went from 279 to 240 us and of 1920 x 1080, which the order
+// keeps busy to its end, from 366 to 373 us (a 65,536 triangle soup: 394 to
+// 353, 468 to 406 us).
 template <int MODE, bool MT, bool PIN, bool COUNT, int LDSD, int BLOCK>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_trace_batch(TraceArgs a) {
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void k_trace_batch(TraceArgs a) {
     __shared__ int s_ref[LDSD * BLOCK];
     __shared__ float s_tn[LDSD * BLOCK];
     const int tid = threadIdx.x;
@@ -1044,7 +1035,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void
         int qsteps = 0;
         if constexpr (QUAD) {
             if (__any(res.open))
-                qsteps = finish_quads<MODE, PIN, LDSD, BLOCK>(a, res.open, anyFlat, res.ref, res.tn, res.sp, res.t, res.u,
+                qsteps = finish_quads<MODE, PIN, LDSD, BLOCK>(a, res.open, res.ref, res.tn, res.sp, res.t, res.u,
                                                               res.v, res.id, ri, s_ref, s_tn, tid, gtid);
         }
         // a cost-ordered launch records the batch's step count (its slowest
@@ -1684,19 +1675,26 @@ static int launch_tuned(const CudaBVHHandle* h, rt::TraceScratch& sc, TraceArgs&
     return launch_depth<MODE, PIN, rt::kScheduleBatch>(h, sc, a, cfg, s);
 }
 
-// Launches of up to this many rays (a queue's capacity where the rays are
-// queued) give each ray four lanes from its root on (k_trace_quad): such a
-// launch leaves the chip's waves short of work, and its time is the chain of
-// steps of its longest rays. Larger ones fill the chip, and there the batch
-// and refill kernels, which hand a wave's last rays to quads, take fewer
-// instructions per ray. Measured, quads from the root / hand-over / neither
-// (us; a 0.5 M triangle terrain and a 1 M triangle soup of camera, secondary
-// and shadow rays):
-//   pinhole    0.26 M rays 152 / 190 / 242, 210 / 252 / 304; 0.41 M 186 / 214 / 243,
-//              257 / 271 / 329; 0.59 M 237 / 233 / 270, 311 / 306 / 344
-//   closest    0.22 M rays 198 / 214 / 273, 273 / 270 / 357; 0.35 M 257 / 231 / 298
-//   any hit    0.35 M rays 108 / 140 / 161; 0.50 M 135 / 161 / 183; 0.57 M (soup) 345 / 343 / 383
-constexpr int kQuadPinhole = 7 << 16, kQuadClosest = 1 << 18, kQuadAny = 1 << 19;
+// Launches of up to this many rays give each ray four lanes from its root on
+// (k_trace_quad): such a launch leaves the chip's waves short of work, and its
+// time is the chain of steps of its longest rays. Larger ones fill the chip,
+// and there the batch and refill kernels, which hand a wave's last rays to
+// quads, take fewer instructions per ray; the pinhole cost order, which only
+// those take, brings its line forward. A queue's capacity is an upper bound of
+// its rays (some 55 to 85 % of it in a frame), so its line lies higher.
+// Measured, quads from the root / hand-over (us; a 0.5 M triangle terrain,
+// then a 65,536 triangle soup; camera, secondary and shadow rays; launches
+// without either took 242 and 304 us for 0.26 M pinhole rays, 273 and 357 us
+// for 0.22 M closest hits):
+//   pinhole     0.26 M rays 131 / 190, 183 / 252; 0.59 M 197 / 246, 261 / 310;
+//               0.79 M 235 / 260, 268 / 326; 1.05 M 296 / 298, 377 / 391
+//   cost order  0.59 M rays 198 / 219, 262 / 269; 0.79 M 234 / 228, 266 / 272
+//   closest     0.22 M rays 165 / 214, 238 / 268; 0.35 M 215 / 234, 0.32 M
+//               311 / 291; 0.50 M 289 / 263
+//   any hit     0.50 M rays 136 / 160, 0.32 M 241 / 261; 0.64 M 168 / 189,
+//               0.57 M 354 / 325; 0.88 M 212 / 210
+constexpr int kQuadPinhole = 1 << 20, kQuadCostOrder = 11 << 16, kQuadClosest = 9 << 15, kQuadQueue = 25 << 14,
+              kQuadAny = 9 << 16;
 
 int launch_trace(const CudaBVHHandle* h, rt::TraceScratch& sc, TraceArgs& a, int mode, bool mt, bool pinhole,
                  bool counted, hipStream_t s) {
@@ -1704,7 +1702,9 @@ int launch_trace(const CudaBVHHandle* h, rt::TraceScratch& sc, TraceArgs& a, int
     if (a.n <= 0) return 0;
     const rt::TraceConfig& cfg = h->tune[mode == kModeAny ? rt::kClassAny : (pinhole ? rt::kClassCoherent : rt::kClassIncoherent)];
     if (!mt && !counted && mode != kModeShade && !cfg.chosen &&
-        a.n <= (mode == kModeAny ? kQuadAny : pinhole ? kQuadPinhole : kQuadClosest) && rtq::fits(h->numNodes4, h->numOrdered)) {
+        a.n <= (mode == kModeAny ? kQuadAny
+                : pinhole        ? (a.costOrder ? kQuadCostOrder : kQuadPinhole)
+                                 : (a.nDev ? kQuadQueue : kQuadClosest)) && rtq::fits(h->numNodes4, h->numOrdered)) {
         const int d = cfg.ldsDepth;
         if (mode == kModeClosest) return pinhole ? launch_quads<kModeClosest, true>(h, sc, a, d, s)
                                                  : launch_quads<kModeClosest, false>(h, sc, a, d, s);

@@ -173,3 +173,75 @@ def test_pinhole_images(pkg, oracle, scenes, dev, W, H):
             got = {k: hb[k].cpu().numpy() for k in KEYS}
             _same({k: got[k][:W * H] for k in KEYS}, ref)
             assert all((got[k][W * H:] == -3).all() for k in KEYS)
+
+
+KEYS2 = ("t", "inst", "prim_id", "u", "v")
+
+
+@pytest.fixture(scope="module")
+def two_level(pkg, dev):
+    """Three meshes (one of a single triangle) in 40 instances: rotated, scaled,
+    mirrored, axis-aligned ones, and pairs of the same transform (ties in t,
+    decided by the instance)."""
+    rng = np.random.default_rng(12)
+    meshes = [_soup(4000, 1), _soup(1, 2, size=0.5), _soup(60, 3, size=0.4, grid=True)]
+    blas = [pkg.BVH.build(m) for m in meshes]
+    o2w = np.zeros((40, 3, 4), np.float32)
+    for k in range(40):
+        q, _ = np.linalg.qr(rng.normal(size=(3, 3)))
+        m = np.eye(3) if k % 4 == 0 else q * rng.uniform(0.3, 1.0) * (1 if k % 3 else -1)
+        o2w[k, :, :3], o2w[k, :, 3] = m, rng.uniform(-0.5, 0.5, 3)
+    o2w[21:31] = o2w[1:11]
+    of = [k % 3 if k < 20 else (k - 20) % 3 for k in range(40)]
+    s = pkg.Scene(blas, o2w.reshape(40, 12), of)
+    yield s
+    s.destroy()
+    for b in blas:
+        b.destroy()
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 64, 65, 3001, 200000])
+def test_two_level(pkg, two_level, dev, n):
+    """Ray counts at and beside a wave's 16 rays, launches whose rays all start
+    in quads and one whose last rays of each wave do, at every stack depth, and
+    queues of one ray less; against the counted traversal."""
+    import torch
+    s, rays = two_level, _rays(n, 3 * n + 1, flat=0.2)
+    R = to_dev(rays, dev)
+
+    def buffers():
+        f = {k: torch.full((n + 64,), -3, dtype=torch.int32 if k in ("inst", "prim_id") else torch.float32, device=dev)
+             for k in KEYS2}
+        return f, torch.full((n + 64,), 7, dtype=torch.uint8, device=dev)
+
+    def check(f, occ, m):
+        torch.cuda.synchronize()
+        for k in KEYS2:
+            got = f[k].cpu().numpy()
+            assert np.array_equal(_bits(got[:m]), _bits(ref[k][:m])) and (got[m:] == -3).all(), k
+        got = occ.cpu().numpy()
+        assert np.array_equal(got[:m], hit[:m]) and (got[m:] == 7).all()
+
+    f, _ = buffers()
+    c = [torch.empty(n, dtype=torch.int32, device=dev) for _ in range(2)]
+    s.trace_closest_counted(R, *[f[k][:n] for k in KEYS2], *c)
+    torch.cuda.synchronize()
+    ref = {k: f[k][:n].cpu().numpy() for k in KEYS2}
+    hit = (ref["prim_id"] >= 0).astype(np.uint8)
+    cnt = torch.tensor([n - 1], dtype=torch.int32, device=dev)
+    saved = [s.trace_config(k) for k in (0, 1)]
+    for depth in (None, 4, 8, 12, 16):
+        if depth:
+            s.set_trace_config(0, 1, depth, 1)
+            s.set_trace_config(1, 2 if depth == 8 else 1, depth, 1)
+        f, occ = buffers()
+        s.trace_closest(R, *[f[k][:n] for k in KEYS2])
+        s.trace_any(R, occ[:n])
+        check(f, occ, n)
+        f, occ = buffers()
+        s.trace_closest_queued(n, cnt, R, *[f[k][:n] for k in KEYS2])
+        s.trace_any_queued(n, cnt, R, occ[:n])
+        check(f, occ, n - 1)
+    for k in (0, 1):
+        s.set_trace_config(k, *saved[k])
+    assert s.trace_status() == 0

@@ -11,9 +11,9 @@
 // direction signs) and its child word, or the vertex components of its
 // triangle already in the order of the ray's watertight axis permutation.
 //
-// Node and triangle addresses are 32-bit offsets from the arrays' (uniform)
-// bases, which keeps a lane's addresses in single registers: the caller uses
-// quads only where both arrays fit (fits()).
+// In the one-level traversal node and triangle addresses are 32-bit offsets
+// from the arrays' (uniform) bases, which keeps a lane's addresses in single
+// registers: its callers use quads only where both arrays fit (fits()).
 //
 // Every value is computed by the expressions of rt_device.h, and a ray's hit
 // is the lexicographic minimum of (t, ID) over the triangles whose boxes pass,
@@ -26,6 +26,12 @@
 #include "rt_device.h"
 
 namespace rtq {
+
+// Global memory: loads through a pointer that was itself loaded would
+// otherwise be flat ones.
+typedef const __attribute__((address_space(1))) char* gptr;
+template <class T>
+__device__ __forceinline__ T gload(gptr p) { return *(const __attribute__((address_space(1))) T*)p; }
 
 inline bool fits(long long nodes, long long tris) { return nodes * 64 <= 0xffffffffll && tris * 48 <= 0xffffffffll; }
 
@@ -65,16 +71,15 @@ __device__ __forceinline__ void set_ray(Ray4& q, const rtd::Ray& r) {
     q.far = rtd::ray_flat(r) ? INFINITY : NAN;
 }
 
-// Watertight test of triangle ti (3 x float4), components addressed in the
-// ray's axis order; the arithmetic of rtd::isect_watertight.
-__device__ __forceinline__ bool isect(const Ray4& q, const void* tris, int ti, float& t, float& u, float& v, int& id) {
-    const char* tb = (const char*)tris;
-    const uint32_t o = (uint32_t)ti * 48u, ox = o + 4u * q.kx, oy = o + 4u * q.ky, oz = o + 4u * q.kz;
-    auto ld = [&](uint32_t off, int vertex) { return *(const float*)(tb + off + 16 * vertex); };
+// Watertight test of the triangle (3 x float4) at tb + o, components addressed
+// in the ray's axis order; the arithmetic of rtd::isect_watertight.
+__device__ __forceinline__ bool isect(const Ray4& q, gptr tb, uint32_t o, float& t, float& u, float& v, int& id) {
+    const uint32_t ox = o + 4u * q.kx, oy = o + 4u * q.ky, oz = o + 4u * q.kz;
+    auto ld = [&](uint32_t off, int vertex) { return gload<float>(tb + off + 16 * vertex); };
     const float ax = ld(ox, 0), bx = ld(ox, 1), cx = ld(ox, 2);
     const float ay = ld(oy, 0), by = ld(oy, 1), cy = ld(oy, 2);
     const float az = ld(oz, 0), bz = ld(oz, 1), cz = ld(oz, 2);
-    id = *(const int*)(tb + o + 12);
+    id = gload<int>(tb + o + 12);
     const float Akz = az - q.oz, Bkz = bz - q.oz, Ckz = cz - q.oz;
     const float Ax = (ax - q.ox) - q.Sx * Akz, Ay = (ay - q.oy) - q.Sy * Akz;
     const float Bx = (bx - q.ox) - q.Sx * Bkz, By = (by - q.oy) - q.Sy * Bkz;
@@ -98,18 +103,39 @@ __device__ __forceinline__ bool isect(const Ray4& q, const void* tris, int ti, f
     return true;
 }
 
-// Offsets in a node of a lane's child: its entry and exit bound per axis
-// (exit: entry with bit 3 turned) and its child word.
-struct Slot { uint32_t x, y, z, child; };
+// This lane's child of a node: the entry and exit bound per axis, in the ray's
+// axis order, and the child word.
+struct Slot { uint32_t hx, hy, hz, gx, gy, gz; int child; };
 
-__device__ __forceinline__ Slot slot(const Ray4& q, int c) {
+// Offsets in a node of a lane's bounds of entry (exit: bit 3 turned) and of
+// its child word.
+struct Offsets { uint32_t x, y, z, child; };
+
+__device__ __forceinline__ Offsets offsets(const Ray4& q, int c) {
     auto entry = [&](float inv, uint32_t axis) { return 16u * axis + 2u * c + (__float_as_uint(inv) >> 31) * 8u; };
     return {entry(q.ix, q.kx), entry(q.iy, q.ky), entry(q.iz, q.kz), 48u + 4u * c};
 }
 
-// Visits node `node` of the array at nb: this lane's child, then the quad's
-// order of the hit ones. The nearest becomes q.ref, the others are pushed.
-// False when no child is hit.
+// The slot of the node at nb + o (nb uniform): one 32-bit offset per load.
+__device__ __forceinline__ Slot slot_at(gptr nb, uint32_t o, const Offsets& e) {
+    auto half = [&](uint32_t off) { return (uint32_t)gload<uint16_t>(nb + off); };
+    const uint32_t x = o + e.x, y = o + e.y, z = o + e.z;
+    return {half(x), half(y), half(z), half(x ^ 8u), half(y ^ 8u), half(z ^ 8u), gload<int>(nb + (o + e.child))};
+}
+
+// The slot of the node at nb (different per quad): one 64-bit address per axis
+// for both bounds, exchanged by the direction's sign.
+__device__ __forceinline__ Slot slot_of(const Ray4& q, gptr nb, int c) {
+    auto half = [&](gptr p) { return (uint32_t)gload<uint16_t>(p); };
+    const gptr x = nb + (16u * q.kx + 2u * c), y = nb + (16u * q.ky + 2u * c), z = nb + (16u * q.kz + 2u * c);
+    const uint32_t lx = half(x), ux = half(x + 8), ly = half(y), uy = half(y + 8), lz = half(z), uz = half(z + 8);
+    const bool sx = __float_as_int(q.ix) < 0, sy = __float_as_int(q.iy) < 0, sz = __float_as_int(q.iz) < 0;
+    return {sx ? ux : lx, sy ? uy : ly, sz ? uz : lz, sx ? lx : ux, sy ? ly : uy, sz ? lz : uz,
+            gload<int>(nb + (48u + 4u * c))};
+}
+
+// Visits a node: this lane's child, then the quad's order of the hit ones. The
+// nearest becomes q.ref, the others are pushed. False when no child is hit.
 //
 // Of a flat ray (an infinite reciprocal) the distance to a plane through its
 // origin is 0 * inf = NaN: such an axis bounds nothing, and the NaN-ignoring
@@ -117,20 +143,14 @@ __device__ __forceinline__ Slot slot(const Ray4& q, int c) {
 // with its -inf / +inf; q.far and tmin stand in where all three are NaN. (An
 // origin and direction of NaN themselves still hit nothing: q.far is NaN.)
 template <bool ANY, class Push>
-__device__ __forceinline__ bool visit(Ray4& q, int c, int sh, const char* nb, uint32_t o, const Slot& e, int maxStack,
-                                      int* status, Push&& push) {
-    auto half = [&](uint32_t off) { return (uint32_t)*(const uint16_t*)(nb + off); };
-    const uint32_t oX = o + e.x, oY = o + e.y, oZ = o + e.z;
-    const uint32_t hx = half(oX), hy = half(oY), hz = half(oZ);
-    const uint32_t gx = half(oX ^ 8u), gy = half(oY ^ 8u), gz = half(oZ ^ 8u);
-    const int child = *(const int*)(nb + (o + e.child));
-    const float t1x = rtd::h_sub<false>(hx, q.ox) * q.ix, t2x = rtd::h_sub<false>(gx, q.ox) * q.ix;
-    const float t1y = rtd::h_sub<false>(hy, q.oy) * q.iy, t2y = rtd::h_sub<false>(gy, q.oy) * q.iy;
-    const float t1z = rtd::h_sub<false>(hz, q.oz) * q.iz, t2z = rtd::h_sub<false>(gz, q.oz) * q.iz;
+__device__ __forceinline__ bool visit(Ray4& q, int c, int sh, const Slot& s, int maxStack, int* status, Push&& push) {
+    const float t1x = rtd::h_sub<false>(s.hx, q.ox) * q.ix, t2x = rtd::h_sub<false>(s.gx, q.ox) * q.ix;
+    const float t1y = rtd::h_sub<false>(s.hy, q.oy) * q.iy, t2y = rtd::h_sub<false>(s.gy, q.oy) * q.iy;
+    const float t1z = rtd::h_sub<false>(s.hz, q.oz) * q.iz, t2z = rtd::h_sub<false>(s.gz, q.oz) * q.iz;
     const float tN = fmaxf(fmaxf(fmaxf(t1x, t1y), t1z), q.tmin);
     const float tF = fminf(fminf(fminf(t2x, t2y), t2z), q.far) * RT_ROBUST_TFAR;
     const float limit = ANY ? q.tmax : q.best;
-    const bool hit = (tN <= tF) && (tN <= limit) && child != -1;
+    const bool hit = (tN <= tF) && (tN <= limit) && s.child != -1;
     const uint32_t hm = (uint32_t)(__ballot(hit) >> sh) & 15u;
     if (!hm) return false;
     // rank of this lane's child among the quad's hits, nearest first: keys of
@@ -141,29 +161,28 @@ __device__ __forceinline__ bool visit(Ray4& q, int c, int sh, const char* nb, ui
     const int rank = -(((k1 - key) >> 31) + ((k2 - key) >> 31) + ((k3 - key) >> 31));
     const int n = __popc(hm);
     const int at = q.sp + n - 1 - rank;
-    if (hit && rank > 0 && at < maxStack) push(q, at, child, tN);
+    if (hit && rank > 0 && at < maxStack) push(q, at, s.child, tN);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the quad's lanes read each other's entries
     q.sp += n - 1;
     if (q.sp > maxStack) { q.sp = maxStack; atomicOr(status, 1); }
     const bool first = hit && rank == 0;
-    int rf = first ? child : 0, tb = first ? __float_as_int(tN) : 0;
+    int rf = first ? s.child : 0, tb = first ? __float_as_int(tN) : 0;
     rf |= quad_perm<kXor1>(rf); tb |= quad_perm<kXor1>(tb);
     q.ref = rf | quad_perm<kXor2>(rf);
     q.tn = __int_as_float(tb | quad_perm<kXor2>(tb));
     return true;
 }
 
-// Tests leaf `ref`, a triangle per lane. closer(t, id): whether a hit replaces
-// this lane's candidate. True when an any-hit ray is done.
+// Tests the cnt triangles from tb + o on, one per lane. closer(t, id): whether
+// a hit replaces this lane's candidate. True when an any-hit ray is done.
 template <bool ANY, class Closer>
-__device__ __forceinline__ bool leaf(Ray4& q, int c, int sh, const void* tris, int ref, Closer&& closer) {
-    const int enc = -(ref + 2), ts = enc >> 3, cnt = (enc & 7) + 1;
+__device__ __forceinline__ bool leaf(Ray4& q, int c, int sh, gptr tb, uint32_t o, int cnt, Closer&& closer) {
     bool hit = false;
     for (int b = 0; b < cnt; b += 4) {
         if (b + c < cnt) {
             float t, u, v;
             int id;
-            if (isect(q, tris, ts + b + c, t, u, v, id) && t > q.tmin) {
+            if (isect(q, tb, o + 48u * (b + c), t, u, v, id) && t > q.tmin) {
                 if (ANY) hit |= t < q.tmax;
                 else if (closer(t, id)) { q.t = t; q.id = id; q.u = u; q.v = v; }
             }
@@ -185,19 +204,22 @@ template <bool ANY, class Push, class Pop>
 __device__ __forceinline__ int traverse(Ray4& q, int lane, const void* nodes, const void* tris, int maxStack, int* status,
                                         Push&& push, Pop&& pop) {
     const int c = lane & 3, sh = lane & 60;
-    const Slot e = slot(q, c);
+    const Offsets e = offsets(q, c);
     int steps = 0;
     for (;;) {
         steps++;
         if (q.ref < 0) {
             if (ANY || q.tn <= q.best) {
-                if (leaf<ANY>(q, c, sh, tris, q.ref, [&](float t, int id) { return t < q.t || (t == q.t && id < q.id); })) {
+                const int enc = -(q.ref + 2);
+                if (leaf<ANY>(q, c, sh, (gptr)tris, (uint32_t)(enc >> 3) * 48u, (enc & 7) + 1, [&](float t, int id) {
+                        return t < q.t || (t == q.t && id < q.id);
+                    })) {
                     q.found = true;
                     break;
                 }
             }
         } else if (ANY || q.tn <= q.best) {
-            if (visit<ANY>(q, c, sh, (const char*)nodes, (uint32_t)q.ref << 6, e, maxStack, status, push)) continue;
+            if (visit<ANY>(q, c, sh, slot_at((gptr)nodes, (uint32_t)q.ref << 6, e), maxStack, status, push)) continue;
         }
         if (q.sp == 0) break;
         q.sp--;

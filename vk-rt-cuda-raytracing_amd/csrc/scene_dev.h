@@ -1,6 +1,6 @@
 // scene_dev.h — device pieces of the two-level traversal shared by the
-// persistent traversal kernel (scene.hip) and the path tracer's tail kernel
-// (pt.hip): the instance transform, the node visit, and a one-ray traversal.
+// traversal kernels (scene.hip) and the path tracer's tail kernel (pt.hip): the
+// instance transform, the node visit, and a traversal with four lanes per ray.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -8,6 +8,7 @@
 #include <climits>
 
 #include "rt_device.h"
+#include "rt_quad.h"
 #include "scene.h"
 
 namespace rtk {
@@ -105,166 +106,133 @@ __device__ __forceinline__ void visit2w(const uint4* __restrict__ nodes, const R
 }
 
 
-// Stack in global memory: entries base[k * stride], k < max.
-struct GlobalStack {
-    int2* base;
-    int stride, max, sp;
-    int* status;                        // bit 0 set on overflow (nullable)
-    __device__ __forceinline__ void push(int rf, float t) {
-        if (sp < max) { base[(size_t)sp * stride] = make_int2(rf, __float_as_int(t)); sp++; }
-        else if (status) atomicOr(status, 1);
-    }
-    __device__ __forceinline__ bool pop(int& rf, float& t) {
-        if (sp == 0) return false;
-        sp--;
-        const int2 e = base[(size_t)sp * stride];
-        rf = e.x; t = __int_as_float(e.y);
-        return true;
-    }
+// A two-level traversal held by the four lanes of a quad (rt_quad.h): the
+// current ray, in world or object space. The world ray stays in LDS (at w:
+// three components of the origin, then of the direction, `stride` apart).
+struct Quad2 : rtq::Ray4 {
+    int inst, hinst;                    // current instance (-1: world), instance of this lane's candidate
+    rtq::gptr nodes, tris;
 };
 
-// Stack in LDS ([LDSD][BLOCK]) spilling to global memory beyond LDSD entries.
-template <int LDSD, int BLOCK>
-struct LdsStack {
-    int* sref;
-    float* stn;
-    int2* spill;
-    size_t stride;
-    int tid, gtid, max, sp;
-    int* status;
-    __device__ __forceinline__ void push(int rf, float t) {
-        if (sp < LDSD) {
-            sref[sp * BLOCK + tid] = rf;
-            stn[sp * BLOCK + tid] = t;
-        } else if (sp < max) {
-            spill[(size_t)(sp - LDSD) * stride + gtid] = make_int2(rf, __float_as_int(t));
-        } else {
-            atomicOr(status, 1);   // unreachable: max bounds a DFS of the two levels
-            return;
-        }
-        sp++;
-    }
-    __device__ __forceinline__ bool pop(int& rf, float& t) {
-        if (sp == 0) return false;
-        sp--;
-        if (sp < LDSD) {
-            rf = sref[sp * BLOCK + tid];
-            t = stn[sp * BLOCK + tid];
-        } else {
-            const int2 e = spill[(size_t)(sp - LDSD) * stride + gtid];
-            rf = e.x; t = __int_as_float(e.y);
-        }
-        return true;
-    }
-};
+// Lane C's value in every lane of a quad.
+template <int C>
+__device__ __forceinline__ float quad_bcast(float v) { return rtq::quad_perm<C * 0x55>(v); }
 
-// One ray through TLAS and BLAS: the traversal of k_trace2l for a single ray
-// (same culling and tie rule; any hit may visit children nearest first,
-// ORD). Closest hit: returns whether something was hit and (t, inst, id, u,
-// v); any hit: whether the ray is occluded. Each loop iteration is one short
-// step — a node visit, an instance entry, or the next one or two triangles
-// of the current BLAS leaf (leaf cursor; the two fetched together) — so
-// lanes of a wave at different kinds of step do not wait for whole leaf
-// loops. As in the one-level batch kernel, the wave's priority rises one
-// level per 32 steps, so that long walks (grazing rays) issue ahead of short
-// ones; it starts at 0 with each call.
-template <bool ANY, bool ORD, class Stack>
-__device__ __forceinline__ bool trace2l_ray(const uint4* tlasNodes, const float4* tlasTris, const InstanceDev* insts,
-                                            const BlasDev* blas, const Ray& rw, Stack& st, float& bt, int& binst,
-                                            int& bid, float& bu, float& bv, int* stepsOut = nullptr) {
-    Ray ro;
-    int ref = 0, inst = -1;
-    int lts = 0, ltc = 0;                   // leaf cursor: next triangle, triangles left
-    float tn = -INFINITY, best = rw.tmax;
-    const bool flatW = rtd::ray_flat(rw);
-    bool flatO = false;
-    const uint4* nodes = tlasNodes;
-    const float4* tris = nullptr;
-    bid = -1; binst = -1; bt = rw.tmax; bu = 0.f; bv = 0.f;
-    auto push = [&](int rf, float t) { st.push(rf, t); };
-    constexpr int kPrio2 = 32;
-    __builtin_amdgcn_s_setprio(0);
-    int steps = 0;
-    for (;;) {
-        if ((++steps & 15) == 0) {
-            const int s = __builtin_amdgcn_readfirstlane(steps);
-            if (s == kPrio2) __builtin_amdgcn_s_setprio(1);
-            else if (s == 2 * kPrio2) __builtin_amdgcn_s_setprio(2);
-            else if (s == 3 * kPrio2) __builtin_amdgcn_s_setprio(3);
-        }
-        if (ltc == 0) {
-            while (ref == -1 || ref == kReturnMark || (!ANY && tn > best)) {
-                if (ref == kReturnMark) { inst = -1; nodes = tlasNodes; ref = -1; continue; }
-                if (!st.pop(ref, tn)) {
-                    if (stepsOut) *stepsOut = steps;
-                    return ANY ? false : bid >= 0;
-                }
-            }
-            if (ref < 0 && inst >= 0) {         // BLAS leaf: start its cursor
-                const int enc = -(ref + 2);
-                lts = enc >> 3; ltc = (enc & 7) + 1;
-                ref = -1;
-            }
-        }
-        if (ltc > 0) {
-            const int ti = lts;
-            const bool two = ltc > 1;
-            const int tj = two ? ti + 1 : ti;
-            const float4 p0 = rtd::ldg_f4(tris + 3 * ti), p1 = rtd::ldg_f4(tris + 3 * ti + 1), p2 = rtd::ldg_f4(tris + 3 * ti + 2);
-            const float4 q0 = rtd::ldg_f4(tris + 3 * tj), q1 = rtd::ldg_f4(tris + 3 * tj + 1), q2 = rtd::ldg_f4(tris + 3 * tj + 2);
-            lts += two ? 2 : 1;
-            ltc -= two ? 2 : 1;
-            // leaf order: the first triangle, then the second (a closest-hit
-            // update of the first is seen by the second's tie rule)
-            auto test = [&](const float4& a0, const float4& a1, const float4& a2) {
-                float t, u, v;
-                if (rtd::isect_watertight(ro, a0, a1, a2, t, u, v) && t > ro.tmin && t < ro.tmax) {
-                    if constexpr (ANY) {
-                        return true;
-                    } else {
-                        const int id = __float_as_int(a0.w);
-                        if (t < best || (t == best && (inst < binst || (inst == binst && id < bid)))) {
-                            best = t; bid = id; binst = inst; bt = t; bu = u; bv = v;
-                        }
-                    }
-                }
-                return false;
-            };
-            if ((test(p0, p1, p2)) || (two && test(q0, q1, q2))) {
-                if (stepsOut) *stepsOut = steps;
-                return true;
-            }
-        } else if (ref >= 0) {
-            const bool w = inst < 0;
-            const Ray& r = w ? rw : ro;
-            if constexpr (ANY && ORD) visit2w<false>(nodes, r, w ? flatW : flatO, r.tmax, ref, tn, push);
-            else visit2w<ANY>(nodes, r, w ? flatW : flatO, ANY ? r.tmax : best, ref, tn, push);
-        } else {
-            // TLAS leaf: enter its instance
-            const int enc = -(ref + 2);
-            const int k = __float_as_int(tlasTris[3 * (enc >> 3)].w);
-            push(kReturnMark, -INFINITY);
-            inst = k;
-            const InstanceDev& I = insts[k];
-            xform(I.w2o, rw, ro);
-            flatO = rtd::ray_flat(ro);
-            const BlasDev& B = blas[I.blas];
-            nodes = B.nodes;
-            tris = B.tris;
-            ref = 0;
-            tn = -INFINITY;
-        }
-    }
+// Makes the world ray current (TLAS nodes; no triangles are tested in it, so
+// the shear is not set up). Each lane divides for its own axis.
+__device__ __forceinline__ void quad_world(Quad2& q, int c, const float* w, int stride, const void* tlasNodes) {
+    const float inv = 1.0f / w[(3 + min(c, 2)) * stride];
+    q.ox = w[0]; q.oy = w[stride]; q.oz = w[2 * stride];
+    q.ix = quad_bcast<0>(inv); q.iy = quad_bcast<1>(inv); q.iz = quad_bcast<2>(inv);
+    q.kx = 0; q.ky = 1; q.kz = 2;
+    q.far = __builtin_isinf(q.ix) || __builtin_isinf(q.iy) || __builtin_isinf(q.iz) ? INFINITY : NAN;
+    q.inst = -1;
+    q.nodes = (rtq::gptr)tlasNodes;
 }
 
-// Global-stack form used by the path tracer's tail kernel.
-template <bool ANY>
-__device__ __forceinline__ bool trace2l_one(const uint4* tlasNodes, const float4* tlasTris, const InstanceDev* insts,
-                                            const BlasDev* blas, const Ray& rw, int2* stk, int stride, int maxStack,
-                                            int* status, float& bt, int& binst, int& bid) {
-    GlobalStack st{stk, stride, maxStack, 0, status};
-    float bu, bv;
-    return trace2l_ray<ANY, false>(tlasNodes, tlasTris, insts, blas, rw, st, bt, binst, bid, bu, bv);
+// Makes instance k's object-space ray current: xform and rtd::ray_setup with
+// the same operations, each lane transforming and dividing for its own axis.
+__device__ __forceinline__ void quad_enter(Quad2& q, int c, const float* w, int stride, int k, const InstanceDev* insts,
+                                           const BlasDev* blas) {
+    const InstanceDev& I = insts[k];
+    const float4 M = ((const float4*)I.w2o)[min(c, 2)];
+    const BlasDev& B = blas[I.blas];
+    const float o = ((M.x * w[0] + M.y * w[stride]) + M.z * w[2 * stride]) + M.w;
+    const float d = (M.x * w[3 * stride] + M.y * w[4 * stride]) + M.z * w[5 * stride];
+    const float inv = 1.0f / d;
+    const float dx = quad_bcast<0>(d), dy = quad_bcast<1>(d), dz = quad_bcast<2>(d);
+    const float ix = quad_bcast<0>(inv), iy = quad_bcast<1>(inv), iz = quad_bcast<2>(inv);
+    const float ax = fabsf(dx), ay = fabsf(dy), az = fabsf(dz);
+    int kz = 0;
+    if (ay > ax) kz = 1;
+    if (az > (kz == 0 ? ax : ay)) kz = 2;
+    int kx = kz + 1; if (kx == 3) kx = 0;
+    int ky = kx + 1; if (ky == 3) ky = 0;
+    const float dkz = rtd::sel3(kz, dx, dy, dz);
+    if (dkz < 0.0f) { const int t = kx; kx = ky; ky = t; }
+    const float S = (c == 0 ? rtd::sel3(kx, dx, dy, dz) : c == 1 ? rtd::sel3(ky, dx, dy, dz) : 1.0f) / dkz;
+    q.Sx = quad_bcast<0>(S); q.Sy = quad_bcast<1>(S); q.Sz = quad_bcast<2>(S);
+    const float ox = quad_bcast<0>(o), oy = quad_bcast<1>(o), oz = quad_bcast<2>(o);
+    q.ox = rtd::sel3(kx, ox, oy, oz); q.oy = rtd::sel3(ky, ox, oy, oz); q.oz = rtd::sel3(kz, ox, oy, oz);
+    q.ix = rtd::sel3(kx, ix, iy, iz); q.iy = rtd::sel3(ky, ix, iy, iz); q.iz = rtd::sel3(kz, ix, iy, iz);
+    q.kx = kx; q.ky = ky; q.kz = kz;
+    q.far = __builtin_isinf(ix) || __builtin_isinf(iy) || __builtin_isinf(iz) ? INFINITY : NAN;
+    q.inst = k;
+    q.nodes = (rtq::gptr)B.nodes;
+    q.tris = (rtq::gptr)B.tris;
+}
+
+// Two-level traversal of the rays of quads with `has`, from q.ref (a node or
+// leaf code, a return marker, or -1: what the stack holds next) until they are
+// done; the current ray is set up. Culling and tie rule of k_trace2l; the
+// stack as in rtq::traverse. Returns the steps taken; q.found: an any-hit
+// ray's result. The loop has one way through and ends for all quads at once:
+// with quads leaving it, or continuing it, from within, each of the some 30
+// registers of state had a second one and was copied in every step.
+template <bool ANY, class Push, class Pop>
+__device__ __forceinline__ int quad_trace2(Quad2& q, bool has, int c, int sh, const float* w, int stride,
+                                           const void* tlasNodes, const float4* tlasTris, const InstanceDev* insts,
+                                           const BlasDev* blas, int maxStack, int* status, Push&& push, Pop&& pop) {
+    int steps = 0;
+    while (__any(has)) {
+        steps++;
+        bool next = false;
+        if (has) {
+            if (q.ref >= 0) {
+                if (ANY || q.tn <= q.best)
+                    next = rtq::visit<ANY>(q, c, sh, rtq::slot_of(q, q.nodes + ((size_t)(uint32_t)q.ref << 6), c), maxStack,
+                                           status, push);
+            } else if (q.ref == kReturnMark) {
+                quad_world(q, c, w, stride, tlasNodes);
+            } else if (q.ref != -1 && (ANY || q.tn <= q.best)) {
+                const int enc = -(q.ref + 2);
+                if (q.inst < 0) {
+                    // TLAS leaf: enter its instance
+                    const int k = __float_as_int(tlasTris[3 * (enc >> 3)].w);
+                    if (q.sp < maxStack) {
+                        if (c == 0) push(q, q.sp, kReturnMark, -INFINITY);
+                        q.sp++;
+                    } else {
+                        atomicOr(status, 1);   // unreachable: maxStack bounds a DFS of the two levels
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    quad_enter(q, c, w, stride, k, insts, blas);
+                    q.ref = 0;
+                    q.tn = -INFINITY;
+                    next = true;
+                } else {
+                    q.found = rtq::leaf<ANY>(q, c, sh, q.tris + (size_t)(enc >> 3) * 48, 0, (enc & 7) + 1, [&](float t, int id) {
+                        const bool closer =
+                            t < q.t || (t == q.t && (q.inst < q.hinst || (q.inst == q.hinst && id < q.id)));
+                        if (closer) q.hinst = q.inst;
+                        return closer;
+                    });
+                }
+            }
+            if (!next) {
+                has = q.sp > 0 && !(ANY && q.found);
+                if (has) {
+                    q.sp--;
+                    pop(q, q.sp, q.ref, q.tn);
+                }
+            }
+        }
+    }
+    return steps;
+}
+
+// The quad's closest hit into every lane (ties: the lowest instance, then ID).
+__device__ __forceinline__ void quad_reduce2(Quad2& q) {
+#define RT_QSTEP(P)                                                                                          \
+    {                                                                                                        \
+        const float t = rtq::quad_perm<P>(q.t), u = rtq::quad_perm<P>(q.u), v = rtq::quad_perm<P>(q.v);      \
+        const int id = rtq::quad_perm<P>(q.id), in = rtq::quad_perm<P>(q.hinst);                             \
+        if (t < q.t || (t == q.t && (in < q.hinst || (in == q.hinst && id < q.id)))) {                       \
+            q.t = t; q.u = u; q.v = v; q.id = id; q.hinst = in;                                              \
+        }                                                                                                    \
+    }
+    RT_QSTEP(rtq::kXor1) RT_QSTEP(rtq::kXor2)
+#undef RT_QSTEP
 }
 
 }  // namespace rtk

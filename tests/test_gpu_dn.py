@@ -194,3 +194,34 @@ def test_weight_gradients_do_not_depend_on_the_split(pkg, dn_ref, dev, H, W):
         cout = dn_ref.LAYERS[i][1]
         assert _rel(grads[1][wo:bo], grads[0][wo:bo]) < 1e-4, i
         assert _rel(grads[1][bo:bo + cout], grads[0][bo:bo + cout]) < 1e-4, i
+
+
+@pytest.mark.parametrize("layer", range(14))
+def test_relu_stops_gradients(pkg, dev, layer):
+    """With a layer's outputs all 0 (a large negative bias) its ReLU lets no
+    gradient through, in whichever kernel that is done: the layer's own weight
+    and bias gradients are exactly 0. The biases are 0 otherwise, so everything
+    is when one of the first or last two layers is (all else passes through
+    them); the other layers leave a path through a skip connection."""
+    import torch
+    shapes = [(16, 32, 9), (32, 32, 9), (32, 64, 9), (64, 64, 9), (64, 128, 9), (128, 128, 9), (128, 256, 9),
+              (256, 256, 9), (384, 128, 9), (128, 128, 9), (192, 64, 9), (64, 64, 9), (96, 32, 9), (32, 32, 9), (32, 3, 1)]
+    sizes = [ci * co * t + co for ci, co, t in shapes]
+    off = np.concatenate([[0], np.cumsum(sizes)])
+    B, H, W = 2, 24, 40
+    d = pkg.Denoiser(B * H * W, seed=3)
+    try:
+        w = d.params(0)
+        w[off[layer + 1] - shapes[layer][1]:off[layer + 1]] = -1e3
+        d.set_params(w)
+        g = torch.Generator(device=dev).manual_seed(layer)
+        x = (torch.randn(B * H * W, 16, device=dev, generator=g) * 0.5).to(torch.bfloat16).view(torch.int16)
+        y = torch.randn(B * H * W, 3, device=dev, generator=g)
+        d.train_step(B, H, W, x, y, 0.0)
+        grad = d.params(1)
+        assert not grad[off[layer]:off[layer + 1]].any()
+        assert grad[-3:].any()
+        alive = [k for k in range(14) if grad[off[k]:off[k + 1]].any()]
+        assert not alive if layer in (0, 1, 12, 13) else 13 in alive
+    finally:
+        d.destroy()

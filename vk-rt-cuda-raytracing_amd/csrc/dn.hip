@@ -103,6 +103,10 @@ struct ConvArgs {
     const uint16_t* hw; const float* hbias; float* head; const float* rgbIn; float* rgbOut;
     // k_conv3r only: x stores input channels [xc0, cin) (channel c at c - xc0)
     int xc0;
+    // the BF16 output is zero where ym is not positive (stride n; nullable,
+    // MASK for k_conv3r): the ReLU backward of the tensor whose gradient the
+    // output is
+    const uint16_t* ym;
 };
 
 // Block: 4 waves x (16*WM) pixels; each wave (16*WM) pixels x (16*WN)
@@ -197,7 +201,7 @@ __global__ __launch_bounds__(kBlock) void k_conv(ConvArgs a) {
                 if (p >= P) continue;
                 float v = acc[r][j][i] + b;
                 if (a.relu) v = fmaxf(v, 0.0f);
-                if (a.y) a.y[(size_t)p * a.ldy + col] = f2bf(v);
+                if (a.y) a.y[(size_t)p * a.ldy + col] = !a.ym || bf2f(a.ym[(size_t)p * a.n + col]) > 0.0f ? f2bf(v) : (uint16_t)0;
                 if (a.yf) a.yf[(size_t)p * a.ldyf + col] = v;
             }
         }
@@ -248,7 +252,7 @@ __device__ __forceinline__ void halo_row_order() {
     }
 }
 
-template <int R, int WGX, int WGC, int OCC, int PD, bool BL, int CS = 32, bool HD = false>
+template <int R, int WGX, int WGC, int OCC, int PD, bool BL, int CS = 32, bool HD = false, bool MASK = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(OCC))) void k_conv3r(ConvArgs a) {
     static_assert(WGX * WGC == kBlock / 64, "four waves");
     static_assert(!BL || WGC == 1, "weights are shared through LDS only when every wave has the same channels");
@@ -421,9 +425,18 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(OCC))) v
                     if (a.relu) v[j][i] = fmaxf(v[j][i], 0.0f);
                 }
                 const bool ok = y < a.H && x < a.W && col < a.n;
-                if (ok && a.y)
-                    *(uint2*)(a.y + p * a.ldy + col) = make_uint2(f2bf(v[j][0]) | ((uint32_t)f2bf(v[j][1]) << 16),
-                                                                  f2bf(v[j][2]) | ((uint32_t)f2bf(v[j][3]) << 16));
+                if (ok && a.y) {
+                    uint2 o = make_uint2(f2bf(v[j][0]) | ((uint32_t)f2bf(v[j][1]) << 16),
+                                         f2bf(v[j][2]) | ((uint32_t)f2bf(v[j][3]) << 16));
+                    if constexpr (MASK) {
+                        const uint2 m = *(const uint2*)(a.ym + p * a.n + col);
+                        if (!(bf2f((uint16_t)m.x) > 0.0f)) o.x &= 0xffff0000u;
+                        if (!(bf2f((uint16_t)(m.x >> 16)) > 0.0f)) o.x &= 0xffffu;
+                        if (!(bf2f((uint16_t)m.y) > 0.0f)) o.y &= 0xffff0000u;
+                        if (!(bf2f((uint16_t)(m.y >> 16)) > 0.0f)) o.y &= 0xffffu;
+                    }
+                    *(uint2*)(a.y + p * a.ldy + col) = o;
+                }
                 if (ok && a.yf) *(float4*)(a.yf + p * a.ldyf + col) = make_float4(v[j][0], v[j][1], v[j][2], v[j][3]);
                 if constexpr (R % 2 == 0) {
                     if (a.yp) {
@@ -899,23 +912,8 @@ __global__ __launch_bounds__(kBlock) void k_reduce_splits(const float* part, int
 }
 
 // ---------------------------------------------------------- elementwise ----
-// g *= (y > 0), 8 channels per thread
-__global__ __launch_bounds__(kBlock) void k_relu_bwd(uint16_t* g, int ldg, const uint16_t* y, int ldy, int c, int P) {
-    const int cg = c / 8;
-    for (size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x; i < (size_t)P * cg; i += (size_t)gridDim.x * kBlock) {
-        const size_t p = i / cg;
-        const int k = 8 * (int)(i % cg);
-        uint4 gv = *(uint4*)(g + p * ldg + k);
-        const uint4 yv = *(const uint4*)(y + p * ldy + k);
-        uint16_t* ge = (uint16_t*)&gv;
-        const uint16_t* ye = (const uint16_t*)&yv;
-        for (int e = 0; e < 8; e++)
-            if (!(bf2f(ye[e]) > 0.0f)) ge[e] = 0;
-        *(uint4*)(g + p * ldg + k) = gv;
-    }
-}
-
-// pool backward: gin[argmax] += gout (first maximum in window order)
+// pool backward: gin[argmax] += gout (first maximum in window order), then the
+// ReLU of the pooled tensor itself: gin *= (in > 0)
 __global__ __launch_bounds__(kBlock) void k_pool_bwd(const uint16_t* in, int ldi, const uint16_t* gout, int ldgo,
                                                      uint16_t* gin, int ldgi, int c, int B, int H, int W) {
     const int Ho = H / 2, Wo = W / 2, cg = c / 8;
@@ -927,11 +925,12 @@ __global__ __launch_bounds__(kBlock) void k_pool_bwd(const uint16_t* in, int ldi
         float m[8];
         int arg[8];
         size_t pis[4];
+        uint4 vs[4];
         for (int e = 0; e < 8; e++) { m[e] = -INFINITY; arg[e] = 0; }
         for (int s = 0; s < 4; s++) {
             pis[s] = ((size_t)(b * H + 2 * yo + (s >> 1)) * W + 2 * xo + (s & 1));
-            const uint4 v = *(const uint4*)(in + pis[s] * ldi + k);
-            const uint16_t* ve = (const uint16_t*)&v;
+            vs[s] = *(const uint4*)(in + pis[s] * ldi + k);
+            const uint16_t* ve = (const uint16_t*)&vs[s];
             for (int e = 0; e < 8; e++) {
                 const float f = bf2f(ve[e]);
                 if (f > m[e]) { m[e] = f; arg[e] = s; }
@@ -942,8 +941,11 @@ __global__ __launch_bounds__(kBlock) void k_pool_bwd(const uint16_t* in, int ldi
         for (int s = 0; s < 4; s++) {
             uint4 d = *(uint4*)(gin + pis[s] * ldgi + k);
             uint16_t* de = (uint16_t*)&d;
-            for (int e = 0; e < 8; e++)
+            const uint16_t* ve = (const uint16_t*)&vs[s];
+            for (int e = 0; e < 8; e++) {
                 if (arg[e] == s) de[e] = f2bf(bf2f(de[e]) + bf2f(gve[e]));
+                if (!(bf2f(ve[e]) > 0.0f)) de[e] = 0;
+            }
             *(uint4*)(gin + pis[s] * ldgi + k) = d;
         }
     }
@@ -963,9 +965,10 @@ __global__ __launch_bounds__(kBlock) void k_up(const uint16_t* in, int ldi, uint
     }
 }
 
-// upsampling backward: gin[p] = sum of the 4 gout children (window order)
-__global__ __launch_bounds__(kBlock) void k_up_bwd(const uint16_t* gout, int ldgo, uint16_t* gin, int ldgi, int c,
-                                                   int B, int H, int W) {
+// upsampling backward: gin[p] = sum of the 4 gout children (window order),
+// then the ReLU of the upsampled tensor act (row stride c): gin *= (act > 0)
+__global__ __launch_bounds__(kBlock) void k_up_bwd(const uint16_t* gout, int ldgo, uint16_t* gin, int ldgi,
+                                                   const uint16_t* act, int c, int B, int H, int W) {
     const int cg = c / 8;
     const size_t n = (size_t)B * H * W * cg;
     for (size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock) {
@@ -981,7 +984,9 @@ __global__ __launch_bounds__(kBlock) void k_up_bwd(const uint16_t* gout, int ldg
         }
         uint4 o;
         uint16_t* oe = (uint16_t*)&o;
-        for (int e = 0; e < 8; e++) oe[e] = f2bf(s[e]);
+        const uint4 av = *(const uint4*)(act + pi * c + k);
+        const uint16_t* ae = (const uint16_t*)&av;
+        for (int e = 0; e < 8; e++) oe[e] = bf2f(ae[e]) > 0.0f ? f2bf(s[e]) : (uint16_t)0;
         *(uint4*)(gin + pi * ldgi + k) = o;
     }
 }
@@ -1027,50 +1032,78 @@ __global__ __launch_bounds__(kBlock) void k_adam(float* w, float* m, float* v, c
     }
 }
 
-// master [cout][taps][cin] -> forward BF16 [rowsF][taps*cin] and the flipped
-// transpose for input gradients [rowsB][taps*coutK]: wb[ci][t][co] = w[co][taps-1-t][ci]
-__global__ __launch_bounds__(kBlock) void k_wlayout(const float* w, int cout, int taps, int cin, uint16_t* wf,
-                                                    uint16_t* wb, int coutK) {
-    const size_t n = (size_t)cout * taps * cin;
-    for (size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock) {
-        const int ci = (int)(i % cin);
-        const int t = (int)((i / cin) % taps);
-        const int co = (int)(i / ((size_t)cin * taps));
-        const uint16_t h = f2bf(w[i]);
-        wf[i] = h;
-        wb[((size_t)ci * taps + (taps - 1 - t)) * coutK + co] = h;
-    }
-}
+// BF16 weight layouts from the FP32 master parameters ([cout][taps][cin]), all
+// layers in one launch: laid out one after the other, after every optimizer
+// step, they were 43 launches of 3-4 us.
+//   kForward    [rowsF][taps * cin], the master's order
+//   kBackward   [rowsB][taps * coutK], the flipped transpose for input
+//               gradients: [ci][t][co] = w[co][taps - 1 - t][ci]
+//   kFrag       kForward of a 3x3 layer (cin a multiple of 32) in MFMA
+//               fragment order [rows/16][cin/32][9][lane][8]: lane = row%16 +
+//               16*kg holds the 8 consecutive input channels 32*chunk + 8*kg
+//               .. +7 of tap t of that row (the B operand of
+//               mfma_f32_16x16x32_bf16 for one tap and channel chunk)
+//   kFragB      kBackward in the same order (coutK a multiple of 32)
+//   kFrag16     kForward of a 3x3 layer of 16 channels in fragment order
+//               [rows/16][3 dy][2 tap pairs][lane][8]: lane = row%16 + 16*kg
+//               holds input channels 8 (kg & 1) .. +7 of tap (dy, 2 pair +
+//               (kg >> 1)); tap column 3 (the second half of the last pair) is
+//               zero
+// One thread makes 8 consecutive elements; rows past the layer's are zero.
+enum LayoutKind { kForward, kBackward, kFrag, kFragB, kFrag16 };
+struct LayoutJob {
+    const float* w;
+    uint16_t* out;
+    int kind, cout, taps, cin, coutK;
+    int groups, block0;                     // threads, first workgroup
+};
+constexpr int kMaxJobs = 60;
+struct LayoutArgs {
+    LayoutJob job[kMaxJobs];
+    int jobs;
+};
 
-// [rows][9*cin] (row-major 3x3 weights, cin a multiple of 32) -> MFMA
-// fragment order [rows/16][cin/32][9][lane][8]: lane = row%16 + 16*kg holds
-// the 8 consecutive input channels 32*chunk + 8*kg .. +7 of tap t of that row
-// (the B operand of mfma_f32_16x16x32_bf16 for one tap and channel chunk).
-__global__ __launch_bounds__(kBlock) void k_wfrag(const uint16_t* w, int rows, int cin, uint16_t* out) {
-    const size_t n = (size_t)rows * 9 * cin;
-    const int nch = cin / 32;
-    for (size_t o = blockIdx.x * (size_t)kBlock + threadIdx.x; o < n; o += (size_t)gridDim.x * kBlock) {
-        const int e = (int)(o & 7), lane = (int)((o >> 3) & 63);
-        const size_t q = o >> 9;
-        const int t = (int)(q % 9), c = (int)((q / 9) % nch), blk = (int)(q / 9 / nch);
-        const int row = blk * 16 + (lane & 15), kg = lane >> 4;
-        out[o] = w[(size_t)row * 9 * cin + t * cin + c * 32 + kg * 8 + e];
+__global__ __launch_bounds__(kBlock) void k_layouts(LayoutArgs a) {
+    int j = 0;
+    while (j + 1 < a.jobs && (int)blockIdx.x >= a.job[j + 1].block0) j++;
+    const LayoutJob& J = a.job[j];
+    const int g = ((int)blockIdx.x - J.block0) * kBlock + (int)threadIdx.x;
+    if (g >= J.groups) return;
+    // the 8 elements are base + e * stride, all or none inside the layer but
+    // for a channel count that is no multiple of 8 (limit)
+    size_t base = 0;
+    int stride = 1, limit = 8;
+    if (J.kind == kForward) {
+        base = (size_t)g * 8;
+    } else if (J.kind == kBackward) {
+        const int cg = J.coutK / 8, co = 8 * (g % cg), t = (g / cg) % J.taps, ci = g / (cg * J.taps);
+        base = ((size_t)co * J.taps + (J.taps - 1 - t)) * J.cin + ci;
+        stride = J.taps * J.cin;
+        limit = J.cout - co;
+    } else {
+        const int lane = g & 63, q = g >> 6, kg = lane >> 4;
+        if (J.kind == kFrag16) {
+            const int pr = q % 2, dy = (q / 2) % 3, row = (q / 6) * 16 + (lane & 15), dx = 2 * pr + (kg >> 1);
+            base = (size_t)row * 144 + (dy * 3 + dx) * 16 + 8 * (kg & 1);
+            limit = dx < 3 && row < J.cout ? 8 : 0;
+        } else {
+            const int nch = (J.kind == kFrag ? J.cin : J.coutK) / 32;
+            const int t = q % 9, k = (q / 9) % nch * 32 + kg * 8, row = q / (9 * nch) * 16 + (lane & 15);
+            if (J.kind == kFrag) {
+                base = ((size_t)row * 9 + t) * J.cin + k;
+                limit = row < J.cout ? 8 : 0;
+            } else {
+                base = ((size_t)k * 9 + (8 - t)) * J.cin + row;
+                stride = 9 * J.cin;
+                limit = row < J.cin ? J.cout - k : 0;
+            }
+        }
     }
-}
-
-// [rows][9*16] (3x3 weights of a 16-channel input) -> fragment order
-// [rows/16][3 dy][2 tap pairs][lane][8]: lane = row%16 + 16*kg holds input
-// channels 8 (kg & 1) .. +7 of tap (dy, 2 pair + (kg >> 1)); tap column 3
-// (the second half of the last pair) is zero.
-__global__ __launch_bounds__(kBlock) void k_wfrag16(const uint16_t* w, int rows, uint16_t* out) {
-    const size_t n = (size_t)rows * 6 * 64;
-    for (size_t o = blockIdx.x * (size_t)kBlock + threadIdx.x; o < n; o += (size_t)gridDim.x * kBlock) {
-        const int e = (int)(o & 7), lane = (int)((o >> 3) & 63);
-        const size_t q = o >> 9;
-        const int pr = (int)(q % 2), dy = (int)((q / 2) % 3), blk = (int)(q / 6);
-        const int row = blk * 16 + (lane & 15), kg = lane >> 4, dx = 2 * pr + (kg >> 1);
-        out[o] = dx < 3 ? w[(size_t)row * 144 + (dy * 3 + dx) * 16 + 8 * (kg & 1) + e] : (uint16_t)0;
-    }
+    uint4 o;
+    uint16_t* oe = (uint16_t*)&o;
+#pragma unroll
+    for (int e = 0; e < 8; e++) oe[e] = e < limit ? f2bf(J.w[base + (size_t)e * stride]) : (uint16_t)0;
+    *(uint4*)(J.out + (size_t)g * 8) = o;
 }
 
 // planes (rgb, albedo, normal: 3 x P; depth: P) -> 16-channel BF16 pixels
@@ -1154,20 +1187,21 @@ static void launch_conv(const ConvArgs& a, int P, int n, hipStream_t s) {
 // staged once per workgroup in LDS when there is more than one channel chunk
 // (all four waves use the same 32 channels; 12 % faster on the 96-channel
 // decoder layer).
-template <int R, int WGX, int WGC, int OCC, int PD, bool BL, int CS = 32, bool HD = false>
+template <int R, int WGX, int WGC, int OCC, int PD, bool BL, int CS = 32, bool HD = false, bool MASK = false>
 static void launch_r(const ConvArgs& a, int chanTiles, hipStream_t s) {
     constexpr int TX = 16 * WGX;
     const dim3 grid(((a.W + TX - 1) / TX) * ((a.H + R - 1) / R) * a.B, chanTiles);
-    hipLaunchKernelGGL((k_conv3r<R, WGX, WGC, OCC, PD, BL, CS, HD>), grid, dim3(kBlock), 0, s, a);
+    hipLaunchKernelGGL((k_conv3r<R, WGX, WGC, OCC, PD, BL, CS, HD, MASK>), grid, dim3(kBlock), 0, s, a);
 }
 
+template <bool MASK>
 static void launch_conv3(const ConvArgs& a, int n, hipStream_t s) {
-    if (n % 128 == 0) launch_r<8, 1, 4, 2, 3, false>(a, n / 128, s);
-    else if (n % 64 == 0 && a.cin >= 128) launch_r<8, 2, 2, 2, 3, false>(a, n / 64, s);
-    else if (n % 64 == 0 && a.cin == 64) launch_r<4, 2, 2, 3, 2, false>(a, n / 64, s);
-    else if (a.cin > 32) launch_r<4, 4, 1, 3, 2, true>(a, (n + 31) / 32, s);
+    if (n % 128 == 0) launch_r<8, 1, 4, 2, 3, false, 32, false, MASK>(a, n / 128, s);
+    else if (n % 64 == 0 && a.cin >= 128) launch_r<8, 2, 2, 2, 3, false, 32, false, MASK>(a, n / 64, s);
+    else if (n % 64 == 0 && a.cin == 64) launch_r<4, 2, 2, 3, 2, false, 32, false, MASK>(a, n / 64, s);
+    else if (a.cin > 32) launch_r<4, 4, 1, 3, 2, true, 32, false, MASK>(a, (n + 31) / 32, s);
     else if (a.hw) launch_r<4, 4, 1, 2, 2, false, 32, true>(a, 1, s);
-    else launch_r<4, 4, 1, 3, 2, false>(a, (n + 31) / 32, s);
+    else launch_r<4, 4, 1, 3, 2, false, 32, false, MASK>(a, (n + 31) / 32, s);
 }
 
 // Optional fusions (3x3 layers with 32-channel chunks): `up` supplies input
@@ -1185,7 +1219,7 @@ static void conv_fwd(Net& N, int li, const uint16_t* x, int ldx, uint16_t* y, in
     ConvArgs a{x, ldx, L.d.cin, L.wf, L.wfF, N.w + L.bOff, y, ldy, yf, ldyf, L.d.cout, B, H, W, relu ? 1 : 0,
                up.x, up.ld, up.cup, yp, ldyp,
                Lh ? Lh->wf : nullptr, Lh ? N.w + Lh->bOff : nullptr, hf.head, hf.rgbIn, hf.rgbOut,
-               up.skipOnly ? up.cup : 0};
+               up.skipOnly ? up.cup : 0, nullptr};
     if (Lh && !(L.d.taps == 9 && L.d.cin == 32 && L.d.cout == 32 && Lh->d.cin == 32 && Lh->d.cout == 3)) {
         rt::set_error("denoiser: head fusion needs a 32 -> 32 3x3 layer and a 32 -> 3 head");
         return;
@@ -1204,7 +1238,7 @@ static void conv_fwd(Net& N, int li, const uint16_t* x, int ldx, uint16_t* y, in
     } else if (L.d.cin % 32) {
         if (WN == 2) launch_conv<9, 16, 2>(a, P, L.d.cout, s);
         else launch_conv<9, 16, 4>(a, P, L.d.cout, s);
-    } else launch_conv3(a, L.d.cout, s);
+    } else launch_conv3<false>(a, L.d.cout, s);
 }
 
 // The first two layers (16 -> 32 -> 32 channels, ReLU after each) in one
@@ -1218,14 +1252,19 @@ static void conv01_fwd(Net& N, uint16_t* y0out, uint16_t* y, int ldy, uint16_t* 
 }
 
 // input gradient: dx = conv(g, flipped transposed weights)
-static void conv_dx(Net& N, int li, const uint16_t* g, int ldg, uint16_t* dx, int lddx, int B, int H, int W) {
+// y: the layer's input where that is a ReLU's output (dense), whose backward is
+// then part of dx
+static void conv_dx(Net& N, int li, const uint16_t* g, int ldg, uint16_t* dx, int lddx, int B, int H, int W,
+                    const uint16_t* y = nullptr) {
     const Layer& L = N.L[li];
     ConvArgs a{g, ldg, L.coutK, L.wb, L.wfB, nullptr, dx, lddx, nullptr, 0, L.d.cin, B, H, W, 0};
+    a.ym = y;
     const int P = B * H * W;
     const int WN = L.d.cin >= 64 ? 4 : 2;
     hipStream_t s = N.stream;
     if (L.d.taps == 1) launch_conv<1, 16, 2>(a, P, L.d.cin, s);
-    else launch_conv3(a, L.d.cin, s);
+    else if (y) launch_conv3<true>(a, L.d.cin, s);
+    else launch_conv3<false>(a, L.d.cin, s);
 }
 
 // Weight and bias gradient of layer li into N.g (weights, then biases, as the
@@ -1261,9 +1300,6 @@ static void conv_dw(Net& N, int li, const uint16_t* g, int ldg, const uint16_t* 
     else launch_wgrad<9, 2, 2, 2, 2>(N, a, n, grad);
 }
 
-static void relu_bwd(Net& N, uint16_t* g, int ldg, const uint16_t* y, int ldy, int c, int P) {
-    hipLaunchKernelGGL(k_relu_bwd, dim3(grid_for((size_t)P * c / 8)), dim3(kBlock), 0, N.stream, g, ldg, y, ldy, c, P);
-}
 static void pool_bwd(Net& N, const uint16_t* in, int ldi, const uint16_t* go, int ldgo, uint16_t* gi, int ldgi, int c,
                      int B, int H, int W) {
     hipLaunchKernelGGL(k_pool_bwd, dim3(grid_for((size_t)B * H * W / 4 * c / 8)), dim3(kBlock), 0, N.stream, in, ldi,
@@ -1273,27 +1309,31 @@ static void up(Net& N, const uint16_t* in, int ldi, uint16_t* out, int ldo, int 
     hipLaunchKernelGGL(k_up, dim3(grid_for((size_t)B * H * W * 4 * c / 8)), dim3(kBlock), 0, N.stream, in, ldi, out,
                        ldo, c, B, H, W);
 }
-static void up_bwd(Net& N, const uint16_t* go, int ldgo, uint16_t* gi, int ldgi, int c, int B, int H, int W) {
+static void up_bwd(Net& N, const uint16_t* go, int ldgo, uint16_t* gi, int ldgi, const uint16_t* y, int c, int B, int H,
+                   int W) {
     hipLaunchKernelGGL(k_up_bwd, dim3(grid_for((size_t)B * H * W * c / 8)), dim3(kBlock), 0, N.stream, go, ldgo, gi,
-                       ldgi, c, B, H, W);
+                       ldgi, y, c, B, H, W);
 }
 
 static void update_layouts(Net& N) {
+    LayoutArgs a;
+    a.jobs = 0;
+    int blocks = 0;
     for (int i = 0; i < kNumLayers; i++) {
         const Layer& L = N.L[i];
-        const size_t n = (size_t)L.d.cout * L.d.taps * L.d.cin;
-        hipLaunchKernelGGL(k_wlayout, dim3(grid_for(n)), dim3(kBlock), 0, N.stream, N.w + L.wOff, L.d.cout, L.d.taps,
-                           L.d.cin, L.wf, L.wb, L.coutK);
-        if (L.wfF && L.d.cin == 16)
-            hipLaunchKernelGGL(k_wfrag16, dim3(grid_for((size_t)L.rowsF * 6 * 64)), dim3(kBlock), 0, N.stream, L.wf,
-                               L.rowsF, L.wfF);
-        else if (L.wfF)
-            hipLaunchKernelGGL(k_wfrag, dim3(grid_for((size_t)L.rowsF * 9 * L.d.cin)), dim3(kBlock), 0, N.stream, L.wf,
-                               L.rowsF, L.d.cin, L.wfF);
-        if (L.wfB)
-            hipLaunchKernelGGL(k_wfrag, dim3(grid_for((size_t)L.rowsB * 9 * L.coutK)), dim3(kBlock), 0, N.stream,
-                               L.wb, L.rowsB, L.coutK, L.wfB);
+        auto add = [&](int kind, uint16_t* out, size_t elems) {
+            if (!out) return;
+            LayoutJob& J = a.job[a.jobs++];
+            J = {N.w + L.wOff, out, kind, L.d.cout, L.d.taps, L.d.cin, L.coutK, (int)(elems / 8), blocks};
+            blocks += (J.groups + kBlock - 1) / kBlock;
+        };
+        add(kForward, L.wf, (size_t)L.d.cout * L.d.taps * L.d.cin);
+        add(kBackward, L.wb, (size_t)L.d.cin * L.d.taps * L.coutK);
+        if (L.d.cin == 16) add(kFrag16, L.wfF, (size_t)L.rowsF * 6 * 64);
+        else add(kFrag, L.wfF, (size_t)L.rowsF * 9 * L.d.cin);
+        add(kFragB, L.wfB, (size_t)L.rowsB * 9 * L.coutK);
     }
+    hipLaunchKernelGGL(k_layouts, dim3(blocks), dim3(kBlock), 0, N.stream, a);
 }
 
 // forward from N.X (B x H x W x 16) to N.head (P x 3 FP32, before the
@@ -1343,58 +1383,45 @@ static void forward(Net& N, int B, int H, int W, bool train, float* rgbOut = nul
     }
 }
 
-// backward from N.gHead (P x 16, loss gradient in channels 0-2) to N.g
+// backward from N.gHead (P x 16, loss gradient in channels 0-2) to N.g. The ReLU
+// backward of each tensor is part of the kernel that writes its gradient (14
+// passes of 5-20 us on 8 x 256 x 256 when they were launches of their own).
 static void backward(Net& N, int B, int H, int W) {
     const int H1 = H / 2, W1 = W / 2, H2 = H / 4, W2 = W / 4, H3 = H / 8, W3 = W / 8;
-    const int P0 = B * H * W, P1 = B * H1 * W1, P2 = B * H2 * W2, P3 = B * H3 * W3;
     conv_dw(N, 14, N.gHead, 16, N.D1, 32, B, H, W);
-    conv_dx(N, 14, N.gHead, 16, N.gD1, 32, B, H, W);
-    relu_bwd(N, N.gD1, 32, N.D1, 32, 32, P0);
+    conv_dx(N, 14, N.gHead, 16, N.gD1, 32, B, H, W, N.D1);
     conv_dw(N, 13, N.gD1, 32, N.A12, 32, B, H, W);
-    conv_dx(N, 13, N.gD1, 32, N.gA12, 32, B, H, W);
-    relu_bwd(N, N.gA12, 32, N.A12, 32, 32, P0);
+    conv_dx(N, 13, N.gD1, 32, N.gA12, 32, B, H, W, N.A12);
     conv_dw(N, 12, N.gA12, 32, N.CAT1, 96, B, H, W);
     conv_dx(N, 12, N.gA12, 32, N.gCAT1, 96, B, H, W);
-    up_bwd(N, N.gCAT1, 96, N.gD2, 64, 64, B, H1, W1);
-    relu_bwd(N, N.gD2, 64, N.D2, 64, 64, P1);
+    up_bwd(N, N.gCAT1, 96, N.gD2, 64, N.D2, 64, B, H1, W1);
     conv_dw(N, 11, N.gD2, 64, N.A10, 64, B, H1, W1);
-    conv_dx(N, 11, N.gD2, 64, N.gA10, 64, B, H1, W1);
-    relu_bwd(N, N.gA10, 64, N.A10, 64, 64, P1);
+    conv_dx(N, 11, N.gD2, 64, N.gA10, 64, B, H1, W1, N.A10);
     conv_dw(N, 10, N.gA10, 64, N.CAT2, 192, B, H1, W1);
     conv_dx(N, 10, N.gA10, 64, N.gCAT2, 192, B, H1, W1);
-    up_bwd(N, N.gCAT2, 192, N.gD3, 128, 128, B, H2, W2);
-    relu_bwd(N, N.gD3, 128, N.D3, 128, 128, P2);
+    up_bwd(N, N.gCAT2, 192, N.gD3, 128, N.D3, 128, B, H2, W2);
     conv_dw(N, 9, N.gD3, 128, N.A8, 128, B, H2, W2);
-    conv_dx(N, 9, N.gD3, 128, N.gA8, 128, B, H2, W2);
-    relu_bwd(N, N.gA8, 128, N.A8, 128, 128, P2);
+    conv_dx(N, 9, N.gD3, 128, N.gA8, 128, B, H2, W2, N.A8);
     conv_dw(N, 8, N.gA8, 128, N.CAT3, 384, B, H2, W2);
     conv_dx(N, 8, N.gA8, 128, N.gCAT3, 384, B, H2, W2);
-    up_bwd(N, N.gCAT3, 384, N.gE4, 256, 256, B, H3, W3);
-    relu_bwd(N, N.gE4, 256, N.E4, 256, 256, P3);
+    up_bwd(N, N.gCAT3, 384, N.gE4, 256, N.E4, 256, B, H3, W3);
     conv_dw(N, 7, N.gE4, 256, N.A6, 256, B, H3, W3);
-    conv_dx(N, 7, N.gE4, 256, N.gA6, 256, B, H3, W3);
-    relu_bwd(N, N.gA6, 256, N.A6, 256, 256, P3);
+    conv_dx(N, 7, N.gE4, 256, N.gA6, 256, B, H3, W3, N.A6);
     conv_dw(N, 6, N.gA6, 256, N.P3, 128, B, H3, W3);
     conv_dx(N, 6, N.gA6, 256, N.gP3, 128, B, H3, W3);
     pool_bwd(N, N.CAT3 + 256, 384, N.gP3, 128, N.gCAT3 + 256, 384, 128, B, H2, W2);
-    relu_bwd(N, N.gCAT3 + 256, 384, N.CAT3 + 256, 384, 128, P2);
     conv_dw(N, 5, N.gCAT3 + 256, 384, N.A4, 128, B, H2, W2);
-    conv_dx(N, 5, N.gCAT3 + 256, 384, N.gA4, 128, B, H2, W2);
-    relu_bwd(N, N.gA4, 128, N.A4, 128, 128, P2);
+    conv_dx(N, 5, N.gCAT3 + 256, 384, N.gA4, 128, B, H2, W2, N.A4);
     conv_dw(N, 4, N.gA4, 128, N.P2, 64, B, H2, W2);
     conv_dx(N, 4, N.gA4, 128, N.gP2, 64, B, H2, W2);
     pool_bwd(N, N.CAT2 + 128, 192, N.gP2, 64, N.gCAT2 + 128, 192, 64, B, H1, W1);
-    relu_bwd(N, N.gCAT2 + 128, 192, N.CAT2 + 128, 192, 64, P1);
     conv_dw(N, 3, N.gCAT2 + 128, 192, N.A2, 64, B, H1, W1);
-    conv_dx(N, 3, N.gCAT2 + 128, 192, N.gA2, 64, B, H1, W1);
-    relu_bwd(N, N.gA2, 64, N.A2, 64, 64, P1);
+    conv_dx(N, 3, N.gCAT2 + 128, 192, N.gA2, 64, B, H1, W1, N.A2);
     conv_dw(N, 2, N.gA2, 64, N.P1, 32, B, H1, W1);
     conv_dx(N, 2, N.gA2, 64, N.gP1, 32, B, H1, W1);
     pool_bwd(N, N.CAT1 + 64, 96, N.gP1, 32, N.gCAT1 + 64, 96, 32, B, H, W);
-    relu_bwd(N, N.gCAT1 + 64, 96, N.CAT1 + 64, 96, 32, P0);
     conv_dw(N, 1, N.gCAT1 + 64, 96, N.A0, 32, B, H, W);
-    conv_dx(N, 1, N.gCAT1 + 64, 96, N.gA0, 32, B, H, W);
-    relu_bwd(N, N.gA0, 32, N.A0, 32, 32, P0);
+    conv_dx(N, 1, N.gCAT1 + 64, 96, N.gA0, 32, B, H, W, N.A0);
     conv_dw(N, 0, N.gA0, 32, N.X, 16, B, H, W);
 }
 

@@ -225,3 +225,28 @@ def test_relu_stops_gradients(pkg, dev, layer):
         assert not alive if layer in (0, 1, 12, 13) else 13 in alive
     finally:
         d.destroy()
+
+
+def test_bf16_rounding(pkg, dev):
+    """Every BF16 value with the low halves where rounding to nearest even can
+    go wrong: ties, their neighbours, zeros and denormals of both signs, the
+    step to infinity, infinities, NaN (which stays NaN)."""
+    import torch
+    hi = np.arange(65536, dtype=np.uint32) << 16
+    u = np.concatenate([hi | lo for lo in (0, 1, 0x7fff, 0x8000, 0x8001, 0xffff)]).astype(np.uint32)
+    n = u.size
+    z = torch.zeros(3, n, device=dev)
+    alb, nrm = z.clone(), z.clone()
+    alb[0] = torch.from_numpy(u.view(np.float32)).to(dev)
+    nrm[2] = torch.from_numpy(u[::-1].copy().view(np.float32)).to(dev)
+    out = torch.empty(n, 16, dtype=torch.int16, device=dev)
+    d = pkg.Denoiser(64, seed=1)
+    d.pack(n, z, alb, nrm, torch.zeros(n, device=dev), out)
+    torch.cuda.synchronize()
+    d.destroy()
+    got = out.cpu().numpy().view(np.uint16)
+    nan = (u & 0x7fffffff) > 0x7f800000
+    ref = np.where(nan, (u >> 16) | 0x40, (u.astype(np.uint64) + 0x7fff + ((u >> 16) & 1)) >> 16).astype(np.uint16)
+    assert np.array_equal(got[:, 3], ref)
+    assert np.array_equal(got[:, 8], ref[::-1])
+    assert not got[:, [0, 1, 2, 4, 5, 6, 7] + list(range(9, 16))].any()

@@ -43,11 +43,16 @@ namespace dn {
 
 constexpr int kBlock = 256;
 
-__device__ __forceinline__ uint16_t f2bf(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40u);   // NaN stays NaN
-    u += 0x7fffu + ((u >> 16) & 1u);                                              // round to nearest even
-    return (uint16_t)(u >> 16);
+// To BF16, round to nearest even, NaN stays NaN: one v_cvt_pk_bf16_f32 for two
+// values. (With integer operations, six per value, the conversions were a
+// third of the vector instructions of the full-resolution convolutions, which
+// are bound by those and not by the matrix cores.)
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
+__device__ __forceinline__ uint32_t f2bf2(float lo, float hi) {
+    const f32x2 v = {lo, hi};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
 }
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
@@ -59,14 +64,11 @@ __device__ __forceinline__ uint16_t log_rgb_bf(float v) { return f2bf(log1pf(fma
 // v = rgb[3], albedo[3], normal[3], depth: log(1 + rgb), albedo, normal,
 // log(1 + depth) / 4, zeros.
 __device__ __forceinline__ void pack_pixel(const float (&v)[10], uint4& o0, uint4& o1) {
-    uint32_t h[10];
+    float l[4];
 #pragma unroll
-    for (int c = 0; c < 3; c++) h[c] = log_rgb_bf(v[c]);
-#pragma unroll
-    for (int c = 3; c < 9; c++) h[c] = f2bf(v[c]);
-    h[9] = f2bf(0.25f * log1pf(fmaxf(v[9], 0.0f)));
-    o0 = make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16));
-    o1 = make_uint4(h[8] | (h[9] << 16), 0, 0, 0);
+    for (int c = 0; c < 4; c++) l[c] = log1pf(fmaxf(v[c < 3 ? c : 9], 0.0f));
+    o0 = make_uint4(f2bf2(l[0], l[1]), f2bf2(l[2], v[3]), f2bf2(v[4], v[5]), f2bf2(v[6], v[7]));
+    o1 = make_uint4(f2bf2(v[8], 0.25f * l[3]), 0, 0, 0);
 }
 __device__ __forceinline__ void load_pixel(const float* rgb, const float* alb, const float* nrm, const float* dep,
                                            size_t P, size_t p, float (&v)[10]) {
@@ -395,13 +397,21 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(OCC))) v
         // are even) and lane pair (l, l ^ 1: pixels 2m, 2m + 1) is written too:
         // rounding to BF16 is monotonic, so this equals pooling the BF16 output.
         const int x = x0 + wx * 16 + row;
-        float pool[2][4];
+        float pool[2][4], bias[2][4];
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int col = n0 + j * 16 + 4 * kg;
+                bias[j][i] = a.bias && col < a.n ? a.bias[col + i] : 0.0f;
+            }
         // HD: the head as one MFMA per output row. K slots 8k .. 8k + 7 of lane
         // group k hold channels 4k .. 4k + 3 and 16 + 4k .. 16 + 4k + 3, which is
         // what a lane of D already holds (tiles j = 0, 1); the A operand row 4c
         // holds head output c's weights for the same channels (other rows
         // zero), so output c lands in item 0 of lane group c.
         bf16x8 hwa;
+        float noisy[R], hbias;
         if constexpr (HD) {
             uint2 w0 = make_uint2(0, 0), w1 = make_uint2(0, 0);
             if ((row & 3) == 0 && row < 12) {
@@ -410,6 +420,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(OCC))) v
                 w1 = *(const uint2*)(a.hw + c * 32 + 16 + 4 * kg);
             }
             hwa = __builtin_bit_cast(bf16x8, make_uint4(w0.x, w0.y, w1.x, w1.y));
+            hbias = kg < 3 ? a.hbias[kg] : 0.0f;
+            if (a.rgbOut && kg < 3 && x < a.W) {
+                // every row's noisy radiance in flight at once
+                const float* in = a.rgbIn + ((size_t)(kg * a.B + bb) * a.H + y0) * a.W + x;
+#pragma unroll
+                for (int r = 0; r < R; r++) noisy[r] = y0 + r < a.H ? in[(size_t)r * a.W] : 0.0f;
+            }
         }
 #pragma unroll
         for (int r = 0; r < R; r++) {
@@ -421,13 +438,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(OCC))) v
                 const int col = n0 + j * 16 + 4 * kg;
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    v[j][i] = acc[r][j][i] + (a.bias && col < a.n ? a.bias[col + i] : 0.0f);
+                    v[j][i] = acc[r][j][i] + bias[j][i];
                     if (a.relu) v[j][i] = fmaxf(v[j][i], 0.0f);
                 }
                 const bool ok = y < a.H && x < a.W && col < a.n;
                 if (ok && a.y) {
-                    uint2 o = make_uint2(f2bf(v[j][0]) | ((uint32_t)f2bf(v[j][1]) << 16),
-                                         f2bf(v[j][2]) | ((uint32_t)f2bf(v[j][3]) << 16));
+                    uint2 o = make_uint2(f2bf2(v[j][0], v[j][1]),
+                                         f2bf2(v[j][2], v[j][3]));
                     if constexpr (MASK) {
                         const uint2 m = *(const uint2*)(a.ym + p * a.n + col);
                         if (!(bf2f((uint16_t)m.x) > 0.0f)) o.x &= 0xffff0000u;
@@ -450,23 +467,23 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(OCC))) v
                         }
                         if ((r & 1) && ok && !(row & 1)) {
                             const size_t q = (size_t)(bb * (a.H >> 1) + (y >> 1)) * (a.W >> 1) + (x >> 1);
-                            *(uint2*)(a.yp + q * a.ldyp + col) = make_uint2(f2bf(m[0]) | ((uint32_t)f2bf(m[1]) << 16),
-                                                                            f2bf(m[2]) | ((uint32_t)f2bf(m[3]) << 16));
+                            *(uint2*)(a.yp + q * a.ldyp + col) = make_uint2(f2bf2(m[0], m[1]),
+                                                                            f2bf2(m[2], m[3]));
                         }
                     }
                 }
             }
             if constexpr (HD) {
                 const bf16x8 act = __builtin_bit_cast(
-                    bf16x8, make_uint4(f2bf(v[0][0]) | ((uint32_t)f2bf(v[0][1]) << 16), f2bf(v[0][2]) | ((uint32_t)f2bf(v[0][3]) << 16),
-                                       f2bf(v[1][0]) | ((uint32_t)f2bf(v[1][1]) << 16), f2bf(v[1][2]) | ((uint32_t)f2bf(v[1][3]) << 16)));
+                    bf16x8, make_uint4(f2bf2(v[0][0], v[0][1]), f2bf2(v[0][2], v[0][3]),
+                                       f2bf2(v[1][0], v[1][1]), f2bf2(v[1][2], v[1][3])));
                 const f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hwa, act, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
                 if (kg < 3 && y < a.H && x < a.W) {
-                    const float hv = d[0] + a.hbias[kg];
+                    const float hv = d[0] + hbias;
                     if (a.head) a.head[p * 3 + kg] = hv;
                     if (a.rgbOut) {
                         const size_t pc = (size_t)kg * a.B * a.H * a.W + p;
-                        a.rgbOut[pc] = fmaxf(expm1f(hv + bf2f(log_rgb_bf(a.rgbIn[pc]))), 0.0f);
+                        a.rgbOut[pc] = fmaxf(expm1f(hv + bf2f(log_rgb_bf(noisy[r]))), 0.0f);
                     }
                 }
             }
@@ -617,8 +634,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
                 float v[4];
 #pragma unroll
                 for (int i = 0; i < 4; i++) v[i] = fmaxf(acc0[r][j][i] + bias0[j][i], 0.0f);
-                const uint2 w = in ? make_uint2(f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16),
-                                                f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16))
+                const uint2 w = in ? make_uint2(f2bf2(v[0], v[1]),
+                                                f2bf2(v[2], v[3]))
                                    : make_uint2(0, 0);
                 const int q = 2 * j + (kg >> 1);
                 ((uint2*)h1)[(hp * 4 + (q ^ (hp & 2))) * 2 + (kg & 1)] = w;
@@ -677,8 +694,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
 #pragma unroll
             for (int i = 0; i < 4; i++) v[i] = fmaxf(acc[r][j][i] + bias1[j][i], 0.0f);
             if (ok)
-                *(uint2*)(a.y + p * a.ldy + col) = make_uint2(f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16),
-                                                              f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16));
+                *(uint2*)(a.y + p * a.ldy + col) = make_uint2(f2bf2(v[0], v[1]),
+                                                              f2bf2(v[2], v[3]));
             float m[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
@@ -688,8 +705,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
             }
             if ((r & 1) && ok && !(row & 1)) {
                 const size_t q = (size_t)(bb * (a.H >> 1) + (y >> 1)) * (a.W >> 1) + (x >> 1);
-                *(uint2*)(a.yp + q * a.ldyp + col) = make_uint2(f2bf(m[0]) | ((uint32_t)f2bf(m[1]) << 16),
-                                                                f2bf(m[2]) | ((uint32_t)f2bf(m[3]) << 16));
+                *(uint2*)(a.yp + q * a.ldyp + col) = make_uint2(f2bf2(m[0], m[1]),
+                                                                f2bf2(m[2], m[3]));
             }
         }
     }

@@ -250,3 +250,22 @@ def test_bf16_rounding(pkg, dev):
     assert np.array_equal(got[:, 3], ref)
     assert np.array_equal(got[:, 8], ref[::-1])
     assert not got[:, [0, 1, 2, 4, 5, 6, 7] + list(range(9, 16))].any()
+
+
+def test_very_wide_image(pkg, dev):
+    """An image wider than the convolutions' 32-bit offsets allow (2^18 pixels)
+    takes their 64-bit form: its left part equals that of the same image cut
+    off beyond the network's reach (a pixel's value does not depend on where
+    the tiles lie)."""
+    import torch
+    H, W, cut, same = 8, (1 << 18) + 8, 2048, 1024
+    g = torch.Generator(device=dev).manual_seed(4)
+    planes = [torch.rand(c, H, W, device=dev, generator=g) for c in (3, 3, 3, 1)]
+    d = pkg.Denoiser(H * W, seed=5)
+    wide, narrow = torch.empty(3, H, W, device=dev), torch.empty(3, H, cut, device=dev)
+    d.denoise(W, H, *planes, wide)
+    d.denoise(cut, H, *[p[:, :, :cut].contiguous() for p in planes], narrow)
+    torch.cuda.synchronize()
+    d.destroy()
+    assert torch.equal(wide[:, :, :same], narrow[:, :, :same])
+    assert wide.std().item() > 0.1

@@ -71,7 +71,7 @@ struct PtArgs {
     rtd::Cam cam;
     int W, H, N, maxDepth, rrStart, tailPaths;
     float sun[3], sunRad[3], skyZ[3], skyH[3], clampMax;
-    // tail kernel: the scene and a stack of tailDepth entries per path in flight
+    // tail kernel: the scene and a stack of tailDepth entries per quad in flight
     const uint4* tlasNodes;
     const float4* tlasTris;
     int2* tailStack;
@@ -83,7 +83,7 @@ struct PtResources {
     int cap = 0;
     void* block = nullptr;            // one allocation for every per-ray buffer
     int* small = nullptr;             // counters, totals, frame
-    int2* tailStack = nullptr;        // tail kernel: [depth][paths] stack entries
+    int2* tailStack = nullptr;        // tail kernel: [depth][quads] stack entries
     size_t tailBytes = 0;
     hipStream_t own = nullptr;        // stream for graph capture when the scene has none
     hipStream_t side = nullptr;       // shadow traces, concurrent with the next bounce's extension trace
@@ -366,16 +366,21 @@ __global__ __launch_bounds__(kPtBlock) void k_pt_octsort(PtArgs a, int b) {
     }
 }
 
-// Tail: at the first bounce b0 with at most tailPaths live paths, four lanes
-// per path run all of its remaining bounces (closest hit, shading, shadow ray,
-// next ray). Each pixel's contributions are added in the wavefront order, so
-// the image is the same; the launch's duration is one longest path instead of
-// one slowest ray per bounce and stage. Shading is the same work in the four
-// lanes, the first of which writes. The chain of one path's traversal steps is
-// the launch's time; four lanes shorten each step: 830 to 350 us for the tail
-// of a 1080p sample against one thread per path. Stack entries from kTailLds on are in
-// a.tailStack, one column per path in flight.
+// Tail: at the first bounce b0 with at most tailPaths live paths, eight lanes
+// per path run all of its remaining bounces: the first four trace the next
+// extension ray while the other four trace the shadow ray of the event before
+// it (both need only that event's shading). Each pixel's contributions are
+// added in the wavefront order, so the image is the same; the launch's
+// duration is one longest path instead of one slowest ray per bounce and
+// stage. Shading is the same work in the eight lanes, the first of which
+// writes. Stack entries from kTailLds on are in a.tailStack, one column per
+// quad.
+//
+// The chain of one path's traversal steps is the launch's time: for the tail
+// of a 1080p sample one thread per path took 830 us, four lanes per path 350
+// to 440, eight 300 us.
 constexpr int kTailLds = 24;
+constexpr int kTailPaths = 8;            // per workgroup
 
 __global__ __launch_bounds__(64) void k_pt_tail(PtArgs a, int b0) {
     const int n0 = a.cnt[b0];
@@ -385,10 +390,10 @@ __global__ __launch_bounds__(64) void k_pt_tail(PtArgs a, int b0) {
     __shared__ float s_w[6 * 16];                // the rays being traced: origins, directions
     const bool sample0 = a.frame[0] == 0;
     const PtQueue& q = a.q[b0 & 1];
-    const int stride = gridDim.x * 16;
+    const int stride = gridDim.x * kTailPaths;
     const int lane = threadIdx.x, c = lane & 3, sh = lane & 60, col = lane >> 2;
-    const int g = blockIdx.x * 16 + col;
-    int2* stk = a.tailStack + g;
+    const bool shadowLane = lane & 4, writer = (lane & 7) == 0;
+    int2* stk = a.tailStack + (blockIdx.x * 16 + col);
     auto push = [&](rtq::Ray4&, int at, int rf, float t) {
         if (at < kTailLds) {
             s_ref[at * 16 + col] = rf;
@@ -408,42 +413,43 @@ __global__ __launch_bounds__(64) void k_pt_tail(PtArgs a, int b0) {
             rf = e.x; t = __int_as_float(e.y);
         }
     };
-    auto start = [&](Quad2& z, const float o[3], float dx, float dy, float dz) {
-        s_w[col] = o[0]; s_w[16 + col] = o[1]; s_w[32 + col] = o[2];
-        s_w[48 + col] = dx; s_w[64 + col] = dy; s_w[80 + col] = dz;
-        z.tmin = 0.0f; z.tmax = RT_MISS_T;
-        z.best = z.t = RT_MISS_T; z.u = z.v = 0.0f; z.id = z.hinst = -1;
-        z.ref = 0; z.sp = 0; z.col = 0; z.tn = -INFINITY; z.found = false;
-        quad_world(z, c, s_w + col, 16, a.tlasNodes);
-    };
-    for (int i = g; i < n0; i += stride) {
+    for (int i = blockIdx.x * kTailPaths + (lane >> 3); i < n0; i += stride) {
         const int pix = q.pix[i];
         float o[3] = {q.r[0][i], q.r[1][i], q.r[2][i]}, d[3] = {q.r[3][i], q.r[4][i], q.r[5][i]};
         float thr[3] = {q.thr[0][i], q.thr[1][i], q.thr[2][i]};
         rtd::Pcg32 rng;
         rng.state = q.rng[i];
         rng.inc = ((uint64_t)pix << 1u) | 1u;
-        for (int b = b0; b < a.maxDepth; b++) {
-            if (b > b0 && c == 0) atomicAdd(&a.cnt[b], 1);
+        ShadeOut so;
+        so.shadow = false;
+        bool path = true;                        // an extension ray is to be traced
+        for (int b = b0; path || so.shadow; b++) {
+            if (path && b > b0 && writer) atomicAdd(&a.cnt[b], 1);
             Quad2 z;
-            start(z, o, d[0], d[1], d[2]);
-            quad_trace2<false>(z, true, c, sh, s_w + col, 16, a.tlasNodes, a.tlasTris, a.inst, a.blas, a.tailDepth,
-                               a.status, push, pop);
+            // both rays start at the last event's point
+            s_w[col] = o[0]; s_w[16 + col] = o[1]; s_w[32 + col] = o[2];
+            s_w[48 + col] = shadowLane ? a.sun[0] : d[0];
+            s_w[64 + col] = shadowLane ? a.sun[1] : d[1];
+            s_w[80 + col] = shadowLane ? a.sun[2] : d[2];
+            z.tmin = 0.0f; z.tmax = RT_MISS_T;
+            z.best = z.t = RT_MISS_T; z.u = z.v = 0.0f; z.id = z.hinst = -1;
+            z.ref = 0; z.sp = 0; z.col = 0; z.tn = -INFINITY; z.found = false;
+            quad_world(z, c, s_w + col, 16, a.tlasNodes);
+            quad_trace2<false>(z, shadowLane ? so.shadow : path, c, sh, s_w + col, 16, a.tlasNodes, a.tlasTris, a.inst,
+                               a.blas, a.tailDepth, a.status, push, pop, shadowLane);
             quad_reduce2(z);
-            ShadeOut so;
-            shade_event(a, b, b == 0 && sample0, c == 0, pix, o, d, thr, rng, z.id >= 0 ? z.t : RT_MISS_T, z.hinst,
-                        z.id, so);
-            if (so.shadow) {
-                if (c == 0) atomicAdd(&a.cnt[kPtMaxDepth + b], 1);
-                Quad2 y;
-                start(y, so.so, a.sun[0], a.sun[1], a.sun[2]);
-                quad_trace2<true>(y, true, c, sh, s_w + col, 16, a.tlasNodes, a.tlasTris, a.inst, a.blas, a.tailDepth,
-                                  a.status, push, pop);
-                if (!y.found && c == 0) {
-                    a.rgb[0][pix] += so.c[0]; a.rgb[1][pix] += so.c[1]; a.rgb[2][pix] += so.c[2];
-                }
+            // the extension ray's hit and whether the shadow ray is blocked, to all eight
+            const int ext = lane & ~4, shd = lane | 4;
+            const int id = __shfl(z.id, ext), inst = __shfl(z.hinst, ext), blocked = __shfl(z.id, shd);
+            const float t = __shfl(z.t, ext);
+            if (so.shadow && blocked < 0 && writer) {
+                a.rgb[0][pix] += so.c[0]; a.rgb[1][pix] += so.c[1]; a.rgb[2][pix] += so.c[2];
             }
-            if (!so.next) break;
+            so.shadow = false;
+            if (!path) break;
+            shade_event(a, b, b == 0 && sample0, writer, pix, o, d, thr, rng, id >= 0 ? t : RT_MISS_T, inst, id, so);
+            path = so.next;
+            if (so.shadow && writer) atomicAdd(&a.cnt[kPtMaxDepth + b], 1);
             for (int k = 0; k < 3; k++) { o[k] = so.so[k]; d[k] = so.nd[k]; }
         }
     }
@@ -665,7 +671,7 @@ int path_trace(CudaSceneHandle* sc, const CudaCamera& cam, const CudaPathParams&
     a.tlasNodes = (const uint4*)sc->tlas->d_nodes4;
     a.tlasTris = (const float4*)sc->tlas->d_tris;
     if (a.tailPaths > 0) {
-        a.tailStride = std::min(64 * 1024, (a.tailPaths + 63) / 64 * 64);
+        a.tailStride = std::min(128 * 1024, (a.tailPaths + kTailPaths - 1) / kTailPaths * 16);   // two quads per path
         a.tailDepth = trace2l_max_stack(sc);
         const size_t need = (size_t)a.tailStride * std::max(a.tailDepth - kTailLds, 1) * sizeof(int2);
         if (need > R.tailBytes) {

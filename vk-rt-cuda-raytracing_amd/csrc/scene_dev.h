@@ -166,13 +166,15 @@ __device__ __forceinline__ void quad_enter(Quad2& q, int c, const float* w, int 
 // leaf code, a return marker, or -1: what the stack holds next) until they are
 // done; the current ray is set up. Culling and tie rule of k_trace2l; the
 // stack as in rtq::traverse. Returns the steps taken; q.found: an any-hit
-// ray's result. The loop has one way through and ends for all quads at once:
+// ray's result. A closest-hit ray with `first` also ends at its first hit (one
+// below q.tmax). The loop has one way through and ends for all quads at once:
 // with quads leaving it, or continuing it, from within, each of the some 30
 // registers of state had a second one and was copied in every step.
 template <bool ANY, class Push, class Pop>
 __device__ __forceinline__ int quad_trace2(Quad2& q, bool has, int c, int sh, const float* w, int stride,
                                            const void* tlasNodes, const float4* tlasTris, const InstanceDev* insts,
-                                           const BlasDev* blas, int maxStack, int* status, Push&& push, Pop&& pop) {
+                                           const BlasDev* blas, int maxStack, int* status, Push&& push, Pop&& pop,
+                                           bool first = false) {
     int steps = 0;
     while (__any(has)) {
         steps++;
@@ -210,7 +212,7 @@ __device__ __forceinline__ int quad_trace2(Quad2& q, bool has, int c, int sh, co
                 }
             }
             if (!next) {
-                has = q.sp > 0 && !(ANY && q.found);
+                has = q.sp > 0 && !(ANY ? q.found : first && q.best < q.tmax);
                 if (has) {
                     q.sp--;
                     pop(q, q.sp, q.ref, q.tn);

@@ -15,10 +15,11 @@
 // from the arrays' (uniform) bases, which keeps a lane's addresses in single
 // registers: its callers use quads only where both arrays fit (fits()).
 //
-// Every value is computed by the expressions of rt_device.h, and a ray's hit
-// is the lexicographic minimum of (t, ID) over the triangles whose boxes pass,
-// in any visiting order, so results equal those of the one-lane traversal bit
-// for bit.
+// Every value is computed by the expressions of rt_device.h, children are
+// visited in the same order, and a ray's hit is the lexicographic minimum of
+// (t, ID) over the triangles whose boxes pass, so results equal those of the
+// one-lane traversal bit for bit. (The order matters for triangles at equal t
+// whose boxes' entry rounds above it: the first one visited hides the others.)
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -153,12 +154,21 @@ __device__ __forceinline__ bool visit(Ray4& q, int c, int sh, const Slot& s, int
     const bool hit = (tN <= tF) && (tN <= limit) && s.child != -1;
     const uint32_t hm = (uint32_t)(__ballot(hit) >> sh) & 15u;
     if (!hm) return false;
-    // rank of this lane's child among the quad's hits, nearest first: keys of
-    // the entry distance (from 0 up) with the lane in the two low bits, so
-    // that no two are equal
-    const int key = hit ? (__float_as_int(fmaxf(tN, 0.0f)) & ~3) | c : 0x7ffffffc | c;
-    const int k1 = quad_perm<kRot1>(key), k2 = quad_perm<kRot2>(key), k3 = quad_perm<kRot3>(key);
-    const int rank = -(((k1 - key) >> 31) + ((k2 - key) >> 31) + ((k3 - key) >> 31));
+    // rank of this lane's child among the quad's hits, nearest first, equal
+    // ones in slot order: lane (c + k) & 3 comes before lane c when it wraps.
+    // (Any hit: in any order, so the lane is in the key's low bits.)
+    int rank;
+    if constexpr (ANY) {
+        const int key = hit ? (__float_as_int(fmaxf(tN, 0.0f)) & ~3) | c : 0x7ffffffc | c;
+        const int k1 = quad_perm<kRot1>(key), k2 = quad_perm<kRot2>(key), k3 = quad_perm<kRot3>(key);
+        rank = -(((k1 - key) >> 31) + ((k2 - key) >> 31) + ((k3 - key) >> 31));
+    } else {
+        const int key = hit ? __float_as_int(fmaxf(tN, 0.0f)) : 0x7fffffff;
+        const int k1 = quad_perm<kRot1>(key), k2 = quad_perm<kRot2>(key), k3 = quad_perm<kRot3>(key);
+        int cc = c;
+        asm volatile("" : "+v"(cc));             // its three terms are not held through the traversal
+        rank = -(((k1 - key - ((cc + 1) >> 2)) >> 31) + ((k2 - key - (cc >> 1)) >> 31) + ((k3 - key - min(cc, 1)) >> 31));
+    }
     const int n = __popc(hm);
     const int at = q.sp + n - 1 - rank;
     if (hit && rank > 0 && at < maxStack) push(q, at, s.child, tN);

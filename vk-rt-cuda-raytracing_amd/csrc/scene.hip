@@ -315,8 +315,14 @@ __device__ __forceinline__ void trace2l_wave(const Trace2LArgs& a, Ray& r, bool 
             };
             if (test(p0, p1, p2) || (two && test(q0, q1, q2))) { found = true; has = false; }
         } else if (ref >= 0) {
-            if constexpr (ANY && ORD) visit2w<false>(nodes, r, flat, r.tmax, ref, tn, push);
-            else visit2w<ANY>(nodes, r, flat, ANY ? r.tmax : best, ref, tn, push);
+            const uint4* np = nodes + 4 * (size_t)ref;
+            const uint4 qc = rtd::ldg_u4(np + 3), nx = rtd::ldg_u4(np), ny = rtd::ldg_u4(np + 1), nz = rtd::ldg_u4(np + 2);
+            constexpr bool SLOTS = ANY && !ORD;     // children in slot order
+            const float limit = ANY ? r.tmax : best;
+            const bool down = __any(flat)
+                ? rtd::visit_free<SLOTS, true, LDSD, BLOCK>(r, nx, ny, nz, qc, limit, ref, tn, s_ref, s_tn, tid, sp, push)
+                : rtd::visit_free<SLOTS, false, LDSD, BLOCK>(r, nx, ny, nz, qc, limit, ref, tn, s_ref, s_tn, tid, sp, push);
+            if (!down) ref = -1;
         } else {
             // TLAS leaf: enter its instance
             const int enc = -(ref + 2);

@@ -503,16 +503,12 @@ __device__ __forceinline__ void trace_wave(const TraceArgs& a, const Ray& r, boo
             ltc -= two ? 2 : 1;
             cont = ltc > 0;
         } else if (ref >= 0 && (MODE == kModeAny || tn <= best)) {
-            int nxt = ref;
-            float nt = 0.f;
-            if constexpr (MODE == kModeAny) {
-                if (flat) visit_any<true>(nodes, r, nxt, push);
-                else visit_any<false>(nodes, r, nxt, push);
-            } else {
-                if (flat) visit_closest<true>(nodes, r, best, nxt, nt, push);
-                else visit_closest<false>(nodes, r, best, nxt, nt, push);
-            }
-            if (nxt != -1) { ref = nxt; tn = nt; cont = true; }
+            const uint4* np = nodes + 4 * (size_t)ref;
+            const uint4 nx = np[0], ny = np[1], nz = np[2], qc = np[3];
+            const float limit = MODE == kModeAny ? r.tmax : best;
+            constexpr bool ANY = MODE == kModeAny;
+            if (flat) cont = rtd::visit_free<ANY, true, LDSD, BLOCK>(r, nx, ny, nz, qc, limit, ref, tn, s_ref, s_tn, tid, sp, push);
+            else cont = rtd::visit_free<ANY, false, LDSD, BLOCK>(r, nx, ny, nz, qc, limit, ref, tn, s_ref, s_tn, tid, sp, push);
         }
         if (!cont) {
             if (sp == 0) {
@@ -809,16 +805,12 @@ __global__ __launch_bounds__(BLOCK) void k_trace_refill(TraceArgs a) {
             ltc -= two ? 2 : 1;
             if (!fin && ltc > 0) cont = true;
         } else if (ref >= 0 && (MODE == kModeAny || tn <= best)) {
-            int nxt = ref;
-            float nt = 0.f;
-            if constexpr (MODE == kModeAny) {
-                if (waveFlat) visit_any<true>(nodes, r, nxt, push);
-                else visit_any<false>(nodes, r, nxt, push);
-            } else {
-                if (waveFlat) visit_closest<true>(nodes, r, best, nxt, nt, push);
-                else visit_closest<false>(nodes, r, best, nxt, nt, push);
-            }
-            if (nxt != -1) { ref = nxt; tn = nt; cont = true; }
+            const uint4* np = nodes + 4 * (size_t)ref;
+            const uint4 nx = np[0], ny = np[1], nz = np[2], qc = np[3];
+            const float limit = MODE == kModeAny ? r.tmax : best;
+            constexpr bool ANY = MODE == kModeAny;
+            if (waveFlat) cont = rtd::visit_free<ANY, true, LDSD, BLOCK>(r, nx, ny, nz, qc, limit, ref, tn, s_ref, s_tn, tid, sp, push);
+            else cont = rtd::visit_free<ANY, false, LDSD, BLOCK>(r, nx, ny, nz, qc, limit, ref, tn, s_ref, s_tn, tid, sp, push);
         }
         if (!cont && !fin) {
             if (sp == 0) {
@@ -956,9 +948,9 @@ __global__ __launch_bounds__(64) void k_trace_quad(TraceArgs a) {
 // of steps of its slowest tiles, mostly run by waves with few rays left. That
 // takes 79 VGPRs, six waves per SIMD instead of seven (at seven it spilled up
 // to 7 to scratch): on a 0.5 M triangle terrain the cost-ordered pinhole launch
-// of 1024 x 1024 went from 279 to 240 us and of 1920 x 1080, which the order
-// keeps busy to its end, from 366 to 373 us (a 65,536 triangle soup: 394 to
-// 353, 468 to 406 us).
+// of 1024 x 1024 went from 279 to 236 us and of 1920 x 1080, which the order
+// keeps busy to its end, from 366 to 362 us (a 65,536 triangle soup: 394 to
+// 342, 468 to 391 us).
 template <int MODE, bool MT, bool PIN, bool COUNT, int LDSD, int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void k_trace_batch(TraceArgs a) {
     __shared__ int s_ref[LDSD * BLOCK];

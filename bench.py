@@ -463,7 +463,7 @@ def bench_path_tracer(pkg, scenes, dev, args):
     nrm = torch.empty(3 * n, device=dev)
     dep = torch.empty(n, device=dev)
     if not args.no_tune:
-        # queue size: below how many live paths one thread per path finishes the bounces
+        # queue size: below how many live paths the tail kernel finishes the bounces
         best_tail, table = gs.autotune_path_tracer(c, pkg.path_params(W, H, spp=1, seed=1), rgb, alb, nrm, dep, reps=4)
         tuning["tail_paths"] = {"chosen": best_tail, "sweep_ms": {str(t): round(ms, 4) for t, ms in table}}
         log(f"pt autotune tail paths: {best_tail}  " + " ".join(f"{t}:{ms:.3f}" for t, ms in table))

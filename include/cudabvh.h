@@ -120,8 +120,9 @@ int cudaBVH_getStacklessBVH2(CudaBVH_t bvh, uint32_t** outData);
 int cudaBVH_getPackedTris(CudaBVH_t bvh, float** outData);
 
 /* layer/cuda_bvh_backend.h:116. Waits for all library work and releases
- * library-global device resources. The device itself is not reset because
- * the library shares it with its host process. */
+ * library-global device resources (among them the freed blocks kept for
+ * reuse). The device itself is not reset because the library shares it with
+ * its host process. */
 void cudaBVH_resetDevice(void);
 
 /* layer/cuda_bvh_backend.h:123. One degenerate triangle per AABB (backend
@@ -491,7 +492,7 @@ typedef struct CudaBVHBatchHandle* CudaBVHBatch_t;
 
 /* Builds the BVHs of numScenes scenes (triangles concatenated; scene k is
  * [triOffsets[k], triOffsets[k+1]), each with more than 4 triangles) in one
- * level-synchronous GPU pass: one forest, each tree identical to the scene's
+ * GPU pass: one forest, each tree identical to the scene's
  * own cudaBVH_build tree, leaf triangles carrying their index within the
  * scene. Host inputs. */
 CudaBVHBatch_t cudaBVH_buildBatch(const CudaTri* tris, const int* triOffsets, int numScenes);

@@ -24,8 +24,9 @@
 //     channels, K = pixels; tiles with their halo staged once for all taps and
 //     read with transposing LDS reads, split over pixel ranges into partials
 //     reduced in a fixed order (deterministic).
-//   * upsampling (training), pooling / upsampling backward, ReLU-mask, loss,
-//     Adam and weight layout kernels.
+//   * upsampling (training), pooling / upsampling backward, loss, Adam and
+//     weight layout kernels (ReLU backward is part of the kernels that write
+//     the gradients).
 #include <hip/hip_runtime.h>
 
 #include <cmath>

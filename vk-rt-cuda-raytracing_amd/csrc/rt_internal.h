@@ -52,7 +52,7 @@ struct GpuBVH {
     float bmin[3], bmax[3];                        // mesh bounds (mesh_bounds' values)
 };
 // Builds one BVH, or with sceneOff (numScenes+1 host offsets into d_tris) a
-// forest of numScenes independent BVHs in one level-synchronous pass: node
+// forest of numScenes independent BVHs in one pass: node
 // arrays shared, each tree contiguous in pre-order, leaf triangles carrying
 // their index within their scene; roots4 receives each tree's BVH4 root.
 int gpu_build(const float* d_tris, int n, int maxLeaf, hipStream_t s, GpuBVH& out, const int* sceneOff = nullptr,

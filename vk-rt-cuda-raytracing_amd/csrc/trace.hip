@@ -947,7 +947,7 @@ __global__ __launch_bounds__(64) void k_trace_quad(TraceArgs a) {
 // last kQuadRays rays to quads, four lanes each: a launch's end is the chain
 // of steps of its slowest tiles, mostly run by waves with few rays left. That
 // takes 79 VGPRs, six waves per SIMD instead of seven (at seven it spilled up
-// to 7 to scratch): on a 0.5 M triangle terrain the cost-ordered pinhole launch
+// to 7 to scratch): on a 3.4 M triangle terrain the cost-ordered pinhole launch
 // of 1024 x 1024 went from 279 to 236 us and of 1920 x 1080, which the order
 // keeps busy to its end, from 366 to 362 us (a 65,536 triangle soup: 394 to
 // 342, 468 to 391 us).
@@ -1682,7 +1682,7 @@ static int launch_tuned(const CudaBVHHandle* h, rt::TraceScratch& sc, TraceArgs&
 // quads, take fewer instructions per ray; the pinhole cost order, which only
 // those take, brings its line forward. A queue's capacity is an upper bound of
 // its rays (some 55 to 85 % of it in a frame), so its line lies higher.
-// Measured, quads from the root / hand-over (us; a 0.5 M triangle terrain,
+// Measured, quads from the root / hand-over (us; a 3.4 M triangle terrain,
 // then a 65,536 triangle soup; camera, secondary and shadow rays; launches
 // without either took 242 and 304 us for 0.26 M pinhole rays, 273 and 357 us
 // for 0.22 M closest hits):

@@ -624,7 +624,12 @@ __device__ __forceinline__ int finish_quads(const TraceArgs& a, bool open, int r
 // are idle, so a wave does not wait for the slowest ray of its batch and
 // the ray set-up of new rays is shared by many lanes. Same depth-first order
 // per ray as trace_ray; uncounted.
-constexpr int kRefillMin = 8;   // 8 measured ~1 % faster than 4, 16 or 24 on the 1080p diffuse rays
+// Idle lanes at which a wave takes new rays: a refill costs every lane its
+// instructions, waiting costs the idle ones theirs. 23 M rays of 64 scenes at
+// 5, 8, 12, 14, 16, 20, 24: 5.27, 4.95, 4.78, 4.74, 4.72, 4.73, 4.78 ms; the
+// 1080p frame (whose diffuse rays stay in step longer) 1.147, 1.137, 1.137,
+// 1.139, 1.145, 1.146, 1.150 ms.
+constexpr int kRefillMin = 14;
 
 template <int MODE, bool MT, bool PIN, int LDSD, int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_trace_refill(TraceArgs a) {

@@ -40,8 +40,7 @@ template <int CTRL>
 __device__ __forceinline__ int quad_perm(int v) { return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, false); }
 template <int CTRL>
 __device__ __forceinline__ float quad_perm(float v) { return __int_as_float(quad_perm<CTRL>(__float_as_int(v))); }
-constexpr int kXor1 = 0xb1, kXor2 = 0x4e;             // quad_perm [1,0,3,2], [2,3,0,1]
-constexpr int kRot1 = 0x39, kRot2 = 0x4e, kRot3 = 0x93;   // lane c reads lane (c + k) & 3
+constexpr int kXor1 = 0xb1, kXor2 = 0x4e, kMid = 0xd8;   // quad_perm [1,0,3,2], [2,3,0,1], [0,2,1,3]
 
 // A ray held by the four lanes of a quad, in the axis order (x, y, z here) of
 // its watertight test throughout: the slab test is the same in any order. t,
@@ -49,7 +48,6 @@ constexpr int kRot1 = 0x39, kRot2 = 0x4e, kRot3 = 0x93;   // lane c reads lane (
 // -1) in every lane; best: the quad's closest distance. tmax: any hit only.
 struct Ray4 {
     float ox, oy, oz, ix, iy, iz, Sx, Sy, Sz, tmin, tmax;
-    float far;                                        // infinite for a flat ray, else NaN (see visit)
     uint32_t kx, ky, kz;                              // the axes
     float t, u, v, best;
     int id;
@@ -69,7 +67,6 @@ __device__ __forceinline__ void set_ray(Ray4& q, const rtd::Ray& r) {
     q.Sx = r.Sx; q.Sy = r.Sy; q.Sz = r.Sz;
     q.tmin = r.tmin; q.tmax = r.tmax;
     q.kx = r.kx; q.ky = r.ky; q.kz = r.kz;
-    q.far = rtd::ray_flat(r) ? INFINITY : NAN;
 }
 
 // Watertight test of the triangle (3 x float4) at tb + o, components addressed
@@ -88,12 +85,15 @@ __device__ __forceinline__ bool isect(const Ray4& q, gptr tb, uint32_t o, float&
     float U = Cx * By - Cy * Bx;
     float V = Ax * Cy - Ay * Cx;
     float W = Bx * Ay - By * Ax;
-    if (U == 0.0f || V == 0.0f || W == 0.0f) {         // one after the other: fewer registers at once
-        U = (float)((double)Cx * (double)By - (double)Cy * (double)Bx);
+    if (U == 0.0f || V == 0.0f || W == 0.0f) {
+        // one after the other, and fused (a product of two floats is exact in
+        // 64 bits, so the bits are those of product and difference): fewer
+        // registers at once
+        U = (float)__builtin_fma(-(double)Cy, (double)Bx, (double)Cx * (double)By);
         __builtin_amdgcn_sched_barrier(0);
-        V = (float)((double)Ax * (double)Cy - (double)Ay * (double)Cx);
+        V = (float)__builtin_fma(-(double)Ay, (double)Cx, (double)Ax * (double)Cy);
         __builtin_amdgcn_sched_barrier(0);
-        W = (float)((double)Bx * (double)Ay - (double)By * (double)Ax);
+        W = (float)__builtin_fma(-(double)By, (double)Ax, (double)Bx * (double)Ay);
     }
     if ((U < 0.0f || V < 0.0f || W < 0.0f) && (U > 0.0f || V > 0.0f || W > 0.0f)) return false;
     const float det = U + V + W;
@@ -135,51 +135,60 @@ __device__ __forceinline__ Slot slot_of(const Ray4& q, gptr nb, int c) {
             gload<int>(nb + (48u + 4u * c))};
 }
 
+// One compare-exchange of the children's order: this lane keeps the smaller
+// distance of its own and lane P's (low -INFINITY) or the larger one
+// (INFINITY), and the child with it; equal ones stay.
+template <int P>
+__device__ __forceinline__ void exchange(float low, float& d, int& child) {
+    const float m = __builtin_amdgcn_fmed3f(d, quad_perm<P>(d), low);
+    const int other = quad_perm<P>(child);
+    child = m != d ? other : child;
+    d = m;
+}
+
 // Visits a node: this lane's child, then the quad's order of the hit ones. The
 // nearest becomes q.ref, the others are pushed. False when no child is hit.
+//
+// The order is that of the one-lane visits' network (compare-exchanges 01, 23,
+// 02, 13, 12 on the entry distances, misses at infinity), taken literally: it
+// is not stable, and the order of boxes at equal distances decides between
+// triangles at equal t (see above). Any hit may use any order.
 //
 // Of a flat ray (an infinite reciprocal) the distance to a plane through its
 // origin is 0 * inf = NaN: such an axis bounds nothing, and the NaN-ignoring
 // max / min leave it out, which is what rt_device.h's FLAT variant computes
-// with its -inf / +inf; q.far and tmin stand in where all three are NaN. (An
-// origin and direction of NaN themselves still hit nothing: q.far is NaN.)
+// with its -inf / +inf. Where all three are NaN no box is hit: such a ray has
+// no finite reciprocal, so its triangle tests give no finite t either.
 template <bool ANY, class Push>
 __device__ __forceinline__ bool visit(Ray4& q, int c, int sh, const Slot& s, int maxStack, int* status, Push&& push) {
     const float t1x = rtd::h_sub<false>(s.hx, q.ox) * q.ix, t2x = rtd::h_sub<false>(s.gx, q.ox) * q.ix;
     const float t1y = rtd::h_sub<false>(s.hy, q.oy) * q.iy, t2y = rtd::h_sub<false>(s.gy, q.oy) * q.iy;
     const float t1z = rtd::h_sub<false>(s.hz, q.oz) * q.iz, t2z = rtd::h_sub<false>(s.gz, q.oz) * q.iz;
-    const float tN = fmaxf(fmaxf(fmaxf(t1x, t1y), t1z), q.tmin);
-    const float tF = fminf(fminf(fminf(t2x, t2y), t2z), q.far) * RT_ROBUST_TFAR;
+    const float tN = fmaxf(fmaxf(t1x, t1y), t1z);
+    const float tF = fminf(fminf(t2x, t2y), t2z) * RT_ROBUST_TFAR;
     const float limit = ANY ? q.tmax : q.best;
-    const bool hit = (tN <= tF) && (tN <= limit) && s.child != -1;
+    const bool hit = (tN <= tF) && (tF >= q.tmin) && (tN <= limit) && s.child != -1;
     const uint32_t hm = (uint32_t)(__ballot(hit) >> sh) & 15u;
     if (!hm) return false;
-    // rank of this lane's child among the quad's hits, nearest first, equal
-    // ones in slot order: lane (c + k) & 3 comes before lane c when it wraps.
-    // (Any hit: in any order, so the lane is in the key's low bits.)
-    int rank;
-    if constexpr (ANY) {
-        const int key = hit ? (__float_as_int(fmaxf(tN, 0.0f)) & ~3) | c : 0x7ffffffc | c;
-        const int k1 = quad_perm<kRot1>(key), k2 = quad_perm<kRot2>(key), k3 = quad_perm<kRot3>(key);
-        rank = -(((k1 - key) >> 31) + ((k2 - key) >> 31) + ((k3 - key) >> 31));
-    } else {
-        const int key = hit ? __float_as_int(fmaxf(tN, 0.0f)) : 0x7fffffff;
-        const int k1 = quad_perm<kRot1>(key), k2 = quad_perm<kRot2>(key), k3 = quad_perm<kRot3>(key);
-        int cc = c;
-        asm volatile("" : "+v"(cc));             // its three terms are not held through the traversal
-        rank = -(((k1 - key - ((cc + 1) >> 2)) >> 31) + ((k2 - key - (cc >> 1)) >> 31) + ((k3 - key - min(cc, 1)) >> 31));
-    }
+    // Missed children sort last. (Opaque copies of c and the infinity: held
+    // through the traversal, what is made of them would cost registers.)
+    int lo = c, hi = c >> 1, inf = 0x7f800000;
+    asm volatile("" : "+v"(lo), "+v"(hi), "+v"(inf));
+    float d = __int_as_float(hit ? min(__float_as_int(tN), 0x7f7fffff) : inf);
+    int child = s.child;
+    const float low1 = __int_as_float((lo << 31) ^ (int)0xff800000), low2 = __int_as_float((hi << 31) ^ (int)0xff800000);
+    exchange<kXor1>(low1, d, child);
+    exchange<kXor2>(low2, d, child);
+    exchange<kMid>(low2, d, child);
+    // lane c holds the c-th of them
     const int n = __popc(hm);
-    const int at = q.sp + n - 1 - rank;
-    if (hit && rank > 0 && at < maxStack) push(q, at, s.child, tN);
+    const int at = q.sp + n - 1 - c;
+    if (c > 0 && c < n && at < maxStack) push(q, at, child, d);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the quad's lanes read each other's entries
     q.sp += n - 1;
     if (q.sp > maxStack) { q.sp = maxStack; atomicOr(status, 1); }
-    const bool first = hit && rank == 0;
-    int rf = first ? s.child : 0, tb = first ? __float_as_int(tN) : 0;
-    rf |= quad_perm<kXor1>(rf); tb |= quad_perm<kXor1>(tb);
-    q.ref = rf | quad_perm<kXor2>(rf);
-    q.tn = __int_as_float(tb | quad_perm<kXor2>(tb));
+    q.ref = quad_perm<0x00>(child);
+    q.tn = quad_perm<0x00>(d);
     return true;
 }
 

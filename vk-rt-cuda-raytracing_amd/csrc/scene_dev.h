@@ -125,7 +125,6 @@ __device__ __forceinline__ void quad_world(Quad2& q, int c, const float* w, int 
     q.ox = w[0]; q.oy = w[stride]; q.oz = w[2 * stride];
     q.ix = quad_bcast<0>(inv); q.iy = quad_bcast<1>(inv); q.iz = quad_bcast<2>(inv);
     q.kx = 0; q.ky = 1; q.kz = 2;
-    q.far = __builtin_isinf(q.ix) || __builtin_isinf(q.iy) || __builtin_isinf(q.iz) ? INFINITY : NAN;
     q.inst = -1;
     q.nodes = (rtq::gptr)tlasNodes;
 }
@@ -156,7 +155,6 @@ __device__ __forceinline__ void quad_enter(Quad2& q, int c, const float* w, int 
     q.ox = rtd::sel3(kx, ox, oy, oz); q.oy = rtd::sel3(ky, ox, oy, oz); q.oz = rtd::sel3(kz, ox, oy, oz);
     q.ix = rtd::sel3(kx, ix, iy, iz); q.iy = rtd::sel3(ky, ix, iy, iz); q.iz = rtd::sel3(kz, ix, iy, iz);
     q.kx = kx; q.ky = ky; q.kz = kz;
-    q.far = __builtin_isinf(ix) || __builtin_isinf(iy) || __builtin_isinf(iz) ? INFINITY : NAN;
     q.inst = k;
     q.nodes = (rtq::gptr)B.nodes;
     q.tris = (rtq::gptr)B.tris;

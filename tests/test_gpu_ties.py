@@ -103,3 +103,28 @@ def test_two_level_four_lanes_per_ray_from_the_root(scene, dev, n):
     got = _out(KEYS2, n, dev)
     s.trace_closest(R, *got)
     assert _differing(got, _counted(s, R, KEYS2, n, dev)) == {}
+
+
+@pytest.mark.parametrize("config", [(0, 8, 0), (0, 12, 2), (3, 8, 2), (3, 12, 0)])
+@pytest.mark.parametrize("n", [200000, 1000000])
+def test_hand_over_within_a_leaf(mesh, pkg, dev, config, n):
+    """A wave's last rays change to four lanes each wherever they are: also
+    between two triangles of a leaf, all of which are still to be tested."""
+    tris, b = mesh
+    R = to_dev(_rays(n, tris, n + 1), dev)
+    ref = _counted(b, R, KEYS, n, dev)
+    saved = b.trace_config(pkg.CLASS_INCOHERENT)
+    b.set_trace_config(pkg.CLASS_INCOHERENT, *config)
+    got = _out(KEYS, n, dev)
+    b.trace_closest(R, *got)
+    b.set_trace_config(pkg.CLASS_INCOHERENT, *saved)
+    assert _differing(got, ref) == {}
+
+
+@pytest.mark.parametrize("n", [200000, 600000])
+def test_two_level_hand_over_within_a_leaf(scene, dev, n):
+    pts, s = scene
+    R = to_dev(_rays(n, pts, n + 1), dev)
+    got = _out(KEYS2, n, dev)
+    s.trace_closest(R, *got)
+    assert _differing(got, _counted(s, R, KEYS2, n, dev)) == {}

@@ -346,9 +346,9 @@ __device__ __forceinline__ void trace2l_wave(const Trace2LArgs& a, Ray& r, bool 
     __builtin_amdgcn_s_setprio(0);
     res.t = best; res.u = bu; res.v = bv; res.id = bid; res.hinst = binst;
     res.occluded = found; res.steps = steps; res.open = has;
-    // a leaf cursor as a leaf code
+    // a leaf cursor as a leaf code, which is not tested against the closest hit again
     res.ref = ltc > 0 ? -((lts << 3) | (ltc - 1)) - 2 : ref;
-    res.tn = tn; res.inst = inst; res.sp = sp;
+    res.tn = ltc > 0 ? -INFINITY : tn; res.inst = inst; res.sp = sp;
 }
 
 // Rays that a wave has left (lanes with w.open, at most kQuadRays2 of them) go

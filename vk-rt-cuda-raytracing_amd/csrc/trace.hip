@@ -532,7 +532,7 @@ __device__ __forceinline__ void trace_wave(const TraceArgs& a, const Ray& r, boo
     res.occluded = found; res.steps = steps;
     res.open = has;
     res.ref = ltc > 0 ? cursor_code(lts, ltc) : ref;
-    res.tn = tn;
+    res.tn = ltc > 0 ? -INFINITY : tn;     // a leaf under way is not tested against the closest hit again
     res.sp = sp;
 }
 
@@ -864,8 +864,8 @@ __global__ __launch_bounds__(BLOCK) void k_trace_refill(TraceArgs a) {
                 if (sbase[sl] >= 0) flush(sl);
         }
         if (__any(has))
-            finish_quads<MODE, PIN, LDSD, BLOCK>(a, has, ltc > 0 ? cursor_code(lts, ltc) : ref, tn, sp,
-                                                 best, bu, bv, bid, ri, s_ref, s_tn, tid, gtid);
+            finish_quads<MODE, PIN, LDSD, BLOCK>(a, has, ltc > 0 ? cursor_code(lts, ltc) : ref, ltc > 0 ? -INFINITY : tn,
+                                                 sp, best, bu, bv, bid, ri, s_ref, s_tn, tid, gtid);
     }
 }
 

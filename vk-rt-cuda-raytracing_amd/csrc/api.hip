@@ -35,13 +35,13 @@ static int ensure_cwbvh(CudaBVH_t bvh);
 static void async_release(CudaBVH_t bvh);
 
 static void free_handle_device(CudaBVHHandle* h) {
-    hipDeviceSynchronize();          // traces on any stream may still read the arrays
-    rt::dev_free(h->d_nodes4); rt::dev_free(h->d_tris); rt::dev_free(h->d_leafOfPrim);
+    // traces on any stream may still read the arrays
+    rt::dev_release(h->d_nodes4); rt::dev_release(h->d_tris); rt::dev_release(h->d_leafOfPrim);
     hipFree(h->d_work); hipFree(h->d_sortWs);
     h->d_sortWs = nullptr; h->sortWsBytes = 0;
     hipFree(h->d_cwNodes); hipFree(h->d_cwTris);
     h->d_cwNodes = h->d_cwTris = nullptr;
-    rt::dev_free(h->d_nodes2); rt::dev_free(h->d_ordered);
+    rt::dev_release(h->d_nodes2); rt::dev_release(h->d_ordered);
     h->d_nodes2 = nullptr; h->d_ordered = nullptr;
     rtk::free_scratch(h->scratch);
     hipHostFree(h->h_pinned);
@@ -170,8 +170,7 @@ static CudaBVHHandle* build_impl(const float* tri9, int n, int maxLeaf, const in
     hipStreamSynchronize(s);          // the build syncs anyway; this separates the upload time
     t1 = clk();
     if (rt::gpu_build(d_in, n, maxLeaf, s, g, sceneOff, numScenes, roots4) != 0) {
-        hipDeviceSynchronize();
-        for (void* p : {(void*)d_own, (void*)g.nodes2, g.nodes4, g.tris, (void*)g.leafOf, (void*)g.ordered}) rt::dev_free(p);
+        for (void* p : {(void*)d_own, (void*)g.nodes2, g.nodes4, g.tris, (void*)g.leafOf, (void*)g.ordered}) rt::dev_release(p);
         goto fail;
     }
     rt::dev_free(d_own);                // the build has waited for its stream
@@ -376,7 +375,8 @@ CudaBVH_t cudaBVH_buildDevice(const void* d_vertices, int numVertices, int verte
         return nullptr;
     }
     CudaBVHHandle* h = build_impl(nullptr, numTris, 4, nullptr, 1, nullptr, d_tri);
-    rt::dev_free(d_tri);                // the build has waited for its stream
+    if (h) rt::dev_free(d_tri);         // the build has waited for its stream
+    else rt::dev_release(d_tri);
     return h;
 }
 
@@ -532,6 +532,7 @@ int cudaBVH_buildManyDevice(const CudaGeometry* geoms, const int* geomOffsets, i
 void cudaBVH_destroy(CudaBVH_t bvh) {
     if (!bvh) return;
     async_release(bvh);          // the background tracer no longer renders from it
+    if (bvh->stream) hipStreamSynchronize(hstream(bvh)); else hipDeviceSynchronize();
     free_handle_device(bvh);
     delete bvh;
 }

@@ -12,9 +12,11 @@
 // back, and so does an allocation that fails. Smaller blocks cost under 3 us
 // and go to the runtime directly.
 //
-// A block enters the cache only when no device work uses it any longer: the
-// caller has waited for that work (dev_free), or dev_release waits for the
-// device as hipFree does. So a later owner may use it on any stream.
+// A block is handed out again only when no device work uses it any longer: the
+// caller has waited for that work (dev_free), or the block is pending
+// (dev_release) until its device has been waited for, which the next
+// allocation that could take it does. So a later owner may use it on any
+// stream. Blocks leave the cache through hipFree, which waits by itself.
 #include <hip/hip_runtime.h>
 
 #include <list>
@@ -28,11 +30,13 @@ namespace rt {
 namespace {
 constexpr size_t kCacheMin = size_t(1) << 20, kCacheMax = size_t(2) << 30;
 
-struct Block { void* p; size_t bytes; int device; };
+// seq: number of the release after which it has not been waited for (0: idle)
+struct Block { void* p; size_t bytes; int device; unsigned long long seq; };
 struct Cache {
     std::mutex mu;
     std::list<Block> free;                          // oldest first
     size_t freeBytes = 0;
+    unsigned long long releases = 0;
     std::unordered_map<void*, Block> live;          // blocks of at least kCacheMin bytes in use
 };
 // never destroyed: handles may be freed while the process tears down
@@ -45,65 +49,62 @@ size_t rounded(size_t bytes) {
     while (step * 16 < bytes) step *= 2;            // at most an eighth over
     return (bytes + step - 1) / step * step;
 }
-}  // namespace
 
-void dev_trim() {
-    std::list<Block> out;
-    {
-        std::lock_guard<std::mutex> g(cache().mu);
-        out.swap(cache().free);
-        cache().freeBytes = 0;
-    }
-    for (const Block& b : out) hipFree(b.p);
-}
-
-void* dev_alloc(size_t bytes) {
+// hipMalloc whose failure leaves no error behind for a later launch check.
+void* raw_alloc(size_t bytes) {
     void* p = nullptr;
-    if (bytes < kCacheMin) {
-        if (hipMalloc(&p, bytes ? bytes : 1) == hipSuccess) return p;
-        dev_trim();
-        return hipMalloc(&p, bytes ? bytes : 1) == hipSuccess ? p : nullptr;
-    }
-    const size_t need = rounded(bytes);
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
-    Cache& c = cache();
-    {
-        std::lock_guard<std::mutex> g(c.mu);
-        auto best = c.free.end();
-        for (auto it = c.free.begin(); it != c.free.end(); ++it)
-            if (it->device == dev && it->bytes >= need && it->bytes <= need + need / 4 &&
-                (best == c.free.end() || it->bytes < best->bytes))
-                best = it;
-        if (best != c.free.end()) {
-            const Block b = *best;
-            c.freeBytes -= b.bytes;
-            c.free.erase(best);
-            c.live.emplace(b.p, b);
-            return b.p;
-        }
-    }
-    if (hipMalloc(&p, need) != hipSuccess) {
-        dev_trim();
-        if (hipMalloc(&p, need) != hipSuccess) return nullptr;
-    }
-    std::lock_guard<std::mutex> g(c.mu);
-    c.live.emplace(p, Block{p, need, dev});
-    return p;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
 }
 
-void dev_free(void* p) {
+// Frees blocks taken out of the cache; those that cannot be freed now (a stream
+// capture that forbids it) go back as pending.
+void give_back(std::list<Block>& out) {
+    for (auto it = out.begin(); it != out.end();) {
+        if (hipFree(it->p) == hipSuccess) { it = out.erase(it); continue; }
+        (void)hipGetLastError();
+        ++it;
+    }
+    if (out.empty()) return;
+    Cache& c = cache();
+    std::lock_guard<std::mutex> g(c.mu);
+    for (Block& b : out) { b.seq = ++c.releases; c.freeBytes += b.bytes; }
+    c.free.splice(c.free.begin(), out);
+}
+
+// Waits for all work of the current device as hipFree does, by freeing a block.
+// (hipDeviceSynchronize ends a capture in relaxed mode on any thread; this does
+// not, and still waits.) False where it cannot wait.
+bool wait_device() {
+    void* p = raw_alloc(1);
+    if (p && hipFree(p) == hipSuccess) return true;
+    if (p) (void)hipGetLastError();
+    return false;
+}
+
+// The smallest cached block of device dev that serves need bytes, idle or pending.
+std::list<Block>::iterator best_fit(Cache& c, int dev, size_t need, bool idle) {
+    auto best = c.free.end();
+    for (auto it = c.free.begin(); it != c.free.end(); ++it)
+        if (it->device == dev && (it->seq == 0) == idle && it->bytes >= need && it->bytes <= need + need / 4 &&
+            (best == c.free.end() || it->bytes < best->bytes))
+            best = it;
+    return best;
+}
+
+void put(void* p, bool idle) {
     if (!p) return;
     Cache& c = cache();
     std::list<Block> out;
     {
         std::lock_guard<std::mutex> g(c.mu);
         auto it = c.live.find(p);
-        if (it == c.live.end()) {
-            out.push_back(Block{p, 0, 0});
-        } else {
-            const Block b = it->second;
+        if (it != c.live.end()) {
+            Block b = it->second;
             c.live.erase(it);
+            b.seq = idle ? 0 : ++c.releases;
+            p = nullptr;
             if (b.bytes > kCacheMax) {
                 out.push_back(b);
             } else {
@@ -116,13 +117,69 @@ void dev_free(void* p) {
             }
         }
     }
-    for (const Block& b : out) hipFree(b.p);
+    if (p && hipFree(p) != hipSuccess) (void)hipGetLastError();   // a small block
+    give_back(out);
+}
+}  // namespace
+
+void dev_trim() {
+    std::list<Block> out;
+    {
+        std::lock_guard<std::mutex> g(cache().mu);
+        out.swap(cache().free);
+        cache().freeBytes = 0;
+    }
+    give_back(out);
 }
 
-void dev_release(void* p) {
-    if (!p) return;
-    hipDeviceSynchronize();
-    dev_free(p);
+void* dev_alloc(size_t bytes) {
+    if (bytes < kCacheMin) {
+        void* p = raw_alloc(bytes ? bytes : 1);
+        if (p) return p;
+        dev_trim();
+        return raw_alloc(bytes ? bytes : 1);
+    }
+    const size_t need = rounded(bytes);
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+    Cache& c = cache();
+    {
+        std::unique_lock<std::mutex> g(c.mu);
+        auto it = best_fit(c, dev, need, true);
+        if (it == c.free.end() && best_fit(c, dev, need, false) != c.free.end()) {
+            // one wait serves every block released before it
+            const unsigned long long upTo = c.releases;
+            g.unlock();
+            const bool waited = wait_device();
+            g.lock();
+            if (waited) {
+                for (Block& b : c.free)
+                    if (b.device == dev && b.seq <= upTo) b.seq = 0;
+                it = best_fit(c, dev, need, true);
+            } else {
+                it = c.free.end();
+            }
+        }
+        if (it != c.free.end()) {
+            const Block b = *it;
+            c.freeBytes -= b.bytes;
+            c.free.erase(it);
+            c.live.emplace(b.p, b);
+            return b.p;
+        }
+    }
+    void* p = raw_alloc(need);
+    if (!p) {
+        dev_trim();
+        p = raw_alloc(need);
+        if (!p) return nullptr;
+    }
+    std::lock_guard<std::mutex> g(c.mu);
+    c.live.emplace(p, Block{p, need, dev, 0});
+    return p;
 }
+
+void dev_free(void* p) { put(p, true); }
+void dev_release(void* p) { put(p, false); }
 
 }  // namespace rt

@@ -63,7 +63,8 @@ int gpu_build(const float* d_tris, int n, int maxLeaf, hipStream_t s, GpuBVH& ou
 int mesh_bounds(const float* d_tris, int n, hipStream_t s, float* mn, float* mx);
 // Device memory with a bounded cache of freed blocks (devmem.hip). nullptr when
 // out of memory. dev_free: no device work uses the block any longer;
-// dev_release waits for the device first (as hipFree does). Both accept nullptr.
+// dev_release: some may, and its device is waited for before the block is used
+// again. Both accept nullptr.
 void* dev_alloc(size_t bytes);
 void dev_free(void* p);
 void dev_release(void* p);

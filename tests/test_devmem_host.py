@@ -150,10 +150,20 @@ static void full_device() {
     rt::dev_free(c);
     CHECK(R.freed.count(c));                        // small blocks are not kept
 }
+static void full_device_other_memory() {
+    void* a = rt::dev_alloc(64 * MB);
+    rt::dev_free(a);
+    R.room = 96 * MB;
+    int *p = nullptr, *q = (int*)1, *r = nullptr;
+    CHECK(rt::dev_malloc(&p, 80 * MB) && p && R.held == 80 * MB);
+    CHECK(!rt::dev_malloc(&q, 80 * MB) && !q && hipGetLastError() == 0);
+    CHECK(rt::dev_malloc(&r, 0) && r);
+}
 int main(int, char** v) {
 #define RUN(f) if (!strcmp(v[1], #f)) { f(); return 0; }
     RUN(released_block_waits) RUN(idle_block_does_not_wait) RUN(other_device) RUN(release_after_the_wait)
     RUN(no_wait_possible) RUN(bound_oldest_first) RUN(bound_after_a_refused_free) RUN(full_device)
+    RUN(full_device_other_memory)
     return 2;
 }
 """
@@ -174,7 +184,8 @@ def driver(tmp_path_factory):
 
 @pytest.mark.parametrize("case", ["released_block_waits", "idle_block_does_not_wait", "other_device",
                                   "release_after_the_wait", "no_wait_possible", "bound_oldest_first",
-                                  "bound_after_a_refused_free", "full_device"])
+                                  "bound_after_a_refused_free", "full_device",
+                                  "full_device_other_memory"])
 def test_cache(driver, case):
     r = subprocess.run([driver, case], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout

@@ -274,7 +274,7 @@ static void* work_buffer(CudaBVHHandle* h, size_t bytes) {
     if (bytes > h->workBytes) {
         hipFree(h->d_work);
         h->d_work = nullptr; h->workBytes = 0;
-        if (hipMalloc(&h->d_work, bytes) != hipSuccess) { set_error("cannot allocate %zu staging bytes", bytes); return nullptr; }
+        if (!rt::dev_malloc(&h->d_work, bytes)) { set_error("cannot allocate %zu staging bytes", bytes); return nullptr; }
         h->workBytes = bytes;
     }
     return h->d_work;
@@ -285,7 +285,7 @@ static void* sort_workspace(CudaBVHHandle* h, int n) {
     if (bytes > h->sortWsBytes) {
         hipFree(h->d_sortWs);
         h->d_sortWs = nullptr; h->sortWsBytes = 0;
-        if (hipMalloc(&h->d_sortWs, bytes) != hipSuccess) { set_error("cannot allocate %zu sort bytes", bytes); return nullptr; }
+        if (!rt::dev_malloc(&h->d_sortWs, bytes)) { set_error("cannot allocate %zu sort bytes", bytes); return nullptr; }
         h->sortWsBytes = bytes;
     }
     return h->d_sortWs;
@@ -356,7 +356,7 @@ CudaBVH_t cudaBVH_buildDevice(const void* d_vertices, int numVertices, int verte
     }
     float* d_tri = nullptr;
     int* d_bad = nullptr;
-    if (!(d_tri = (float*)rt::dev_alloc(size_t(numTris) * 36)) || hipMalloc((void**)&d_bad, sizeof(int)) != hipSuccess) {
+    if (!(d_tri = (float*)rt::dev_alloc(size_t(numTris) * 36)) || !rt::dev_malloc(&d_bad, sizeof(int))) {
         rt::dev_free(d_tri);
         set_error("cudaBVH_buildDevice: cannot allocate %zu bytes", size_t(numTris) * 36);
         return nullptr;
@@ -430,7 +430,7 @@ int cudaBVH_buildManyDevice(const CudaGeometry* geoms, const int* geomOffsets, i
     if (total > (1ll << 28)) { set_error("%s: %lld triangles in all", fn, total); return -1; }
     float* dTri = nullptr;
     int* dBad = nullptr;
-    if (!(dTri = (float*)rt::dev_alloc(size_t(total) * 36)) || hipMalloc((void**)&dBad, sizeof(int)) != hipSuccess) {
+    if (!(dTri = (float*)rt::dev_alloc(size_t(total) * 36)) || !rt::dev_malloc(&dBad, sizeof(int))) {
         rt::dev_free(dTri);
         set_error("%s: cannot allocate %lld triangles", fn, total);
         return -1;
@@ -689,7 +689,7 @@ struct AsyncTracer {
                 shade_to_device(b, scratch, stream, W, H, X, Y, Z, tgt, F);
                 hipStreamSynchronize(stream);
             } else {
-                if (dbytes < sz) { hipFree(dbuf); dbuf = nullptr; dbytes = 0; if (hipMalloc(&dbuf, sz) == hipSuccess) dbytes = sz; }
+                if (dbytes < sz) { hipFree(dbuf); dbuf = nullptr; dbytes = 0; if (rt::dev_malloc(&dbuf, sz)) dbytes = sz; }
                 if (dbuf && shade_to_device(b, scratch, stream, W, H, X, Y, Z, dbuf, F) == 0) {
                     hipMemcpyAsync(host[wi].data(), dbuf, sz, hipMemcpyDeviceToHost, stream);
                     hipStreamSynchronize(stream);
@@ -927,7 +927,7 @@ int cudaBVH_buildTLASFast(const float* aabbs, int numAABBs, uint32_t** outNodes,
     const size_t n = size_t(numAABBs), total = 2 * n - 1;
     const size_t inB = n * 24, nodeB = total * 32, ordB = n * 4, wsB = rtk::lbvh_scratch_bytes(numAABBs);
     char* d = nullptr;
-    if (hipMalloc((void**)&d, inB + nodeB + ordB + wsB + 256) != hipSuccess) {
+    if (!rt::dev_malloc(&d, inB + nodeB + ordB + wsB + 256)) {
         set_error("cudaBVH_buildTLASFast: cannot allocate %zu device bytes", inB + nodeB + ordB + wsB);
         return 0;
     }
@@ -992,8 +992,8 @@ static int ensure_cwbvh(CudaBVH_t bvh) {
         const int id = bvh->h_ordered[li];
         memcpy(&o[3], &id, 4);
     }
-    if (hipMalloc(&bvh->d_cwNodes, bvh->h_cw.size() * 4) != hipSuccess ||
-        hipMalloc(&bvh->d_cwTris, tri.size() * 4) != hipSuccess ||
+    if (!rt::dev_malloc(&bvh->d_cwNodes, bvh->h_cw.size() * 4) ||
+        !rt::dev_malloc(&bvh->d_cwTris, tri.size() * 4) ||
         hipMemcpy(bvh->d_cwNodes, bvh->h_cw.data(), bvh->h_cw.size() * 4, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(bvh->d_cwTris, tri.data(), tri.size() * 4, hipMemcpyHostToDevice) != hipSuccess) {
         hipFree(bvh->d_cwNodes); hipFree(bvh->d_cwTris);
@@ -1266,7 +1266,7 @@ int cudaBVH_autotune(CudaBVH_t bvh, int rayClass, int width, int height, const C
     const int n = coherent ? width * height : numRays;
     hipStream_t s = hstream(bvh);
     void* out = nullptr;
-    HIP_TRY(hipMalloc(&out, size_t(n) * 16), return -1);
+    if (!rt::dev_malloc(&out, size_t(n) * 16)) { set_error("cudaBVH_autotune: cannot allocate %d results", n); return -1; }
     rtk::TraceArgs base;
     base.n = n;
     // coherent candidates of the batch schedule run in the cost order, as
@@ -1425,8 +1425,8 @@ CudaScene_t cudaBVH_sceneCreate(const CudaBVH_t* blas, int numBlas, const CudaIn
     for (int b = 0; b < numBlas; b++)
         bd[b] = rtk::BlasDev{(const uint4*)blas[b]->d_nodes4, (const float4*)blas[b]->d_tris, blas[b]->d_leafOfPrim,
                              blas[b]->depth4, blas[b]->numTris};
-    if (hipMalloc((void**)&sc->d_inst, sizeof(rtk::InstanceDev) * numInst) != hipSuccess ||
-        hipMalloc((void**)&sc->d_blas, sizeof(rtk::BlasDev) * numBlas) != hipSuccess ||
+    if (!rt::dev_malloc(&sc->d_inst, sizeof(rtk::InstanceDev) * numInst) ||
+        !rt::dev_malloc(&sc->d_blas, sizeof(rtk::BlasDev) * numBlas) ||
         hipMemcpy(sc->d_inst, sc->inst.data(), sizeof(rtk::InstanceDev) * numInst, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(sc->d_blas, bd.data(), sizeof(rtk::BlasDev) * numBlas, hipMemcpyHostToDevice) != hipSuccess) {
         set_error("cudaBVH_sceneCreate: device allocation failed");
@@ -1590,7 +1590,7 @@ CudaBVHBatch_t cudaBVH_buildBatch(const CudaTri* tris, const int* triOffsets, in
     b->forest = build_impl(reinterpret_cast<const float*>(tris), triOffsets[numScenes], 4, triOffsets, numScenes,
                            &b->roots4);
     if (!b->forest) { delete b; return nullptr; }
-    if (hipMalloc((void**)&b->d_roots, sizeof(int) * numScenes) != hipSuccess ||
+    if (!rt::dev_malloc(&b->d_roots, sizeof(int) * numScenes) ||
         hipMemcpy(b->d_roots, b->roots4.data(), sizeof(int) * numScenes, hipMemcpyHostToDevice) != hipSuccess) {
         set_error("cudaBVH_buildBatch: device allocation failed");
         cudaBVH_destroy(b->forest);
@@ -1735,7 +1735,7 @@ int cudaBVH_sceneAutotune(CudaScene_t sc, int rayClass, int numRays, const CudaR
     }
     hipStream_t s = (hipStream_t)sc->stream;
     void* buf = nullptr;
-    if (hipMalloc(&buf, (size_t)numRays * 20) != hipSuccess) { set_error("cudaBVH_sceneAutotune: no memory"); return -1; }
+    if (!rt::dev_malloc(&buf, (size_t)numRays * 20)) { set_error("cudaBVH_sceneAutotune: no memory"); return -1; }
     CudaSceneHit hit{(float*)buf, (int*)buf + numRays, (int*)buf + 2 * (size_t)numRays,
                      (float*)buf + 3 * (size_t)numRays, (float*)buf + 4 * (size_t)numRays};
     hipEvent_t e0, e1;

@@ -151,7 +151,7 @@ int launch_bounce(const CudaBVHHandle* h, rt::TraceScratch& sc, const rtd::Cam& 
         hipFree(sc.tiles);
         sc.tiles = nullptr; sc.tileCap = 0;
         sc.gen++;
-        if (hipMalloc((void**)&sc.tiles, (size_t)tiles * sizeof(int)) != hipSuccess) {
+        if (!rt::dev_malloc(&sc.tiles, (size_t)tiles * sizeof(int))) {
             rt::set_error("cannot allocate %d tile counters", tiles);
             return -1;
         }

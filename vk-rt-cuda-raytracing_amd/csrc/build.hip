@@ -1512,7 +1512,7 @@ struct Slab {
 
 int mesh_bounds(const float* d_tris, int n, hipStream_t s, float* mn, float* mx) {
     unsigned long long* key = nullptr;
-    if (hipMalloc((void**)&key, 128) != hipSuccess) { set_error("mesh bounds: out of device memory"); return -1; }
+    if (!rt::dev_malloc(&key, 128)) { set_error("mesh bounds: out of device memory"); return -1; }
     float* out = (float*)(key + 8);
     float h[6];
     hipLaunchKernelGGL(rtb::k_keys_init, dim3(1), dim3(64), 0, s, key);

@@ -8,8 +8,9 @@
 // allocation of about their size on their device, at most kCacheMax bytes in
 // all over the process (the oldest go first; a 3.4 M-triangle scene rebuilt and
 // traced every frame holds 1.0 GiB of them between frames, which a bound of
-// 1 GiB gave back and took again each time, 0.34 of 4.3 ms); cudaBVH_resetDevice gives them
-// back, and so does an allocation that fails. Smaller blocks cost under 3 us
+// 1 GiB gave back and took again each time, 0.34 of 4.3 ms).
+// cudaBVH_resetDevice gives them back, and so does every device allocation of
+// the library that finds no memory (dev_plain). Smaller blocks cost under 3 us
 // and go to the runtime directly.
 //
 // A block is handed out again only when no device work uses it any longer: the
@@ -132,13 +133,18 @@ void dev_trim() {
     give_back(out);
 }
 
-void* dev_alloc(size_t bytes) {
-    if (bytes < kCacheMin) {
-        void* p = raw_alloc(bytes ? bytes : 1);
-        if (p) return p;
+void* dev_plain(size_t bytes) {
+    if (bytes == 0) bytes = 1;
+    void* p = raw_alloc(bytes);
+    if (!p) {
         dev_trim();
-        return raw_alloc(bytes ? bytes : 1);
+        p = raw_alloc(bytes);
     }
+    return p;
+}
+
+void* dev_alloc(size_t bytes) {
+    if (bytes < kCacheMin) return dev_plain(bytes);
     const size_t need = rounded(bytes);
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return nullptr;
@@ -168,12 +174,8 @@ void* dev_alloc(size_t bytes) {
             return b.p;
         }
     }
-    void* p = raw_alloc(need);
-    if (!p) {
-        dev_trim();
-        p = raw_alloc(need);
-        if (!p) return nullptr;
-    }
+    void* p = dev_plain(need);
+    if (!p) return nullptr;
     std::lock_guard<std::mutex> g(c.mu);
     c.live.emplace(p, Block{p, need, dev, 0});
     return p;

@@ -1544,8 +1544,8 @@ CudaDenoiser_t cudaBVH_denoiserCreate(int maxPixels, uint64_t seed) {
     for (auto& b : bufs) actBytes += (b.elems * 2 + 255) & ~(size_t)255;
     N.partFloats = 16u << 20;
     const size_t fBytes = (lv0 * 3 * 2 + N.partFloats + 8192) * 4;
-    if (hipMalloc(&N.act, actBytes + fBytes) != hipSuccess ||
-        hipMalloc((void**)&N.w, N.nParams * 4 * 4) != hipSuccess || hipMalloc((void**)&N.wbuf, wbytes) != hipSuccess) {
+    if (!rt::dev_malloc(&N.act, actBytes + fBytes) ||
+        !rt::dev_malloc(&N.w, N.nParams * 4 * 4) || !rt::dev_malloc(&N.wbuf, wbytes)) {
         rt::set_error("cudaBVH_denoiserCreate: cannot allocate %zu bytes", actBytes + fBytes + N.nParams * 16 + wbytes);
         hipFree(N.act); hipFree(N.w); hipFree(N.wbuf);
         delete h;

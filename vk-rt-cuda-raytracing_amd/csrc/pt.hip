@@ -559,11 +559,11 @@ static int pt_alloc(PtResources& R, int N) {
     const size_t per = 3 * (11 * 4 + 4 + 8) + (11 * 4 + 4 + 1) + 12;
     const size_t chunkBytes = 2 * ((size_t)(N + 63) / 64 * 4 + 256);     // camera-ray chunk costs and order
     const size_t bytes = per * (size_t)N + chunkBytes + 4096;
-    if (hipMalloc(&R.block, bytes) != hipSuccess) {
+    if (!rt::dev_malloc(&R.block, bytes)) {
         rt::set_error("path tracer: cannot allocate %zu bytes of queues", bytes);
         return -1;
     }
-    if (!R.small && hipMalloc((void**)&R.small, 4096) != hipSuccess) {
+    if (!R.small && !rt::dev_malloc(&R.small, 4096)) {
         rt::set_error("path tracer: cannot allocate counters");
         return -1;
     }
@@ -677,7 +677,7 @@ int path_trace(CudaSceneHandle* sc, const CudaCamera& cam, const CudaPathParams&
         if (need > R.tailBytes) {
             hipFree(R.tailStack);
             R.tailStack = nullptr; R.tailBytes = 0;
-            if (hipMalloc((void**)&R.tailStack, need) != hipSuccess) {
+            if (!rt::dev_malloc(&R.tailStack, need)) {
                 rt::set_error("scenePathTrace: cannot allocate %zu stack bytes", need);
                 return -1;
             }

@@ -69,6 +69,12 @@ void* dev_alloc(size_t bytes);
 void dev_free(void* p);
 void dev_release(void* p);
 void dev_trim();                                   // gives the cached blocks back
+// Device memory outside the cache (hipFree), for everything else: where there
+// is none, the cache's blocks are given back first. False (and nullptr) when
+// out of memory.
+void* dev_plain(size_t bytes);
+template <class T>
+bool dev_malloc(T** p, size_t bytes) { return (*p = (T*)dev_plain(bytes)) != nullptr; }
 void scan_exclusive(const int* in, int* out, int n, int* total, int* tiles, hipStream_t s);
 int scan_tiles_needed(int n);
 

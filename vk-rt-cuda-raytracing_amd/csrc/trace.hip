@@ -1467,9 +1467,9 @@ static int launch_kernel(const CudaBVHHandle* h, rt::TraceScratch& sc, TraceArgs
             hipFree(sc.tileCost); hipFree(sc.tileOrder); hipFree(sc.tilePred);
             sc.tileCost = sc.tileOrder = sc.tilePred = nullptr; sc.costCap = 0; sc.costW = sc.costH = 0;
             sc.gen++;
-            if (hipMalloc((void**)&sc.tileCost, (size_t)a.nTiles * sizeof(int)) != hipSuccess ||
-                hipMalloc((void**)&sc.tileOrder, (size_t)a.nTiles * sizeof(int)) != hipSuccess ||
-                hipMalloc((void**)&sc.tilePred, (size_t)a.nTiles * sizeof(int)) != hipSuccess) {
+            if (!rt::dev_malloc(&sc.tileCost, (size_t)a.nTiles * sizeof(int)) ||
+                !rt::dev_malloc(&sc.tileOrder, (size_t)a.nTiles * sizeof(int)) ||
+                !rt::dev_malloc(&sc.tilePred, (size_t)a.nTiles * sizeof(int))) {
                 hipFree(sc.tileCost); hipFree(sc.tileOrder); hipFree(sc.tilePred);
                 sc.tileCost = sc.tileOrder = sc.tilePred = nullptr;
                 rt::set_error("cannot allocate the tile cost order of %d tiles", a.nTiles);
@@ -1578,7 +1578,7 @@ int launch_chunk_order(const int* cost, int nChunks, int* order, hipStream_t s) 
 
 int alloc_scratch(rt::TraceScratch& sc) {
     if (sc.counter) return 0;
-    if (hipMalloc((void**)&sc.counter, rtd::kBands * rtd::kBandStride * sizeof(uint32_t)) != hipSuccess || hipMalloc((void**)&sc.status, 64) != hipSuccess ||
+    if (!rt::dev_malloc(&sc.counter, rtd::kBands * rtd::kBandStride * sizeof(uint32_t)) || !rt::dev_malloc(&sc.status, 64) ||
         hipMemset(sc.status, 0, 64) != hipSuccess) {
         free_scratch(sc);
         rt::set_error("cannot allocate traversal scratch");
@@ -1602,7 +1602,7 @@ int grow_hits(rt::TraceScratch& sc, size_t need) {
     hipFree(sc.hits);
     sc.hits = nullptr; sc.hitsBytes = 0;
     sc.gen++;
-    if (hipMalloc(&sc.hits, need) != hipSuccess) {
+    if (!rt::dev_malloc(&sc.hits, need)) {
         rt::set_error("cannot allocate %zu bytes of staged hit records", need);
         return -1;
     }

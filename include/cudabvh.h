@@ -257,7 +257,8 @@ int cudaBVH_genPinholeRays(int width, int height, const CudaCamera* cam,
  * CUDABVH_FLAG_COST_ORDER (batch schedule): the handle keeps each 8x8 tile's
  * step count of the last launch of this image size, and the next launch
  * starts the tiles predicted slowest first (a renderer tracing consecutive
- * frames; the hits are the same in any order). Extension of this build:
+ * frames; the hits are the same in any order). Small launches that give each
+ * ray four lanes (cudaBVH_setTraceConfig) ignore it. Extension of this build:
  * the reference's primary trace (layer/cuda_bvh_backend.cu:761-800) has
  * no tile order. */
 int cudaBVH_tracePinholeClosest(CudaBVH_t bvh, int width, int height, const CudaCamera* cam,
@@ -295,7 +296,13 @@ int cudaBVH_traceAnyQueued(CudaBVH_t bvh, int capacity, const int* d_count,
  * refilled from the wave-local pool),
  * LDS stack depth per lane (4, 8, 12 or 16 entries; deeper entries spill to
  * HBM) and resident workgroups per CU (0 = occupancy limit). Defaults after a
- * build: batch / 12 / 0 for classes 0 and 2, refill / 8 / 0 for class 1. */
+ * build: batch / 12 / 0 for classes 0 and 2, refill / 8 / 0 for class 1.
+ * With the default configuration, uncounted watertight launches of few rays
+ * give each ray four lanes instead (same hits): up to 1,048,576 pinhole rays
+ * (720,896 with CUDABVH_FLAG_COST_ORDER), 294,912 rays of class 1 (a queue's
+ * capacity: 409,600) and 589,824 of class 2. Any other configuration holds for
+ * launches of every size. Setting the default one returns to this; setting the
+ * one that is set changes nothing. */
 int cudaBVH_setTraceConfig(CudaBVH_t bvh, int rayClass, int schedule, int ldsDepth, int blocksPerCU);
 int cudaBVH_getTraceConfig(CudaBVH_t bvh, int rayClass, int* schedule, int* ldsDepth, int* blocksPerCU);
 
@@ -305,7 +312,9 @@ int cudaBVH_getTraceConfig(CudaBVH_t bvh, int rayClass, int* schedule, int* ldsD
  * handle. results (nullable, room for 192 floats: schedule, ldsDepth,
  * blocksPerCU, ms per candidate) and *numResults report the sweep. The
  * coherent class's batch candidates are timed in the tile cost order of
- * CUDABVH_FLAG_COST_ORDER. */
+ * CUDABVH_FLAG_COST_ORDER. The default configuration is timed as it runs on
+ * that many rays; tuned on more than it would give four lanes each, smaller
+ * launches stay as they were. */
 int cudaBVH_autotune(CudaBVH_t bvh, int rayClass, int width, int height, const CudaCamera* cam,
                      int numRays, const CudaRayPacket* rays, int reps, float* results, int* numResults);
 

@@ -129,13 +129,7 @@ static CudaBVHHandle* make_handle(CudaBVHHandle* h, const float* bmin, const flo
         delete h;
         return nullptr;
     }
-    // defaults: the configurations the autotuner picks most often on the
-    // 1080p terrain frame (refill / 8: its 16 KB of stack plus 8 KB of
-    // gathered results per workgroup leave room for six workgroups per CU)
-    h->tune[rt::kClassIncoherent].schedule = rt::kScheduleRefill;
-    h->tune[rt::kClassIncoherent].ldsDepth = 8;
-    h->tune[rt::kClassCoherent].ldsDepth = 12;
-    h->tune[rt::kClassAny].ldsDepth = 12;
+    for (int k = 0; k < rt::kNumClasses; k++) h->tune[k] = rt::default_config(k);
     if (rt::verbose())
         fprintf(stderr, "[CudaBVH] built %d tris: %d BVH4 nodes (depth %d), %d BVH2 nodes\n", n, h->numNodes4,
                 h->depth4, h->numNodes2);
@@ -1233,10 +1227,10 @@ int cudaBVH_setTraceConfig(CudaBVH_t bvh, int rayClass, int schedule, int ldsDep
                   schedule, ldsDepth, blocksPerCU);
         return -1;
     }
-    bvh->tune[rayClass].schedule = schedule;
-    bvh->tune[rayClass].ldsDepth = ldsDepth;
-    bvh->tune[rayClass].blocksPerCU = blocksPerCU;
-    bvh->tune[rayClass].chosen = true;
+    rt::TraceConfig c;
+    c.schedule = schedule; c.ldsDepth = ldsDepth; c.blocksPerCU = blocksPerCU;
+    c.everySize = !c.same(rt::default_config(rayClass));
+    if (!c.same(bvh->tune[rayClass])) bvh->tune[rayClass] = c;     // setting what is set changes nothing
     return 0;
 }
 
@@ -1250,7 +1244,8 @@ int cudaBVH_getTraceConfig(CudaBVH_t bvh, int rayClass, int* schedule, int* ldsD
 
 // Autotuner: times every candidate launch configuration of one ray class on
 // the caller's workload (a pinhole frame for the coherent class, a device ray
-// packet otherwise) and keeps the fastest in the handle. results (nullable,
+// packet otherwise) and keeps the fastest in the handle; the default one is
+// timed as it runs there, with four lanes per ray in small launches. results (nullable,
 // room for 4 floats x 36 candidates) receives {schedule, ldsDepth,
 // blocksPerCU, milliseconds} per candidate.
 int cudaBVH_autotune(CudaBVH_t bvh, int rayClass, int width, int height, const CudaCamera* cam, int numRays,
@@ -1296,7 +1291,8 @@ int cudaBVH_autotune(CudaBVH_t bvh, int rayClass, int width, int height, const C
                 bvh->tune[rayClass].schedule = sch;
                 bvh->tune[rayClass].ldsDepth = d;
                 bvh->tune[rayClass].blocksPerCU = b;
-                bvh->tune[rayClass].chosen = true;       // times this schedule whatever the ray count
+                // (the default configuration as it runs at this ray count)
+                bvh->tune[rayClass].everySize = !bvh->tune[rayClass].same(rt::default_config(rayClass));
                 rtk::TraceArgs a = base;
                 rc = rtk::launch_trace(bvh, bvh->scratch, a, mode, false, coherent, false, s);   // warm-up
                 hipEventRecord(e0, s);
@@ -1323,8 +1319,10 @@ int cudaBVH_autotune(CudaBVH_t bvh, int rayClass, int width, int height, const C
     }
     hipEventDestroy(e0); hipEventDestroy(e1);
     hipFree(out);
+    // A workload that four lanes per ray would not take by default says nothing
+    // about the smaller ones that they would.
+    if (!rtk::small_launch(bvh, base, mode, coherent)) best.everySize = saved.everySize;
     bvh->tune[rayClass] = rc == 0 ? best : saved;
-    bvh->tune[rayClass].chosen = saved.chosen;
     if (numResults) *numResults = row;
     return rc;
 }

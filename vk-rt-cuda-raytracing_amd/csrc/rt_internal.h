@@ -103,8 +103,23 @@ struct TraceConfig {
     int schedule = kScheduleBatch;
     int ldsDepth = 16;
     int blocksPerCU = 0;
-    bool chosen = false;                // set by the caller: small launches keep this schedule too
+    // Holds for launches of every size. Otherwise those up to a ray count give
+    // each ray four lanes from its root on (launch_trace) and larger ones run so.
+    bool everySize = false;
+    bool same(const TraceConfig& o) const {
+        return schedule == o.schedule && ldsDepth == o.ldsDepth && blocksPerCU == o.blocksPerCU;
+    }
 };
+
+// After a build: the configurations the autotuner picks most often on the 1080p
+// terrain frame (refill / 8: its 16 KB of stack plus 8 KB of gathered results
+// per workgroup leave room for six workgroups per CU).
+inline TraceConfig default_config(int rayClass) {
+    TraceConfig c;
+    c.schedule = rayClass == kClassIncoherent ? kScheduleRefill : kScheduleBatch;
+    c.ldsDepth = rayClass == kClassIncoherent ? 8 : 12;
+    return c;
+}
 
 // Resources of one traversal kernel, read once per kernel (hipFuncGetAttributes
 // and the occupancy calculator).

@@ -1701,15 +1701,19 @@ static int launch_tuned(const CudaBVHHandle* h, rt::TraceScratch& sc, TraceArgs&
 constexpr int kQuadPinhole = 1 << 20, kQuadCostOrder = 11 << 16, kQuadClosest = 9 << 15, kQuadQueue = 25 << 14,
               kQuadAny = 9 << 16;
 
+bool small_launch(const CudaBVHHandle* h, const TraceArgs& a, int mode, bool pinhole) {
+    return a.n <= (mode == kModeAny ? kQuadAny
+                   : pinhole        ? (a.costOrder ? kQuadCostOrder : kQuadPinhole)
+                                    : (a.nDev ? kQuadQueue : kQuadClosest)) &&
+           rtq::fits(h->numNodes4, h->numOrdered);
+}
+
 int launch_trace(const CudaBVHHandle* h, rt::TraceScratch& sc, TraceArgs& a, int mode, bool mt, bool pinhole,
                  bool counted, hipStream_t s) {
     if (alloc_scratch(sc) != 0) return -1;
     if (a.n <= 0) return 0;
     const rt::TraceConfig& cfg = h->tune[mode == kModeAny ? rt::kClassAny : (pinhole ? rt::kClassCoherent : rt::kClassIncoherent)];
-    if (!mt && !counted && mode != kModeShade && !cfg.chosen &&
-        a.n <= (mode == kModeAny ? kQuadAny
-                : pinhole        ? (a.costOrder ? kQuadCostOrder : kQuadPinhole)
-                                 : (a.nDev ? kQuadQueue : kQuadClosest)) && rtq::fits(h->numNodes4, h->numOrdered)) {
+    if (!mt && !counted && mode != kModeShade && !cfg.everySize && small_launch(h, a, mode, pinhole)) {
         const int d = cfg.ldsDepth;
         if (mode == kModeClosest) return pinhole ? launch_quads<kModeClosest, true>(h, sc, a, d, s)
                                                  : launch_quads<kModeClosest, false>(h, sc, a, d, s);

@@ -66,6 +66,9 @@ struct TraceArgs {
     const int* rayOff = nullptr; const int* roots = nullptr; int numScenes = 0;
 };
 
+// Whether a launch with these arguments takes four lanes per ray from the root
+// on unless its class's configuration holds for every size (trace.hip).
+bool small_launch(const CudaBVHHandle* h, const TraceArgs& a, int mode, bool pinhole);
 int launch_trace(const CudaBVHHandle* h, rt::TraceScratch& sc, TraceArgs& a, int mode, bool mt, bool pinhole,
                  bool counted, hipStream_t s);
 int alloc_scratch(rt::TraceScratch& sc);

@@ -142,7 +142,8 @@ static CudaBVHHandle* make_handle(CudaBVHHandle* h, const float* bmin, const flo
 static CudaBVHHandle* build_impl(const float* tri9, int n, int maxLeaf, const int* sceneOff = nullptr,
                                  int numScenes = 1, std::vector<int>* roots4 = nullptr,
                                  const float* d_tri9 = nullptr, std::vector<rt::Node2>* forestNodes2 = nullptr,
-                                 std::vector<int>* forestOrdered = nullptr) {
+                                 std::vector<int>* forestOrdered = nullptr,
+                                 std::vector<float>* forestBounds = nullptr) {
     rt::clear_error();
     if ((!tri9 && !d_tri9) || n <= 0) { set_error("cudaBVH_build: need tris != NULL and numTris > 0 (got %d)", n); return nullptr; }
     if (n > (1 << 27)) { set_error("cudaBVH_build: %d triangles exceed the leaf encoding (2^27)", n); return nullptr; }
@@ -188,6 +189,7 @@ static CudaBVHHandle* build_impl(const float* tri9, int n, int maxLeaf, const in
             forestOrdered->resize(n);
             e = hipMemcpy(forestOrdered->data(), g.ordered, size_t(n) * 4, hipMemcpyDeviceToHost);
         }
+        if (forestBounds) forestBounds->swap(g.sceneBounds);
         rt::dev_free(g.nodes2);
         if (e != hipSuccess) { set_error("copying the forest back failed: %s", hipGetErrorString(e)); goto fail; }
     }
@@ -464,7 +466,8 @@ int cudaBVH_buildManyDevice(const CudaGeometry* geoms, const int* geomOffsets, i
         for (int i = 0; i < R; i++) off[i + 1] = off[i] + (int)count[big[i]];
         std::vector<int> roots4, ford;
         std::vector<rt::Node2> fn2;
-        CudaBVHHandle* forest = build_impl(nullptr, off[R], 4, off.data(), R, &roots4, dTri, &fn2, &ford);
+        std::vector<float> bounds;
+        CudaBVHHandle* forest = build_impl(nullptr, off[R], 4, off.data(), R, &roots4, dTri, &fn2, &ford, &bounds);
         if (!forest) return fail_all();
         // BVH2 subtree sizes: the trees lie one after another in pre-order
         std::vector<int> sz(fn2.size(), 1);
@@ -508,13 +511,7 @@ int cudaBVH_buildManyDevice(const CudaGeometry* geoms, const int* geomOffsets, i
             }
             h->depth4 = bvh4_depth(hn4);
             root2 += sz[root2];
-            float bmin[3], bmax[3];
-            if (rt::mesh_bounds(dTri + 9 * size_t(t0), nt, nullptr, bmin, bmax) == 0) {
-                out[k] = make_handle(h, bmin, bmax, nt);
-            } else {
-                free_handle_device(h);
-                delete h;
-            }
+            out[k] = make_handle(h, &bounds[6 * size_t(i)], &bounds[6 * size_t(i) + 3], nt);
             if (!out[k]) { cudaBVH_destroy(forest); return fail_all(); }
         }
         cudaBVH_destroy(forest);

@@ -144,7 +144,7 @@ struct Build {
     const int* primBase;     // [numScenes + 1] chunks of kChunk primitives before each scene
     int* rootAcc;            // [numScenes][12] root bounds (ordered ints)
     int* rootRef;            // [numScenes] top node or -1 - subtree
-    unsigned long long* bnd; // [6] mesh bounds as (ordered value, first position) keys
+    unsigned long long* bnd; // [numScenes][6] scene bounds as (ordered value, first position) keys
     // active nodes of a level (ping-pong)
     Seg* act[2];             // [maxBig]
     int* actAcc[2];          // [maxBig][12]
@@ -251,7 +251,7 @@ __device__ __forceinline__ int empty_bin(int i) {
 __global__ void k_build_init(Build b, int slots) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < b.numScenes * 12) b.rootAcc[i] = (i % 6) < 3 ? kOrdPosInf : kOrdNegInf;
-    if (i < 6) b.bnd[i] = ~0ull;
+    if (i < b.numScenes * 6) b.bnd[i] = ~0ull;
     if (i < 8) b.count[i] = 0;
     if (i == 0) b.topLevel[0] = 0;
     if (i < slots * kSlotInts) {
@@ -260,11 +260,11 @@ __global__ void k_build_init(Build b, int slots) {
 }
 
 // ------------------------------- top phase -----------------------------------
-// Primitive boxes and identity order, the scenes' root bounds and the bounds
-// of the whole mesh. The mesh bounds keep, as a sequential std::min / std::max
-// pass over the triangles would, the first of equal values (the sign of a
-// zero) and skip NaN: each axis reduces a 64-bit key of the ordered value and
-// the position of the coordinate.
+// Primitive boxes and identity order, the scenes' root bounds and their exact
+// bounds. The latter keep, as a sequential std::min / std::max pass over the
+// scene's triangles would, the first of equal values (the sign of a zero) and
+// skip NaN: each axis reduces a 64-bit key of the ordered value and the
+// position of the coordinate.
 __global__ __launch_bounds__(kTopThreads) void k_prims(Build b, const float* __restrict__ tris) {
     __shared__ int lds[kTopThreads / 64 * 12];
     __shared__ unsigned long long lk[kTopThreads / 64][6];
@@ -320,56 +320,22 @@ __global__ __launch_bounds__(kTopThreads) void k_prims(Build b, const float* __r
     if (threadIdx.x < 6) {
         unsigned long long v = lk[0][threadIdx.x];
         for (int w = 1; w < kTopThreads / 64; w++) v = min(v, lk[w][threadIdx.x]);
-        atomicMin(&b.bnd[threadIdx.x], v);
+        atomicMin(&b.bnd[6 * (size_t)j + threadIdx.x], v);
     }
 }
 
-// Bounds of n triangles alone (one tree of a forest): the keys of k_prims.
-__global__ __launch_bounds__(kTopThreads) void k_mesh_keys(const float* __restrict__ tris, int n,
-                                                           unsigned long long* bnd) {
-    unsigned long long key[6];
-#pragma unroll
-    for (int k = 0; k < 6; k++) key[k] = ~0ull;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-#pragma unroll
-        for (int e = 0; e < 9; e++) {
-            const float x = tris[9 * (size_t)i + e];
-            if (x == x) {
-                const int a = e % 3;
-                const unsigned int o = (unsigned int)f2o(x + 0.0f) ^ 0x80000000u;
-                const unsigned int pos = 3u * (unsigned int)i + (unsigned int)(e / 3);
-                const unsigned long long lo = (unsigned long long)o << 32 | pos;
-                const unsigned long long hi = (unsigned long long)~o << 32 | pos;
-                if (lo < key[a]) key[a] = lo;
-                if (hi < key[3 + a]) key[3 + a] = hi;
-            }
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < 6; k++) {
-        unsigned long long v = key[k];
-        for (int d = 32; d > 0; d >>= 1) {
-            const unsigned long long o = __shfl_xor(v, d, 64);
-            if (o < v) v = o;
-        }
-        if ((threadIdx.x & 63) == 0) atomicMin(&bnd[k], v);
-    }
-}
-__global__ void k_keys_init(unsigned long long* bnd) {
-    if (threadIdx.x < 6) bnd[threadIdx.x] = ~0ull;
-}
-// Keys -> the coordinates they name; an axis without a value below 1e30
-// (above -1e30) keeps that bound, as the sequential pass does.
-__global__ void k_mesh_bounds(const float* tris, const unsigned long long* bnd, float* out) {
-    const int k = threadIdx.x;
-    if (k >= 6) return;
+// Keys -> the coordinates they name (n of them, six per scene); an axis without
+// a value below 1e30 (above -1e30) keeps that bound, as the sequential pass does.
+__global__ void k_scene_bounds(const float* tris, const unsigned long long* bnd, int n, float* out) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, k = i % 6;
+    if (i >= n) return;
     float r = k < 3 ? 1e30f : -1e30f;
-    if (bnd[k] != ~0ull) {
-        const unsigned int pos = (unsigned int)bnd[k];
+    if (bnd[i] != ~0ull) {
+        const unsigned int pos = (unsigned int)bnd[i];
         const float x = tris[9 * (size_t)(pos / 3) + 3 * (pos % 3) + k % 3];
         if (k < 3 ? x < r : r < x) r = x;
     }
-    out[k] = r;
+    out[i] = r;
 }
 
 // Next level's active nodes: the children (2 m of them, or with `init` the
@@ -1510,22 +1476,6 @@ struct Slab {
         if (!(cond)) { set_error("%s", msg); return -1; } \
     } while (0)
 
-int mesh_bounds(const float* d_tris, int n, hipStream_t s, float* mn, float* mx) {
-    unsigned long long* key = nullptr;
-    if (!rt::dev_malloc(&key, 128)) { set_error("mesh bounds: out of device memory"); return -1; }
-    float* out = (float*)(key + 8);
-    float h[6];
-    hipLaunchKernelGGL(rtb::k_keys_init, dim3(1), dim3(64), 0, s, key);
-    hipLaunchKernelGGL(rtb::k_mesh_keys, dim3(std::min((n + 511) / 512, 1024)), dim3(rtb::kTopThreads), 0, s, d_tris, n, key);
-    hipLaunchKernelGGL(rtb::k_mesh_bounds, dim3(1), dim3(64), 0, s, d_tris, key, out);
-    hipError_t e = hipMemcpyAsync(h, out, sizeof h, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    hipFree(key);
-    if (e != hipSuccess) { set_error("mesh bounds: %s", hipGetErrorString(e)); return -1; }
-    for (int a = 0; a < 3; a++) { mn[a] = h[a]; mx[a] = h[3 + a]; }
-    return 0;
-}
-
 // Builds the BVH on the device from d_tris (n x 9 floats, original order).
 // Outputs (device, allocated here): nodes4 (numNodes4 x 64 B), leaf-order
 // triangles (n x 48 B), leafOf (n ints), ordered (n ints, leaf order ->
@@ -1573,7 +1523,7 @@ static int build_with_room(const float* d_tris, int n, int maxLeaf, hipStream_t 
     slab.add(&b.pbox, 2 * N);
     slab.add(&b.idx[0], N); slab.add(&b.idx[1], N);
     slab.add(&b.leafFlag, N); slab.add(&b.leafRank, N);
-    slab.add(&b.rootAcc, 12 * (size_t)R); slab.add(&b.rootRef, R); slab.add(&b.bnd, 6);
+    slab.add(&b.rootAcc, 12 * (size_t)R); slab.add(&b.rootRef, R); slab.add(&b.bnd, 6 * (size_t)R);
     for (int k = 0; k < 2; k++) {
         slab.add(&b.act[k], b.maxBig); slab.add(&b.actAcc[k], 12 * (size_t)b.maxBig);
         slab.add(&b.chunkBase[k], b.maxBig + 1); slab.add(&b.bins[k], 2 * (size_t)b.maxBig * kSlotInts);
@@ -1589,7 +1539,7 @@ static int build_with_room(const float* d_tris, int n, int maxLeaf, hipStream_t 
     slab.add(&head, 2 * N); slab.add(&assign, 2 * N); slab.add(&b4id, 2 * N);
     slab.add(&tiles, scan_tiles_needed((int)std::min<size_t>(2 * N, 0x7fffffff)) + 8);
     slab.add(&dRoot4, R);
-    slab.add(&dBounds, 8);
+    slab.add(&dBounds, 6 * (size_t)R);
     BUILD_CHECK(slab.alloc(), "gpu build: out of device memory");
     out.ordered = (int*)dev_alloc(N * 4);
     out.tris = dev_alloc(N * 48);
@@ -1609,7 +1559,7 @@ static int build_with_room(const float* d_tris, int n, int maxLeaf, hipStream_t 
     const int slots0 = std::max(big0, 1);
     hipLaunchKernelGGL(k_build_init, grid(std::max(R * 12, slots0 * kSlotInts)), dim3(T), 0, s, b, slots0);
     hipLaunchKernelGGL(k_prims, dim3(hBase[R]), dim3(kTopThreads), 0, s, b, d_tris);
-    hipLaunchKernelGGL(k_mesh_bounds, dim3(1), dim3(64), 0, s, d_tris, b.bnd, dBounds);
+    hipLaunchKernelGGL(k_scene_bounds, grid(6 * (long long)R), dim3(T), 0, s, d_tris, b.bnd, 6 * R, dBounds);
     hipLaunchKernelGGL(k_top_next, dim3(1), dim3(1024), 0, s, b, 0, 1, 0);
     // Levels until no node of more than kSmall primitives is left. The
     // largest scene needs at least log2(c / kSmall) levels, so the first
@@ -1672,15 +1622,20 @@ static int build_with_room(const float* d_tris, int n, int maxLeaf, hipStream_t 
     hipLaunchKernelGGL(k_sub_emit, dim3(numSmall), dim3(T), 0, s, b, em);
     scan_exclusive(head, b4id, nodeCount, b.count + 5, tiles, s);
     hipLaunchKernelGGL(k_leaf_tris, grid(n), dim3(T), 0, s, d_tris, b.ordered, n, (float4*)out.tris, out.leafOf, b.off, R);
-    float hb[6];
+    out.sceneBounds.resize(6 * (size_t)R);
     int fin[3] = {0, 0, 0};                       // heads, BVH4 and BVH2 levels
     if (hipMemcpyAsync(fin, b.count + 5, sizeof fin, hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipMemcpyAsync(hb, dBounds, sizeof hb, hipMemcpyDeviceToHost, s) != hipSuccess ||
+        hipMemcpyAsync(out.sceneBounds.data(), dBounds, 24 * (size_t)R, hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess) {
         set_error("gpu build: numbering failed");
         return -1;
     }
-    for (int a = 0; a < 3; a++) { out.bmin[a] = hb[a]; out.bmax[a] = hb[3 + a]; }
+    for (int a = 0; a < 3; a++) { out.bmin[a] = 1e30f; out.bmax[a] = -1e30f; }
+    for (int k = 0; k < R; k++)
+        for (int a = 0; a < 3; a++) {
+            out.bmin[a] = std::min(out.bmin[a], out.sceneBounds[6 * (size_t)k + a]);
+            out.bmax[a] = std::max(out.bmax[a], out.sceneBounds[6 * (size_t)k + 3 + a]);
+        }
     const int heads = fin[0];
     out.numNodes4 = std::max(heads, 1);
     out.depth4 = std::max(fin[1], 1);             // a leaf root is one node

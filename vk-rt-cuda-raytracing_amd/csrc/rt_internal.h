@@ -49,7 +49,11 @@ struct GpuBVH {
     int* leafOf = nullptr;                         // original index -> leaf position
     int* ordered = nullptr;                        // leaf position -> original index
     int levels = 0;                                // BVH2 levels
-    float bmin[3], bmax[3];                        // mesh bounds (mesh_bounds' values)
+    // Bounds as a sequential std::min / std::max pass over the triangles computes
+    // them (from 1e30 / -1e30; the first of equal values, NaN skipped): of the
+    // whole mesh and of each scene (min xyz, max xyz)
+    float bmin[3], bmax[3];
+    std::vector<float> sceneBounds;
 };
 // Builds one BVH, or with sceneOff (numScenes+1 host offsets into d_tris) a
 // forest of numScenes independent BVHs in one pass: node
@@ -57,10 +61,6 @@ struct GpuBVH {
 // their index within their scene; roots4 receives each tree's BVH4 root.
 int gpu_build(const float* d_tris, int n, int maxLeaf, hipStream_t s, GpuBVH& out, const int* sceneOff = nullptr,
               int numScenes = 1, std::vector<int>* roots4 = nullptr);
-// Bounds of n x 9 device floats as a sequential std::min / std::max pass over
-// the triangles computes them (from 1e30 / -1e30; the first of equal values,
-// NaN skipped). Waits for stream s. 0 on success.
-int mesh_bounds(const float* d_tris, int n, hipStream_t s, float* mn, float* mx);
 // Device memory with a bounded cache of freed blocks (devmem.hip). nullptr when
 // out of memory. dev_free: no device work uses the block any longer;
 // dev_release: some may, and its device is waited for before the block is used

@@ -397,7 +397,9 @@ int cudaBVH_sceneTraceAnyQueued(CudaScene_t scene, int capacity, const int* d_co
 /* Resources of the last traversal launch on the handle / scene (8 ints):
  * VGPRs per lane, static LDS bytes per workgroup, scratch bytes per lane,
  * workgroups per CU launched, workgroups per CU that fit, total workgroups,
- * threads per workgroup, waves per SIMD. Zeros before the first launch.
+ * threads per workgroup, waves per SIMD. Zeros before the first launch. A
+ * launch with four lanes per ray has as many workgroups as its rays take: per
+ * CU, those of them that are resident at once are reported.
  * No backend counterpart (the reference fixes __launch_bounds__(256, 5),
  * layer/cuda_bvh_backend.cu:104); it reports the occupancy that the launch
  * configuration and the autotuner's choice give. */

@@ -77,3 +77,17 @@ def test_autotune_on_a_large_workload(pkg, bvh, threads, dev):
     bvh.set_trace_config(cls, 0, 16, 0)
     bvh.autotune(cls, reps=1, rays=big)
     assert threads() == 256
+
+
+@pytest.mark.parametrize("n", [1, 3000, 100000])
+def test_launch_info_of_small_launches(pkg, bvh, dev, n):
+    """Workgroups and waves as many as the rays take, up to what fits."""
+    import torch
+    R, H = _rays(n, dev), hit_buffers(n, dev)
+    bvh.trace_closest(R, H["t"], H["prim_id"], H["u"], H["v"])
+    torch.cuda.synchronize()
+    info = bvh.launch_info()
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert info["threads_per_workgroup"] == 64 and info["workgroups"] == (n + 15) // 16
+    assert info["blocks_per_cu"] == min(info["max_blocks_per_cu"], -(-info["workgroups"] // cus))
+    assert info["waves_per_simd"] == -(-info["blocks_per_cu"] // 4)

@@ -1536,7 +1536,7 @@ static int launch_quads(const CudaBVHHandle* h, rt::TraceScratch& sc, TraceArgs&
         if (grid < 1) { rt::set_error("fixed traversal scratch too small for a tree of depth %d", h->depth4); return -1; }
     }
     rt::note_launch(kern, 64, ki, 0, 0, nullptr);
-    rt::note_launch(kern, 64, ki, ki.maxBlocks, grid, sc.launchInfo);
+    rt::note_launch(kern, 64, ki, std::min(ki.maxBlocks, (grid + num_cus() - 1) / num_cus()), grid, sc.launchInfo);
     a.spill = (int2*)sc.spill;
     a.spillStride = grid * 16;
     a.status = sc.status;

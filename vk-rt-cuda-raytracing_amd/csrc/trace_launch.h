@@ -26,7 +26,7 @@ inline void note_launch(K kern, int block, KernelInfo& ki, int blocksPerCU, int 
     if (!info) return;
     info[0] = ki.vgprs; info[1] = ki.ldsBytes; info[2] = ki.scratchBytes;
     info[3] = blocksPerCU; info[4] = ki.maxBlocks; info[5] = grid; info[6] = block;
-    info[7] = blocksPerCU * (block / 64) / 4;
+    info[7] = (blocksPerCU * (block / 64) + 3) / 4;
 }
 
 }  // namespace rt

@@ -668,8 +668,9 @@ def load_traffic(config):
 
 def build_report(bvh, tris, build_s):
     """The GPU build of the frame's BVH against its roofline: algorithmic bytes
-    per triangle 36 (read) + 36 (reordered write) + 36 per binning pass (one
-    per BVH2 level), plus 64 per BVH4 node, over the device build time."""
+    per triangle 36 (read) + 36 (reordered write) + 36 per BVH2 level (what
+    binning level by level reads; the subtrees' lower levels stay in LDS),
+    plus 64 per BVH4 node, over the device build time."""
     st = bvh.build_stats()
     n = int(tris.shape[0])
     alg = n * (36 + 36 + 36 * st["levels"]) + 64 * bvh.num_bvh4_nodes
@@ -681,7 +682,7 @@ def build_report(bvh, tris, build_s):
             "device_ms": round(st["device_ms"], 2), "handle_ms": round(st["handle_ms"], 2),
             "levels": st["levels"], "bvh4_nodes": bvh.num_bvh4_nodes, "alg_bytes": int(alg),
             "achieved_GBps": round(gbs, 1), "peak_GBps": HBM_PEAK_GBS, "frac": round(gbs / HBM_PEAK_GBS, 4),
-            "bound": "launch/latency (one pass per BVH2 level)"}
+            "bound": "dependent LDS steps of the subtrees; two box gathers and four launches per top level"}
 
 
 def cpu_build_baseline(bvh, tris):

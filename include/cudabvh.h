@@ -460,8 +460,8 @@ typedef struct {
     float skyZenith[3];   /* escaped-ray radiance: horizon + (zenith - horizon) * max(d.y, 0) */
     float skyHorizon[3];
     float clampMax;       /* per-contribution max-channel clamp; <= 0 disables */
-    int tailPaths;        /* from the first bounce with at most this many live paths on, one
-                             thread per path runs all remaining bounces (0: wavefront only;
+    int tailPaths;        /* from the first bounce with at most this many live paths on, eight
+                             lanes per path run all remaining bounces (0: wavefront only;
                              < 0: the scene's tuned value, 32768 until
                              cudaBVH_sceneAutotunePathTracer); the image does not depend on it */
 } CudaPathParams;

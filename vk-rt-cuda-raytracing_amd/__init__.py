@@ -704,8 +704,8 @@ Scene.path_trace = _scene_path_trace
 
 def _scene_autotune_path_tracer(self, cam: CudaCamera, params: CudaPathParams, rgb, albedo, normal, depth,
                                 reps: int = 4):
-    """Tunes the tail threshold (the queue size below which one thread per
-    path finishes the bounces) on this frame; returns (chosen, [(threshold,
+    """Tunes the tail threshold (the queue size below which eight lanes per
+    path finish the bounces) on this frame; returns (chosen, [(threshold,
     ms per sample)]). Later renders use it with tail_paths=-1."""
     img = CudaPathImage(_ptr(rgb), _ptr(albedo), _ptr(normal), _ptr(depth))
     res = np.zeros(12, np.float32)

@@ -953,9 +953,11 @@ __global__ __launch_bounds__(64) void k_trace_quad(TraceArgs a) {
 // of steps of its slowest tiles, mostly run by waves with few rays left. That
 // takes 79 VGPRs, six waves per SIMD instead of seven (at seven it spilled up
 // to 7 to scratch): on a 3.4 M triangle terrain the cost-ordered pinhole launch
-// of 1024 x 1024 went from 279 to 236 us and of 1920 x 1080, which the order
-// keeps busy to its end, from 366 to 362 us (a 65,536 triangle soup: 394 to
-// 342, 468 to 391 us).
+// of 1024 x 1024 went from 308 to 256 us and of 1920 x 1080, which the order
+// keeps busy to its end, stayed at 372 (a 65,536 triangle soup: 408 to 339, 468
+// to 406 us). The counted and Moller-Trumbore forms, which have no hand-over,
+// take as long as at seven waves (1 M rays 759 / 760 us Moller-Trumbore, 787 /
+// 785 counted).
 template <int MODE, bool MT, bool PIN, bool COUNT, int LDSD, int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void k_trace_batch(TraceArgs a) {
     __shared__ int s_ref[LDSD * BLOCK];

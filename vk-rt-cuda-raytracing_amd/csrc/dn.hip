@@ -799,6 +799,19 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
         struct { s16x4 a, b; } f{h[0], h[1]};
         return __builtin_bit_cast(bf16x8, f);
     };
+    // A gradient of zero times an infinite or NaN input would be NaN where the
+    // pixel lies outside the image. That can happen only just past its right
+    // and bottom edge, for the taps that look back into it: those inputs are
+    // cleared (element e of a fragment) and those rows left out.
+    auto without = [](bf16x8 v, int e) {
+        uint4 w = __builtin_bit_cast(uint4, v);
+        const uint32_t keep = (e & 1) ? 0xffffu : 0xffff0000u;
+        if (e >> 1 == 0) w.x &= keep;
+        if (e >> 1 == 1) w.y &= keep;
+        if (e >> 1 == 2) w.z &= keep;
+        if (e >> 1 == 3) w.w &= keep;
+        return __builtin_bit_cast(bf16x8, w);
+    };
     f32x4 acc[TAPS][MT][NT], accb[MT];
 #pragma unroll
     for (int t = 0; t < TAPS; t++)
@@ -850,10 +863,15 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
                 bf16x8 xb[NT];
 #pragma unroll
                 for (int j = 0; j < NT; j++) xb[j] = frag(sx + (wk * RW + xr) * (XW * XC / 8), dx, wi * NT + j, XC / 8);
+                if (HALO && dx == 0 && x0 + kWgPx > a.W) {
+#pragma unroll
+                    for (int j = 0; j < NT; j++) xb[j] = without(xb[j], a.W - x0 - 8 * kg);
+                }
 #pragma unroll
                 for (int dy = 0; dy < NR; dy++) {
                     const int ro = xr - dy;        // output row whose tap dy reads this input row
                     if (ro < 0 || ro >= RW) continue;
+                    if (HALO && dy == 0 && y0 + wk * RW + ro == a.H) continue;
 #pragma unroll
                     for (int r = 0; r < MT; r++)
 #pragma unroll
